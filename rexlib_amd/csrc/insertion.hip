@@ -89,23 +89,19 @@ __global__ void settle_kernel(insertion_params p)
 			}
 			// A non-finite frame bounds no rows (src/backends/cpu/kernels/row_interval.cpp).
 			e.last_shell = finite ? last : -1;
-			e.ctf_radial = e.ctf_axial = e.ctf_diagonal = e.ctf_aberration = e.ctf_phase = 0.0f;
-			// Two samples of one parity class differ by 2 a X + 2 b Y; when the
-			// smallest eigenvalue of the Gram matrix of (X, Y) exceeds 3/4, that
-			// is at least one voxel along some axis, so no two of them fall in
-			// the same voxel cell.
+			e.ctf_radial = e.ctf_axial = e.ctf_diagonal = e.ctf_phase = 0.0f;
 			{
-				double xx = 0.0, xy = 0.0, yy = 0.0;
-				for (int a = 0; a < 3; ++a)
-				{
-					xx += static_cast<double>(e.x_step[a]) * e.x_step[a];
-					xy += static_cast<double>(e.x_step[a]) * e.y_step[a];
-					yy += e.y_step[a] * e.y_step[a];
-				}
-				const double trace = xx + yy;
-				const double gap = sqrt(fmax(0.0, (xx - yy) * (xx - yy) + 4.0 * xy * xy));
-				const double smallest = 0.5 * (trace - gap);
-				e.lattice_free = finite && smallest > 0.76 ? 1 : 0;
+				const float x0 = e.x_step[0], x1 = e.x_step[1], x2 = e.x_step[2];
+				const float y0 = static_cast<float>(e.y_step[0]);
+				const float y1 = static_cast<float>(e.y_step[1]);
+				const float y2 = static_cast<float>(e.y_step[2]);
+				slice_plane plane;
+				plane.normal[0] = x1 * y2 - x2 * y1;
+				plane.normal[1] = x2 * y0 - x0 * y2;
+				plane.normal[2] = x0 * y1 - x1 * y0;
+				plane.reach = e.last_shell < 0 ? -1.0e30f : (static_cast<float>(e.last_shell) + 0.5f) * 1.001f *
+					sqrtf(x0 * x0 + x1 * x1 + x2 * x2 + y0 * y0 + y1 * y1 + y2 * y2) + 1e-3f;
+				p.planes[s] = plane;
 			}
 			e.extra_offset = p.extra != nullptr ? offset(slot_extra) : 0;
 			if (p.variant == variant_ctf)
@@ -122,14 +118,12 @@ __global__ void settle_kernel(insertion_params p)
 				e.ctf_axial = static_cast<float>(p.ctf_defocus_scale * half_difference * cos(2.0 * angle));
 				e.ctf_diagonal = static_cast<float>(
 					2.0 * p.ctf_defocus_scale * half_difference * sin(2.0 * angle));
-				e.ctf_aberration = static_cast<float>(p.ctf_aberration);
 				e.ctf_phase = static_cast<float>(phase + p.ctf_phase0);
 			}
 			e.slice_offset = offset(slot_slices);
 			e.radial_offset = radial_offset;
 			e.numerator_offset = kept_offset(p.map, slot_numerator_out, kept);
 			e.denominator_offset = kept_offset(p.map, slot_denominator_out, kept);
-			e.kept = kept;
 			p.entries[s] = e;
 		}
 
@@ -211,25 +205,44 @@ __global__ void volume_phase_kernel(float2 *table, int big)
 	table[j] = make_float2(static_cast<float>(cs), static_cast<float>(sn));
 }
 
-// Out-of-place insertions start from a copy of the accumulators.
-__global__ void copy_accumulators_kernel(insertion_params p, const float2 *num_in, int64_t ni0, int64_t ni1,
-	int64_t ni2, const float *den_in, int64_t di0, int64_t di1, int64_t di2)
+// Out-of-place insertions start from a copy of the accumulators: a wavefront
+// copies a row (kept, z, y), so that the batch offsets and the divisions are
+// made once per row. SHARED copies only the rows that hold the frequencies
+// +-N/2 of an even N along y or z (2 N - 1 of a volume's N^2): what bricks
+// that own voxels need. A row per wavefront moves 1.6 GB at 512^3 in 0.29 ms
+// where a division chain per voxel took 0.36 ms.
+template <bool SHARED>
+__global__ __launch_bounds__(256) void copy_accumulators_kernel(insertion_params p, const float2 *num_in, int64_t ni0,
+	int64_t ni1, int64_t ni2, const float *den_in, int64_t di0, int64_t di1, int64_t di2)
 {
-	const int64_t volume = static_cast<int64_t>(p.big) * p.big * p.half;
-	const int64_t total = volume * p.map.kept_count;
-	for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < total;
-		i += static_cast<int64_t>(gridDim.x) * blockDim.x)
+	const int lane = threadIdx.x & 63;
+	const int big = p.big;
+	const int64_t rows = SHARED ? 2 * static_cast<int64_t>(big) - 1 : static_cast<int64_t>(big) * big;
+	const int64_t total = rows * p.map.kept_count;
+	for (int64_t i = blockIdx.x * 4ll + (threadIdx.x >> 6); i < total; i += gridDim.x * 4ll)
 	{
-		const int64_t kept = i / volume;
-		int64_t v = i % volume;
-		const int64_t x = v % p.half;
-		v /= p.half;
-		const int64_t y = v % p.big;
-		const int64_t z = v / p.big;
-		const float2 a = num_in[kept_offset(p.map, slot_numerator, kept) + z * ni0 + y * ni1 + x * ni2];
-		const float b = den_in[kept_offset(p.map, slot_denominator, kept) + z * di0 + y * di1 + x * di2];
-		p.numerator[kept_offset(p.map, slot_numerator_out, kept) + z * p.num_s0 + y * p.num_s1 + x * p.num_s2] = a;
-		p.denominator[kept_offset(p.map, slot_denominator_out, kept) + z * p.den_s0 + y * p.den_s1 + x * p.den_s2] = b;
+		const int64_t kept = i / rows;
+		const int64_t r = i - kept * rows;
+		int64_t z, y;
+		if (SHARED)
+		{
+			z = r < big ? big / 2 : (r - big < big / 2 ? r - big : r - big + 1);
+			y = r < big ? r : big / 2;
+		}
+		else
+		{
+			z = r / big;
+			y = r - z * big;
+		}
+		const float2 *num = num_in + kept_offset(p.map, slot_numerator, kept) + z * ni0 + y * ni1;
+		const float *den = den_in + kept_offset(p.map, slot_denominator, kept) + z * di0 + y * di1;
+		float2 *num_out = p.numerator + kept_offset(p.map, slot_numerator_out, kept) + z * p.num_s0 + y * p.num_s1;
+		float *den_out = p.denominator + kept_offset(p.map, slot_denominator_out, kept) + z * p.den_s0 + y * p.den_s1;
+		for (int x = lane; x < p.half; x += 64)
+		{
+			num_out[x * p.num_s2] = num[x * ni2];
+			den_out[x * p.den_s2] = den[x * di2];
+		}
 	}
 }
 
@@ -243,7 +256,6 @@ __global__ __launch_bounds__(256) void scatter_kernel(insertion_params p)
 	// A slice holds n (n/2 + 1) < 2^31 elements: 32-bit indices (a 64-bit
 	// division per element would cost more than the sample itself).
 	const int elements32 = p.n * p.h;
-	const int64_t elements = elements32;
 	const int idx = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
 	if (idx >= elements32)
 	{
@@ -371,14 +383,18 @@ void dispatch_scatter(const insertion_params &p, hipStream_t stream)
 // brick; the brick's LDS holds its cells and the taps - 1 voxels above them.
 //
 // The wavefront tests 64 slices at a time for planes that pass near the
-// brick; for each such slice it bounds the rows that can hold its samples and
-// clips each row to them -- bound_rows and clip_row of
-// src/backends/cpu/kernels/row_interval.cpp, restated per brick as the
-// reference restates them per tile (slice_insertion_functor.inl:391-440).
-// The rows of all hit slices are then packed densely over the lanes (64
-// rows at a time, each with its base position, step and first sample in a
-// small LDS table), and their samples over the lanes (64 at a time), so a
-// lane carries a sample whatever slice it comes from.
+// brick and queues the few that do; for 64 queued slices at once it bounds
+// the rows that can hold their samples (bound_section, bound_rows) and clips
+// each row to them (clip_row of src/backends/cpu/kernels/row_interval.cpp,
+// restated per brick as the reference restates it per tile,
+// slice_insertion_functor.inl:391-440). The rows of the queued slices are
+// packed densely over the lanes (64 rows at a time, each with its base
+// position, step and first sample in its lane's registers), and their samples
+// over the lanes (64 at a time), so a lane carries a sample whatever slice it
+// comes from. The kernel is bound by its vector instructions (88 % of the
+// SIMD cycles at 4,096 slices of 256^2 into 256^3): bounding the 2.2 hits of
+// each 64 slices on their own spent half of them, and the queue took the
+// launch from 1.9 to 1.2 ms.
 //
 // The samples are added by plain LDS read-modify-write, not LDS float
 // atomics (which retire at about a third of a lane per clock per CU on
@@ -386,7 +402,8 @@ void dispatch_scatter(const insertion_params &p, hipStream_t stream)
 // holding a sample claims its first-tap cell (a byte per cell: it writes its
 // lane, then reads it back); the lanes that read their own lane add their
 // taps one after another, the others keep their sample for the next round,
-// whose new samples go to the free lanes only. No two lanes of one tap
+// whose new samples go to the free lanes only. (With 4 taps the 64 lanes are
+// the taps of one sample instead: wide_round.) No two lanes of one tap
 // instruction then touch one voxel (a tap is a constant offset from the
 // cell). LDS runs a wavefront's accesses in program order and lds_order
 // keeps the compiler from moving them; the wavefront is the brick's only
@@ -404,7 +421,8 @@ void dispatch_scatter(const insertion_params &p, hipStream_t stream)
 // by plain read-add-write; the others (the taps - 1 layers at each face that
 // the neighbouring bricks also reach, every voxel of a split brick, and bricks
 // holding the y or z frequency +-N/2 of an even N, two signed frequencies of
-// one stored element) add with atomics.
+// one stored element) add with atomics. Sparse calls take bricks that own
+// voxels instead and write each once (bricks_own_voxels).
 // ---------------------------------------------------------------------------
 
 
@@ -416,28 +434,34 @@ struct brick_reach
 	static constexpr int taps = PROFILE == REXLIB_HIP_BOX ? 1 : (PROFILE == REXLIB_HIP_TRIANGLE ? 2 : 4);
 };
 
+// LDS pitches of a brick of lx x ly voxels per plane. Up to 2 taps: odd, so
+// that lanes stepping along any axis fall in different banks. With 4 taps the
+// 64 lanes of an access are the 4 x 4 x 4 taps of one sample: a y pitch of 4
+// modulo 8 and a z pitch of 16 modulo 32 put every 32 of them in 32 different
+// residues, without a bank conflict.
+constexpr int brick_pitch_y(int taps, int lx)
+{
+	return taps == 4 ? (lx + 3) / 8 * 8 + 4 : (lx % 2 == 0 ? lx + 1 : lx);
+}
+
+constexpr int brick_pitch_z(int taps, int pitch_y, int ly)
+{
+	return taps == 4 ? (pitch_y * ly + 15) / 32 * 32 + 16 : (pitch_y * ly) % 2 == 0 ? pitch_y * ly + 1 : pitch_y * ly;
+}
+
 // LDS layout of a brick of first-tap cells EX x EY x EZ with the taps - 1
-// voxels above them: odd pitches, so that lanes stepping along any axis fall
-// in different banks.
+// voxels above them.
 template <int T, int EX, int EY, int EZ>
 struct brick_layout
 {
 	static constexpr int lx = EX + T - 1;
 	static constexpr int ly = EY + T - 1;
 	static constexpr int lz = EZ + T - 1;
-	static constexpr int pitch_y = lx % 2 == 0 ? lx + 1 : lx;
-	static constexpr int pitch_z = (pitch_y * ly) % 2 == 0 ? pitch_y * ly + 1 : pitch_y * ly;
+	static constexpr int pitch_y = brick_pitch_y(T, lx);
+	static constexpr int pitch_z = brick_pitch_z(T, pitch_y, ly);
+	static_assert(pitch_y >= lx && pitch_z >= pitch_y * ly, "the pitches hold a row and a plane");
 	static constexpr int voxels = pitch_z * lz;
 	static constexpr int cells = EX * EY * EZ;
-};
-
-// A voxel of a brick in LDS: 12 bytes. (16-byte voxels, one 128-bit access
-// per tap, measured slower: the larger brick costs wavefronts per CU.)
-struct brick_voxel
-{
-	float re;
-	float im;
-	float den;
 };
 
 struct brick_box
@@ -445,6 +469,19 @@ struct brick_box
 	int lo[3];  // signed (x, y, z) of the first cell
 	int ext[3]; // cells along (x, y, z)
 	bool alias_free;
+};
+
+// The accumulators the sums are added to, read by bricks that own voxels:
+// the caller's inputs (first chunk of an out-of-place call), else the outputs.
+struct accumulator_input
+{
+	const float2 *numerator;
+	int64_t num_s0, num_s1, num_s2;
+	const float *denominator;
+	int64_t den_s0, den_s1, den_s2;
+	int num_slot; // whose batch offsets the pointers take
+	int den_slot;
+	bool in_place;
 };
 
 __device__ inline brick_box unpack_brick(int4 b)
@@ -656,22 +693,54 @@ __global__ __launch_bounds__(256) void columns_prepare_kernel(insertion_params p
 	}
 }
 
-// bound_rows of one slice and sign: the rows [r0, r1) whose samples k_x in
-// [first, widest] can reach the box [lower, upper]; r0 >= r1 when none.
-// Evaluated per lane, one slice per lane.
-// `inv_y` and `inv_x` hold 1 / y_step_f and 1 / x_step per axis (0 where the
-// step is 0); a product with them stands for the division, the box being
-// widened far beyond its rounding.
-//
-// The reference bounds each axis separately over the whole k_x range
-// (row_interval.cpp:34-136), which keeps rows whose line meets the box only
-// at k_x the slice does not hold. Here the bound is refined once: the k_x
-// (integers) that can reach the box from those rows, then the rows again
-// for that k_x range. Each step keeps every row holding a sample in the
-// box, and about half the rows go.
-__device__ inline void bound_rows(const insertion_params &p, const float *x_step, const float *y_step_f,
-	const float *inv_y, const float *inv_x, int last_shell, const float *lower, const float *upper, int sign_index,
-	int &r0, int &r1)
+// The section of a slice's plane with the box [lower, upper], as real ranges
+// of k_x and k_y (of the +k copy; the -k copy's are the negated ones). With
+// p = k_x X + k_y Y, eliminating k_x or k_y between the axes a and b gives
+//   k_y n = X_a p_b - X_b p_a,  k_x n = Y_b p_a - Y_a p_b,  n = X_a Y_b - X_b Y_a,
+// and the three pairs of axes bound each frequency exactly: the section is
+// the intersection of three strips, whose projections are the intersections
+// of the strips' pairwise ones. The per-axis bound of the reference
+// (row_interval.cpp:34-136) takes each axis over the whole k_x range; it kept
+// 28 rows per (slice, brick) at 256^3 where 7.4 hold samples, these keep 9.
+// The box is widened by 0.01 voxel, the roundings here stay within
+// 1e-4 (|X_a| + |X_b|) of the products, which the widening covers.
+__device__ inline void bound_section(const float *x_step, const float *y_step, const float *normal, const float *lower,
+	const float *upper, float *kx, float *ky)
+{
+	kx[0] = ky[0] = -3.0e38f;
+	kx[1] = ky[1] = 3.0e38f;
+#pragma unroll
+	for (int c = 0; c < 3; ++c)
+	{
+		const int a = (c + 1) % 3;
+		const int b = (c + 2) % 3;
+		if (fabsf(normal[c]) > 1e-30f)
+		{
+			const float inv = __builtin_amdgcn_rcpf(normal[c]);
+			const auto narrow = [&](float p, float q, int i, int j, float *range)
+			{
+				// p [lower_i, upper_i] - q [lower_j, upper_j], over the normal.
+				const float p0 = p * lower[i], p1 = p * upper[i];
+				const float q0 = q * lower[j], q1 = q * upper[j];
+				const float l = (fminf(p0, p1) - fmaxf(q0, q1)) * inv;
+				const float u = (fmaxf(p0, p1) - fminf(q0, q1)) * inv;
+				range[0] = fmaxf(range[0], fminf(l, u));
+				range[1] = fminf(range[1], fmaxf(l, u));
+			};
+			narrow(x_step[a], x_step[b], b, a, ky);
+			narrow(y_step[b], y_step[a], a, b, kx);
+		}
+	}
+}
+
+// The rows [r0, r1) of one sign of a slice whose samples k_x in [first,
+// widest] can reach the box [lower, upper], given the section's ranges of
+// k_x and k_y (all already of that sign: the -k copy passes the negated box
+// and ranges); r0 >= r1 when none. `inv_y` holds 1 / y_step (0 where the step
+// is 0). Evaluated per lane, one slice per lane.
+__device__ inline void bound_rows(const insertion_params &p, const float *x_step, const float *y_step,
+	const float *inv_y, int last_shell, const float *lower, const float *upper, float kx_low, float kx_high,
+	float ky_low, float ky_high, int first, int &r0, int &r1)
 {
 	r0 = 0;
 	r1 = 0;
@@ -681,34 +750,27 @@ __device__ inline void bound_rows(const insertion_params &p, const float *x_step
 	const int last_column = h - (even ? 2 : 1);
 	const int highest_row = even ? n / 2 - 1 : n / 2;
 	const int widest = min(last_column, last_shell);
-	const int first_row = max(-highest_row, -widest);
 	const int last_row = min(highest_row, widest);
-	const float sign = sign_index == 0 ? 1.0f : -1.0f;
-	const int first = sign_index;
-	if (last_shell < 0 || first > widest || first_row > last_row)
-	{
-		return;
-	}
-	float low = static_cast<float>(first_row);
-	float high = static_cast<float>(last_row);
-	bool none = false;
+	const float k_low = ceilf(fmaxf(kx_low, static_cast<float>(first)));
+	const float k_high = floorf(fminf(kx_high, static_cast<float>(widest)));
+	float low = fmaxf(ky_low, -static_cast<float>(last_row));
+	float high = fminf(ky_high, static_cast<float>(last_row));
+	bool none = last_shell < 0 || k_low > k_high;
+#pragma unroll
 	for (int a = 0; a < 3; ++a)
 	{
-		const float step = sign * x_step[a];
-		const float y_step = sign * y_step_f[a];
-		const float at_first = static_cast<float>(first) * step;
-		const float at_last = static_cast<float>(widest) * step;
+		const float at_first = k_low * x_step[a];
+		const float at_last = k_high * x_step[a];
 		const float lo = lower[a] - fmaxf(at_first, at_last);
 		const float hi = upper[a] - fminf(at_first, at_last);
-		if (y_step == 0.0f)
+		if (y_step[a] == 0.0f)
 		{
 			none = none || !(lo <= 0.0f && 0.0f <= hi);
 		}
 		else
 		{
-			const float inv = sign * inv_y[a];
-			const float l = lo * inv;
-			const float u = hi * inv;
+			const float l = lo * inv_y[a];
+			const float u = hi * inv_y[a];
 			low = fmaxf(low, fminf(l, u));
 			high = fminf(high, fmaxf(l, u));
 		}
@@ -717,52 +779,10 @@ __device__ inline void bound_rows(const insertion_params &p, const float *x_step
 	{
 		return;
 	}
-	float k_low = static_cast<float>(first);
-	float k_high = static_cast<float>(widest);
-	for (int a = 0; a < 3; ++a)
-	{
-		const float step = sign * x_step[a];
-		if (step != 0.0f)
-		{
-			const float y_step = sign * y_step_f[a];
-			const float b0 = low * y_step;
-			const float b1 = high * y_step;
-			const float inv = sign * inv_x[a];
-			const float l = (lower[a] - fmaxf(b0, b1)) * inv;
-			const float u = (upper[a] - fminf(b0, b1)) * inv;
-			k_low = fmaxf(k_low, fminf(l, u));
-			k_high = fminf(k_high, fmaxf(l, u));
-		}
-	}
-	k_low = ceilf(k_low);
-	k_high = floorf(k_high);
-	if (k_low > k_high)
-	{
-		return;
-	}
-	for (int a = 0; a < 3; ++a)
-	{
-		const float step = sign * x_step[a];
-		const float y_step = sign * y_step_f[a];
-		if (y_step != 0.0f)
-		{
-			const float at_first = k_low * step;
-			const float at_last = k_high * step;
-			const float inv = sign * inv_y[a];
-			const float l = (lower[a] - fmaxf(at_first, at_last)) * inv;
-			const float u = (upper[a] - fminf(at_first, at_last)) * inv;
-			low = fmaxf(low, fminf(l, u));
-			high = fminf(high, fmaxf(l, u));
-		}
-	}
-	if (low > high)
-	{
-		return;
-	}
 	// The box is already widened past the window, so rounding inwards keeps
 	// every sample that can reach it.
-	r0 = max(static_cast<int>(ceilf(low)), first_row);
-	r1 = min(static_cast<int>(floorf(high)) + 1, last_row + 1);
+	r0 = static_cast<int>(ceilf(low));
+	r1 = static_cast<int>(floorf(high)) + 1;
 }
 
 // Position of sample k_x along one axis from its row's base and step (the
@@ -819,20 +839,62 @@ __device__ inline void clip_row(int ky, int first, int widest, float radius, con
 	}
 }
 
+// The inputs of the bricks that own voxels but are split into shares (the
+// first `gridDim.x` tasks hold them all): their shares add with atomics.
+template <int T>
+__global__ __launch_bounds__(64) void copy_split_bricks_kernel(insertion_params p, const int4 *tasks,
+	accumulator_input input)
+{
+	const brick_box box = unpack_brick(tasks[2 * blockIdx.x]);
+	const int4 share = tasks[2 * blockIdx.x + 1];
+	if (share.x != 0 || share.y == 1)
+	{
+		return;
+	}
+	const int64_t kept = blockIdx.y;
+	const int he = p.big / 2;
+	const int ex = box.ext[0] - (T - 1), ey = box.ext[1] - (T - 1), ez = box.ext[2] - (T - 1);
+	for (int v = threadIdx.x; v < ex * ey * ez; v += 64)
+	{
+		const int x = box.lo[0] + T - 1 + v % ex;
+		const int y = box.lo[1] + T - 1 + (v / ex) % ey;
+		const int z = box.lo[2] + T - 1 + v / (ex * ey);
+		if (x <= he && y <= he && z <= he)
+		{
+			const int64_t sy = y < 0 ? y + p.big : y;
+			const int64_t sz = z < 0 ? z + p.big : z;
+			p.numerator[kept_offset(p.map, slot_numerator_out, kept) + sz * p.num_s0 + sy * p.num_s1 + x * p.num_s2] =
+				input.numerator[kept_offset(p.map, input.num_slot, kept) + sz * input.num_s0 + sy * input.num_s1 +
+					x * input.num_s2];
+			p.denominator[kept_offset(p.map, slot_denominator_out, kept) + sz * p.den_s0 + sy * p.den_s1 + x * p.den_s2] =
+				input.denominator[kept_offset(p.map, input.den_slot, kept) + sz * input.den_s0 + sy * input.den_s1 +
+					x * input.den_s2];
+		}
+	}
+}
+
 // A wavefront owns the brick of one task (a brick and a share of the
 // slices): EX x EY x EZ first-tap cells and the voxels their taps reach, in
 // LDS.
-template <int PROFILE, bool ODD, int EX, int EY, int EZ>
+template <int PROFILE, bool ODD, bool VOXELS, int EX, int EY, int EZ>
 __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chunk chunk, const prepared_sample *prepared,
-	const int4 *tasks, int task_count)
+	const int4 *tasks, int task_count, accumulator_input input)
 {
 	constexpr int T = brick_reach<PROFILE>::taps;
 	using L = brick_layout<T, EX, EY, EZ>;
-	__shared__ brick_voxel acc[L::voxels];
-	// Per first-tap cell: the lane that last claimed it.
-	__shared__ unsigned char claim[L::cells];
+	// The voxels as two arrays, value and weight. A tap is then a 64-bit and a
+	// 32-bit access at even and odd bank pitches; one array of 12-byte voxels
+	// took 217 cycles per CU for the 8 taps of 48 lanes, the two arrays 184.
+	__shared__ float2 acc_value[L::voxels];
+	__shared__ float acc_weight[L::voxels];
+	// Up to 2 taps, per first-tap cell: the lane that last claimed it.
+	__shared__ unsigned char claim[T == 4 ? 1 : L::cells];
+	// 4 taps: the axis weights of the samples in the lanes, x, y, z.
+	__shared__ float4 axis_weights[T == 4 ? 64 * 3 : 1];
 	// Per lane: the last row (or slice) starting at or before it.
 	__shared__ int marker[64];
+	// Slices that hit the brick, waiting for their rows to be bounded.
+	__shared__ int queue[64];
 
 	const int lane = threadIdx.x;
 	const int big = p.big;
@@ -840,7 +902,6 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 	const int h = p.h;
 	const int64_t elements = static_cast<int64_t>(n) * h;
 	const int64_t kept = blockIdx.y;
-	const int taps = PROFILE == REXLIB_HIP_KAISER_BESSEL ? p.taps : T;
 	const int last_column = h - (n % 2 == 0 ? 2 : 1);
 	// A first tap f holds the positions [f + offset, f + 1 + offset).
 	const float cell_offset = PROFILE == REXLIB_HIP_BOX ? -0.5f :
@@ -853,11 +914,6 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 		const int4 share = tasks[2 * ti + 1];
 		const int64_t share_begin = chunk.count * share.x / share.y;
 		const int64_t share_end = chunk.count * (share.x + 1) / share.y;
-		for (int v = lane; v < L::voxels; v += 64)
-		{
-			acc[v] = brick_voxel{0.0f, 0.0f, 0.0f};
-		}
-		lds_order();
 		// The positions whose first tap lies in the brick, widened so that
 		// rounding never drops a sample (each sample is then tested exactly).
 		float lower[3];
@@ -875,13 +931,20 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 		}
 		const float half_diagonal = sqrtf(half_diagonal2);
 		const float centre_norm = sqrtf(centre[0] * centre[0] + centre[1] * centre[1] + centre[2] * centre[2]);
+		const float nearest = centre_norm - half_diagonal - 1e-3f;
+		// The middle of the first taps of the brick's EX x EY x EZ cells: a
+		// first tap f is the brick's when |f - middle| < E / 2 along each axis.
+		// (A brick cut short at the volume's end may take cells beyond its own
+		// extents, which no other brick owns: their rows end at `upper`.)
+		const float middle[3] = {static_cast<float>(box.lo[0]) + 0.5f * (EX - 1),
+			static_cast<float>(box.lo[1]) + 0.5f * (EY - 1), static_cast<float>(box.lo[2]) + 0.5f * (EZ - 1)};
 
-		// The sample this lane holds, not yet added: value, cell (bits 0-23,
-		// bit 24 set while held) and per axis the fraction past the first tap
-		// (triangle) or the position (Kaiser-Bessel).
+		// The sample this lane holds, not yet added: value, its first-tap cell
+		// and voxel, and per axis the fraction past the first tap.
 		bool pending = false;
 		float held_re = 0.0f, held_im = 0.0f, held_den = 0.0f;
 		int held_cell = 0;
+		int held_voxel = 0;
 		float held_w[3] = {0.0f, 0.0f, 0.0f};
 
 		// One round: every holding lane claims its cell and the winners add
@@ -901,6 +964,91 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 		float4 row_base = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 		float4 row_step = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 		uint32_t row_index = 0;
+		// With 4 taps a sample's 64 taps are the 64 lanes: each lane takes one
+		// sample of the rows, puts its 12 axis weights in LDS, and the wavefront
+		// then adds the samples one after another, each by one read-add-write
+		// of 64 different voxels (no claims, no bank conflicts, every lane
+		// busy). 64 serial taps per lane, claimed as below, took 48 cycles per
+		// CU and sample; this is bound by the LDS pipeline at about 20.
+		const int tap_x = lane & 3;
+		const int tap_y = (lane >> 2) & 3;
+		const int tap_z = lane >> 4;
+		const int tap_voxel = tap_x + L::pitch_y * tap_y + L::pitch_z * tap_z;
+		auto wide_round = [&]()
+		{
+			if constexpr (T == 4)
+			{
+				const int take = min(64, total - next);
+				marker[lane] = lane == 0 ? current : 0;
+				lds_order();
+				if (row_count > 0 && row_start >= next && row_start < next + 64)
+				{
+					marker[row_start - next] = lane;
+				}
+				lds_order();
+				const int row = wave_prefix_max(marker[lane]);
+				lds_order();
+				current = __builtin_amdgcn_readlane(row, take - 1);
+				const float4 b = make_float4(__shfl(row_base.x, row, 64), __shfl(row_base.y, row, 64),
+					__shfl(row_base.z, row, 64), __shfl(row_base.w, row, 64));
+				const float4 st = make_float4(__shfl(row_step.x, row, 64), __shfl(row_step.y, row, 64),
+					__shfl(row_step.z, row, 64), 0.0f);
+				const uint32_t ix = static_cast<uint32_t>(__shfl(static_cast<int>(row_index), row, 64));
+				const int kx = __float_as_int(b.w) + next + lane;
+				const bool mine = lane < take;
+				prepared_sample q{0.0f, 0.0f, 0.0f};
+				if (mine)
+				{
+					q = prepared[(ix & 0x7fffffffu) + static_cast<uint32_t>(kx)];
+				}
+				const float c[3] = {row_position(b.x, st.x, kx), row_position(b.y, st.y, kx), row_position(b.z, st.z, kx)};
+				float f[3];
+#pragma unroll
+				for (int a = 0; a < 3; ++a)
+				{
+					float w[4];
+					window_taps<PROFILE>::template place<4>(p, mine ? c[a] : 0.0f, w);
+					axis_weights[lane * 3 + a] = make_float4(w[0], w[1], w[2], w[3]);
+					f[a] = window_taps<PROFILE>::first_float(p, c[a]) - middle[a];
+				}
+				const bool own = mine && fabsf(f[0]) < 0.5f * EX && fabsf(f[1]) < 0.5f * EY && fabsf(f[2]) < 0.5f * EZ &&
+					!(q.re == 0.0f && q.im == 0.0f && q.den == 0.0f);
+				constexpr float first_voxel = 0.5f * ((EX - 1) + L::pitch_y * (EY - 1) + L::pitch_z * (EZ - 1));
+				const int voxel = static_cast<int>(fmaf(f[2], L::pitch_z, fmaf(f[1], L::pitch_y, f[0] + first_voxel)));
+				const float im = __uint_as_float(__float_as_uint(q.im) ^ (ix & 0x80000000u));
+				lds_order();
+				const float *weights = reinterpret_cast<const float *>(axis_weights);
+				// The weights of the next sample are read before the taps of this
+				// one, so a sample waits for LDS once.
+				uint64_t left = __ballot(own);
+				int s = left != 0 ? __builtin_ctzll(left) : 0;
+				float wx = weights[12 * s + tap_x];
+				float wy = weights[12 * s + 4 + tap_y];
+				float wz = weights[12 * s + 8 + tap_z];
+				while (left != 0)
+				{
+					const int at = __builtin_amdgcn_readlane(voxel, s) + tap_voxel;
+					const float wt = wz * wy * wx;
+					const float re = lane_value(q.re, s);
+					const float imaginary = lane_value(im, s);
+					const float den = lane_value(q.den, s);
+					left &= left - 1;
+					s = left != 0 ? __builtin_ctzll(left) : 0;
+					wx = weights[12 * s + tap_x];
+					wy = weights[12 * s + 4 + tap_y];
+					wz = weights[12 * s + 8 + tap_z];
+					float2 v = acc_value[at];
+					float d = acc_weight[at];
+					v.x += re * wt;
+					v.y += imaginary * wt;
+					d += den * wt;
+					acc_value[at] = v;
+					acc_weight[at] = d;
+					lds_order();
+				}
+				next += take;
+			}
+		};
 		auto round = [&](bool fill)
 		{
 			// Claim: each holding lane writes its lane into the byte of its
@@ -908,16 +1056,12 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 			// store (lds_order keeps the compiler from reusing the stored
 			// value); a volatile pointer would turn it into a flat load, which
 			// is not ordered after the LDS store.
-			const int lx = held_cell & 0xff;
-			const int ly = (held_cell >> 8) & 0xff;
-			const int lz = (held_cell >> 16) & 0xff;
-			const int cell = lx + EX * (ly + EY * lz);
 			if (pending)
 			{
-				claim[cell] = static_cast<unsigned char>(lane);
+				claim[held_cell] = static_cast<unsigned char>(lane);
 			}
 			lds_order();
-			const bool win = pending && claim[cell] == lane;
+			const bool win = pending && claim[held_cell] == lane;
 			lds_order();
 
 			// The fill starts before the winners' taps: the lanes free after
@@ -972,7 +1116,7 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 
 			if (win)
 			{
-				const int base = lx + L::pitch_y * ly + L::pitch_z * lz;
+				const int base = held_voxel;
 				float wx[T], wy[T], wz[T];
 				if constexpr (PROFILE == REXLIB_HIP_TRIANGLE)
 				{
@@ -983,17 +1127,11 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 					wz[0] = 1.0f - held_w[2];
 					wz[1] = held_w[2];
 				}
-				else if constexpr (PROFILE == REXLIB_HIP_BOX)
+				else
 				{
 					wx[0] = 1.0f;
 					wy[0] = 1.0f;
 					wz[0] = 1.0f;
-				}
-				else
-				{
-					window_taps<PROFILE>::template place<T>(p, held_w[0], wx);
-					window_taps<PROFILE>::template place<T>(p, held_w[1], wy);
-					window_taps<PROFILE>::template place<T>(p, held_w[2], wz);
 				}
 #pragma unroll
 				for (int tz = 0; tz < T; ++tz)
@@ -1005,15 +1143,16 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 #pragma unroll
 						for (int tx = 0; tx < T; ++tx)
 						{
-							if (tx < taps && ty < taps && tz < taps)
 							{
 								const float wt = wzy * wx[tx];
-								brick_voxel &a = acc[base + tx + L::pitch_y * ty + L::pitch_z * tz];
-								brick_voxel v = a;
-								v.re += held_re * wt;
-								v.im += held_im * wt;
-								v.den += held_den * wt;
-								a = v;
+								const int at = base + tx + L::pitch_y * ty + L::pitch_z * tz;
+								float2 v = acc_value[at];
+								float d = acc_weight[at];
+								v.x += held_re * wt;
+								v.y += held_im * wt;
+								d += held_den * wt;
+								acc_value[at] = v;
+								acc_weight[at] = d;
 							}
 							lds_order();
 						}
@@ -1027,26 +1166,28 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 			{
 				const float c[3] = {row_position(b.x, st.x, kx), row_position(b.y, st.y, kx),
 					row_position(b.z, st.z, kx)};
-				int local[3];
+				// First taps in float (whole numbers, exact), less the middle.
+				float f[3];
 				float w[3];
 #pragma unroll
 				for (int a = 0; a < 3; ++a)
 				{
-					const int f = window_taps<PROFILE>::first(p, c[a]);
-					local[a] = f - box.lo[a];
-					w[a] = PROFILE == REXLIB_HIP_TRIANGLE ? c[a] - static_cast<float>(f) : c[a];
+					f[a] = window_taps<PROFILE>::first_float(p, c[a]);
+					w[a] = c[a] - f[a];
+					f[a] -= middle[a];
 				}
-				const bool own = static_cast<unsigned>(local[0]) < static_cast<unsigned>(box.ext[0]) &&
-					static_cast<unsigned>(local[1]) < static_cast<unsigned>(box.ext[1]) &&
-					static_cast<unsigned>(local[2]) < static_cast<unsigned>(box.ext[2]);
-				const bool value = !(q.re == 0.0f && q.im == 0.0f && q.den == 0.0f);
-				if (mine && own && value)
+				const bool own = fabsf(f[0]) < 0.5f * EX && fabsf(f[1]) < 0.5f * EY && fabsf(f[2]) < 0.5f * EZ;
+				if (mine && own)
 				{
 					pending = true;
 					held_re = q.re;
-					held_im = (ix >> 31) != 0 ? -q.im : q.im;
+					held_im = __uint_as_float(__float_as_uint(q.im) ^ (ix & 0x80000000u));
 					held_den = q.den;
-					held_cell = local[0] | (local[1] << 8) | (local[2] << 16) | (1 << 24);
+					constexpr float first_cell = 0.5f * ((EX - 1) + EX * (EY - 1) + EX * EY * (EZ - 1));
+					constexpr float first_voxel =
+						0.5f * ((EX - 1) + L::pitch_y * (EY - 1) + L::pitch_z * (EZ - 1));
+					held_cell = static_cast<int>(fmaf(f[2], EX * EY, fmaf(f[1], EX, f[0] + first_cell)));
+					held_voxel = static_cast<int>(fmaf(f[2], L::pitch_z, fmaf(f[1], L::pitch_y, f[0] + first_voxel)));
 					held_w[0] = w[0];
 					held_w[1] = w[1];
 					held_w[2] = w[2];
@@ -1055,39 +1196,27 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 			}
 		};
 
-		for (int64_t window = share_begin; window < share_end; window += 64)
+		const slice_plane *planes = p.planes + kept * p.map.reduced_count + chunk.begin;
+		const slice_entry *entries = p.entries + kept * p.map.reduced_count + chunk.begin;
+
+		// The rows of the `hits` slices in the queue: one slice per lane.
+		const auto insert_hits = [&](int hits)
 		{
-			// Slices whose plane passes near the brick, one per lane.
-			const int64_t j = window + lane;
-			bool near = false;
+			const bool near = lane < hits;
+			const int js_lane = near ? queue[lane] : 0;
+			lds_order();
 			float x0 = 0.0f, x1 = 0.0f, x2 = 0.0f, y0 = 0.0f, y1 = 0.0f, y2 = 0.0f;
 			int last_shell = -1;
-			if (j < share_end)
+			if (near)
 			{
-				const slice_entry &e = p.entries[kept * p.map.reduced_count + chunk.begin + j];
+				const slice_entry &e = entries[js_lane];
 				last_shell = e.last_shell;
-				if (e.last_shell >= 0)
-				{
-					x0 = e.x_step[0];
-					x1 = e.x_step[1];
-					x2 = e.x_step[2];
-					y0 = static_cast<float>(e.y_step[0]);
-					y1 = static_cast<float>(e.y_step[1]);
-					y2 = static_cast<float>(e.y_step[2]);
-					const float nx = x1 * y2 - x2 * y1;
-					const float ny = x2 * y0 - x0 * y2;
-					const float nz = x0 * y1 - x1 * y0;
-					// The plane meets the box iff |n . c| is at most the box's
-					// support sum_a |n_a| h_a along the normal n.
-					const float distance = fabsf(nx * centre[0] + ny * centre[1] + nz * centre[2]);
-					const float support = fabsf(nx) * half_extent[0] + fabsf(ny) * half_extent[1] +
-						fabsf(nz) * half_extent[2];
-					const float radius = static_cast<float>(e.last_shell) + 0.5f;
-					const float spread =
-						radius * sqrtf(x0 * x0 + x1 * x1 + x2 * x2 + y0 * y0 + y1 * y1 + y2 * y2);
-					near = distance <= support * 1.001f + 1e-3f &&
-						centre_norm <= spread * 1.001f + half_diagonal + 1e-3f;
-				}
+				x0 = e.x_step[0];
+				x1 = e.x_step[1];
+				x2 = e.x_step[2];
+				y0 = static_cast<float>(e.y_step[0]);
+				y1 = static_cast<float>(e.y_step[1]);
+				y2 = static_cast<float>(e.y_step[2]);
 			}
 			// bound_rows of both signs, one slice per lane, and the
 			// reciprocal steps of the frame (shared by both signs).
@@ -1107,9 +1236,15 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 				ix0 = x0 == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(x0);
 				ix1 = x1 == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(x1);
 				ix2 = x2 == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(x2);
-				const float ixs[3] = {ix0, ix1, ix2};
-				bound_rows(p, xs, ys, iy, ixs, last_shell, lower, upper, 0, r0_plus, r1_plus);
-				bound_rows(p, xs, ys, iy, ixs, last_shell, lower, upper, 1, r0_minus, r1_minus);
+				const float normal[3] = {x1 * y2 - x2 * y1, x2 * y0 - x0 * y2, x0 * y1 - x1 * y0};
+				float kx[2];
+				float ky[2];
+				bound_section(xs, ys, normal, lower, upper, kx, ky);
+				bound_rows(p, xs, ys, iy, last_shell, lower, upper, kx[0], kx[1], ky[0], ky[1], 0, r0_plus, r1_plus);
+				const float mirrored_lower[3] = {-upper[0], -upper[1], -upper[2]};
+				const float mirrored_upper[3] = {-lower[0], -lower[1], -lower[2]};
+				bound_rows(p, xs, ys, iy, last_shell, mirrored_lower, mirrored_upper, -kx[1], -kx[0], -ky[1], -ky[0], 1,
+					r0_minus, r1_minus);
 			}
 			const int plus_rows = near ? max(r1_plus - r0_plus, 0) : 0;
 			const int minus_rows = near ? max(r1_minus - r0_minus, 0) : 0;
@@ -1146,7 +1281,7 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 				const float frame_y[3] = {__shfl(y0, s, 64), __shfl(y1, s, 64), __shfl(y2, s, 64)};
 				const float frame_ix[3] = {__shfl(ix0, s, 64), __shfl(ix1, s, 64), __shfl(ix2, s, 64)};
 				const int shell = __shfl(last_shell, s, 64);
-				const int64_t js = window + s;
+				const int js = __shfl(js_lane, s, 64);
 				float step[3];
 				float y_step[3];
 				float inv_step[3];
@@ -1155,7 +1290,7 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 				int end = 0;
 				if (r < total_rows)
 				{
-					const slice_entry &e = p.entries[kept * p.map.reduced_count + chunk.begin + js];
+					const slice_entry &e = entries[js];
 					for (int a = 0; a < 3; ++a)
 					{
 						step[a] = sign * frame_x[a];
@@ -1189,26 +1324,152 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 				current = 0;
 				while (next < total)
 				{
-					round(true);
+					if constexpr (T == 4)
+					{
+						wide_round();
+					}
+					else
+					{
+						round(true);
+					}
 				}
 				lds_order();
 			}
+		};
+
+		// Slices whose plane passes near the brick: 64 planes are tested at a
+		// time (one 16-byte word a lane, the next 64 already in flight), and
+		// the few that hit (3.5 % at 256^3) collect in `queue` until 64 wait or
+		// the share ends, so that the bounds and rows below run on full lanes.
+		int queued = 0;
+		// Whether any slice hit the brick (its LDS is cleared for the first).
+		bool touched = false;
+		slice_plane plane = planes[min(share_begin + lane, chunk.count - 1)];
+		for (int64_t window = share_begin;; window += 64)
+		{
+			const bool last = window >= share_end;
+			uint64_t hits = 0;
+			bool hit = false;
+			if (!last)
+			{
+				const slice_plane tested = plane;
+				plane = planes[min(window + 64 + lane, chunk.count - 1)];
+				// The plane meets the box iff |n . c| is at most the box's
+				// support sum_a |n_a| h_a along the normal n.
+				const float distance = fabsf(tested.normal[0] * centre[0] + tested.normal[1] * centre[1] +
+					tested.normal[2] * centre[2]);
+				const float support = fabsf(tested.normal[0]) * half_extent[0] + fabsf(tested.normal[1]) * half_extent[1] +
+					fabsf(tested.normal[2]) * half_extent[2];
+				hit = window + lane < share_end && distance <= support * 1.001f + 1e-3f && nearest <= tested.reach;
+				hits = __ballot(hit);
+			}
+			const int count = static_cast<int>(__popcll(hits));
+			if (queued > 0 && (last || queued + count > 64))
+			{
+				if (!touched)
+				{
+					for (int v = lane; v < L::voxels; v += 64)
+					{
+						acc_value[v] = make_float2(0.0f, 0.0f);
+						acc_weight[v] = 0.0f;
+					}
+					touched = true;
+				}
+				lds_order();
+				insert_hits(queued);
+				queued = 0;
+			}
+			if (last)
+			{
+				break;
+			}
+			lds_order();
+			if (hit)
+			{
+				queue[queued + static_cast<int>(__popcll(hits & below))] = static_cast<int>(window) + lane;
+			}
+			queued += count;
 		}
 		// Samples still held after the last rows.
-		while (__ballot(pending) != 0)
+		if constexpr (T < 4)
 		{
-			round(false);
+			while (__ballot(pending) != 0)
+			{
+				round(false);
+			}
 		}
 		lds_order();
 
 		// Add the brick to the accumulators of its kept batch element.
+		if (!touched && !(VOXELS && share.x == 0 && !input.in_place))
+		{
+			continue;
+		}
+		const int he = big / 2;
+		const int64_t num_base = kept_offset(p.map, slot_numerator_out, kept);
+		const int64_t den_base = kept_offset(p.map, slot_denominator_out, kept);
+		if constexpr (VOXELS)
+		{
+			// The voxels past the T - 1 lower faces are this brick's alone: out =
+			// in + sum, written once. Atomics go to the voxels of a brick split
+			// into shares and to +-N/2 of an even N (one stored element that
+			// two bricks reach), whose inputs are in the outputs already.
+			const bool split = share.y > 1;
+			if (split && !touched)
+			{
+				continue;
+			}
+			const int64_t num_in = kept_offset(p.map, input.num_slot, kept);
+			const int64_t den_in = kept_offset(p.map, input.den_slot, kept);
+			const int x_count = min(box.ext[0] - (T - 1), he + 1 - (box.lo[0] + T - 1));
+			const int y_count = min(box.ext[1] - (T - 1), he + 1 - (box.lo[1] + T - 1));
+			const int z_count = min(box.ext[2] - (T - 1), he + 1 - (box.lo[2] + T - 1));
+			constexpr int row = EX - T + 1 <= 8 ? 8 : 16; // lanes along x
+			const int lx = lane % row;
+			if (lx < x_count)
+			{
+				const int x = box.lo[0] + T - 1 + lx;
+				for (int r = lane / row; r < y_count * z_count; r += 64 / row)
+				{
+					const int lz = r / y_count;
+					const int ly = r - lz * y_count;
+					const int v = (lx + T - 1) + L::pitch_y * (ly + T - 1) + L::pitch_z * (lz + T - 1);
+					const float2 sum = touched ? acc_value[v] : make_float2(0.0f, 0.0f);
+					const float weight = touched ? acc_weight[v] : 0.0f;
+					const int y = box.lo[1] + T - 1 + ly;
+					const int z = box.lo[2] + T - 1 + lz;
+					const int sy = y < 0 ? y + big : y;
+					const int sz = z < 0 ? z + big : z;
+					const float2 value = volume_phase<ODD>(p, sum, x, sy, sz);
+					float2 *target = p.numerator + num_base + sz * p.num_s0 + sy * p.num_s1 + x * p.num_s2;
+					float *dtarget = p.denominator + den_base + sz * p.den_s0 + sy * p.den_s1 + x * p.den_s2;
+					const bool shared = split || (big % 2 == 0 && (sy == he || sz == he));
+					const bool none = sum.x == 0.0f && sum.y == 0.0f && weight == 0.0f;
+					if (shared)
+					{
+						if (!none)
+						{
+							atomicAdd(&target->x, value.x);
+							atomicAdd(&target->y, value.y);
+							atomicAdd(dtarget, weight);
+						}
+					}
+					else if (!(none && input.in_place))
+					{
+						const float2 a = input.numerator[num_in + sz * input.num_s0 + sy * input.num_s1 + x * input.num_s2];
+						const float d = input.denominator[den_in + sz * input.den_s0 + sy * input.den_s1 + x * input.den_s2];
+						*target = make_float2(a.x + value.x, a.y + value.y);
+						*dtarget = d + weight;
+					}
+				}
+			}
+			lds_order();
+			continue;
+		}
 		// Voxels no other task touches (at least taps - 1 past the lower faces,
 		// inside the cells, a brick of one task without aliasing) take a plain
 		// read-add-write, the others atomics.
 		const bool single = share.y == 1 && box.alias_free;
-		const int he = big / 2;
-		const int64_t num_base = kept_offset(p.map, slot_numerator_out, kept);
-		const int64_t den_base = kept_offset(p.map, slot_denominator_out, kept);
 		for (int v = lane; v < L::voxels; v += 64)
 		{
 			const int lz = v / L::pitch_z;
@@ -1219,8 +1480,9 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 			{
 				continue;
 			}
-			const brick_voxel sum = acc[v];
-			if (sum.re == 0.0f && sum.im == 0.0f && sum.den == 0.0f)
+			const float2 sum = acc_value[v];
+			const float weight = acc_weight[v];
+			if (sum.x == 0.0f && sum.y == 0.0f && weight == 0.0f)
 			{
 				continue;
 			}
@@ -1233,7 +1495,7 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 			}
 			const int sy = y < 0 ? y + big : y;
 			const int sz = z < 0 ? z + big : z;
-			const float2 value = volume_phase<ODD>(p, make_float2(sum.re, sum.im), x, sy, sz);
+			const float2 value = volume_phase<ODD>(p, sum, x, sy, sz);
 			float2 *target = p.numerator + num_base + sz * p.num_s0 + sy * p.num_s1 + x * p.num_s2;
 			float *dtarget = p.denominator + den_base + sz * p.den_s0 + sy * p.den_s1 + x * p.den_s2;
 			const bool exclusive = single && lx >= T - 1 && ly >= T - 1 && lz >= T - 1 && lx < box.ext[0] &&
@@ -1244,20 +1506,20 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 				t.x += value.x;
 				t.y += value.y;
 				*target = t;
-				*dtarget += sum.den;
+				*dtarget += weight;
 			}
 			else
 			{
 				atomicAdd(&target->x, value.x);
 				atomicAdd(&target->y, value.y);
-				atomicAdd(dtarget, sum.den);
+				atomicAdd(dtarget, weight);
 			}
 		}
 		lds_order();
 	}
 }
 
-// Brick shapes (first-tap cells along x, y, z): 16 x 8 x 6 (the default),
+// Brick shapes (first-tap cells along x, y, z): 16 x 8 x 6,
 // 16 x 8 x 8, 16 x 16 x 8, 8 x 8 x 8, 8 x 8 x 6, 8 x 6 x 6 and 8 x 8 x 4, and
 // the expected plane hits per task that splits busy bricks. Smaller bricks
 // take less LDS (more wavefronts per CU) but hold more halo voxels per cell.
@@ -1272,7 +1534,20 @@ struct brick_tuning
 	int share;
 };
 
+// What the getter reports for an extent without an entry.
 constexpr brick_tuning default_brick_tuning{16, 8, 6, 256};
+
+// What calls take without an entry: over 64 to 512 voxels and 16 to 2,048
+// slices, 8 x 8 x 8 bricks and 512 plane hits per task stay within a tenth of
+// the fastest shape for up to two taps per axis, and 8 x 6 x 6 for four (16 x
+// 8 x 6 and 256, the default before the slices were culled 64 at a time, is up
+// to a third slower on dense stacks).
+constexpr brick_tuning untuned_bricks{8, 8, 8, 512};
+constexpr brick_tuning untuned_wide_bricks{8, 6, 6, 512};
+
+// Bricks that own voxels: a cell shell of T - 1 is walked twice, so the brick
+// has to be a large one of the small ones.
+constexpr brick_tuning voxel_tuning{8, 8, 8, 512};
 
 std::mutex tuning_mutex;
 std::map<int, brick_tuning> tuning_table;
@@ -1289,8 +1564,8 @@ constexpr int taps_key = 1 << 20;
 
 // The tuning of an extent for a window of `taps` per axis (0: any window):
 // the window's own entry, else the extent's, else the entry for every
-// extent, else the built-in default.
-brick_tuning tuning_for(int extent, int taps = 0)
+// extent, else `fallback`.
+brick_tuning tuning_for(int extent, int taps, const brick_tuning &fallback)
 {
 	std::lock_guard<std::mutex> lock(tuning_mutex);
 	auto found = taps > 0 ? tuning_table.find(extent + taps * taps_key) : tuning_table.end();
@@ -1302,71 +1577,79 @@ brick_tuning tuning_for(int extent, int taps = 0)
 	{
 		found = tuning_table.find(0);
 	}
-	return found != tuning_table.end() ? found->second : default_brick_tuning;
+	return found != tuning_table.end() ? found->second : fallback;
 }
 
 template <int PROFILE, int EX, int EY, int EZ>
 void launch_brick_shape(const insertion_params &p, slice_chunk chunk, const prepared_sample *prepared, const int4 *tasks,
-	int task_count, hipStream_t stream)
+	int task_count, const accumulator_input *input, hipStream_t stream)
 {
 	const dim3 grid(static_cast<unsigned>(task_count), static_cast<unsigned>(p.map.kept_count));
-	if (p.big % 2 == 1)
+	const auto launch = [&](auto odd, auto voxels)
 	{
-		brick_kernel<PROFILE, true, EX, EY, EZ><<<grid, 64, 0, stream>>>(p, chunk, prepared, tasks, task_count);
-	}
-	else
+		brick_kernel<PROFILE, decltype(odd)::value, decltype(voxels)::value, EX, EY, EZ><<<grid, 64, 0, stream>>>(p, chunk,
+			prepared, tasks, task_count, input != nullptr ? *input : accumulator_input{});
+	};
+	if constexpr (PROFILE != REXLIB_HIP_KAISER_BESSEL && EX == voxel_tuning.ex && EY == voxel_tuning.ey &&
+		EZ == voxel_tuning.ez)
 	{
-		brick_kernel<PROFILE, false, EX, EY, EZ><<<grid, 64, 0, stream>>>(p, chunk, prepared, tasks, task_count);
+		if (input != nullptr)
+		{
+			p.big % 2 == 1 ? launch(std::true_type(), std::true_type()) : launch(std::false_type(), std::true_type());
+			return;
+		}
 	}
+	p.big % 2 == 1 ? launch(std::true_type(), std::false_type()) : launch(std::false_type(), std::false_type());
 }
 
 template <int PROFILE>
 void launch_brick(const insertion_params &p, slice_chunk chunk, const prepared_sample *prepared, const int4 *tasks,
-	int task_count, const brick_tuning &t, hipStream_t stream)
+	int task_count, const brick_tuning &t, const accumulator_input *input, hipStream_t stream)
 {
 	if (t.ex == 16 && t.ey == 8 && t.ez == 8)
 	{
-		launch_brick_shape<PROFILE, 16, 8, 8>(p, chunk, prepared, tasks, task_count, stream);
+		launch_brick_shape<PROFILE, 16, 8, 8>(p, chunk, prepared, tasks, task_count, input, stream);
 	}
 	else if (t.ex == 16 && t.ey == 16)
 	{
-		launch_brick_shape<PROFILE, 16, 16, 8>(p, chunk, prepared, tasks, task_count, stream);
+		launch_brick_shape<PROFILE, 16, 16, 8>(p, chunk, prepared, tasks, task_count, input, stream);
 	}
 	else if (t.ex == 8 && t.ey == 8 && t.ez == 8)
 	{
-		launch_brick_shape<PROFILE, 8, 8, 8>(p, chunk, prepared, tasks, task_count, stream);
+		launch_brick_shape<PROFILE, 8, 8, 8>(p, chunk, prepared, tasks, task_count, input, stream);
 	}
 	else if (t.ex == 8 && t.ey == 8 && t.ez == 6)
 	{
-		launch_brick_shape<PROFILE, 8, 8, 6>(p, chunk, prepared, tasks, task_count, stream);
+		launch_brick_shape<PROFILE, 8, 8, 6>(p, chunk, prepared, tasks, task_count, input, stream);
 	}
 	else if (t.ex == 8 && t.ey == 8)
 	{
-		launch_brick_shape<PROFILE, 8, 8, 4>(p, chunk, prepared, tasks, task_count, stream);
+		launch_brick_shape<PROFILE, 8, 8, 4>(p, chunk, prepared, tasks, task_count, input, stream);
 	}
 	else if (t.ex == 8)
 	{
-		launch_brick_shape<PROFILE, 8, 6, 6>(p, chunk, prepared, tasks, task_count, stream);
+		launch_brick_shape<PROFILE, 8, 6, 6>(p, chunk, prepared, tasks, task_count, input, stream);
 	}
 	else
 	{
-		launch_brick_shape<PROFILE, 16, 8, 6>(p, chunk, prepared, tasks, task_count, stream);
+		launch_brick_shape<PROFILE, 16, 8, 6>(p, chunk, prepared, tasks, task_count, input, stream);
 	}
 }
 
 void dispatch_brick(const insertion_params &p, slice_chunk chunk, const prepared_sample *prepared, const int4 *tasks,
-	int task_count, const brick_tuning &tuning, hipStream_t stream)
+	int task_count, const brick_tuning &tuning, const accumulator_input *input,
+	hipStream_t stream)
 {
 	switch (p.profile)
 	{
 	case REXLIB_HIP_BOX:
-		launch_brick<REXLIB_HIP_BOX>(p, chunk, prepared, tasks, task_count, tuning, stream);
+		launch_brick<REXLIB_HIP_BOX>(p, chunk, prepared, tasks, task_count, tuning, input, stream);
 		break;
 	case REXLIB_HIP_TRIANGLE:
-		launch_brick<REXLIB_HIP_TRIANGLE>(p, chunk, prepared, tasks, task_count, tuning, stream);
+		launch_brick<REXLIB_HIP_TRIANGLE>(p, chunk, prepared, tasks, task_count, tuning, input, stream);
 		break;
 	default:
-		launch_brick<REXLIB_HIP_KAISER_BESSEL>(p, chunk, prepared, tasks, task_count, tuning, stream);
+		launch_brick<REXLIB_HIP_KAISER_BESSEL>(p, chunk, prepared, tasks, task_count, tuning, input, stream);
 		break;
 	}
 }
@@ -1468,7 +1751,8 @@ void dispatch_columns_prepare(const insertion_params &p, slice_chunk chunk, prep
 // split into shares of at most `target` of them -- or fewer, so that no task
 // carries more than the average load of a slot (the total over `slots`):
 // a task longer than that would outlast the rest of the launch.
-std::vector<int4> brick_task_items(int big, int64_t bucket, int target, int ex, int ey, int ez, int taps, int slots)
+std::vector<int4> brick_task_items(int big, int64_t bucket, int target, int ex, int ey, int ez, int taps, int slots,
+	bool voxels)
 {
 	const int half = big / 2;
 	// First-tap cells: x in [-(taps - 1), N/2]; y, z in [-(N/2) - (taps - 1),
@@ -1481,10 +1765,13 @@ std::vector<int4> brick_task_items(int big, int64_t bucket, int target, int ex, 
 		const int end = first + count + reach;
 		return (first <= -half && -half < end) || (first <= half && half < end);
 	};
-	const auto starts = [](int low, int high, int edge)
+	// Bricks that own voxels overlap by the taps - 1 cells whose samples reach
+	// the next brick's first voxels.
+	const int overlap = voxels ? reach : 0;
+	const auto starts = [overlap](int low, int high, int edge)
 	{
 		std::vector<std::pair<int, int>> out;
-		for (int s = low; s <= high; s += edge)
+		for (int s = low; s + overlap <= high; s += edge - overlap)
 		{
 			out.emplace_back(s, std::min(edge, high - s + 1));
 		}
@@ -1548,59 +1835,73 @@ std::vector<int4> brick_task_items(int big, int64_t bucket, int target, int ex, 
 struct task_list
 {
 	std::vector<int4> host;
+	int split = 0; // the tasks up to the last one of a split brick
 	int4 *device = nullptr;
 };
 
 std::mutex task_mutex;
-std::map<std::tuple<int, int, int64_t, int, int, int, int, int>, task_list> task_cache;
+std::map<std::tuple<int, int, int64_t, int, int, int, int, int, bool>, task_list> task_cache;
 
-// The cached list for a call (made on first use); the caller holds task_mutex.
-task_list &brick_task_list(int big, int64_t slices, const brick_tuning &tuning, int taps)
+int64_t slice_bucket(int64_t slices)
 {
-	int device = 0;
-	REXLIB_HIP_CHECK(hipGetDevice(&device));
 	int64_t bucket = 1;
 	while (bucket < slices)
 	{
 		bucket *= 2;
 	}
-	const auto key = std::make_tuple(device, big, bucket, tuning.share, tuning.ex, tuning.ey, tuning.ez, taps);
+	return bucket;
+}
+
+// The cached list for a call (made on first use); the caller holds task_mutex.
+task_list &brick_task_list(int big, int64_t slices, const brick_tuning &tuning, int taps, bool voxels)
+{
+	int device = 0;
+	REXLIB_HIP_CHECK(hipGetDevice(&device));
+	const int64_t bucket = slice_bucket(slices);
+	const auto key = std::make_tuple(device, big, bucket, tuning.share, tuning.ex, tuning.ey, tuning.ez, taps, voxels);
 	auto found = task_cache.find(key);
 	if (found == task_cache.end())
 	{
 		// Brick wavefronts resident at once: as many per CU as its 160 KiB of
-		// LDS holds (the brick's voxels, claim bytes and 64 markers, in
-		// 512-byte granules).
+		// LDS holds (the brick's voxels, claim bytes or axis weights, 64
+		// markers and 64 queued slices, in 512-byte granules).
 		int units = 0;
 		REXLIB_HIP_CHECK(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device));
 		const int lx = tuning.ex + taps - 1, ly = tuning.ey + taps - 1, lz = tuning.ez + taps - 1;
-		const int pitch_y = lx % 2 == 0 ? lx + 1 : lx;
-		const int pitch_z = (pitch_y * ly) % 2 == 0 ? pitch_y * ly + 1 : pitch_y * ly;
+		const int pitch_z = brick_pitch_z(taps, brick_pitch_y(taps, lx), ly);
 		const int lds = static_cast<int>(align_up(static_cast<std::size_t>(pitch_z * lz * 12 +
-			tuning.ex * tuning.ey * tuning.ez + 64 * 4), 512));
+			(taps == 4 ? 64 * 48 : tuning.ex * tuning.ey * tuning.ez) + 2 * 64 * 4), 512));
 		found = task_cache.emplace(key, task_list{}).first;
 		found->second.host = brick_task_items(big, bucket, tuning.share, tuning.ex, tuning.ey, tuning.ez, taps,
-			units * std::max(1, (160 * 1024) / lds));
+			units * std::max(1, (160 * 1024) / lds), voxels);
+		for (std::size_t i = 0; i < found->second.host.size(); i += 2)
+		{
+			if (found->second.host[i + 1].y > 1)
+			{
+				found->second.split = static_cast<int>(i / 2) + 1;
+			}
+		}
 	}
 	return found->second;
 }
 
 // Workspace bytes the task list of a call takes (with its alignment).
-std::size_t brick_task_bytes(int big, int64_t slices, const brick_tuning &tuning, int taps)
+std::size_t brick_task_bytes(int big, int64_t slices, const brick_tuning &tuning, int taps, bool voxels)
 {
 	std::lock_guard<std::mutex> lock(task_mutex);
-	return align_up(sizeof(int4) * brick_task_list(big, slices, tuning, taps).host.size(), 256) + 256;
+	return align_up(sizeof(int4) * brick_task_list(big, slices, tuning, taps, voxels).host.size(), 256) + 256;
 }
 
 // The device copy of a call's tasks. With a fixed workspace buffer the list
 // is copied into it from the host copy the cache keeps (nothing allocated);
 // otherwise the device copy is made once and cached.
-const int4 *brick_tasks(int big, int64_t slices, const brick_tuning &tuning, int taps, workspace_source &workspace,
-	hipStream_t stream, int &count)
+const int4 *brick_tasks(int big, int64_t slices, const brick_tuning &tuning, int taps, bool voxels,
+	workspace_source &workspace, hipStream_t stream, int &count, int &split)
 {
 	std::lock_guard<std::mutex> lock(task_mutex);
-	task_list &list = brick_task_list(big, slices, tuning, taps);
+	task_list &list = brick_task_list(big, slices, tuning, taps, voxels);
 	count = static_cast<int>(list.host.size() / 2);
+	split = list.split;
 	const std::size_t bytes = sizeof(int4) * list.host.size();
 	if (workspace.arena != nullptr)
 	{
@@ -1614,6 +1915,24 @@ const int4 *brick_tasks(int big, int64_t slices, const brick_tuning &tuning, int
 		REXLIB_HIP_CHECK(hipMemcpy(list.device, list.host.data(), bytes, hipMemcpyHostToDevice));
 	}
 	return list.device;
+}
+
+// Whether the bricks of a call own voxels rather than first-tap cells. A brick
+// of cells adds its voxels on the faces that other bricks also reach by
+// atomics (they bypass the L2 of an XCD), after a copy of the inputs; a brick
+// of voxels writes each of them once, input plus sum, but inserts the samples
+// of its T - 1 lower cell layers a second time (512 / 343 of the samples for 8
+// x 8 x 8 and two taps). The line is at the density where the one costs what
+// the other does, in samples per voxel of the stored half: 256 slices of 256^2
+// into 512^3 (0.1 samples per voxel) take 1.25 against 1.75 ms, 512 of 256^2
+// into 256^3 (1.6) 0.47 against 0.51 ms, 1,024 (3.1) 0.75 against 0.71 ms. Four
+// taps would insert 4 times the samples; a fixed workspace buffer keeps the
+// smaller task list of cells.
+bool bricks_own_voxels(const insertion_params &p, int64_t slices, int taps, const workspace_source &workspace)
+{
+	const double samples = 0.125 * 3.14159265 * p.n * p.n * static_cast<double>(slice_bucket(slices));
+	const double voxels = 0.5 * p.big * p.big * static_cast<double>(p.big);
+	return taps <= 2 && workspace.arena == nullptr && samples < 1.6 * voxels;
 }
 
 } // anonymous namespace
@@ -1645,7 +1964,7 @@ void set_insertion_tuning(int extent, int taps, int extent_x, int extent_y, int 
 
 void get_insertion_tuning(int extent, int *extent_x, int *extent_y, int *extent_z, int *share)
 {
-	const brick_tuning t = tuning_for(extent);
+	const brick_tuning t = tuning_for(extent, 0, default_brick_tuning);
 	*extent_x = t.ex;
 	*extent_y = t.ey;
 	*extent_z = t.ez;
@@ -1687,32 +2006,39 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 	const int h = p.h;
 
 	// Workspace: entries, phase tables, the window table, the volume phases.
-	const std::size_t entry_bytes = align_up(sizeof(slice_entry) * std::max<int64_t>(slices, 1), 256);
+	static_assert(sizeof(slice_entry) == 96 && sizeof(slice_plane) == 16, "an entry and its plane take 112 bytes");
+	const std::size_t entry_bytes = align_up((sizeof(slice_entry) + sizeof(slice_plane)) *
+		std::max<int64_t>(slices, 1), 256);
 	const std::size_t table_bytes = align_up(sizeof(float2) * (h + n) * std::max<int64_t>(slices, 1), 256);
 	const std::size_t kb_bytes = align_up(sizeof(float) * (p.kb_count + 3), 256);
 	const std::size_t phase_bytes = align_up(sizeof(float2) * p.big, 256);
 	char *base = static_cast<char *>(
 		workspace.take(area_insertion, entry_bytes + table_bytes + kb_bytes + phase_bytes, stream));
 	p.entries = reinterpret_cast<slice_entry *>(base);
+	p.planes = reinterpret_cast<slice_plane *>(p.entries + slices);
 	p.tables = reinterpret_cast<float2 *>(base + entry_bytes);
 	float *kb = reinterpret_cast<float *>(base + entry_bytes + table_bytes);
 	float2 *vphase = reinterpret_cast<float2 *>(base + entry_bytes + table_bytes + kb_bytes);
 	p.kb_table = kb;
 	p.volume_phase = vphase;
 
-	if (!in_place)
+	const auto copy_inputs = [&](bool shared_only)
 	{
-		const int64_t total = static_cast<int64_t>(p.big) * p.big * p.half * p.map.kept_count;
-		if (total > 0)
+		const int64_t rows = (shared_only ? 2 * static_cast<int64_t>(p.big) - 1 : static_cast<int64_t>(p.big) * p.big) *
+			p.map.kept_count;
+		if (in_place || rows == 0)
 		{
-			const unsigned blocks = static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 1 << 20));
-			copy_accumulators_kernel<<<blocks, 256, 0, stream>>>(p, num_in, num_in_strides[0], num_in_strides[1],
-				num_in_strides[2], den_in, den_in_strides[0], den_in_strides[1], den_in_strides[2]);
-			REXLIB_HIP_CHECK(hipGetLastError());
+			return;
 		}
-	}
+		const unsigned blocks = static_cast<unsigned>(std::min<int64_t>((rows + 3) / 4, 1 << 20));
+		const auto kernel = shared_only ? copy_accumulators_kernel<true> : copy_accumulators_kernel<false>;
+		kernel<<<blocks, 256, 0, stream>>>(p, num_in, num_in_strides[0], num_in_strides[1], num_in_strides[2], den_in,
+			den_in_strides[0], den_in_strides[1], den_in_strides[2]);
+		REXLIB_HIP_CHECK(hipGetLastError());
+	};
 	if (slices == 0)
 	{
+		copy_inputs(false);
 		return;
 	}
 
@@ -1737,7 +2063,7 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 	const int64_t limit = int64_t(4) << 30;
 	// Taps per axis of the brick layout: 1, 2, or 4 for every Kaiser-Bessel window.
 	const int layout_taps = p.profile == REXLIB_HIP_BOX ? 1 : (p.profile == REXLIB_HIP_TRIANGLE ? 2 : 4);
-	const brick_tuning tuning = tuning_for(p.big, layout_taps);
+	brick_tuning tuning = tuning_for(p.big, layout_taps, layout_taps == 4 ? untuned_wide_bricks : untuned_bricks);
 	int64_t chunk_count = 0;
 	if (schedule != schedule_scatter && p.taps <= 4 && p.map.kept_count <= 65535)
 	{
@@ -1754,10 +2080,21 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 			// Tasks made for more slices stay valid for fewer (their shares
 			// are fractions of a chunk).
 			chunk_count = std::min<int64_t>(chunk_count,
-				room(brick_task_bytes(p.big, chunk_count, tuning, layout_taps)) / per_slice);
+				room(brick_task_bytes(p.big, chunk_count, tuning, layout_taps, false)) / per_slice);
 		}
 	}
 	const bool brick = chunk_count >= 1;
+	const bool voxels = brick && bricks_own_voxels(p, chunk_count, layout_taps, workspace);
+	if (voxels)
+	{
+		tuning = voxel_tuning;
+	}
+	// Bricks that own voxels read the inputs themselves, but for the elements
+	// that two of them add to.
+	if (!voxels || p.big % 2 == 0)
+	{
+		copy_inputs(voxels);
+	}
 	// Pending column transforms run inside the preparation of each chunk on
 	// the brick schedule; on the scatter schedule they run here, in place.
 	const bool fused_columns = columns != nullptr && brick;
@@ -1780,7 +2117,8 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 	if (brick)
 	{
 		int count = 0;
-		const int4 *tasks = brick_tasks(p.big, chunk_count, tuning, layout_taps, workspace, stream, count);
+		int split = 0; // tasks of split bricks, the first ones
+		const int4 *tasks = brick_tasks(p.big, chunk_count, tuning, layout_taps, voxels, workspace, stream, count, split);
 		prepared_sample *prepared = static_cast<prepared_sample *>(workspace.take(area_prepared,
 			static_cast<std::size_t>(per_slice * chunk_count), stream));
 		for (int64_t begin = 0; begin < p.map.reduced_count; begin += chunk_count)
@@ -1802,7 +2140,21 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 			REXLIB_HIP_CHECK(hipGetLastError());
 			timing_end(prepare_token, stream);
 			const int brick_token = timing_begin(REXLIB_HIP_KERNEL_BRICK, stream);
-			dispatch_brick(p, chunk, prepared, tasks, count, tuning, stream);
+			const bool from_outputs = in_place || begin > 0;
+			const accumulator_input input = from_outputs ?
+				accumulator_input{p.numerator, p.num_s0, p.num_s1, p.num_s2, p.denominator, p.den_s0, p.den_s1, p.den_s2,
+					slot_numerator_out, slot_denominator_out, true} :
+				accumulator_input{num_in, num_in_strides[0], num_in_strides[1], num_in_strides[2], den_in,
+					den_in_strides[0], den_in_strides[1], den_in_strides[2], slot_numerator, slot_denominator, false};
+			if (voxels && !input.in_place && split > 0)
+			{
+				const dim3 grid(static_cast<unsigned>(split), static_cast<unsigned>(p.map.kept_count));
+				const auto kernel = layout_taps == 1 ? copy_split_bricks_kernel<1> :
+					(layout_taps == 2 ? copy_split_bricks_kernel<2> : copy_split_bricks_kernel<4>);
+				kernel<<<grid, 64, 0, stream>>>(p, tasks, input);
+				REXLIB_HIP_CHECK(hipGetLastError());
+			}
+			dispatch_brick(p, chunk, prepared, tasks, count, tuning, voxels ? &input : nullptr, stream);
 			REXLIB_HIP_CHECK(hipGetLastError());
 			timing_end(brick_token, stream);
 		}

@@ -25,15 +25,22 @@ struct alignas(16) slice_entry
 	float ctf_radial;  // pi L D s^2 = radial |k|^2 + axial (kx^2 - ky^2) + diagonal kx ky
 	float ctf_axial;
 	float ctf_diagonal;
-	float ctf_aberration; // (pi / 2) Cs L^3 s^4 = aberration |k|^4
 	float ctf_phase;      // phase shift + asin(Q)
-	int32_t lattice_free; // 1: samples two steps apart on both axes never share a voxel cell
 	int64_t slice_offset;  // elements of the complex slices
 	int64_t extra_offset;  // elements of the weights (weighted) or CTF parameters
 	int64_t radial_offset;
 	int64_t numerator_offset;   // of the output numerator
 	int64_t denominator_offset; // of the output denominator
-	int64_t kept;
+};
+
+// The plane of a slice, for the brick schedule's first test: the normal
+// X x Y and how far from the origin the slice's disk reaches (negative:
+// nothing to insert). 16 bytes beside the 96 of the entry, so that a wavefront
+// reads 64 planes as 64 consecutive 16-byte words.
+struct alignas(16) slice_plane
+{
+	float normal[3];
+	float reach;
 };
 
 // The range of slices one launch covers, per kept accumulator: reduced
@@ -74,10 +81,11 @@ struct insertion_params
 	int64_t den_s0, den_s1, den_s2;
 	// CTF constants, computed in double on the host.
 	double ctf_defocus_scale; // pi L / (n p)^2
-	double ctf_aberration;    // (pi / 2) Cs L^3 / (n p)^4
+	double ctf_aberration;    // (pi / 2) Cs L^3 / (n p)^4 = aberration |k|^4
 	double ctf_phase0;        // asin(Q)
 	// Workspace.
 	slice_entry *entries;
+	slice_plane *planes;      // one per slice
 	float2 *tables;           // per slice: h x phases then n y phases
 	const float *kb_table;    // kb_count + 3 entries
 	const float2 *volume_phase; // N entries: exp(-2 pi i f(j) C / N) (odd N)

@@ -1,0 +1,77 @@
+"""Insertions on either side of the density at which the bricks own voxels
+rather than first-tap cells (sparse calls write each voxel once, input plus
+sum), and the Kaiser-Bessel bricks whose lanes are the taps of one sample:
+against the float64 oracle at volume extents that cut the bricks short, in
+place and out of place, with strided and batched accumulators."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from cases import make_case
+from gpu_helpers import OPTICS, hip_insert, hip_window, to_device
+from rexlib_amd import em
+
+pytestmark = pytest.mark.gpu
+
+# The reference's float32 bar (max-abs 1e-4 of accumulators of order one).
+BAR = 1e-4
+
+
+def geometry(inputs, rng):
+    """Rotations with shifts in place of the fixture's random matrices."""
+    from rexlib_amd import synthetic
+    count = inputs[2].shape[0]
+    inputs[3][...] = synthetic.transforms_of(synthetic.uniform_rotations(count, rng))
+    inputs[3][:, :2, 3] = rng.uniform(-2, 2, (count, 2))
+    return inputs
+
+
+# 1.6 samples per voxel of the stored half divide the two: n = N = 16 with 5
+# slices (0.4: bucket 8) and with 60 (3.1); N around 7 (voxels per brick), 8 and
+# 14; odd and even.
+@pytest.mark.parametrize("n,big,slices", [(16, 16, 5), (16, 16, 60), (6, 7, 2), (7, 13, 3), (8, 14, 3), (9, 15, 1),
+                                          (12, 24, 9), (12, 29, 9), (20, 33, 4)])
+@pytest.mark.parametrize("in_place", [True, False])
+def test_sparse_and_dense_insertions_match_the_oracle(n, big, slices, in_place):
+    inputs = geometry(make_case("plain", n, big, seed=n + big, slices=slices), np.random.default_rng(big))
+    ref = oracle.insert_f64("plain", inputs, oracle.Window.linear())
+    num, den = hip_insert("plain", inputs, oracle.Window.linear(), in_place=in_place)
+    scale = max(1.0, float(np.abs(ref[0]).max()))
+    assert np.abs(num - ref[0]).max() <= BAR * scale
+    assert np.abs(den - ref[1]).max() <= BAR * max(1.0, float(np.abs(ref[1]).max()))
+
+
+def test_sparse_insertion_into_strided_batched_accumulators():
+    n, big, kept, slices = 10, 20, 2, 3
+    rng = np.random.default_rng(4)
+    inputs = make_case("plain", n, big, seed=9, slices=slices, accumulator_batch=(kept, 1))
+    inputs = geometry(inputs, rng)
+    inputs[2] = rng.uniform(-1, 1, (kept, slices, n, n // 2 + 1)) + 0j
+    ref = oracle.insert_f64("plain", inputs, oracle.Window.linear())
+    t = [to_device(a) for a in inputs]
+    # The accumulators transposed in memory, the outputs padded along x.
+    num = t[0].transpose(-3, -2).contiguous().transpose(-3, -2)
+    den = t[1].transpose(-3, -2).contiguous().transpose(-3, -2)
+    num_out = torch.full((kept, 1, big, big, big // 2 + 4), 7.0, dtype=torch.complex64, device="cuda")
+    den_out = torch.full((kept, 1, big, big, big // 2 + 4), 7.0, device="cuda")
+    em.insert_slices(num, den, t[2], t[3], t[4], em.GriddingWindow.linear(),
+                     numerator_out=num_out[..., :big // 2 + 1], denominator_out=den_out[..., :big // 2 + 1])
+    torch.cuda.synchronize()
+    assert np.abs(num_out[..., :big // 2 + 1].cpu().numpy() - ref[0]).max() <= BAR
+    assert np.abs(den_out[..., :big // 2 + 1].cpu().numpy() - ref[1]).max() <= BAR
+    assert bool((num_out[..., big // 2 + 1:] == 7.0).all()) and bool((den_out[..., big // 2 + 1:] == 7.0).all())
+    assert np.array_equal(num.cpu().numpy(), inputs[0].astype(np.complex64))
+
+
+# 3 and 4 taps, one sample per wavefront step; more samples than a wavefront.
+@pytest.mark.parametrize("half_width,shape", [(1.2, 4.0), (1.5, 6.0), (2.0, 9.0)])
+@pytest.mark.parametrize("n,big,slices", [(5, 9, 1), (12, 16, 7), (24, 37, 20)])
+def test_kaiser_bessel_bricks_match_the_oracle(half_width, shape, n, big, slices):
+    window = oracle.Window.kaiser_bessel(half_width, shape)
+    inputs = geometry(make_case("plain", n, big, seed=3 * n, slices=slices), np.random.default_rng(n))
+    ref = oracle.insert_f64("plain", inputs, window)
+    num, den = hip_insert("plain", inputs, window)
+    # The reference's bar for this window (5e-4: its table and its edge).
+    assert np.abs(num - ref[0]).max() <= 5e-4 * max(1.0, float(np.abs(ref[0]).max()))
+    assert np.abs(den - ref[1]).max() <= 5e-4 * max(1.0, float(np.abs(ref[1]).max()))
