@@ -1,8 +1,12 @@
-// Batched FFTs on gfx950: Stockham autosort transforms in LDS.
+// Batched FFTs on gfx950.
 //
-// Every kernel stages a group of lines in LDS, runs the radix-4/2/3/5
-// stages there (ping-pong between two LDS buffers, one butterfly per thread
-// per step), and writes the lines back. Real transforms pack two real rows
+// Lengths of two register factors (every 2-3-5 length from 48 to 625 but 125,
+// 243 and few others, fft_two.hpp) hold a line in the registers of its
+// threads and exchange it once through LDS: 4.5 to 5.5 TB/s of the operand
+// read and written, from 64 to 512 points, where the LDS stages below reach 1.7
+// to 2.9. The other lengths stage a group of lines in LDS, run the
+// radix-4/2/3/5 Stockham stages there (ping-pong between two LDS buffers, one
+// butterfly per thread per step), and write the lines back. Real transforms pack two real rows
 // into one complex line and separate the two half spectra afterwards, so a
 // real row costs half a complex transform.
 //
@@ -14,6 +18,7 @@
 // transform ignores the imaginary parts of the self-conjugate elements.
 #include "fft.hpp"
 #include "fft_device.hpp"
+#include "fft_two.hpp"
 
 #include <hip/hip_bf16.h>
 #include <hip/hip_fp16.h>
@@ -143,16 +148,64 @@ __device__ inline float4 load_real4(const void *base, int64_t index)
 	}
 }
 
+// WIDTH elements of a real row from element c, scaled (zeros when not live):
+// one load of all of them (unit stride, base and row aligned to WIDTH
+// elements) or, for WIDTH 1, one element at any stride.
+template <int KIND, int WIDTH>
+__device__ inline void load_reals(const void *base, bool live, int64_t row, int c, int64_t stride, float scale, float *v)
+{
+#pragma unroll
+	for (int q = 0; q < WIDTH; ++q)
+	{
+		v[q] = 0.0f;
+	}
+	if (!live)
+	{
+		return;
+	}
+	if constexpr (WIDTH == 4)
+	{
+		const float4 f = load_real4<KIND>(base, row + c);
+		v[0] = f.x;
+		v[1] = f.y;
+		v[2] = f.z;
+		v[3] = f.w;
+	}
+	else if constexpr (WIDTH == 2 && KIND == real_f32)
+	{
+		const float2 f = *reinterpret_cast<const float2 *>(static_cast<const float *>(base) + row + c);
+		v[0] = f.x;
+		v[1] = f.y;
+	}
+	else if constexpr (WIDTH == 2)
+	{
+		const unsigned bits = *reinterpret_cast<const unsigned *>(static_cast<const unsigned short *>(base) + row + c);
+		v[0] = KIND == real_bf16 ? __uint_as_float(bits << 16) :
+			__half2float(__ushort_as_half(static_cast<unsigned short>(bits & 0xffff)));
+		v[1] = KIND == real_bf16 ? __uint_as_float(bits & 0xffff0000u) :
+			__half2float(__ushort_as_half(static_cast<unsigned short>(bits >> 16)));
+	}
+	else
+	{
+		v[0] = load_real<KIND>(base, row + c * stride);
+	}
+#pragma unroll
+	for (int q = 0; q < WIDTH; ++q)
+	{
+		v[q] *= scale;
+	}
+}
+
 // Rows of real images, two at a time, to half spectra. Images of extent m
 // are zero-padded to the transform length n with their origin m/2 moved to
 // n/2. `rows` counts the padded rows, n per image, in line set `in` of images
 // (middle = image row, outer = image); the output rows follow line set `out`.
-template <int KIND, int N>
+template <int KIND>
 __global__ void rfft_rows_kernel(const void *in, line_set in_rows, int m, const float *scales,
 	int64_t scale_stride, float2 *out, line_set out_rows, fft_plan plan, const float2 *tw, int pairs)
 {
 	extern __shared__ float2 lds[];
-	const int n = N > 0 ? N : plan.n;
+	const int n = plan.n;
 	const int h = n / 2 + 1;
 	const int stride = n + 1;
 	float2 *a = lds;
@@ -214,7 +267,7 @@ __global__ void rfft_rows_kernel(const void *in, line_set in_rows, int m, const 
 			a[p * stride + i] = make_float2(value[0], value[1]);
 		}
 		__syncthreads();
-		const float2 *z = transform<N>(a, b, pairs, stride, plan, twl, -1.0f);
+		const float2 *z = block_fft(a, b, pairs, stride, plan, twl, -1.0f);
 		for (int t = threadIdx.x; t < pairs * h; t += blockDim.x)
 		{
 			const int p = t / h;
@@ -241,12 +294,11 @@ __global__ void rfft_rows_kernel(const void *in, line_set in_rows, int m, const 
 
 // Complex lines from `src` to `dst` (may be the same memory), `group` lines
 // per step; consecutive lines of a group are loaded by consecutive threads.
-template <int N>
 __global__ void fft_lines_kernel(const float2 *src, line_set src_lines, float2 *dst, line_set dst_lines,
 	fft_plan plan, const float2 *tw, float sign, float scale, int group)
 {
 	extern __shared__ float2 lds[];
-	const int n = N > 0 ? N : plan.n;
+	const int n = plan.n;
 	const int stride = n + 1;
 	float2 *a = lds;
 	float2 *b = lds + group * stride;
@@ -278,7 +330,7 @@ __global__ void fft_lines_kernel(const float2 *src, line_set src_lines, float2 *
 			}
 		}
 		__syncthreads();
-		const float2 *z = transform<N>(a, b, lines, stride, plan, twl, sign);
+		const float2 *z = block_fft(a, b, lines, stride, plan, twl, sign);
 		for (int t = threadIdx.x; t < group * n; t += blockDim.x)
 		{
 			const int e = t / group;
@@ -287,62 +339,6 @@ __global__ void fft_lines_kernel(const float2 *src, line_set src_lines, float2 *
 			{
 				const float2 v = z[l * stride + e];
 				dst[line_dst[l] + e * dst_lines.s_elem] = make_float2(v.x * scale, v.y * scale);
-			}
-		}
-		__syncthreads();
-	}
-}
-
-__global__ __launch_bounds__(256) void fft256_lines_kernel(const float2 *src, line_set src_lines, float2 *dst,
-	line_set dst_lines, const float2 *tw, float sign, float scale)
-{
-	// Per line 16 x 17 values (odd pitches against bank conflicts).
-	__shared__ float2 exchange[fft256_lines * fft256_line_stride];
-	__shared__ float2 twl[256];
-	__shared__ int64_t line_src[fft256_lines];
-	__shared__ int64_t line_dst[fft256_lines];
-	const int t = threadIdx.x;
-	const int l = t & (fft256_lines - 1);
-	const int j = t / fft256_lines; // n1 in the first half, k1 in the second
-	twl[t] = tw[t];
-	const int64_t total = src_lines.count;
-	for (int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(fft256_lines); first < total;
-		first += static_cast<int64_t>(gridDim.x) * fft256_lines)
-	{
-		const int lines = static_cast<int>(total - first < fft256_lines ? total - first : fft256_lines);
-		if (t < fft256_lines)
-		{
-			line_src[t] = t < lines ? line_offset(src_lines, first + t) : 0;
-			line_dst[t] = t < lines ? line_offset(dst_lines, first + t) : 0;
-		}
-		__syncthreads();
-		float2 v[16];
-		const bool live = l < lines;
-		const float2 *in = src + line_src[l];
-#pragma unroll
-		for (int k = 0; k < 16; ++k)
-		{
-			v[k] = live ? in[(j + 16 * k) * src_lines.s_elem] : make_float2(0.0f, 0.0f);
-		}
-		float2 *x = exchange + l * fft256_line_stride;
-		fft256_four_step(v, x, twl, j, sign);
-		// The outputs go back to LDS (each thread to slots only it reads),
-		// so the stores loop over them without holding all 16.
-		__syncthreads();
-#pragma unroll
-		for (int k2 = 0; k2 < 16; ++k2)
-		{
-			x[k2 * 17 + j] = v[k2];
-		}
-		if (live)
-		{
-			float2 *out = dst + line_dst[l] + j * dst_lines.s_elem;
-			const int64_t step = 16 * dst_lines.s_elem;
-#pragma unroll 4
-			for (int k2 = 0; k2 < 16; ++k2)
-			{
-				const float2 y = x[k2 * 17 + j];
-				out[k2 * step] = make_float2(y.x * scale, y.y * scale);
 			}
 		}
 		__syncthreads();
@@ -507,12 +503,11 @@ __global__ __launch_bounds__(256) void rfft256_rows_kernel(const void *in, line_
 }
 
 // Half-spectrum rows, two at a time, to real rows, scaled.
-template <int N>
 __global__ void irfft_rows_kernel(const float2 *src, line_set src_rows, float *dst, line_set dst_rows,
 	fft_plan plan, const float2 *tw, float scale, int pairs)
 {
 	extern __shared__ float2 lds[];
-	const int n = N > 0 ? N : plan.n;
+	const int n = plan.n;
 	const int h = n / 2 + 1;
 	const int stride = n + 1;
 	float2 *a = lds;
@@ -568,7 +563,7 @@ __global__ void irfft_rows_kernel(const float2 *src, line_set src_rows, float *d
 			a[p * stride + k] = make_float2(va.x - vb.y, va.y + vb.x);
 		}
 		__syncthreads();
-		const float2 *z = transform<N>(a, b, pairs, stride, plan, twl, 1.0f);
+		const float2 *z = block_fft(a, b, pairs, stride, plan, twl, 1.0f);
 		for (int t = threadIdx.x; t < pairs * n; t += blockDim.x)
 		{
 			const int p = t / n;
@@ -589,6 +584,192 @@ __global__ void irfft_rows_kernel(const float2 *src, line_set src_rows, float *d
 	}
 }
 
+// ---------------------------------------------------------------------------
+// Lengths of two register factors (fft_two.hpp).
+// ---------------------------------------------------------------------------
+
+// Real rows, two to a complex line, to half spectra, as rfft_rows_kernel: a
+// block of (b, lines) threads stages its rows in LDS (a line's threads load
+// consecutive elements, 4 at a time where VEC), transforms them and separates
+// the two half spectra. Bound by HBM: 1,000 images 320^2 take 0.20 ms against
+// 0.52 ms through the Stockham stages (0.8 GB: 4.0 against 1.6 TB/s).
+template <int KIND, int WIDTH, int CLASS>
+__global__ __launch_bounds__(512, two_factor::waves<CLASS>) void rfft_rows_two_kernel(const void *in, line_set in_rows, int m,
+	const float *scales, int64_t scale_stride, float2 *out, line_set out_rows, two_factor::plan p, const float2 *tw)
+{
+	extern __shared__ float2 lds[];
+	const int j = threadIdx.x;
+	const int l = threadIdx.y;
+	const int threads = blockDim.x;
+	const int n = p.n;
+	const int h = n / 2 + 1;
+	float2 *twl = lds + p.lines * p.line;
+	float2 *x = lds + l * p.line;
+	two_factor::stage_twiddles(p, twl, tw, l * threads + j, threads * blockDim.y);
+	const int64_t total = out_rows.count; // padded rows of all images
+	const int offset = n / 2 - m / 2;
+	// One group of lines per block: a loop over groups would hoist the
+	// twiddles of every register length out of it, into registers.
+	const int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(2 * p.lines);
+	if (first >= total)
+	{
+		return;
+	}
+	// The two rows of the line: first input element (-1: a zero row of the
+	// padding or past the end), first output element, scale.
+	int64_t src[2], dst[2];
+	float scale[2];
+#pragma unroll
+	for (int q = 0; q < 2; ++q)
+	{
+		const int64_t row = first + 2 * l + q;
+		src[q] = -1;
+		dst[q] = -1;
+		scale[q] = 1.0f;
+		if (row < total)
+		{
+			const int64_t image = row / n;
+			const int r = static_cast<int>(row - image * n) - offset;
+			if (r >= 0 && r < m)
+			{
+				src[q] = line_offset(in_rows, image * m + r);
+				if (scales != nullptr)
+				{
+					scale[q] = scales[image * scale_stride];
+				}
+			}
+			dst[q] = line_offset(out_rows, row);
+		}
+	}
+	// Loads of WIDTH elements, two steps of both rows in flight.
+#pragma unroll 2
+	for (int i = WIDTH * j; i < n; i += WIDTH * threads)
+	{
+		const int c = i - offset;
+		const bool inside = c >= 0 && c < m;
+		float a[WIDTH], b[WIDTH];
+		load_reals<KIND, WIDTH>(in, inside && src[0] >= 0, src[0], c, in_rows.s_elem, scale[0], a);
+		load_reals<KIND, WIDTH>(in, inside && src[1] >= 0, src[1], c, in_rows.s_elem, scale[1], b);
+#pragma unroll
+		for (int q = 0; q < WIDTH; ++q)
+		{
+			x[i + q] = make_float2(a[q], b[q]);
+		}
+	}
+	__syncthreads();
+	two_factor::transform_line<CLASS, true, true>(p, x, twl, j, -1.0f, [&](int i) { return x[i]; },
+		[&](int k, float2 v) { x[k] = v; });
+	__syncthreads();
+	for (int k = j; k < h; k += threads)
+	{
+		const float2 zk = x[k];
+		const float2 zm = cconj(x[k == 0 ? 0 : n - k]);
+		if (dst[0] >= 0)
+		{
+			const float2 sum = cadd(zk, zm);
+			out[dst[0] + k * out_rows.s_elem] = make_float2(0.5f * sum.x, 0.5f * sum.y);
+		}
+		if (dst[1] >= 0)
+		{
+			// (zk - zm) / (2 i)
+			const float2 diff = csub(zk, zm);
+			out[dst[1] + k * out_rows.s_elem] = make_float2(0.5f * diff.y, -0.5f * diff.x);
+		}
+	}
+}
+
+// Half-spectrum rows, two at a time, to real rows, scaled, as
+// irfft_rows_kernel: a coefficient is read once and staged with its mirror.
+template <int CLASS>
+__global__ __launch_bounds__(512, two_factor::waves<CLASS>) void irfft_rows_two_kernel(const float2 *src, line_set src_rows, float *dst,
+	line_set dst_rows, two_factor::plan p, const float2 *tw, float scale)
+{
+	extern __shared__ float2 lds[];
+	const int j = threadIdx.x;
+	const int l = threadIdx.y;
+	const int threads = blockDim.x;
+	const int n = p.n;
+	const int h = n / 2 + 1;
+	float2 *twl = lds + p.lines * p.line;
+	float2 *x = lds + l * p.line;
+	two_factor::stage_twiddles(p, twl, tw, l * threads + j, threads * blockDim.y);
+	const int64_t total = src_rows.count;
+	const int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(2 * p.lines);
+	if (first >= total)
+	{
+		return;
+	}
+	const int64_t row = first + 2 * l;
+	const int64_t src0 = row < total ? line_offset(src_rows, row) : -1;
+	const int64_t src1 = row + 1 < total ? line_offset(src_rows, row + 1) : -1;
+	const int64_t dst0 = row < total ? line_offset(dst_rows, row) : -1;
+	const int64_t dst1 = row + 1 < total ? line_offset(dst_rows, row + 1) : -1;
+	for (int k = j; k < h; k += threads)
+	{
+		float2 va = src0 >= 0 ? src[src0 + k * src_rows.s_elem] : make_float2(0.0f, 0.0f);
+		float2 vb = src1 >= 0 ? src[src1 + k * src_rows.s_elem] : make_float2(0.0f, 0.0f);
+		if (k == 0 || 2 * k == n)
+		{
+			va.y = 0.0f;
+			vb.y = 0.0f;
+		}
+		else
+		{
+			// conj A + i conj B at n - k.
+			x[n - k] = make_float2(va.x + vb.y, vb.x - va.y);
+		}
+		x[k] = make_float2(va.x - vb.y, va.y + vb.x); // A + i B
+	}
+	__syncthreads();
+	two_factor::transform_line<CLASS, true, false>(p, x, twl, j, 1.0f, [&](int i) { return x[i]; },
+		[&](int i, float2 v)
+		{
+			if (dst0 >= 0)
+			{
+				dst[dst0 + i * dst_rows.s_elem] = v.x * scale;
+			}
+			if (dst1 >= 0)
+			{
+				dst[dst1 + i * dst_rows.s_elem] = v.y * scale;
+			}
+		});
+}
+
+// Complex lines from `src` to `dst` (may be the same memory). ROWS: the
+// elements of a line are consecutive and so are the threads of a line, else
+// the lines are neighbours in memory and consecutive threads take consecutive
+// lines.
+template <bool ROWS, int CLASS>
+__global__ __launch_bounds__(512, two_factor::waves<CLASS>) void fft_lines_two_kernel(const float2 *src, line_set src_lines, float2 *dst,
+	line_set dst_lines, two_factor::plan p, const float2 *tw, float sign, float scale)
+{
+	extern __shared__ float2 lds[];
+	const int j = ROWS ? threadIdx.x : threadIdx.y;
+	const int l = ROWS ? threadIdx.y : threadIdx.x;
+	float2 *twl = lds + p.lines * p.line;
+	float2 *x = lds + l * p.line;
+	two_factor::stage_twiddles(p, twl, tw, threadIdx.y * blockDim.x + threadIdx.x, blockDim.x * blockDim.y);
+	__syncthreads();
+	const int64_t total = src_lines.count;
+	const int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(p.lines);
+	if (first >= total)
+	{
+		return;
+	}
+	const bool live = first + l < total;
+	const float2 *in = src + (live ? line_offset(src_lines, first + l) : 0);
+	float2 *out = dst + (live ? line_offset(dst_lines, first + l) : 0);
+	two_factor::transform_line<CLASS, false, false>(p, x, twl, j, sign,
+		[&](int i) { return live ? in[i * src_lines.s_elem] : make_float2(0.0f, 0.0f); },
+		[&](int i, float2 v)
+		{
+			if (live)
+			{
+				out[i * dst_lines.s_elem] = make_float2(v.x * scale, v.y * scale);
+			}
+		});
+}
+
 unsigned grid_for(int64_t work, int64_t per_block)
 {
 	const int64_t blocks = (work + per_block - 1) / per_block;
@@ -597,6 +778,52 @@ unsigned grid_for(int64_t work, int64_t per_block)
 
 } // anonymous namespace
 
+namespace two_factor
+{
+
+plan make_plan(int64_t n)
+{
+	// Register lengths per class (with_radix).
+	static const int small[] = {4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16};
+	static const int medium[] = {8, 9, 10, 11, 12, 13, 14, 15, 16, 18, 20, 21, 22};
+	static const int large[] = {10, 12, 13, 14, 15, 16, 18, 20, 21, 22, 24, 25, 26, 27, 28, 30, 32};
+	plan p{};
+	if (n < 48 || n > 1024)
+	{
+		return p;
+	}
+	const auto search = [&](const int *set, int count, int kind)
+	{
+		for (int i = 0; i < count && p.n == 0; ++i)
+		{
+			for (int k = 0; k <= i; ++k)
+			{
+				if (set[i] * set[k] == n)
+				{
+					p.n = static_cast<int32_t>(n);
+					p.a = set[k];
+					p.b = set[i];
+					p.kind = kind;
+				}
+			}
+		}
+	};
+	search(small, 13, 16);
+	search(medium, 13, 22);
+	search(large, 17, 32);
+	if (p.n != 0)
+	{
+		p.pitch = p.b | 1;
+		p.line = (p.a * p.pitch) | 1;
+		// 16 lines read whole 128-byte cache lines of strided operands; past 512
+		// points (32 KiB of exchange per 8 lines) 8 keep two blocks on a CU.
+		p.lines = n <= 512 ? 16 : 8;
+	}
+	return p;
+}
+
+} // namespace two_factor
+
 int lines_per_group(int n)
 {
 	// About 2048 complex elements (16 KiB) per LDS buffer: small blocks keep
@@ -604,25 +831,21 @@ int lines_per_group(int n)
 	return std::max(1, std::min(8, 2048 / std::max(n, 1)));
 }
 
-// Calls f.template operator()<N>() with N the length when it is a power of
-// two from 64 to 512, else 0 (the planned transform).
-template <typename F>
-void with_fixed_length(int64_t n, F &&f)
+// The path's transforms (rfft2, irfft2, irfft3, the image insertion) take
+// lengths with prime factors 2, 3 and 5 and refuse others, as make_fft_plan
+// says; the general transforms also use the kernels of any two-factor length.
+static void check_length(int64_t n, bool any_length)
 {
-	switch (n)
+	if (!(any_length && two_factor::make_plan(n).n != 0))
 	{
-	case 64: f(std::integral_constant<int, 64>()); break;
-	case 128: f(std::integral_constant<int, 128>()); break;
-	case 256: f(std::integral_constant<int, 256>()); break;
-	case 512: f(std::integral_constant<int, 512>()); break;
-	default: f(std::integral_constant<int, 0>()); break;
+		make_fft_plan(n);
 	}
 }
 
 void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, const float *scales,
-	int64_t scale_stride, float2 *out, const line_set &out_rows, int64_t n, hipStream_t stream)
+	int64_t scale_stride, float2 *out, const line_set &out_rows, int64_t n, hipStream_t stream, bool any_length)
 {
-	const fft_plan plan = make_fft_plan(n);
+	check_length(n, any_length);
 	const float2 *tw = twiddles(n);
 	if (n == 256)
 	{
@@ -658,69 +881,130 @@ void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, 
 		REXLIB_HIP_CHECK(hipGetLastError());
 		return;
 	}
+	const two_factor::plan two = two_factor::make_plan(n);
+	if (two.n != 0)
+	{
+		const unsigned blocks = two_factor::blocks_for(out_rows.count, 2 * two.lines);
+		// Rows take loads of 4 (or 2) elements when every run of them is
+		// aligned and contiguous.
+		const std::uintptr_t element = kind == real_f32 ? 4 : 2;
+		const auto runs_of = [&](int64_t width)
+		{
+			return n % width == 0 && in_rows.s_elem == 1 && m % width == 0 && (n / 2 - m / 2) % width == 0 &&
+				in_rows.s_outer % width == 0 && in_rows.s_middle % width == 0 && in_rows.s_inner % width == 0 &&
+				reinterpret_cast<std::uintptr_t>(in) % (width * element) == 0;
+		};
+		const int width = runs_of(4) ? 4 : (runs_of(2) ? 2 : 1);
+		two_factor::with_class(two, [&](auto kind_class)
+			{
+				constexpr int CLASS = decltype(kind_class)::value;
+				const auto launch = [&](auto kind_constant, auto width_constant)
+				{
+					rfft_rows_two_kernel<decltype(kind_constant)::value, decltype(width_constant)::value, CLASS>
+						<<<blocks, dim3(two.b, two.lines), two_factor::shared_bytes(two), stream>>>(in, in_rows, m, scales,
+							scale_stride, out, out_rows, two, tw);
+				};
+				const auto with_width = [&](auto kind_constant)
+				{
+					if (width == 4)
+					{
+						launch(kind_constant, std::integral_constant<int, 4>());
+					}
+					else if (width == 2)
+					{
+						launch(kind_constant, std::integral_constant<int, 2>());
+					}
+					else
+					{
+						launch(kind_constant, std::integral_constant<int, 1>());
+					}
+				};
+				switch (kind)
+				{
+				case real_f32: with_width(std::integral_constant<int, real_f32>()); break;
+				case real_bf16: with_width(std::integral_constant<int, real_bf16>()); break;
+				default: with_width(std::integral_constant<int, real_f16>()); break;
+				}
+			});
+		REXLIB_HIP_CHECK(hipGetLastError());
+		return;
+	}
+	const fft_plan plan = make_fft_plan(n);
 	const int pairs = std::max(1, lines_per_group(static_cast<int>(n)) / 2);
 	// Two buffers, the twiddles, then per row two offsets and a scale.
 	const std::size_t shared = sizeof(float2) * (2 * pairs * (n + 1) + n) + 2 * pairs * (2 * sizeof(int64_t) + 4);
 	const unsigned grid = grid_for(out_rows.count, 2 * pairs);
-	with_fixed_length(n, [&](auto length)
-		{
-			constexpr int N = decltype(length)::value;
-			switch (kind)
-			{
-			case real_f32:
-				rfft_rows_kernel<real_f32, N><<<grid, 256, shared, stream>>>(in, in_rows, m, scales, scale_stride,
-					out, out_rows, plan, tw, pairs);
-				break;
-			case real_bf16:
-				rfft_rows_kernel<real_bf16, N><<<grid, 256, shared, stream>>>(in, in_rows, m, scales, scale_stride,
-					out, out_rows, plan, tw, pairs);
-				break;
-			default:
-				rfft_rows_kernel<real_f16, N><<<grid, 256, shared, stream>>>(in, in_rows, m, scales, scale_stride,
-					out, out_rows, plan, tw, pairs);
-				break;
-			}
-		});
+	const auto launch = [&](auto kind_constant)
+	{
+		rfft_rows_kernel<decltype(kind_constant)::value><<<grid, 256, shared, stream>>>(in, in_rows, m, scales,
+			scale_stride, out, out_rows, plan, tw, pairs);
+	};
+	switch (kind)
+	{
+	case real_f32: launch(std::integral_constant<int, real_f32>()); break;
+	case real_bf16: launch(std::integral_constant<int, real_bf16>()); break;
+	default: launch(std::integral_constant<int, real_f16>()); break;
+	}
 	REXLIB_HIP_CHECK(hipGetLastError());
 }
 
 void launch_fft_lines(const float2 *src, const line_set &src_lines, float2 *dst, const line_set &dst_lines,
-	int64_t n, float sign, float scale, hipStream_t stream)
+	int64_t n, float sign, float scale, hipStream_t stream, bool any_length)
 {
-	const fft_plan plan = make_fft_plan(n);
+	check_length(n, any_length);
 	const float2 *tw = twiddles(n);
-	const int group = lines_per_group(static_cast<int>(n));
-	const std::size_t shared = sizeof(float2) * (2 * group * (n + 1) + n) + 2 * group * sizeof(int64_t);
-	const unsigned grid = grid_for(src_lines.count, group);
-	if (n == 256)
+	const bool rows = src_lines.s_elem == 1 && dst_lines.s_elem == 1;
+	const two_factor::plan two = two_factor::make_plan(n);
+	if (two.n != 0)
 	{
-		const unsigned blocks = xcd_grid(grid_for(src_lines.count, fft256_lines));
-		fft256_lines_kernel<<<blocks, 256, 0, stream>>>(src, src_lines, dst, dst_lines, tw, sign, scale);
+		const unsigned blocks = two_factor::blocks_for(src_lines.count, two.lines);
+		two_factor::with_class(two, [&](auto kind_class)
+			{
+				constexpr int CLASS = decltype(kind_class)::value;
+				if (rows)
+				{
+					fft_lines_two_kernel<true, CLASS><<<blocks, dim3(two.b, two.lines), two_factor::shared_bytes(two),
+						stream>>>(src, src_lines, dst, dst_lines, two, tw, sign, scale);
+				}
+				else
+				{
+					fft_lines_two_kernel<false, CLASS><<<blocks, dim3(two.lines, two.b), two_factor::shared_bytes(two),
+						stream>>>(src, src_lines, dst, dst_lines, two, tw, sign, scale);
+				}
+			});
 		REXLIB_HIP_CHECK(hipGetLastError());
 		return;
 	}
-	with_fixed_length(n, [&](auto length)
-		{
-			constexpr int N = decltype(length)::value;
-			fft_lines_kernel<N><<<grid, 256, shared, stream>>>(src, src_lines, dst, dst_lines, plan, tw, sign, scale,
-				group);
-		});
+	const fft_plan plan = make_fft_plan(n);
+	const int group = lines_per_group(static_cast<int>(n));
+	const std::size_t shared = sizeof(float2) * (2 * group * (n + 1) + n) + 2 * group * sizeof(int64_t);
+	const unsigned grid = grid_for(src_lines.count, group);
+	fft_lines_kernel<<<grid, 256, shared, stream>>>(src, src_lines, dst, dst_lines, plan, tw, sign, scale, group);
 	REXLIB_HIP_CHECK(hipGetLastError());
 }
 
 void launch_irfft_rows(const float2 *src, const line_set &src_rows, float *dst, const line_set &dst_rows,
-	int64_t n, float scale, hipStream_t stream)
+	int64_t n, float scale, hipStream_t stream, bool any_length)
 {
-	const fft_plan plan = make_fft_plan(n);
+	check_length(n, any_length);
 	const float2 *tw = twiddles(n);
+	const two_factor::plan two = two_factor::make_plan(n);
+	if (two.n != 0)
+	{
+		const unsigned blocks = two_factor::blocks_for(src_rows.count, 2 * two.lines);
+		two_factor::with_class(two, [&](auto kind_class)
+			{
+				irfft_rows_two_kernel<decltype(kind_class)::value><<<blocks, dim3(two.b, two.lines),
+					two_factor::shared_bytes(two), stream>>>(src, src_rows, dst, dst_rows, two, tw, scale);
+			});
+		REXLIB_HIP_CHECK(hipGetLastError());
+		return;
+	}
+	const fft_plan plan = make_fft_plan(n);
 	const int pairs = std::max(1, lines_per_group(static_cast<int>(n)) / 2);
 	const std::size_t shared = sizeof(float2) * (2 * pairs * (n + 1) + n) + 2 * pairs * 2 * sizeof(int64_t);
 	const unsigned grid = grid_for(src_rows.count, 2 * pairs);
-	with_fixed_length(n, [&](auto length)
-		{
-			constexpr int N = decltype(length)::value;
-			irfft_rows_kernel<N><<<grid, 256, shared, stream>>>(src, src_rows, dst, dst_rows, plan, tw, scale, pairs);
-		});
+	irfft_rows_kernel<<<grid, 256, shared, stream>>>(src, src_rows, dst, dst_rows, plan, tw, scale, pairs);
 	REXLIB_HIP_CHECK(hipGetLastError());
 }
 

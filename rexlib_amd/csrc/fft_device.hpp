@@ -160,8 +160,7 @@ __device__ inline void fft256_four_step(float2 *v, float2 *line, const float2 *t
 }
 
 // Stockham stages over `lines` lines of an LDS buffer, ping-pong between a
-// and b; the planned form for any length of radices 4, 2, 3, 5, the fixed
-// form for the powers of two with compile-time indices.
+// and b, for any length of radices 4, 2, 3, 5.
 template <int R>
 __device__ inline void stage(const float2 *a, float2 *b, int lines, int n, int line_stride, int ns,
 	const float2 *tw, float sign)
@@ -222,77 +221,6 @@ __device__ inline float2 *block_fft(float2 *a, float2 *b, int lines, int line_st
 		ns *= r;
 	}
 	return a;
-}
-
-// The same transform for a power-of-two length N known at compile time:
-// radix 4 while it divides, then one radix 2 (the order make_fft_plan gives),
-// with every index computed by shifts and masks.
-template <int N, int R, int NS>
-__device__ inline void stage_fixed(const float2 *a, float2 *b, int lines, int line_stride, const float2 *tw,
-	float sign)
-{
-	constexpr int m = N / R;
-	constexpr int twiddle_step = N / (NS * R);
-	for (int t = threadIdx.x; t < lines * m; t += blockDim.x)
-	{
-		const int line = t / m;
-		const int j = t % m;
-		const int k = j % NS;
-		const float2 *src = a + line * line_stride;
-		float2 v[R];
-#pragma unroll
-		for (int r = 0; r < R; ++r)
-		{
-			v[r] = src[j + r * m];
-		}
-#pragma unroll
-		for (int r = 1; r < R; ++r)
-		{
-			float2 w = tw[k * r * twiddle_step];
-			w.y *= -sign; // the table holds exp(-2 pi i m / n)
-			v[r] = cmul(v[r], w);
-		}
-		dft<R>(v, sign);
-		const int d = (j / NS) * NS * R + k;
-		float2 *dst = b + line * line_stride;
-#pragma unroll
-		for (int r = 0; r < R; ++r)
-		{
-			dst[d + r * NS] = v[r];
-		}
-	}
-}
-
-template <int N, int NS = 1>
-__device__ inline float2 *block_fft_fixed(float2 *a, float2 *b, int lines, int line_stride, const float2 *tw,
-	float sign)
-{
-	if constexpr (NS >= N)
-	{
-		return a;
-	}
-	else
-	{
-		constexpr int R = (N / NS) % 4 == 0 ? 4 : 2;
-		stage_fixed<N, R, NS>(a, b, lines, line_stride, tw, sign);
-		__syncthreads();
-		return block_fft_fixed<N, NS * R>(b, a, lines, line_stride, tw, sign);
-	}
-}
-
-// The fixed form for N > 0, the planned one otherwise.
-template <int N>
-__device__ inline float2 *transform(float2 *a, float2 *b, int lines, int line_stride, const fft_plan &plan,
-	const float2 *tw, float sign)
-{
-	if constexpr (N > 0)
-	{
-		return block_fft_fixed<N>(a, b, lines, line_stride, tw, sign);
-	}
-	else
-	{
-		return block_fft(a, b, lines, line_stride, plan, tw, sign);
-	}
 }
 
 // The chip's eight XCDs take workgroups in turn (workgroup b runs on XCD

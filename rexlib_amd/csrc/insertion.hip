@@ -20,6 +20,7 @@
 //     This is the GPU form of the reference's tile-owned schedule
 //     (slice_insertion_functor.inl:105-156, 271-465).
 #include "fft_device.hpp"
+#include "fft_two.hpp"
 #include "launch.hpp"
 #include "sample.hpp"
 
@@ -621,16 +622,15 @@ __global__ __launch_bounds__(256) void columns_prepare256_kernel(insertion_param
 
 // The same fusion for the other lengths the FFT kernels take: a block
 // stages `group` columns of the chunk's slices in LDS, transforms them with
-// the Stockham stages (compile-time for N > 0, planned for N = 0), and
-// prepares every element from LDS. The lines are (slice j of the chunk,
+// the Stockham stages, and prepares every element from LDS. The lines are (slice j of the chunk,
 // column), numbered j columns + column, where columns is n/2 for even n
 // (the Nyquist column, never inserted, is skipped) and n/2 + 1 for odd n.
-template <int VARIANT, int N>
+template <int VARIANT>
 __global__ __launch_bounds__(256) void columns_prepare_kernel(insertion_params p, slice_chunk chunk, fft_plan plan,
 	const float2 *tw, int group, prepared_sample *prepared)
 {
 	extern __shared__ float2 lds[];
-	const int n = N > 0 ? N : plan.n;
+	const int n = plan.n;
 	const int stride = n + 1;
 	float2 *a = lds;
 	float2 *b = lds + group * stride;
@@ -674,7 +674,7 @@ __global__ __launch_bounds__(256) void columns_prepare_kernel(insertion_params p
 			}
 		}
 		__syncthreads();
-		const float2 *z = transform<N>(a, b, lines, stride, plan, twl, -1.0f);
+		const float2 *z = block_fft(a, b, lines, stride, plan, twl, -1.0f);
 		for (int t = threadIdx.x; t < group * n; t += blockDim.x)
 		{
 			const int e = t / group;
@@ -690,6 +690,56 @@ __global__ __launch_bounds__(256) void columns_prepare_kernel(insertion_params p
 			}
 		}
 		__syncthreads();
+	}
+}
+
+// The same fusion for lengths of two register factors (fft_two.hpp): a block
+// of (lines, b) threads transforms `lines` neighbouring columns, and their
+// threads prepare the elements from LDS.
+template <int VARIANT, int CLASS>
+__global__ __launch_bounds__(512, two_factor::waves<CLASS>) void columns_prepare_two_kernel(insertion_params p, slice_chunk chunk,
+	two_factor::plan plan, const float2 *tw, prepared_sample *prepared)
+{
+	extern __shared__ float2 lds[];
+	const int l = threadIdx.x;
+	const int j = threadIdx.y;
+	const int n = plan.n;
+	float2 *twl = lds + plan.lines * plan.line;
+	float2 *x = lds + l * plan.line;
+	two_factor::stage_twiddles(plan, twl, tw, j * blockDim.x + l, blockDim.x * blockDim.y);
+	__syncthreads();
+	const int h = p.h;
+	const int columns = n % 2 == 0 ? n / 2 : h;
+	const int64_t elements = static_cast<int64_t>(n) * h;
+	const int64_t total = p.map.kept_count * chunk.count * columns;
+	const int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(plan.lines);
+	if (first >= total)
+	{
+		return;
+	}
+	const int64_t line = first + l;
+	const bool live = line < total;
+	const int64_t jj = live ? line / columns : 0;
+	const int column = static_cast<int>(live ? line - jj * columns : 0);
+	const int64_t kept = jj / chunk.count;
+	const int64_t slice = kept * p.map.reduced_count + chunk.begin + jj % chunk.count;
+	const slice_entry &e = p.entries[slice];
+	const float2 *in = p.slices + e.slice_offset + column * p.slice_s1;
+	two_factor::transform_line<CLASS, false, true>(plan, x, twl, j, -1.0f,
+		[&](int i) { return live ? in[i * p.slice_s0] : make_float2(0.0f, 0.0f); },
+		[&](int k, float2 v) { x[k] = v; });
+	__syncthreads();
+	if (live)
+	{
+		const float2 *table = p.tables + slice * static_cast<int64_t>(h + n);
+		const float2 x_phase = table[column];
+		const float *radial = p.radial + e.radial_offset;
+		prepared_sample *out = prepared + jj * elements + column;
+#pragma unroll 4
+		for (int row = j; row < n; row += blockDim.y)
+		{
+			out[row * h] = prepare_unbranched<VARIANT>(p, e, radial, table + h, x_phase, row, column, x[row]);
+		}
 	}
 }
 
@@ -1680,26 +1730,23 @@ void launch_columns_prepare(const insertion_params &p, slice_chunk chunk, prepar
 	const int n = p.n;
 	const int columns = n % 2 == 0 ? n / 2 : p.h;
 	const int64_t lines = p.map.kept_count * chunk.count * columns;
-	const fft_plan plan = make_fft_plan(n);
 	const float2 *tw = twiddles(n);
+	const two_factor::plan two = two_factor::make_plan(n);
+	if (two.n != 0)
+	{
+		const unsigned blocks = two_factor::blocks_for(lines, two.lines);
+		two_factor::with_class(two, [&](auto kind_class)
+			{
+				columns_prepare_two_kernel<VARIANT, decltype(kind_class)::value><<<blocks, dim3(two.lines, two.b),
+					two_factor::shared_bytes(two), stream>>>(p, chunk, two, tw, prepared);
+			});
+		return;
+	}
+	const fft_plan plan = make_fft_plan(n);
 	const int group = lines_per_group(n);
 	const std::size_t shared = sizeof(float2) * (2 * group * (n + 1) + n) + group * (3 * sizeof(int64_t) + sizeof(int));
 	const unsigned grid = xcd_grid(static_cast<unsigned>(std::min<int64_t>((lines + group - 1) / group, 1 << 20)));
-	switch (n)
-	{
-	case 64:
-		columns_prepare_kernel<VARIANT, 64><<<grid, 256, shared, stream>>>(p, chunk, plan, tw, group, prepared);
-		break;
-	case 128:
-		columns_prepare_kernel<VARIANT, 128><<<grid, 256, shared, stream>>>(p, chunk, plan, tw, group, prepared);
-		break;
-	case 512:
-		columns_prepare_kernel<VARIANT, 512><<<grid, 256, shared, stream>>>(p, chunk, plan, tw, group, prepared);
-		break;
-	default:
-		columns_prepare_kernel<VARIANT, 0><<<grid, 256, shared, stream>>>(p, chunk, plan, tw, group, prepared);
-		break;
-	}
+	columns_prepare_kernel<VARIANT><<<grid, 256, shared, stream>>>(p, chunk, plan, tw, group, prepared);
 }
 
 void dispatch_columns_prepare(const insertion_params &p, slice_chunk chunk, prepared_sample *prepared,
