@@ -202,7 +202,7 @@ __device__ inline void load_reals(const void *base, bool live, int64_t row, int 
 // (middle = image row, outer = image); the output rows follow line set `out`.
 template <int KIND>
 __global__ void rfft_rows_kernel(const void *in, line_set in_rows, int m, const float *scales,
-	int64_t scale_stride, float2 *out, line_set out_rows, fft_plan plan, const float2 *tw, int pairs)
+	int64_t scale_stride, float2 *out, line_set out_rows, fft_plan plan, const float2 *tw, int pairs, float half)
 {
 	extern __shared__ float2 lds[];
 	const int n = plan.n;
@@ -256,12 +256,12 @@ __global__ void rfft_rows_kernel(const void *in, line_set in_rows, int m, const 
 			const int i = t - p * n;
 			const int c = i - offset;
 			float value[2] = {0.0f, 0.0f};
-			for (int half = 0; half < 2; ++half)
+			for (int q = 0; q < 2; ++q)
 			{
-				const int64_t src = row_in[2 * p + half];
+				const int64_t src = row_in[2 * p + q];
 				if (src >= 0 && c >= 0 && c < m)
 				{
-					value[half] = load_real<KIND>(in, src + c * in_rows.s_elem) * row_scale[2 * p + half];
+					value[q] = load_real<KIND>(in, src + c * in_rows.s_elem) * row_scale[2 * p + q];
 				}
 			}
 			a[p * stride + i] = make_float2(value[0], value[1]);
@@ -279,13 +279,13 @@ __global__ void rfft_rows_kernel(const void *in, line_set in_rows, int m, const 
 			if (dst0 >= 0)
 			{
 				const float2 sum = cadd(zk, zm);
-				out[dst0 + k * out_rows.s_elem] = make_float2(0.5f * sum.x, 0.5f * sum.y);
+				out[dst0 + k * out_rows.s_elem] = make_float2(half * sum.x, half * sum.y);
 			}
 			if (dst1 >= 0)
 			{
-				// (zk - zm) / (2 i)
+				// (zk - zm) / (2 i), times the scale
 				const float2 diff = csub(zk, zm);
-				out[dst1 + k * out_rows.s_elem] = make_float2(0.5f * diff.y, -0.5f * diff.x);
+				out[dst1 + k * out_rows.s_elem] = make_float2(half * diff.y, -half * diff.x);
 			}
 		}
 		__syncthreads();
@@ -356,7 +356,7 @@ __global__ void fft_lines_kernel(const float2 *src, line_set src_lines, float2 *
 // image, are zeros, as in rfft_rows_kernel.
 template <int KIND, bool VEC>
 __global__ __launch_bounds__(256) void rfft256_rows_kernel(const void *in, line_set in_rows, int m,
-	const float *scales, int64_t scale_stride, float2 *out, line_set out_rows, const float2 *tw)
+	const float *scales, int64_t scale_stride, float2 *out, line_set out_rows, const float2 *tw, float half)
 {
 	constexpr int n = 256;
 	constexpr int h = n / 2 + 1;
@@ -488,13 +488,13 @@ __global__ __launch_bounds__(256) void rfft256_rows_kernel(const void *in, line_
 				if (dst_a >= 0)
 				{
 					const float2 sum = cadd(zk, zm);
-					out[dst_a + k * out_rows.s_elem] = make_float2(0.5f * sum.x, 0.5f * sum.y);
+					out[dst_a + k * out_rows.s_elem] = make_float2(half * sum.x, half * sum.y);
 				}
 				if (dst_b >= 0)
 				{
-					// (zk - zm) / (2 i)
+					// (zk - zm) / (2 i), times the scale
 					const float2 diff = csub(zk, zm);
-					out[dst_b + k * out_rows.s_elem] = make_float2(0.5f * diff.y, -0.5f * diff.x);
+					out[dst_b + k * out_rows.s_elem] = make_float2(half * diff.y, -half * diff.x);
 				}
 			}
 		}
@@ -595,7 +595,7 @@ __global__ void irfft_rows_kernel(const float2 *src, line_set src_rows, float *d
 // 0.52 ms through the Stockham stages (0.8 GB: 4.0 against 1.6 TB/s).
 template <int KIND, int WIDTH, int CLASS>
 __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void rfft_rows_two_kernel(const void *in, line_set in_rows, int m,
-	const float *scales, int64_t scale_stride, float2 *out, line_set out_rows, two_factor::plan p, const float2 *tw)
+	const float *scales, int64_t scale_stride, float2 *out, line_set out_rows, two_factor::plan p, const float2 *tw, float half)
 {
 	extern __shared__ float2 lds[];
 	const int j = threadIdx.x;
@@ -667,13 +667,13 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void rfft_rows_two_k
 		if (dst[0] >= 0)
 		{
 			const float2 sum = cadd(zk, zm);
-			out[dst[0] + k * out_rows.s_elem] = make_float2(0.5f * sum.x, 0.5f * sum.y);
+			out[dst[0] + k * out_rows.s_elem] = make_float2(half * sum.x, half * sum.y);
 		}
 		if (dst[1] >= 0)
 		{
-			// (zk - zm) / (2 i)
+			// (zk - zm) / (2 i), times the scale
 			const float2 diff = csub(zk, zm);
-			out[dst[1] + k * out_rows.s_elem] = make_float2(0.5f * diff.y, -0.5f * diff.x);
+			out[dst[1] + k * out_rows.s_elem] = make_float2(half * diff.y, -half * diff.x);
 		}
 	}
 }
@@ -843,7 +843,8 @@ static void check_length(int64_t n, bool any_length)
 }
 
 void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, const float *scales,
-	int64_t scale_stride, float2 *out, const line_set &out_rows, int64_t n, hipStream_t stream, bool any_length)
+	int64_t scale_stride, float2 *out, const line_set &out_rows, int64_t n, hipStream_t stream, bool any_length,
+	float scale)
 {
 	check_length(n, any_length);
 	const float2 *tw = twiddles(n);
@@ -854,12 +855,13 @@ void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, 
 		// aligned and contiguous.
 		const std::uintptr_t element = kind == real_f32 ? 4 : 2;
 		const bool aligned = in_rows.s_elem == 1 && m % 4 == 0 && (n / 2 - m / 2) % 4 == 0 &&
-			in_rows.s_outer % 4 == 0 && in_rows.s_middle % 4 == 0 && in_rows.s_inner % 4 == 0 &&
+			in_rows.s_outer % 4 == 0 && (in_rows.middle_count == 1 || in_rows.s_middle % 4 == 0) &&
+			(in_rows.inner_count == 1 || in_rows.s_inner % 4 == 0) &&
 			reinterpret_cast<std::uintptr_t>(in) % (4 * element) == 0;
 		auto launch = [&](auto kind_constant, auto vec_constant)
 		{
 			rfft256_rows_kernel<decltype(kind_constant)::value, decltype(vec_constant)::value>
-				<<<blocks, 256, 0, stream>>>(in, in_rows, m, scales, scale_stride, out, out_rows, tw);
+				<<<blocks, 256, 0, stream>>>(in, in_rows, m, scales, scale_stride, out, out_rows, tw, 0.5f * scale);
 		};
 		using vec = std::true_type;
 		using scalar = std::false_type;
@@ -891,7 +893,8 @@ void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, 
 		const auto runs_of = [&](int64_t width)
 		{
 			return n % width == 0 && in_rows.s_elem == 1 && m % width == 0 && (n / 2 - m / 2) % width == 0 &&
-				in_rows.s_outer % width == 0 && in_rows.s_middle % width == 0 && in_rows.s_inner % width == 0 &&
+				in_rows.s_outer % width == 0 && (in_rows.middle_count == 1 || in_rows.s_middle % width == 0) &&
+				(in_rows.inner_count == 1 || in_rows.s_inner % width == 0) &&
 				reinterpret_cast<std::uintptr_t>(in) % (width * element) == 0;
 		};
 		const int width = runs_of(4) ? 4 : (runs_of(2) ? 2 : 1);
@@ -902,7 +905,7 @@ void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, 
 				{
 					rfft_rows_two_kernel<decltype(kind_constant)::value, decltype(width_constant)::value, CLASS>
 						<<<blocks, dim3(two.b, two.lines), two_factor::shared_bytes(two), stream>>>(in, in_rows, m, scales,
-							scale_stride, out, out_rows, two, tw);
+							scale_stride, out, out_rows, two, tw, 0.5f * scale);
 				};
 				const auto with_width = [&](auto kind_constant)
 				{
@@ -937,7 +940,7 @@ void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, 
 	const auto launch = [&](auto kind_constant)
 	{
 		rfft_rows_kernel<decltype(kind_constant)::value><<<grid, 256, shared, stream>>>(in, in_rows, m, scales,
-			scale_stride, out, out_rows, plan, tw, pairs);
+			scale_stride, out, out_rows, plan, tw, pairs, 0.5f * scale);
 	};
 	switch (kind)
 	{

@@ -4,20 +4,28 @@
 // reference's CPU backend (src/backends/cpu/kernels/pocketfft_fourier_transform.cpp:74-163,
 // src/ops/fourier/fourier_normalization.cpp:56-71).
 //
-// A complex transform between dense operands over axes of 2-3-5 lengths
-// runs its axis passes from the input straight into the output. Otherwise
-// the operand is gathered into a contiguous complex buffer; each axis is
-// then a batch of lines (outer, line, inner) transformed in place by the
-// Stockham kernels (fft.hip) when its length factors into 2, 3 and 5, and by
-// Bluestein's chirp-z algorithm otherwise: x_k w_k, zero-padded to a power
-// of two m >= 2n - 1, convolved with conj(w) by two length-m transforms, then
-// times w_k, with w_k = exp(-+ i pi k^2 / n) computed in double from k^2
-// mod 2n. A real-to-complex transform transforms the real input as complex
-// and keeps the first n/2 + 1 coefficients of its last axis. A
+// Transforms between dense operands run their axis passes from the input
+// straight into the output: complex ones over any axes, real ones whose halved
+// axis is the last one in memory (its rows go two to a complex line). Other
+// operands are gathered into a contiguous complex buffer; each axis is then a
+// batch of lines (outer, line, inner) transformed in place.
+//
+// A line takes the kernels of fft.hip when its length factors into 2, 3 and 5
+// or into two register factors (primes up to 13), and Bluestein's chirp-z
+// algorithm otherwise: x_k w_k, zero-padded to m >= 2n - 1, convolved with
+// conj(w) by two length-m transforms, then times w_k, with w_k = exp(-+ i pi
+// k^2 / n) computed in double from k^2 mod 2n. For n <= 512, m is the
+// shortest two-factor length and one kernel makes all five steps on a line in
+// LDS and registers (bluestein_*); longer lines pass through memory between
+// them, with m a power of two.
+//
+// On the gathered path a real-to-complex transform transforms the real input
+// as complex and keeps the first n/2 + 1 coefficients of its last axis, and a
 // complex-to-real transform runs the inverse over every axis but the last,
 // extends each last-axis line of n/2 + 1 coefficients to n by Hermitian
 // symmetry (the imaginary parts of the self-conjugate coefficients are
 // dropped, as pocketfft's c2r does), transforms it, and keeps the real part.
+#include "fft_two.hpp"
 #include "launch.hpp"
 
 #include <algorithm>
@@ -241,9 +249,29 @@ bool smooth(int64_t n)
 // lengths up to 4096 (96 KiB).
 constexpr int64_t longest_direct = 4096;
 
+// Whether the kernels of fft.hip take a length without Bluestein's algorithm.
+bool direct_length(int64_t n)
+{
+	return (smooth(n) && n <= longest_direct) || two_factor::make_plan(n).n != 0;
+}
+
+// The longest line whose convolution a block holds (1,024 points).
+constexpr int64_t longest_fused = 512;
+
+// The convolution length of a line of n points: the shortest two-factor
+// length for the fused kernels, else a power of two.
 int64_t bluestein_length(int64_t n)
 {
 	int64_t m = 1;
+	if (n <= longest_fused)
+	{
+		m = std::max<int64_t>(48, 2 * n - 1);
+		while (!smooth(m) || two_factor::make_plan(m).n == 0)
+		{
+			++m;
+		}
+		return m;
+	}
 	while (m < 2 * n - 1)
 	{
 		m *= 2;
@@ -259,6 +287,30 @@ __global__ void chirp_values_kernel(int64_t n, float sign, float2 *w)
 	{
 		w[k] = chirp(k, n, sign);
 	}
+}
+
+// B[k] = sum_j b[j] exp(-2 pi i j k / m) of the wrapped conjugate chirp, in
+// double: one thread per coefficient, m <= 1,024 (built once per length).
+__global__ void chirp_spectrum_kernel(int64_t n, int64_t m, float sign, float2 *b)
+{
+	const int64_t k = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+	if (k >= m)
+	{
+		return;
+	}
+	double re = 0.0, im = 0.0;
+	for (int64_t j = 0; j < n; ++j)
+	{
+		double s, c;
+		sincospi(static_cast<double>(j * j % (2 * n)) / static_cast<double>(n), &s, &c);
+		s *= -static_cast<double>(sign);
+		// b[j] = b[m - j]: exp(-i a) + exp(i a) = 2 cos a.
+		const double turn = cospi(2.0 * static_cast<double>(j * k % m) / static_cast<double>(m));
+		const double factor = j == 0 ? 1.0 : 2.0 * turn;
+		re += c * factor;
+		im += s * factor;
+	}
+	b[k] = make_float2(static_cast<float>(re), static_cast<float>(im));
 }
 
 // B = FFT_m(conjugate chirp) in the first m elements, then the chirp w
@@ -278,13 +330,262 @@ const float2 *chirp_spectrum(int64_t n, int64_t m, float sign, hipStream_t strea
 	}
 	float2 *b = nullptr;
 	REXLIB_HIP_CHECK(hipMalloc(&b, sizeof(float2) * static_cast<std::size_t>(m + n)));
-	chirp_table_kernel<<<blocks_for(m), 256, 0, stream>>>(n, m, sign, b);
 	chirp_values_kernel<<<blocks_for(n), 256, 0, stream>>>(n, sign, b + m);
-	const line_set one{1, 1, 1, 0, 0, 0, 1};
-	launch_fft_lines(b, one, b, one, m, -1.0f, 1.0f, stream);
+	if (n <= longest_fused)
+	{
+		chirp_spectrum_kernel<<<static_cast<unsigned>((m + 63) / 64), 64, 0, stream>>>(n, m, sign, b);
+	}
+	else
+	{
+		chirp_table_kernel<<<blocks_for(m), 256, 0, stream>>>(n, m, sign, b);
+		const line_set one{1, 1, 1, 0, 0, 0, 1};
+		launch_fft_lines(b, one, b, one, m, -1.0f, 1.0f, stream);
+	}
 	REXLIB_HIP_CHECK(hipStreamSynchronize(stream));
 	cache[key] = b;
 	return b;
+}
+
+// Bluestein's five steps on the lines of a block (fft_two.hpp's thread
+// layout, m = p.n): `load(i)` gives element i < n, `store(k, X)` takes
+// coefficient k < n, unscaled. `chirps` holds B (m values), then w (n values).
+// The line crosses memory once where the separate steps crossed it seven
+// times, padded (200 images 252^2 there and back: 2.3 ms).
+template <int CLASS, bool LOAD_LDS, bool STORE_LDS, typename Load, typename Store>
+__device__ __forceinline__ void bluestein_line(const two_factor::plan &p, int n, float2 *x, const float2 *tw, int j,
+	const float2 *chirps, Load &&load, Store &&store)
+{
+	const float2 *w = chirps + p.n;
+	two_factor::transform_line<CLASS, LOAD_LDS, true>(p, x, tw, j, -1.0f,
+		[&](int i) { return i < n ? cmul(load(i), w[i]) : make_float2(0.0f, 0.0f); },
+		[&](int k, float2 v) { x[k] = cmul(v, chirps[k]); });
+	__syncthreads();
+	const float inverse = 1.0f / static_cast<float>(p.n);
+	two_factor::transform_line<CLASS, true, STORE_LDS>(p, x, tw, j, 1.0f, [&](int i) { return x[i]; },
+		[&](int k, float2 v)
+		{
+			if (k < n)
+			{
+				store(k, cscale(cmul(v, w[k]), inverse));
+			}
+		});
+}
+
+// Complex lines (as fft_lines_two_kernel).
+template <bool ROWS, int CLASS>
+__global__ __launch_bounds__(512, two_factor::waves<CLASS>) void bluestein_lines_kernel(const float2 *src,
+	line_set src_lines, float2 *dst, line_set dst_lines, int n, two_factor::plan p, const float2 *tw,
+	const float2 *chirps, float scale)
+{
+	extern __shared__ float2 lds[];
+	const int j = ROWS ? threadIdx.x : threadIdx.y;
+	const int l = ROWS ? threadIdx.y : threadIdx.x;
+	float2 *twl = lds + p.lines * p.line;
+	float2 *x = lds + l * p.line;
+	two_factor::stage_twiddles(p, twl, tw, threadIdx.y * blockDim.x + threadIdx.x, blockDim.x * blockDim.y);
+	__syncthreads();
+	const int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(p.lines);
+	if (first >= src_lines.count)
+	{
+		return;
+	}
+	const bool live = first + l < src_lines.count;
+	const float2 *in = src + (live ? line_offset(src_lines, first + l) : 0);
+	float2 *out = dst + (live ? line_offset(dst_lines, first + l) : 0);
+	bluestein_line<CLASS, false, false>(p, n, x, twl, j, chirps,
+		[&](int i) { return live ? in[i * src_lines.s_elem] : make_float2(0.0f, 0.0f); },
+		[&](int k, float2 v)
+		{
+			if (live)
+			{
+				out[k * dst_lines.s_elem] = cscale(v, scale);
+			}
+		});
+}
+
+// Real rows, two to a complex line, to half spectra (as rfft_rows_two_kernel).
+template <int CLASS>
+__global__ __launch_bounds__(512, two_factor::waves<CLASS>) void bluestein_rfft_rows_kernel(const float *src,
+	line_set src_rows, float2 *dst, line_set dst_rows, int n, two_factor::plan p, const float2 *tw,
+	const float2 *chirps, float scale)
+{
+	extern __shared__ float2 lds[];
+	const int j = threadIdx.x;
+	const int l = threadIdx.y;
+	float2 *twl = lds + p.lines * p.line;
+	float2 *x = lds + l * p.line;
+	two_factor::stage_twiddles(p, twl, tw, l * blockDim.x + j, blockDim.x * blockDim.y);
+	__syncthreads();
+	const int64_t row = (xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(p.lines) + l) * 2;
+	if (row - 2 * l >= src_rows.count)
+	{
+		return;
+	}
+	const bool live0 = row < src_rows.count;
+	const bool live1 = row + 1 < src_rows.count;
+	const float *in0 = src + (live0 ? line_offset(src_rows, row) : 0);
+	const float *in1 = src + (live1 ? line_offset(src_rows, row + 1) : 0);
+	bluestein_line<CLASS, false, true>(p, n, x, twl, j, chirps,
+		[&](int i) { return make_float2(live0 ? in0[i * src_rows.s_elem] : 0.0f, live1 ? in1[i * src_rows.s_elem] : 0.0f); },
+		[&](int k, float2 v) { x[k] = v; });
+	__syncthreads();
+	float2 *out0 = dst + (live0 ? line_offset(dst_rows, row) : 0);
+	float2 *out1 = dst + (live1 ? line_offset(dst_rows, row + 1) : 0);
+	const float half = 0.5f * scale;
+	for (int k = j; k < n / 2 + 1; k += blockDim.x)
+	{
+		const float2 zk = x[k];
+		const float2 zm = cconj(x[k == 0 ? 0 : n - k]);
+		if (live0)
+		{
+			out0[k * dst_rows.s_elem] = cscale(cadd(zk, zm), half);
+		}
+		if (live1)
+		{
+			// (zk - zm) / (2 i), times the scale
+			const float2 diff = csub(zk, zm);
+			out1[k * dst_rows.s_elem] = make_float2(half * diff.y, -half * diff.x);
+		}
+	}
+}
+
+// Half-spectrum rows, two at a time, to real rows (as irfft_rows_two_kernel).
+template <int CLASS>
+__global__ __launch_bounds__(512, two_factor::waves<CLASS>) void bluestein_irfft_rows_kernel(const float2 *src,
+	line_set src_rows, float *dst, line_set dst_rows, int n, two_factor::plan p, const float2 *tw,
+	const float2 *chirps, float scale)
+{
+	extern __shared__ float2 lds[];
+	const int j = threadIdx.x;
+	const int l = threadIdx.y;
+	float2 *twl = lds + p.lines * p.line;
+	float2 *x = lds + l * p.line;
+	two_factor::stage_twiddles(p, twl, tw, l * blockDim.x + j, blockDim.x * blockDim.y);
+	const int64_t row = (xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(p.lines) + l) * 2;
+	if (row - 2 * l >= src_rows.count)
+	{
+		return;
+	}
+	const bool live0 = row < src_rows.count;
+	const bool live1 = row + 1 < src_rows.count;
+	const float2 *in0 = src + (live0 ? line_offset(src_rows, row) : 0);
+	const float2 *in1 = src + (live1 ? line_offset(src_rows, row + 1) : 0);
+	for (int k = j; k < n / 2 + 1; k += blockDim.x)
+	{
+		float2 va = live0 ? in0[k * src_rows.s_elem] : make_float2(0.0f, 0.0f);
+		float2 vb = live1 ? in1[k * src_rows.s_elem] : make_float2(0.0f, 0.0f);
+		if (k == 0 || 2 * k == n)
+		{
+			va.y = 0.0f;
+			vb.y = 0.0f;
+		}
+		else
+		{
+			x[n - k] = make_float2(va.x + vb.y, vb.x - va.y);
+		}
+		x[k] = make_float2(va.x - vb.y, va.y + vb.x);
+	}
+	__syncthreads();
+	float *out0 = dst + (live0 ? line_offset(dst_rows, row) : 0);
+	float *out1 = dst + (live1 ? line_offset(dst_rows, row + 1) : 0);
+	bluestein_line<CLASS, true, false>(p, n, x, twl, j, chirps, [&](int i) { return x[i]; },
+		[&](int k, float2 v)
+		{
+			if (live0)
+			{
+				out0[k * dst_rows.s_elem] = v.x * scale;
+			}
+			if (live1)
+			{
+				out1[k * dst_rows.s_elem] = v.y * scale;
+			}
+		});
+}
+
+// Complex lines of any length the general transforms take, from `src` to
+// `dst`; false when they need scratch (transform_axis then).
+bool launch_lines(const float2 *src, const line_set &src_lines, float2 *dst, const line_set &dst_lines, int64_t n,
+	float sign, float scale, hipStream_t stream)
+{
+	if (direct_length(n))
+	{
+		launch_fft_lines(src, src_lines, dst, dst_lines, n, sign, scale, stream, true);
+		return true;
+	}
+	if (n > longest_fused)
+	{
+		return false;
+	}
+	const int64_t m = bluestein_length(n);
+	const two_factor::plan p = two_factor::make_plan(m);
+	const float2 *chirps = chirp_spectrum(n, m, sign, stream);
+	const float2 *tw = twiddles(m);
+	const bool rows = src_lines.s_elem == 1 && dst_lines.s_elem == 1;
+	const unsigned blocks = two_factor::blocks_for(src_lines.count, p.lines);
+	two_factor::with_class(p, [&](auto kind)
+		{
+			constexpr int CLASS = decltype(kind)::value;
+			if (rows)
+			{
+				bluestein_lines_kernel<true, CLASS><<<blocks, dim3(p.b, p.lines), two_factor::shared_bytes(p), stream>>>(
+					src, src_lines, dst, dst_lines, static_cast<int>(n), p, tw, chirps, scale);
+			}
+			else
+			{
+				bluestein_lines_kernel<false, CLASS><<<blocks, dim3(p.lines, p.b), two_factor::shared_bytes(p), stream>>>(
+					src, src_lines, dst, dst_lines, static_cast<int>(n), p, tw, chirps, scale);
+			}
+		});
+	REXLIB_HIP_CHECK(hipGetLastError());
+	return true;
+}
+
+// Whether real rows of n run without scratch, and their launches.
+bool direct_rows(int64_t n)
+{
+	return n > 1 && (direct_length(n) || n <= longest_fused);
+}
+
+void launch_forward_rows(const float *src, const line_set &src_rows, float2 *dst, const line_set &dst_rows, int64_t n,
+	float scale, hipStream_t stream)
+{
+	if (direct_length(n))
+	{
+		launch_rfft_rows(real_f32, src, src_rows, static_cast<int>(n), nullptr, 0, dst, dst_rows, n, stream, true, scale);
+		return;
+	}
+	const int64_t m = bluestein_length(n);
+	const two_factor::plan p = two_factor::make_plan(m);
+	const float2 *chirps = chirp_spectrum(n, m, -1.0f, stream);
+	const float2 *tw = twiddles(m);
+	two_factor::with_class(p, [&](auto kind)
+		{
+			bluestein_rfft_rows_kernel<decltype(kind)::value><<<two_factor::blocks_for(src_rows.count, 2 * p.lines),
+				dim3(p.b, p.lines), two_factor::shared_bytes(p), stream>>>(src, src_rows, dst, dst_rows,
+				static_cast<int>(n), p, tw, chirps, scale);
+		});
+	REXLIB_HIP_CHECK(hipGetLastError());
+}
+
+void launch_inverse_rows(const float2 *src, const line_set &src_rows, float *dst, const line_set &dst_rows, int64_t n,
+	float sign, float scale, hipStream_t stream)
+{
+	if (direct_length(n))
+	{
+		launch_irfft_rows(src, src_rows, dst, dst_rows, n, scale, stream, true);
+		return;
+	}
+	const int64_t m = bluestein_length(n);
+	const two_factor::plan p = two_factor::make_plan(m);
+	const float2 *chirps = chirp_spectrum(n, m, sign, stream);
+	const float2 *tw = twiddles(m);
+	two_factor::with_class(p, [&](auto kind)
+		{
+			bluestein_irfft_rows_kernel<decltype(kind)::value><<<two_factor::blocks_for(src_rows.count, 2 * p.lines),
+				dim3(p.b, p.lines), two_factor::shared_bytes(p), stream>>>(src, src_rows, dst, dst_rows,
+				static_cast<int>(n), p, tw, chirps, scale);
+		});
+	REXLIB_HIP_CHECK(hipGetLastError());
 }
 
 // Lines along `axis` of a contiguous buffer of `extents`.
@@ -315,9 +616,8 @@ void transform_axis(float2 *buffer, const std::vector<int64_t> &extents, int axi
 	{
 		return;
 	}
-	if (smooth(n) && n <= longest_direct)
+	if (launch_lines(buffer, lines, buffer, lines, n, sign, 1.0f, stream))
 	{
-		launch_fft_lines(buffer, lines, buffer, lines, n, sign, 1.0f, stream);
 		return;
 	}
 	const int64_t m = bluestein_length(n);
@@ -354,7 +654,7 @@ int64_t bluestein_elements(const std::vector<int64_t> &extents, const std::vecto
 	for (const int a : axes)
 	{
 		const int64_t n = extents[a];
-		if (n > 1 && !(smooth(n) && n <= longest_direct))
+		if (n > longest_fused && !direct_length(n))
 		{
 			most = std::max(most, count / n * bluestein_length(n));
 		}
@@ -457,50 +757,116 @@ bool dense(const rexlib_hip_array &a)
 	return true;
 }
 
-// A complex transform between dense operands (the same buffer, or buffers
-// that do not overlap) over axes whose lengths factor into 2, 3 and 5: the
-// first axis pass reads the input and writes the output, the later passes
-// run in place on the output, the last one applying the normalisation. No
-// gather, scatter or workspace. Returns false when the operands do not fit.
-bool direct_complex_transform(const rexlib_hip_array *in, const rexlib_hip_array *out, const std::vector<int> &axes,
-	const std::vector<int64_t> &full, float sign, float scale, int64_t count, hipStream_t stream)
+// Whether two dense operands are one buffer, or do not overlap at all.
+bool separate(const void *a, int64_t a_bytes, const void *b, int64_t b_bytes)
 {
-	if (!dense(*in) || !dense(*out))
-	{
-		return false;
-	}
-	const char *a = static_cast<const char *>(in->data);
-	const char *b = static_cast<const char *>(out->data);
-	const int64_t bytes = count * static_cast<int64_t>(sizeof(float2));
-	if (a != b && a < b + bytes && b < a + bytes)
-	{
-		return false;
-	}
-	std::vector<int> live;
+	const char *p = static_cast<const char *>(a);
+	const char *q = static_cast<const char *>(b);
+	return p >= q + b_bytes || q >= p + a_bytes;
+}
+
+// The axes of a transform that are longer than 1, when every one of them but
+// `skipped` runs without scratch; false when one does not.
+bool direct_axes(const std::vector<int> &axes, const std::vector<int64_t> &full, int skipped, std::vector<int> &live)
+{
 	for (const int axis : axes)
 	{
 		const int64_t n = full[axis];
-		if (n > 1)
+		if (axis != skipped && n > 1)
 		{
-			if (!smooth(n) || n > longest_direct)
+			if (!direct_length(n) && n > longest_fused)
 			{
 				return false;
 			}
 			live.push_back(axis);
 		}
 	}
-	if (live.empty())
+	return true;
+}
+
+// A transform between dense operands whose axes run without scratch: no
+// gather, scatter or extension, each axis costs one read and one write. A
+// complex one (the same buffer, or buffers that do not overlap) runs its first
+// pass from the input into the output and the others in place; a real one
+// (buffers that do not overlap) halves the axis that is last in memory: a
+// forward one first, into the output, an inverse one last, from a workspace
+// that holds the passes of the other axes. The last pass applies the scale.
+// Returns false when the operands do not fit.
+bool direct_transform(int kind, const rexlib_hip_array *in, const rexlib_hip_array *out, const std::vector<int> &axes,
+	const std::vector<int64_t> &full, float sign, float scale, int64_t count, hipStream_t stream)
+{
+	if (!dense(*in) || !dense(*out))
 	{
 		return false;
 	}
-	const float2 *src = static_cast<const float2 *>(in->data);
-	float2 *dst = static_cast<float2 *>(out->data);
-	for (std::size_t i = 0; i < live.size(); ++i)
+	const int last = axes.back();
+	std::vector<int> live;
+	if (!direct_axes(axes, full, kind == 0 ? -1 : last, live))
 	{
-		const line_set lines = axis_lines(full, live[i]);
-		launch_fft_lines(i == 0 ? src : dst, lines, dst, lines, full[live[i]], sign,
-			i + 1 == live.size() ? scale : 1.0f, stream);
+		return false;
 	}
+	if (kind == 0)
+	{
+		const int64_t bytes = count * static_cast<int64_t>(sizeof(float2));
+		if (live.empty() || (in->data != out->data && !separate(in->data, bytes, out->data, bytes)))
+		{
+			return false;
+		}
+		const float2 *src = static_cast<const float2 *>(in->data);
+		float2 *dst = static_cast<float2 *>(out->data);
+		for (std::size_t i = 0; i < live.size(); ++i)
+		{
+			const line_set lines = axis_lines(full, live[i]);
+			launch_lines(i == 0 ? src : dst, lines, dst, lines, full[live[i]], sign,
+				i + 1 == live.size() ? scale : 1.0f, stream);
+		}
+		return true;
+	}
+	// Real: the halved axis is the last one in memory.
+	std::vector<int64_t> half = full;
+	half[last] = full[last] / 2 + 1;
+	for (int a = last + 1; a < in->rank; ++a)
+	{
+		if (full[a] != 1)
+		{
+			return false;
+		}
+	}
+	const int64_t n = full[last];
+	const int64_t half_count = count / n * half[last];
+	const int64_t real_bytes = count * static_cast<int64_t>(sizeof(float));
+	const int64_t half_bytes = half_count * static_cast<int64_t>(sizeof(float2));
+	if (!direct_rows(n) || !separate(in->data, kind == 1 ? real_bytes : half_bytes, out->data,
+		kind == 1 ? half_bytes : real_bytes))
+	{
+		return false;
+	}
+	const line_set rows = axis_lines(full, last);
+	const line_set half_rows = axis_lines(half, last);
+	if (kind == 1)
+	{
+		float2 *dst = static_cast<float2 *>(out->data);
+		launch_forward_rows(static_cast<const float *>(in->data), rows, dst, half_rows, n, live.empty() ? scale : 1.0f,
+			stream);
+		for (std::size_t i = 0; i < live.size(); ++i)
+		{
+			const line_set lines = axis_lines(half, live[i]);
+			launch_lines(dst, lines, dst, lines, full[live[i]], sign, i + 1 == live.size() ? scale : 1.0f, stream);
+		}
+		return true;
+	}
+	const float2 *src = static_cast<const float2 *>(in->data);
+	if (!live.empty())
+	{
+		float2 *work = static_cast<float2 *>(workspace_area_bytes(area_fft, static_cast<std::size_t>(half_bytes), stream));
+		for (const int axis : live)
+		{
+			const line_set lines = axis_lines(half, axis);
+			launch_lines(src, lines, work, lines, full[axis], sign, 1.0f, stream);
+			src = work;
+		}
+	}
+	launch_inverse_rows(src, half_rows, static_cast<float *>(out->data), rows, n, sign, scale, stream);
 	return true;
 }
 
@@ -556,7 +922,7 @@ void general_transform(int kind, const rexlib_hip_array *in, const rexlib_hip_ar
 	}
 	const float scale = static_cast<float>(normalisation_factor(normalization, inverse, points));
 	const float sign = inverse ? 1.0f : -1.0f;
-	if (kind == 0 && direct_complex_transform(in, out, axes, full, sign, scale, count, stream))
+	if (direct_transform(kind, in, out, axes, full, sign, scale, count, stream))
 	{
 		REXLIB_HIP_CHECK(hipGetLastError());
 		return;

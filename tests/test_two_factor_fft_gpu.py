@@ -18,13 +18,16 @@ BAR = 2e-6
 # 243 are taken by the other kernels.
 LENGTHS = [47, 48, 49, 64, 65, 99, 121, 125, 143, 162, 169, 200, 225, 243, 250, 256, 260, 286, 300, 320, 441, 484, 512,
            529, 625, 676, 729, 1024]
+# Chirp-z lengths: convolutions of 48 points (the shortest) to 1,024 in one
+# kernel, and one (521) whose steps pass through memory.
+CHIRP_LENGTHS = [7, 17, 37, 101, 127, 251, 383, 509, 511, 521]
 
 
 def rel(a, b):
     return float(np.linalg.norm(a - b) / np.linalg.norm(b))
 
 
-@pytest.mark.parametrize("n", LENGTHS)
+@pytest.mark.parametrize("n", LENGTHS + CHIRP_LENGTHS)
 @pytest.mark.parametrize("count", [1, 17])
 def test_complex_lines_match_numpy(n, count):
     g = torch.Generator().manual_seed(n + count)
@@ -50,6 +53,38 @@ def test_real_images_match_numpy(n):
         assert rel(spectra.cpu().numpy(), ref) <= BAR
         back = rexlib_amd.irfft2(spectra)
         assert rel(back.cpu().numpy(), operand.numpy().astype(np.float64)) <= BAR
+
+
+# Even, odd and prime halved axes; a strided and a batched other axis; an odd
+# number of rows (one left without a partner); every normalisation.
+@pytest.mark.parametrize("shape,axes", [((3, 7, 64), (-1,)), ((5, 252, 60), (-2, -1)), ((1, 101, 127), (-2, -1)),
+                                        ((3, 50, 251), (0, 2)), ((9, 256, 256), (-2, -1)), ((48, 49, 54), (0, 1, 2)),
+                                        ((2, 33, 521), (-2, -1)), ((60, 5, 48), (2, 0)), ((6, 70, 5), (0, 1))])
+@pytest.mark.parametrize("norm", ["backward", "ortho", "forward"])
+def test_real_transforms_over_any_axes_match_numpy(shape, axes, norm):
+    g = torch.Generator().manual_seed(sum(shape))
+    x = torch.randn(shape, generator=g)
+    ref = np.fft.rfftn(x.numpy().astype(np.float64), axes=axes, norm=norm)
+    spectra = fourier.rfftn(x.cuda(), axes=axes, norm=norm)
+    assert rel(spectra.cpu().numpy(), ref) <= BAR
+    sizes = [shape[a] for a in axes]
+    # Imaginary parts of self-conjugate coefficients do not count.
+    noisy = ref + 1j * 0.1 * np.abs(ref).max()
+    expected = np.fft.irfft(
+        np.fft.ifftn(noisy, axes=axes[:-1], norm=norm) if len(axes) > 1 else noisy, n=sizes[-1], axis=axes[-1], norm=norm)
+    got = fourier.irfftn(torch.from_numpy(noisy.astype(np.complex64)).cuda(), s=sizes, axes=axes, norm=norm)
+    assert rel(got.cpu().numpy(), expected) <= BAR
+
+
+def test_overlapping_real_operands_take_the_general_path():
+    # The output starts inside the input's memory.
+    n, count = 60, 7
+    buffer = torch.zeros(count * n + 2 * count * (n // 2 + 1), device="cuda")
+    x = torch.randn((count, n), generator=torch.Generator().manual_seed(1))
+    buffer[:count * n] = x.reshape(-1).cuda()
+    out = torch.view_as_complex(buffer[count * n // 2:count * n // 2 + 2 * count * (n // 2 + 1)].view(-1, 2))
+    fourier.rfftn(buffer[:count * n].view(count, n), axes=(-1,), out=out.view(count, n // 2 + 1))
+    assert rel(out.view(count, -1).cpu().numpy(), np.fft.rfft(x.numpy().astype(np.float64))) <= BAR
 
 
 def test_lengths_of_other_primes_stay_refused():
