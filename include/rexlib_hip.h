@@ -429,6 +429,18 @@ int rexlib_hip_compensation_features(const rexlib_hip_array *denominator, const 
 	double density_scale, const rexlib_hip_array *features,
 	void *stream);
 
+/* scale[0] (device memory, float64) = 1 / mean of the positive values of a
+ * contiguous float32 array, summed in float64; 1 when none is positive. */
+int rexlib_hip_density_scale(const rexlib_hip_array *denominator, double *scale, void *stream);
+
+/* weights (N, N, N/2+1) float32 = exp(MLP(features)) / denominator within the
+ * Nyquist sphere |g| <= N/2 and 1 / denominator beyond it, 0 where the
+ * denominator is not positive: rexlib_hip_compensation_features and
+ * rexlib_hip_mlp_forward in one pass, without the features in memory. */
+int rexlib_hip_predicted_weights(const rexlib_hip_array *denominator, const rexlib_hip_array *table,
+	double density_scale, const rexlib_hip_array *parameters_f16, const rexlib_hip_array *parameters_f32,
+	const rexlib_hip_array *weights, void *stream);
+
 /* The perceptron 10 -> 64 -> 64 -> 64 -> 1 (ReLU) on v_mfma_f32_16x16x16_f16:
  * parameters are rexlib_hip_mlp_parameter_count() elements, row-major
  * W1 (16x64), W2 (64x64), W3 (64x64), W4 (64x16, column 0), b1, b2, b3 (64)

@@ -83,6 +83,8 @@ EXPORTS = [
     "rexlib_hip_density_compensation",
     "rexlib_hip_coverage_table",
     "rexlib_hip_compensation_features",
+    "rexlib_hip_density_scale",
+    "rexlib_hip_predicted_weights",
     "rexlib_hip_mlp_parameter_count",
     "rexlib_hip_mlp_forward",
     "rexlib_hip_mlp_backward",
@@ -145,6 +147,8 @@ def library() -> ctypes.CDLL:
     lib.rexlib_hip_density_compensation.argtypes = [A, ctypes.c_int32, d, A, vp]
     lib.rexlib_hip_coverage_table.argtypes = [A, ctypes.c_int32, A, vp]
     lib.rexlib_hip_compensation_features.argtypes = [A, A, d, A, vp]
+    lib.rexlib_hip_density_scale.argtypes = [A, vp, vp]
+    lib.rexlib_hip_predicted_weights.argtypes = [A, A, d, A, A, A, vp]
     lib.rexlib_hip_mlp_parameter_count.argtypes = []
     lib.rexlib_hip_mlp_forward.argtypes = [A, A, A, A, vp]
     lib.rexlib_hip_mlp_backward.argtypes = [A, A, A, A, A, A, d, vp]

@@ -1010,6 +1010,72 @@ int rexlib_hip_compensation_features(const rexlib_hip_array *denominator, const 
 	});
 }
 
+int rexlib_hip_density_scale(const rexlib_hip_array *denominator, double *scale, void *stream)
+{
+	return guarded([&]
+	{
+		check_array(denominator, "density_scale denominator", 0);
+		expect_dtype(*denominator, REXLIB_HIP_FLOAT32, "density_scale denominator");
+		if (!contiguous(*denominator))
+		{
+			fail(REXLIB_HIP_UNSUPPORTED, "density_scale: a contiguous operand");
+		}
+		if (scale == nullptr)
+		{
+			fail(REXLIB_HIP_INVALID_ARGUMENT, "density_scale: null output");
+		}
+		int64_t count = 1;
+		for (int i = 0; i < denominator->rank; ++i)
+		{
+			count *= denominator->extents[i];
+		}
+		const hipStream_t s = as_stream(stream);
+		double *scratch = static_cast<double *>(workspace_area_bytes(area_compensation,
+			sizeof(double) * static_cast<std::size_t>(rexlib_hip::density_scratch()), s));
+		launch_density_scale(static_cast<const float *>(denominator->data), count, scratch, scale, s);
+	});
+}
+
+int rexlib_hip_predicted_weights(const rexlib_hip_array *denominator, const rexlib_hip_array *table,
+	double density_scale, const rexlib_hip_array *parameters_f16, const rexlib_hip_array *parameters_f32,
+	const rexlib_hip_array *weights, void *stream)
+{
+	return guarded([&]
+	{
+		check_array(denominator, "predicted_weights denominator", 3);
+		check_array(table, "predicted_weights table", 4);
+		check_array(weights, "predicted_weights output", 3);
+		check_array(parameters_f16, "mlp float16 parameters", 1);
+		check_array(parameters_f32, "mlp float32 parameters", 1);
+		expect_dtype(*denominator, REXLIB_HIP_FLOAT32, "predicted_weights denominator");
+		expect_dtype(*table, REXLIB_HIP_FLOAT32, "predicted_weights table");
+		expect_dtype(*weights, REXLIB_HIP_FLOAT32, "predicted_weights output");
+		expect_dtype(*parameters_f16, REXLIB_HIP_FLOAT16, "mlp float16 parameters");
+		expect_dtype(*parameters_f32, REXLIB_HIP_FLOAT32, "mlp float32 parameters");
+		const int64_t big = core_extent(*denominator, 3);
+		expect_core(*denominator, "predicted_weights denominator", {big, big, big / 2 + 1});
+		expect_core(*table, "predicted_weights table", {8, 33, 64, 8});
+		check_same_shape(*denominator, *weights, "predicted_weights output");
+		const int64_t count = rexlib_hip::mlp_parameter_count();
+		if (denominator->rank != 3 || !contiguous(*denominator) || !contiguous(*weights) || !contiguous(*table))
+		{
+			fail(REXLIB_HIP_UNSUPPORTED, "predicted_weights: contiguous operands of one grid");
+		}
+		if (parameters_f16->extents[0] != count || parameters_f32->extents[0] != count || !contiguous(*parameters_f16) ||
+			!contiguous(*parameters_f32))
+		{
+			fail(REXLIB_HIP_INVALID_ARGUMENT, "mlp: parameters hold rexlib_hip_mlp_parameter_count() elements");
+		}
+		if (!(density_scale > 0.0) || !std::isfinite(density_scale))
+		{
+			fail(REXLIB_HIP_INVALID_ARGUMENT, "predicted_weights: the density scale must be finite and positive");
+		}
+		launch_predicted_weights(static_cast<const float *>(denominator->data), static_cast<const float *>(table->data),
+			static_cast<float>(density_scale), parameters_f16->data, static_cast<const float *>(parameters_f32->data),
+			static_cast<float *>(weights->data), static_cast<int>(big), as_stream(stream));
+	});
+}
+
 int32_t rexlib_hip_mlp_parameter_count(void)
 {
 	return rexlib_hip::mlp_parameter_count();

@@ -146,6 +146,12 @@ void launch_coverage(const float *transforms, int64_t slices, int64_t ts0, int64
 	float *table, hipStream_t stream);
 void launch_features(const float *den, const float *table, float density_scale, void *features, int big,
 	hipStream_t stream);
+// scale[0] = 1 / mean of the positive values (1 without any); `scratch` holds
+// density_scratch() doubles.
+void launch_density_scale(const float *den, int64_t count, double *scratch, double *scale, hipStream_t stream);
+int64_t density_scratch();
+void launch_predicted_weights(const float *den, const float *table, float density_scale, const void *params_h,
+	const float *params_f, float *out, int big, hipStream_t stream);
 void launch_mlp_forward(const void *features, const void *params_h, const float *params_f, float *out, int64_t count,
 	hipStream_t stream);
 void launch_mlp_backward(const void *features, const float *target, const void *params_h, const float *params_f,

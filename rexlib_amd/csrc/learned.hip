@@ -14,10 +14,8 @@
 //     products run on v_mfma_f32_16x16x16_f16 with float32 accumulation, in
 //     the forward pass and in the backward pass that trains it.
 //
-// Features of a voxel g: |g| / (N/2); log(1 + den(g)); for each of the 8
-// octants (sx, sy, sz) in {-1, 1}^3, log(1 + the mean of den over the 7
-// neighbours g + (a sx, b sy, c sz), (a, b, c) in {0, 1}^3 \ 0) -- an 8-bin
-// histogram of where the sampling around g lies.
+// Features of a voxel g: |g| / (N/2); log(1 + den(g) * scale); and the 8
+// coverage fractions of its radius and direction (below).
 //
 // The half spectrum is Hermitian: the full-spectrum element (x, y, z) with x
 // beyond the stored half is the element (N - x, -y, -z), and a real field
@@ -66,31 +64,118 @@ __device__ inline bool voxel_of_thread(int big, int half, int &x, int &y, int &z
 	return true;
 }
 
-__global__ __launch_bounds__(256) void compensation_pass_kernel(const float *den, const float *w_in, float *w_out,
-	int big, float floor_value)
+// One pass of the iteration, on P = W den: P <- P / max(K3 * P, floor) where
+// den > 0, else 0. It starts from P = den (W = 1), and the last pass divides by
+// den; the passes between touch P alone. A block takes a tile of `width` x
+// height voxels (x, y), an even share of the row, and walks
+// compensation_planes planes along z: a plane goes to LDS with its halo of
+// one, is convolved there along x and y, and the three z taps come from
+// registers, so a voxel is loaded once per pass and tile (1.4 times with the
+// halo). 27 gathers of W and den per voxel took 166 us a pass at 256^3; this
+// takes 31 us (68 MB of P read and written), bound by the latency of a plane's
+// loads and barrier.
+constexpr int compensation_planes = 16;
+constexpr int compensation_width = 40; // at most
+
+template <bool FIRST, bool LAST>
+__global__ __launch_bounds__(256) void compensation_pass_kernel(const float *den, const float *p_in, float *out,
+	int big, int width, int height, float floor_value)
 {
+	// A plane of the tile with its halo, at most two elements per thread.
+	__shared__ float product[2][512];
 	const int half = big / 2 + 1;
-	const float t[3] = {1.0f / 6.0f, 2.0f / 3.0f, 1.0f / 6.0f};
-	int x, y, z;
-	if (!voxel_of_thread(big, half, x, y, z))
+	const int t = threadIdx.x;
+	const int ty = t / width;
+	const int tx = t - ty * width;
+	const int x0 = blockIdx.x * width;
+	const int y0 = blockIdx.y * height;
+	const int z0 = blockIdx.z * compensation_planes;
+	const int z1 = min(z0 + compensation_planes, big);
+	const int x = x0 + tx;
+	const int y = y0 + ty;
+	const bool live = ty < height && x < half && y < big;
+	const int pitch = width + 2;
+	const int halo = pitch * (height + 2);
+	// This thread's two elements of the tile with the halo. The frequencies
+	// past the stored half mirror (x, y, z): the y index is fixed per thread,
+	// and the z index flips with it.
+	bool held[2];
+	bool mirrored[2];
+	int64_t offset[2];
+#pragma unroll
+	for (int k = 0; k < 2; ++k)
 	{
-		return;
+		const int q = t + 256 * k;
+		const int hy_tile = q / pitch;
+		const int hx = x0 + (q - hy_tile * pitch) - 1;
+		const int hy = y0 + hy_tile - 1;
+		// Tiles that reach past the volume's end need one column and row more.
+		held[k] = q < halo && hx <= half && hy <= big;
+		const int xw = hx < 0 ? hx + big : hx;
+		const int yw = hy < 0 ? hy + big : (hy >= big ? hy - big : hy);
+		mirrored[k] = xw >= half;
+		const int xs = mirrored[k] ? big - xw : xw;
+		const int ys = mirrored[k] && yw != 0 ? big - yw : yw;
+		offset[k] = static_cast<int64_t>(ys) * half + xs;
 	}
-	const int64_t i = (static_cast<int64_t>(z) * big + y) * half + x;
-	float c = 0.0f;
-	for (int dz = -1; dz <= 1; ++dz)
+	const int64_t plane_size = static_cast<int64_t>(big) * half;
+	float staged[2] = {0.0f, 0.0f};
+	const auto load = [&](int z)
 	{
-		for (int dy = -1; dy <= 1; ++dy)
+		const int zw = z < 0 ? z + big : (z >= big ? z - big : z);
+		const int zm = zw == 0 ? 0 : big - zw;
+#pragma unroll
+		for (int k = 0; k < 2; ++k)
 		{
-			for (int dx = -1; dx <= 1; ++dx)
+			if (held[k])
 			{
-				const int64_t j = neighbour_index(x + dx, y + dy, z + dz, big, half);
-				c += t[dz + 1] * t[dy + 1] * t[dx + 1] * w_in[j] * den[j];
+				staged[k] = p_in[(mirrored[k] ? zm : zw) * plane_size + offset[k]];
 			}
 		}
+	};
+	const float side = 1.0f / 6.0f, middle = 2.0f / 3.0f;
+	float below = 0.0f, here = 0.0f, p_here = 0.0f;
+	load(z0 - 1);
+	for (int z = z0 - 1; z <= z1; ++z)
+	{
+		float *plane = product[z & 1];
+		plane[t] = staged[0];
+		plane[t + 256] = staged[1];
+		if (z < z1)
+		{
+			load(z + 1);
+		}
+		const int64_t i = (z - 1) * plane_size + static_cast<int64_t>(y) * half + x;
+		float d = 1.0f;
+		if (LAST && z > z0 && live)
+		{
+			d = den[i];
+		}
+		__syncthreads();
+		float sum = 0.0f;
+		float p = 0.0f;
+		if (live)
+		{
+			const float *row = plane + ty * pitch + tx;
+#pragma unroll
+			for (int dy = 0; dy < 3; ++dy)
+			{
+				sum += (dy == 1 ? middle : side) * (middle * row[1] + side * (row[0] + row[2]));
+				p = dy == 1 ? row[1] : p;
+				row += pitch;
+			}
+		}
+		// `sum` is plane z convolved along x and y; plane z - 1 is complete.
+		if (z > z0 && live)
+		{
+			const float c = middle * here + side * (below + sum);
+			const float next = (FIRST ? p_here > 0.0f : true) ? p_here / fmaxf(c, floor_value) : 0.0f;
+			out[i] = LAST ? (d > 0.0f ? next / d : 0.0f) : next;
+		}
+		below = here;
+		here = sum;
+		p_here = p;
 	}
-	const float w = w_in[i];
-	w_out[i] = den[i] > 0.0f ? w / fmaxf(c, floor_value) : 0.0f;
 }
 
 __global__ void fill_kernel(float *out, int64_t count, float value)
@@ -232,21 +317,19 @@ __global__ __launch_bounds__(256) void coverage_normalize_kernel(float *table)
 	}
 }
 
-// Features of every voxel, as 16 float16 per voxel (the last 6 zero):
-// the shell radius |g| / (N/2), log(1 + den * density_scale) (the local
-// sample count against the mean of the positive weights), and the 8
-// coverage fractions of the table entry nearest to the voxel's radius and
-// direction. The 32 bytes are stored as two 16-byte words.
-__global__ __launch_bounds__(256) void features_kernel(const float *den, const float *table, float density_scale,
-	__half *features, int big)
+// What the features of voxel (x, sy, sz) need: the shell radius |g| / (N/2),
+// log(1 + den * density_scale) (the local sample count against the mean of the
+// positive weights) and the coverage table's entry nearest to the voxel's
+// radius and direction.
+struct voxel_features
 {
-	const int half = big / 2 + 1;
-	int x, sy, sz;
-	if (!voxel_of_thread(big, half, x, sy, sz))
-	{
-		return;
-	}
-	const int64_t i = (static_cast<int64_t>(sz) * big + sy) * half + x;
+	float radius;
+	float density;
+	int entry;
+};
+
+__device__ inline voxel_features features_of(float den, float density_scale, int x, int sy, int sz, int big)
+{
 	// Signed frequencies as numpy's fftfreq: index N/2 is -N/2.
 	const int y = sy < big / 2 ? sy : sy - big;
 	const int z = sz < big / 2 ? sz : sz - big;
@@ -259,17 +342,38 @@ __global__ __launch_bounds__(256) void features_kernel(const float *den, const f
 		return u == 1.0f ? v : __logf(u) * (v / (u - 1.0f));
 	};
 	const float length = sqrtf(static_cast<float>(x * x + y * y + z * z));
-	float f[16];
-	f[0] = length / (0.5f * static_cast<float>(big));
-	f[1] = log1(fmaxf(den[i], 0.0f) * density_scale);
-	const int r = min(coverage_radii - 1, static_cast<int>(f[0] * coverage_radii));
+	voxel_features f;
+	f.radius = length / (0.5f * static_cast<float>(big));
+	f.density = log1(fmaxf(den, 0.0f) * density_scale);
+	const int r = min(coverage_radii - 1, static_cast<int>(f.radius * coverage_radii));
 	const float theta = length > 0.0f ? acosf(fminf(1.0f, fmaxf(-1.0f, static_cast<float>(z) / length))) : 0.0f;
 	float phi = atan2f(static_cast<float>(y), static_cast<float>(x));
 	phi = phi < 0.0f ? phi + 6.28318530717959f : phi;
 	// The nearest grid direction (phi wraps around).
 	const int it = min(coverage_theta - 1, static_cast<int>(theta * ((coverage_theta - 1) / 3.14159265358979f) + 0.5f));
 	const int ip = static_cast<int>(phi * (coverage_phi / 6.28318530717959f) + 0.5f) % coverage_phi;
-	const float *entry = table + (static_cast<int64_t>(r * coverage_theta + it) * coverage_phi + ip) * coverage_bins;
+	f.entry = (r * coverage_theta + it) * coverage_phi + ip;
+	return f;
+}
+
+// Features of every voxel, as 16 float16 per voxel (the last 6 zero):
+// radius, density and the 8 coverage fractions. The 32 bytes are stored as two
+// 16-byte words.
+__global__ __launch_bounds__(256) void features_kernel(const float *den, const float *table, float density_scale,
+	__half *features, int big)
+{
+	const int half = big / 2 + 1;
+	int x, sy, sz;
+	if (!voxel_of_thread(big, half, x, sy, sz))
+	{
+		return;
+	}
+	const int64_t i = (static_cast<int64_t>(sz) * big + sy) * half + x;
+	const voxel_features v = features_of(den[i], density_scale, x, sy, sz, big);
+	float f[16];
+	f[0] = v.radius;
+	f[1] = v.density;
+	const float *entry = table + static_cast<int64_t>(v.entry) * coverage_bins;
 	for (int b = 0; b < coverage_bins; ++b)
 	{
 		f[2 + b] = entry[b];
@@ -458,12 +562,12 @@ struct tile_lds
 
 constexpr int mlp_waves = 4;
 
-// out[i] = MLP(features[i]) for i < count, in transposed form: each layer
-// computes Y^T = W^T X^T on a tile of 16 samples, the 16 columns of the B
-// operand. The weights are the A operands and stay in registers for the
-// whole kernel. An MFMA's output fragment (lane l: rows 4 (l / 16) + j,
-// column l % 16) is laid out as a B operand, so after bias, ReLU and the
-// float16 rounding the activations never leave registers.
+// The perceptron in transposed form: each layer computes Y^T = W^T X^T on a
+// tile of 16 samples, the 16 columns of the B operand. The weights are the A
+// operands and stay in registers for the whole kernel. An MFMA's output
+// fragment (lane l: rows 4 (l / 16) + j, column l % 16) is laid out as a B
+// operand, so after ReLU and the float16 rounding the activations never leave
+// registers.
 // - The first layer (depth 16) takes mfma16: lane l of A holds
 //   W^T[m0 + l % 16][4 (l / 16) + j] = W[4 (l / 16) + j][m0 + l % 16].
 // - The depth-64 layers take mfma32 over two chunks of 32 hidden units. A
@@ -472,11 +576,46 @@ constexpr int mlp_waves = 4;
 //   (j >= 4): its B operand is the two output fragments of m-tiles 2t and
 //   2t + 1 side by side, and its A operand holds the weights of the same
 //   units.
-__global__ __launch_bounds__(256) void mlp_forward_kernel(const __half *features, const _Float16 *params_h,
-	const float *params_f, float *out, int64_t count)
+// The bias is the accumulator a layer starts from, and ReLU runs on pairs of
+// rounded values (max and rounding commute), so that the vector work between
+// layers is one conversion and one maximum per pair; adding the bias and
+// clamping in float32 took three instructions per value and bound the kernel
+// (0.31 ms for the voxels of 256^3; with two tiles in flight 0.22 ms, the
+// features included).
+struct mlp_weights
 {
-	// Biases per (layer, m-tile, lane group): the 4 rows a lane's output holds.
-	__shared__ float4_t bias[3][4][4];
+	half4_t w1[4];
+	half8_t w2[4][2];
+	half8_t w3[4][2];
+	half8_t w4[2];
+	float b4;
+};
+
+// Biases per (layer, m-tile, lane group): the 4 rows a lane's output holds.
+typedef float4_t mlp_biases[3][4][4];
+
+// The float16 weights pass through LDS, 16 bytes a lane: straight from memory
+// the fragments are 160 scattered 2-byte loads per lane.
+__device__ inline void load_mlp(const _Float16 *weights, const float *params_f, mlp_weights &m, mlp_biases &bias)
+{
+	static_assert(off_b1 % 8 == 0, "whole 16-byte words");
+	__shared__ uint4 staged[off_b1 / 8];
+	const bool aligned = reinterpret_cast<uintptr_t>(weights) % 16 == 0;
+	for (int i = threadIdx.x; i < off_b1 / 8; i += blockDim.x)
+	{
+		if (aligned)
+		{
+			staged[i] = reinterpret_cast<const uint4 *>(weights)[i];
+		}
+		else
+		{
+			for (int k = 0; k < 8; ++k)
+			{
+				reinterpret_cast<_Float16 *>(staged)[8 * i + k] = weights[8 * i + k];
+			}
+		}
+	}
+	const _Float16 *params_h = reinterpret_cast<const _Float16 *>(staged);
 	if (threadIdx.x < 48)
 	{
 		const int layer = threadIdx.x / 16;
@@ -489,17 +628,13 @@ __global__ __launch_bounds__(256) void mlp_forward_kernel(const __half *features
 	const int lane = threadIdx.x & 63;
 	const int g = lane >> 4;
 	const int c = lane & 15;
-	half4_t w1[4];
-	half8_t w2[4][2];
-	half8_t w3[4][2];
-	half8_t w4[2];
 #pragma unroll
 	for (int j = 0; j < 4; ++j)
 	{
 #pragma unroll
 		for (int mt = 0; mt < 4; ++mt)
 		{
-			w1[mt][j] = params_h[off_w1 + (4 * g + j) * hidden + mt * 16 + c];
+			m.w1[mt][j] = params_h[off_w1 + (4 * g + j) * hidden + mt * 16 + c];
 		}
 	}
 #pragma unroll
@@ -513,81 +648,266 @@ __global__ __launch_bounds__(256) void mlp_forward_kernel(const __half *features
 #pragma unroll
 			for (int mt = 0; mt < 4; ++mt)
 			{
-				w2[mt][t][j] = params_h[off_w2 + unit * hidden + mt * 16 + c];
-				w3[mt][t][j] = params_h[off_w3 + unit * hidden + mt * 16 + c];
+				m.w2[mt][t][j] = params_h[off_w2 + unit * hidden + mt * 16 + c];
+				m.w3[mt][t][j] = params_h[off_w3 + unit * hidden + mt * 16 + c];
 			}
-			w4[t][j] = params_h[off_w4 + unit * 16 + c];
+			m.w4[t][j] = params_h[off_w4 + unit * 16 + c];
 		}
 	}
-	const float b4 = params_f[off_b4];
-	const int64_t tiles = (count + 15) / 16;
-	const int64_t waves = static_cast<int64_t>(gridDim.x) * (blockDim.x / 64);
-	for (int64_t tile = static_cast<int64_t>(blockIdx.x) * (blockDim.x / 64) + (threadIdx.x >> 6); tile < tiles;
-		tile += waves)
+	m.b4 = params_f[off_b4];
+}
+
+// Rounds to float16 and clamps at 0.
+__device__ inline half4_t relu_half(float4_t v)
+{
+	typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+	const half2_t zero = {0, 0};
+	const half2_t lo = __builtin_elementwise_max(
+		half2_t{static_cast<_Float16>(v[0]), static_cast<_Float16>(v[1])}, zero);
+	const half2_t hi = __builtin_elementwise_max(
+		half2_t{static_cast<_Float16>(v[2]), static_cast<_Float16>(v[3])}, zero);
+	return half4_t{lo[0], lo[1], hi[0], hi[1]};
+}
+
+// The perceptron on TILES tiles at once (independent chains of MFMAs, so that
+// one tile's fill the gaps of another's): lane (g, c) brings features 4 g ..
+// 4 g + 3 of sample c of each; the output of sample c is in lane c (group 0).
+template <int TILES>
+__device__ __forceinline__ void mlp_tiles(const mlp_weights &m, const mlp_biases &bias, int g, const half4_t *x, float *y)
+{
+	half4_t h1[TILES][4];
+	half4_t h2[TILES][4];
+#pragma unroll
+	for (int mt = 0; mt < 4; ++mt)
 	{
-		const int64_t row = tile * 16 + c;
-		// B fragment of X^T: B[4 g + j][c] = X[row][4 g + j], 8 bytes per lane.
-		half4_t x = {0, 0, 0, 0};
-		if (row < count)
+#pragma unroll
+		for (int i = 0; i < TILES; ++i)
 		{
-			x = *reinterpret_cast<const half4_t *>(features + row * inputs + 4 * g);
+			h1[i][mt] = relu_half(mfma16(m.w1[mt], x[i], bias[0][mt][g]));
 		}
-		half4_t h1[4];
-		half4_t h2[4];
+	}
+	const auto layer = [&](const half8_t (&w)[4][2], int number, const half4_t (*in)[4], half4_t (*out)[4])
+	{
 #pragma unroll
 		for (int mt = 0; mt < 4; ++mt)
 		{
-			const float4_t acc = mfma16(w1[mt], x, float4_t{0.0f, 0.0f, 0.0f, 0.0f});
-			const float4_t b = bias[0][mt][g];
+			float4_t acc[TILES];
 #pragma unroll
-			for (int j = 0; j < 4; ++j)
+			for (int i = 0; i < TILES; ++i)
 			{
-				h1[mt][j] = static_cast<_Float16>(fmaxf(acc[j] + b[j], 0.0f));
+				acc[i] = bias[number][mt][g];
 			}
-		}
-#pragma unroll
-		for (int mt = 0; mt < 4; ++mt)
-		{
-			float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
 			for (int t = 0; t < 2; ++t)
 			{
-				acc = mfma32(w2[mt][t], join(h1[2 * t], h1[2 * t + 1]), acc);
-			}
-			const float4_t b = bias[1][mt][g];
 #pragma unroll
-			for (int j = 0; j < 4; ++j)
+				for (int i = 0; i < TILES; ++i)
+				{
+					acc[i] = mfma32(w[mt][t], join(in[i][2 * t], in[i][2 * t + 1]), acc[i]);
+				}
+			}
+#pragma unroll
+			for (int i = 0; i < TILES; ++i)
 			{
-				h2[mt][j] = static_cast<_Float16>(fmaxf(acc[j] + b[j], 0.0f));
+				out[i][mt] = relu_half(acc[i]);
 			}
 		}
+	};
+	layer(m.w2, 1, h1, h2);
+	layer(m.w3, 2, h2, h1);
 #pragma unroll
-		for (int mt = 0; mt < 4; ++mt)
-		{
-			float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-			for (int t = 0; t < 2; ++t)
-			{
-				acc = mfma32(w3[mt][t], join(h2[2 * t], h2[2 * t + 1]), acc);
-			}
-			const float4_t b = bias[2][mt][g];
-#pragma unroll
-			for (int j = 0; j < 4; ++j)
-			{
-				h1[mt][j] = static_cast<_Float16>(fmaxf(acc[j] + b[j], 0.0f)); // layer 3, reusing h1
-			}
-		}
+	for (int i = 0; i < TILES; ++i)
+	{
 		float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
 		for (int t = 0; t < 2; ++t)
 		{
-			acc = mfma32(w4[t], join(h1[2 * t], h1[2 * t + 1]), acc);
+			acc = mfma32(m.w4[t], join(h1[i][2 * t], h1[i][2 * t + 1]), acc);
 		}
 		// Output row 0 (the one used column of W4) sits in lanes 0..15.
-		if (g == 0 && row < count)
+		y[i] = acc[0] + m.b4;
+	}
+}
+
+// out[i] = MLP(features[i]) for i < count.
+__global__ __launch_bounds__(256, 2) void mlp_forward_kernel(const __half *features, const _Float16 *params_h,
+	const float *params_f, float *out, int64_t count)
+{
+	__shared__ mlp_biases bias;
+	mlp_weights m;
+	load_mlp(params_h, params_f, m, bias);
+	const int lane = threadIdx.x & 63;
+	const int g = lane >> 4;
+	const int c = lane & 15;
+	const int64_t pairs = (count + 31) / 32;
+	const int64_t waves = static_cast<int64_t>(gridDim.x) * (blockDim.x / 64);
+	for (int64_t pair = static_cast<int64_t>(blockIdx.x) * (blockDim.x / 64) + (threadIdx.x >> 6); pair < pairs;
+		pair += waves)
+	{
+		const int64_t row = pair * 32 + c;
+		// B fragment of X^T: B[4 g + j][c] = X[row][4 g + j], 8 bytes per lane.
+		half4_t x[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+		for (int i = 0; i < 2; ++i)
 		{
-			out[row] = acc[0] + b4;
+			if (row + 16 * i < count)
+			{
+				x[i] = *reinterpret_cast<const half4_t *>(features + (row + 16 * i) * inputs + 4 * g);
+			}
 		}
+		float y[2];
+		mlp_tiles<2>(m, bias, g, x, y);
+#pragma unroll
+		for (int i = 0; i < 2; ++i)
+		{
+			if (g == 0 && row + 16 * i < count)
+			{
+				out[row + 16 * i] = y[i];
+			}
+		}
+	}
+}
+
+// The predicted weights of a volume in one pass: W = exp(MLP(features)) / den
+// where den > 0 within the Nyquist sphere, 1 / den beyond it, 0 elsewhere. A
+// lane computes the radius, density and table entry of one of 64 voxels of a
+// plane; four tiles of 16 voxels then take theirs by shuffles, the coverage
+// fractions from the table, and hand the outputs back. The features (270 MB at
+// 256^3), the correction and the masks never reach memory.
+__global__ __launch_bounds__(256, 2) void predicted_weights_kernel(const float *den, const float *table,
+	float density_scale, const _Float16 *params_h, const float *params_f, float *out, int big)
+{
+	__shared__ mlp_biases bias;
+	mlp_weights m;
+	load_mlp(params_h, params_f, m, bias);
+	const int lane = threadIdx.x & 63;
+	const int g = lane >> 4;
+	const int c = lane & 15;
+	const int half = big / 2 + 1;
+	const int plane = big * half;
+	const int groups = (plane + 63) / 64; // of 64 voxels per plane
+	const int waves = gridDim.x * (blockDim.x / 64);
+	// (Plane, group) of this wavefront, stepped without a division.
+	const int first = __builtin_amdgcn_readfirstlane(blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6));
+	const int step_planes = waves / groups;
+	const int step_groups = waves - step_planes * groups;
+	int sz = first / groups;
+	int group = first - sz * groups;
+	for (; sz < big; sz += step_planes + (group + step_groups >= groups ? 1 : 0),
+		group += group + step_groups >= groups ? step_groups - groups : step_groups)
+	{
+		const int xy = group * 64 + lane;
+		const bool live = xy < plane;
+		const int sy = live ? xy / half : 0;
+		const int x = live ? xy - sy * half : 0;
+		const int64_t i = static_cast<int64_t>(sz) * plane + (live ? xy : 0);
+		const float d = den[i];
+		const voxel_features f = features_of(d, density_scale, x, sy, sz, big);
+		const half4_t own = {static_cast<_Float16>(f.radius), static_cast<_Float16>(f.density), 0, 0};
+		const int packed = __builtin_bit_cast(int2, own).x;
+		// Features 4 g .. 4 g + 3 of tile t's voxel c: (radius, density, bins 0,
+		// 1), (bins 2 .. 5), (bins 6, 7, 0, 0), zeros. Every lane loads, so the
+		// loads of the four tiles are in flight together. (The table may lie at
+		// any multiple of 4 bytes.)
+		struct __attribute__((packed, aligned(4))) bin_pair
+		{
+			float x, y;
+		};
+		const bin_pair *pairs = reinterpret_cast<const bin_pair *>(table);
+		const int low = g == 0 ? 0 : (g == 1 ? 1 : 3);
+		bin_pair bins[4][2];
+		int head[4];
+#pragma unroll
+		for (int t = 0; t < 4; ++t)
+		{
+			const int entry = __shfl(f.entry, 16 * t + c, 64) * (coverage_bins / 2);
+			head[t] = __shfl(packed, 16 * t + c, 64);
+			bins[t][0] = pairs[entry + low];
+			bins[t][1] = pairs[entry + 2];
+		}
+		half4_t v[4];
+#pragma unroll
+		for (int t = 0; t < 4; ++t)
+		{
+			typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+			const int first = __builtin_bit_cast(int,
+				half2_t{static_cast<_Float16>(bins[t][0].x), static_cast<_Float16>(bins[t][0].y)});
+			const int second = __builtin_bit_cast(int,
+				half2_t{static_cast<_Float16>(bins[t][1].x), static_cast<_Float16>(bins[t][1].y)});
+			const int a = g == 0 ? head[t] : (g == 3 ? 0 : first);
+			const int b = g == 0 ? first : (g == 1 ? second : 0);
+			v[t] = __builtin_bit_cast(half4_t, make_int2(a, b));
+		}
+		float y4[4];
+		mlp_tiles<2>(m, bias, g, v, y4);
+		mlp_tiles<2>(m, bias, g, v + 2, y4 + 2);
+		float correction = 0.0f;
+#pragma unroll
+		for (int t = 0; t < 4; ++t)
+		{
+			const float mine = __shfl(y4[t], c, 64);
+			correction = g == t ? mine : correction;
+		}
+		if (live)
+		{
+			// numpy's fftfreq (of an odd N, index N/2 is +N/2).
+			const int y = sy < (big + 1) / 2 ? sy : sy - big;
+			const int z = sz < (big + 1) / 2 ? sz : sz - big;
+			const int64_t r2 = static_cast<int64_t>(x) * x + static_cast<int64_t>(y) * y + static_cast<int64_t>(z) * z;
+			const bool inside = r2 <= static_cast<int64_t>(big / 2) * (big / 2);
+			out[i] = d > 0.0f ? (inside ? expf(correction) : 1.0f) / d : 0.0f;
+		}
+	}
+}
+
+// Sum and number of the positive weights, one pair per block in double, then
+// scale = 1 / mean (1 without any).
+constexpr int density_blocks = 1024;
+
+__global__ __launch_bounds__(256) void density_sums_kernel(const float *den, int64_t count, double *partial)
+{
+	__shared__ double sums[2][4];
+	double sum = 0.0, positive = 0.0;
+	for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < count; i += gridDim.x * 256ll)
+	{
+		const float d = den[i];
+		sum += d > 0.0f ? static_cast<double>(d) : 0.0;
+		positive += d > 0.0f ? 1.0 : 0.0;
+	}
+	for (int offset = 32; offset > 0; offset /= 2)
+	{
+		sum += __shfl_down(sum, offset, 64);
+		positive += __shfl_down(positive, offset, 64);
+	}
+	if ((threadIdx.x & 63) == 0)
+	{
+		sums[0][threadIdx.x >> 6] = sum;
+		sums[1][threadIdx.x >> 6] = positive;
+	}
+	__syncthreads();
+	if (threadIdx.x < 2)
+	{
+		const double *s = sums[threadIdx.x];
+		partial[2 * blockIdx.x + threadIdx.x] = s[0] + s[1] + s[2] + s[3];
+	}
+}
+
+__global__ __launch_bounds__(64) void density_scale_kernel(const double *partial, int blocks, double *scale)
+{
+	double sum = 0.0, positive = 0.0;
+	for (int b = threadIdx.x; b < blocks; b += 64)
+	{
+		sum += partial[2 * b];
+		positive += partial[2 * b + 1];
+	}
+	for (int offset = 32; offset > 0; offset /= 2)
+	{
+		sum += __shfl_down(sum, offset, 64);
+		positive += __shfl_down(positive, offset, 64);
+	}
+	if (threadIdx.x == 0)
+	{
+		scale[0] = positive > 0.0 ? positive / sum : 1.0;
 	}
 }
 
@@ -816,10 +1136,19 @@ void launch_compensation(const float *den, float *w, float *scratch, int big, in
 	// writes w.
 	float *a = passes % 2 == 0 ? w : scratch;
 	float *b = passes % 2 == 0 ? scratch : w;
-	fill_kernel<<<blocks_of(count, 256), 256, 0, stream>>>(a, count, 1.0f);
+	const int half = big / 2 + 1;
+	const int columns = (half + compensation_width - 1) / compensation_width;
+	const int width = (half + columns - 1) / columns;
+	// As many rows as 256 threads and 512 halo elements take.
+	const int height = std::min(256 / width, 512 / (width + 2) - 2);
+	const dim3 tiles(static_cast<unsigned>(columns), static_cast<unsigned>((big + height - 1) / height),
+		static_cast<unsigned>((big + compensation_planes - 1) / compensation_planes));
 	for (int p = 0; p < passes; ++p)
 	{
-		compensation_pass_kernel<<<volume_grid(big), 256, 0, stream>>>(den, a, b, big, floor_value);
+		const bool first = p == 0, last = p + 1 == passes;
+		const auto kernel = first ? (last ? compensation_pass_kernel<true, true> : compensation_pass_kernel<true, false>) :
+			(last ? compensation_pass_kernel<false, true> : compensation_pass_kernel<false, false>);
+		kernel<<<tiles, 256, 0, stream>>>(den, first ? den : a, b, big, width, height, floor_value);
 		float *t = a;
 		a = b;
 		b = t;
@@ -857,10 +1186,34 @@ void launch_features(const float *den, const float *table, float density_scale, 
 	REXLIB_HIP_CHECK(hipGetLastError());
 }
 
+void launch_density_scale(const float *den, int64_t count, double *scratch, double *scale, hipStream_t stream)
+{
+	const int blocks = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>((count + 255) / 256, density_blocks)));
+	density_sums_kernel<<<blocks, 256, 0, stream>>>(den, count, scratch);
+	density_scale_kernel<<<1, 64, 0, stream>>>(scratch, blocks, scale);
+	REXLIB_HIP_CHECK(hipGetLastError());
+}
+
+int64_t density_scratch()
+{
+	return 2 * density_blocks;
+}
+
+void launch_predicted_weights(const float *den, const float *table, float density_scale, const void *params_h,
+	const float *params_f, float *out, int big, hipStream_t stream)
+{
+	// Two blocks per CU, the registers' limit: each wavefront loads the weights
+	// once for dozens of groups.
+	const int64_t groups = static_cast<int64_t>((big * (big / 2 + 1) + 63) / 64) * big;
+	predicted_weights_kernel<<<blocks_of(std::min<int64_t>(groups, 2048), 4), 256, 0, stream>>>(den, table, density_scale,
+		static_cast<const _Float16 *>(params_h), params_f, out, big);
+	REXLIB_HIP_CHECK(hipGetLastError());
+}
+
 void launch_mlp_forward(const void *features, const void *params_h, const float *params_f, float *out, int64_t count,
 	hipStream_t stream)
 {
-	mlp_forward_kernel<<<blocks_of((count + 15) / 16, 4 * 32), 256, 0, stream>>>(
+	mlp_forward_kernel<<<static_cast<unsigned>(std::min<int64_t>(blocks_of((count + 31) / 32, 4), 512)), 256, 0, stream>>>(
 		static_cast<const __half *>(features), static_cast<const _Float16 *>(params_h), params_f, out, count);
 	REXLIB_HIP_CHECK(hipGetLastError());
 }

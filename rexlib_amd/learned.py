@@ -23,6 +23,7 @@ Reconstruction with weights W: V = gridding_correct(irfft3(numerator * W)).
 """
 from __future__ import annotations
 
+import ctypes
 import math
 import os
 from dataclasses import dataclass
@@ -64,8 +65,9 @@ def coverage_table(transforms: torch.Tensor, big: int) -> torch.Tensor:
 
 def density_scale(den: torch.Tensor) -> float:
     """1 / mean of the positive weights (1 when there are none)."""
-    positive = den[den > 0]
-    return 1.0 / float(positive.mean()) if positive.numel() else 1.0
+    out = torch.empty(1, dtype=torch.float64, device=den.device)
+    N.check(N.library().rexlib_hip_density_scale(N.array(den.contiguous()), ctypes.c_void_p(out.data_ptr()), _stream()))
+    return float(out)
 
 
 def features(den: torch.Tensor, table: torch.Tensor, scale: float | None = None) -> torch.Tensor:
@@ -168,12 +170,10 @@ class CompensationModel:
     def weights(self, den: torch.Tensor, table: torch.Tensor) -> torch.Tensor:
         """Predicted W = exp(correction) / den on the grid of `den` (0 where
         den <= 0; the plain quotient 1 / den beyond the Nyquist sphere)."""
-        f = features(den, table).reshape(-1, FEATURES)
-        correction = self.predict(f).reshape(den.shape)
-        correction = torch.where(inside_nyquist(den.shape[0], den.device), correction, torch.zeros_like(correction))
-        positive = den > 0
-        return torch.where(positive, torch.exp(correction) / torch.where(positive, den, torch.ones_like(den)),
-                           torch.zeros_like(den))
+        out = torch.empty_like(den)
+        N.check(N.library().rexlib_hip_predicted_weights(N.array(den), N.array(table), density_scale(den),
+                                                         N.array(self.f16), N.array(self.f32), N.array(out), _stream()))
+        return out
 
     def save(self, path: str):
         np.savez(path, parameters=self.parameters())
