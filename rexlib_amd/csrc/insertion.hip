@@ -522,101 +522,94 @@ __global__ __launch_bounds__(256) void prepare_kernel(insertion_params p, slice_
 		// and the rejected ones zeroed afterwards.
 		const float2 *table = p.tables + s * static_cast<int64_t>(p.h + p.n);
 		const float2 x = p.slices[e.slice_offset + row * p.slice_s0 + column * p.slice_s1];
-		prepared[j * elements + idx] = prepare_unbranched<VARIANT>(p, e, p.radial + e.radial_offset, table + p.h,
-			table[column], row, column, x);
+		bool read;
+		const prepared_sample sample = prepare_unbranched<VARIANT>(p, e, p.radial + e.radial_offset, table + p.h,
+			table[column], row, column, x, read);
+		if (read)
+		{
+			prepared[j * elements + idx] = sample;
+		}
 	}
 }
 
 // The column transforms of 256-point slices fused with the preparation.
 // The rows of each slice are transformed already (in p.slices, at the
-// slices' own offsets and strides); a block transforms 16 columns k_x of the
-// chunk's slices by the four-step decomposition and writes the prepared
+// slices' own offsets and strides); a block transforms 16 columns k_x of one of
+// the chunk's slices by the four-step decomposition and writes the prepared
 // samples of those columns directly, so the finished spectra never pass
 // through HBM. The Nyquist column k_x = n/2 holds no inserted sample and the
-// brick schedule never reads it, so it is skipped: the lines are (slice j of
-// the chunk, k_x < n/2), numbered j n/2 + k_x, and a block's 16 columns never
-// straddle two slices.
+// brick schedule never reads it, so it is skipped: slice j of the chunk takes
+// 8 blocks, and everything of the slice is uniform over a block (scalar
+// registers; its row phases and radial weights in LDS). It was bound by its
+// vector instructions (99 per sample and a 64-bit division chain per line, 66
+// % of the SIMD cycles: 0.75 ms for 4,096 slices).
 template <int VARIANT>
 __global__ __launch_bounds__(256) void columns_prepare256_kernel(insertion_params p, slice_chunk chunk,
 	const float2 *tw, prepared_sample *prepared)
 {
+	constexpr int n = 256;
+	constexpr int h = n / 2 + 1;
+	constexpr int groups = n / 2 / fft256_lines; // of 16 columns per slice
 	__shared__ float2 exchange[fft256_lines * fft256_line_stride];
-	__shared__ float2 twl[256];
-	__shared__ int64_t line_slice[fft256_lines];
-	__shared__ int64_t line_src[fft256_lines];
-	__shared__ int64_t line_dst[fft256_lines];
-	__shared__ int line_column[fft256_lines];
+	__shared__ float2 twl[n];
+	__shared__ float2 row_phase[n];
+	__shared__ float radial[h];
 	const int t = threadIdx.x;
 	const int l = t & (fft256_lines - 1);
 	const int j = t / fft256_lines; // n1 in the first half of the transform, k1 in the second
-	twl[t] = tw[t];
-	const int h = p.h;
-	const int columns = p.n / 2;
-	const int64_t elements = static_cast<int64_t>(p.n) * h;
-	const int64_t total = p.map.kept_count * chunk.count * columns;
-	for (int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(fft256_lines); first < total;
-		first += static_cast<int64_t>(gridDim.x) * fft256_lines)
+	const unsigned block = xcd_block(blockIdx.x, gridDim.x);
+	const int64_t jj = block / groups;
+	if (jj >= p.map.kept_count * chunk.count)
 	{
-		const int lines = static_cast<int>(total - first < fft256_lines ? total - first : fft256_lines);
-		if (t < fft256_lines)
-		{
-			int64_t slice = 0;
-			int64_t src = 0;
-			int64_t dst = 0;
-			int column = 0;
-			if (t < lines)
-			{
-				const int64_t line = first + t;
-				const int64_t jj = line / columns;
-				column = static_cast<int>(line - jj * columns);
-				const int64_t kept = jj / chunk.count;
-				slice = kept * p.map.reduced_count + chunk.begin + jj % chunk.count;
-				src = p.entries[slice].slice_offset + column * p.slice_s1;
-				dst = jj * elements + column;
-			}
-			line_slice[t] = slice;
-			line_src[t] = src;
-			line_dst[t] = dst;
-			line_column[t] = column;
-		}
-		__syncthreads();
-		const bool live = l < lines;
-		// Elements j + 16 k of the column, by pointer steps.
-		const float2 *in = p.slices + line_src[l] + j * p.slice_s0;
-		const int64_t in_step = 16 * p.slice_s0;
-		float2 v[16];
+		return;
+	}
+	const int column = static_cast<int>(block % groups) * fft256_lines + l;
+	const int64_t kept = p.map.kept_count == 1 ? 0 : jj / chunk.count;
+	const int64_t slice = kept * p.map.reduced_count + chunk.begin + (jj - kept * chunk.count);
+	const slice_entry &e = p.entries[slice];
+	const float2 *table = p.tables + slice * static_cast<int64_t>(h + n);
+	// Elements j + 16 k of the column, by pointer steps.
+	const float2 *in = p.slices + e.slice_offset + column * p.slice_s1 + j * p.slice_s0;
+	const int64_t in_step = 16 * p.slice_s0;
+	float2 v[16];
 #pragma unroll
-		for (int k = 0; k < 16; ++k)
-		{
-			v[k] = live ? in[k * in_step] : make_float2(0.0f, 0.0f);
-		}
-		float2 *x = exchange + l * fft256_line_stride;
-		fft256_four_step(v, x, twl, j, -1.0f);
-		// The outputs go back to LDS (each thread to slots only it reads), so
-		// the preparation loops over them without holding all 16.
-		__syncthreads();
+	for (int k = 0; k < 16; ++k)
+	{
+		v[k] = in[k * in_step];
+	}
+	twl[t] = tw[t];
+	row_phase[t] = table[h + t];
+	if (t < h)
+	{
+		radial[t] = p.radial[e.radial_offset + t * p.radial_s0];
+	}
+	const float2 x_phase = table[column];
+	__syncthreads();
+	float2 *x = exchange + l * fft256_line_stride;
+	fft256_four_step(v, x, twl, j, -1.0f);
+	// The outputs go back to LDS (each thread to slots only it reads), so
+	// the preparation loops over them without holding all 16.
+	__syncthreads();
 #pragma unroll
-		for (int k2 = 0; k2 < 16; ++k2)
-		{
-			x[k2 * 17 + j] = v[k2];
-		}
-		if (live)
-		{
-			const int64_t slice = line_slice[l];
-			const slice_entry &e = p.entries[slice];
-			const int column = line_column[l];
-			const float2 *table = p.tables + slice * static_cast<int64_t>(h + p.n);
-			const float2 x_phase = table[column];
-			const float *radial = p.radial + e.radial_offset;
-			prepared_sample *out = prepared + line_dst[l] + j * h;
+	for (int k2 = 0; k2 < 16; ++k2)
+	{
+		x[k2 * 17 + j] = v[k2];
+	}
+	prepared_sample *out = prepared + jj * static_cast<int64_t>(n * h) + j * h + column;
+	// (The radial weights are in LDS at unit stride, the extent is 256.)
+	insertion_params q = p;
+	q.n = n;
+	q.radial_s0 = 1;
 #pragma unroll 4
-			for (int k2 = 0; k2 < 16; ++k2)
-			{
-				out[k2 * 16 * h] = prepare_unbranched<VARIANT>(p, e, radial, table + h, x_phase, j + 16 * k2, column,
-					x[k2 * 17 + j]);
-			}
+	for (int k2 = 0; k2 < 16; ++k2)
+	{
+		bool read;
+		const prepared_sample sample = prepare_unbranched<VARIANT>(q, e, radial, row_phase, x_phase, j + 16 * k2, column,
+			x[k2 * 17 + j], read);
+		if (read)
+		{
+			out[k2 * 16 * h] = sample;
 		}
-		__syncthreads();
 	}
 }
 
@@ -685,8 +678,13 @@ __global__ __launch_bounds__(256) void columns_prepare_kernel(insertion_params p
 				const slice_entry &entry = p.entries[slice];
 				const float2 *table = p.tables + slice * static_cast<int64_t>(h + n);
 				const int column = line_column[l];
-				prepared[line_dst[l] + static_cast<int64_t>(e) * h] = prepare_unbranched<VARIANT>(p, entry,
-					p.radial + entry.radial_offset, table + h, table[column], e, column, z[l * stride + e]);
+				bool read;
+				const prepared_sample sample = prepare_unbranched<VARIANT>(p, entry, p.radial + entry.radial_offset, table + h,
+					table[column], e, column, z[l * stride + e], read);
+				if (read)
+				{
+					prepared[line_dst[l] + static_cast<int64_t>(e) * h] = sample;
+				}
 			}
 		}
 		__syncthreads();
@@ -738,7 +736,13 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void columns_prepare
 #pragma unroll 4
 		for (int row = j; row < n; row += blockDim.y)
 		{
-			out[row * h] = prepare_unbranched<VARIANT>(p, e, radial, table + h, x_phase, row, column, x[row]);
+			bool read;
+			const prepared_sample sample =
+				prepare_unbranched<VARIANT>(p, e, radial, table + h, x_phase, row, column, x[row], read);
+			if (read)
+			{
+				out[row * h] = sample;
+			}
 		}
 	}
 }
@@ -1768,9 +1772,8 @@ void dispatch_columns_prepare(const insertion_params &p, slice_chunk chunk, prep
 		}
 		return;
 	}
-	const int64_t lines = p.map.kept_count * chunk.count * (p.n / 2);
-	const unsigned grid = xcd_grid(static_cast<unsigned>(
-		std::min<int64_t>((lines + fft256_lines - 1) / fft256_lines, 1 << 20)));
+	// 8 blocks of 16 columns per slice.
+	const unsigned grid = static_cast<unsigned>(p.map.kept_count * chunk.count * 8);
 	const float2 *tw = twiddles(256);
 	switch (p.variant)
 	{

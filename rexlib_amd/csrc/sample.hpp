@@ -253,34 +253,6 @@ __device__ __forceinline__ int wave_inclusive_scan(int v)
 	return v;
 }
 
-// Exclusive starts and wave totals of two per-lane counts (each at least 0).
-// Two 16-bit counts share an int while every count is below 1024 (64 lanes
-// then sum below 2^16), else each takes a scan of its own. Called with every
-// lane of the wavefront active.
-__device__ __forceinline__ void scan_two(int a, int b, int &start_a, int &start_b, int &total_a, int &total_b)
-{
-	if (__ballot(a > 1023 || b > 1023) == 0)
-	{
-		const int v = a | (b << 16);
-		const int inclusive = wave_inclusive_scan(v);
-		const int exclusive = inclusive - v;
-		const int total = __builtin_amdgcn_readlane(inclusive, 63);
-		start_a = exclusive & 0xffff;
-		start_b = exclusive >> 16;
-		total_a = total & 0xffff;
-		total_b = total >> 16;
-	}
-	else
-	{
-		const int inclusive_a = wave_inclusive_scan(a);
-		const int inclusive_b = wave_inclusive_scan(b);
-		start_a = inclusive_a - a;
-		start_b = inclusive_b - b;
-		total_a = __builtin_amdgcn_readlane(inclusive_a, 63);
-		total_b = __builtin_amdgcn_readlane(inclusive_b, 63);
-	}
-}
-
 // Prefix maximum over the 64 lanes (lane i gets the maximum of lanes 0..i),
 // by DPP row shifts within rows of 16 and row broadcasts across them.
 // Lanes without a source read 0 (bound_ctrl), which leaves the result
@@ -302,24 +274,6 @@ __device__ inline float lane_value(float v, int lane)
 	return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
-// Lane i + 1's value by a DPP wavefront shift (wave_shl:1); lane 63 gets 0
-// (bound_ctrl). Called with every lane of the wavefront active.
-__device__ __forceinline__ int next_lane(int v)
-{
-	return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xf, 0xf, true);
-}
-
-// Lane i - 1's value (wave_shr:1); lane 0 gets 0.
-__device__ __forceinline__ int previous_lane(int v)
-{
-	return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, true);
-}
-
-__device__ __forceinline__ float next_lane(float v)
-{
-	return __int_as_float(next_lane(__float_as_int(v)));
-}
-
 // Keeps the compiler from moving LDS accesses across it: the taps of other
 // lanes may alias, which it cannot see.
 __device__ inline void lds_order()
@@ -327,38 +281,47 @@ __device__ inline void lds_order()
 	__asm__ __volatile__("" ::: "memory");
 }
 
+// The shell of an element of a slice of extent n <= 720, from |k|^2 as a float
+// (exact below 2^24): no |k| is closer than 1 / (8 s) to the boundary s + 1/2,
+// 2.4e-4 for the 509 shells of that extent, and the hardware square root with
+// the addition stays within 5e-5. Three instructions; shell_of takes 30 with
+// its rounded square root and four quarter-rate products.
+constexpr int largest_quick_shell = 720;
+
+__device__ inline int quick_shell(float norm)
+{
+	return static_cast<int>(__builtin_amdgcn_sqrtf(norm) + 0.5f);
+}
+
+// The brick schedule reads the elements of a slice with k_x and k_y inside the
+// Nyquist frequency and shell <= last_shell; up to this extent the clipped
+// rows end exactly at the shell ((2 L + 1)^2 < 2^24 and its square root apart
+// from every integer), so the others are not written.
+constexpr int largest_exact_clip = 4095;
+
 // prepare_value without branches, for prepare_kernel and the fused column
 // passes: every load is in bounds whatever the sample (the radial index is
 // clamped to the last shell, the phase tables cover every row and column),
 // and the sample is zeroed afterwards where prepare_value rejects it, so the
 // loads of several elements can be in flight together. The arithmetic is
-// prepare_value's, in the same order. `radial` is the slice's radial
-// weights, `y_table` its row phases.
-// Whether stored element (row, column) of a slice is inserted at all: not on
-// a Nyquist row or column of an even n, within the last shell, and with a
-// nonzero radial weight (row_insertion_kernel.inl:180-220). The same test as
-// prepare_unbranched's, from the geometry alone.
-__device__ inline bool sample_inserted(const insertion_params &p, const slice_entry &e, const float *radial, int row,
-	int column)
-{
-	const int n = p.n;
-	const int ky = row <= n / 2 ? row : row - n;
-	const int shell = shell_of(column, ky);
-	const bool nyquist = (n % 2 == 0) && (row == n / 2 || column == n / 2);
-	const float r = radial[min(shell, max(e.last_shell, 0)) * p.radial_s0];
-	return !nyquist && shell <= e.last_shell && r != 0.0f;
-}
-
+// prepare_value's, in the same order. `radial` is the slice's radial weights,
+// `y_table` its row phases. `read` says whether the brick schedule reads it.
 template <int VARIANT>
 __device__ inline prepared_sample prepare_unbranched(const insertion_params &p, const slice_entry &e,
-	const float *radial, const float2 *y_table, float2 x_phase, int row, int column, float2 x, bool &inserted_out)
+	const float *radial, const float2 *y_table, float2 x_phase, int row, int column, float2 x, bool &read)
 {
 	const int n = p.n;
 	const int ky = row <= n / 2 ? row : row - n;
-	const int shell = shell_of(column, ky);
+	const float fx = static_cast<float>(column);
+	const float fy = static_cast<float>(ky);
+	const float xx = fx * fx;
+	const float yy = fy * fy;
+	const float norm = xx + yy;
+	const int shell = n <= largest_quick_shell ? quick_shell(norm) : shell_of(column, ky);
 	const bool nyquist = (n % 2 == 0) && (row == n / 2 || column == n / 2);
-	const float r = radial[min(shell, max(e.last_shell, 0)) * p.radial_s0];
-	const float2 y_phase = y_table[row];
+	const int clamped = min(shell, max(e.last_shell, 0));
+	const float r = p.radial_s0 == 1 ? radial[static_cast<unsigned>(clamped)] : radial[clamped * p.radial_s0];
+	const float2 y_phase = y_table[static_cast<unsigned>(row)];
 	float numerator_weight = 1.0f;
 	float denominator_weight = 1.0f;
 	if (VARIANT == variant_weighted)
@@ -367,11 +330,6 @@ __device__ inline prepared_sample prepare_unbranched(const insertion_params &p, 
 	}
 	else if (VARIANT == variant_ctf)
 	{
-		const float fx = static_cast<float>(column);
-		const float fy = static_cast<float>(ky);
-		const float xx = fx * fx;
-		const float yy = fy * fy;
-		const float norm = xx + yy;
 		const float chi = e.ctf_radial * norm + e.ctf_axial * (xx - yy) + e.ctf_diagonal * (fx * fy) -
 			static_cast<float>(p.ctf_aberration) * (norm * norm) + e.ctf_phase;
 		numerator_weight = phase_sin(chi);
@@ -379,18 +337,10 @@ __device__ inline prepared_sample prepare_unbranched(const insertion_params &p, 
 	}
 	const float2 v = cmul(cmul(x, x_phase), y_phase);
 	const float scale = r * numerator_weight;
-	const bool inserted = !nyquist && shell <= e.last_shell && r != 0.0f;
-	inserted_out = inserted;
-	return inserted ? prepared_sample{v.x * scale, v.y * scale, r * denominator_weight} :
+	const bool within = !nyquist && shell <= e.last_shell;
+	read = within || n > largest_exact_clip;
+	return within && r != 0.0f ? prepared_sample{v.x * scale, v.y * scale, r * denominator_weight} :
 		prepared_sample{0.0f, 0.0f, 0.0f};
-}
-
-template <int VARIANT>
-__device__ inline prepared_sample prepare_unbranched(const insertion_params &p, const slice_entry &e,
-	const float *radial, const float2 *y_table, float2 x_phase, int row, int column, float2 x)
-{
-	bool inserted;
-	return prepare_unbranched<VARIANT>(p, e, radial, y_table, x_phase, row, column, x, inserted);
 }
 
 } // namespace rexlib_hip
