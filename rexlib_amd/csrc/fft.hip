@@ -198,11 +198,12 @@ __device__ inline void load_reals(const void *base, bool live, int64_t row, int 
 
 // Rows of real images, two at a time, to half spectra. Images of extent m
 // are zero-padded to the transform length n with their origin m/2 moved to
-// n/2. `rows` counts the padded rows, n per image, in line set `in` of images
-// (middle = image row, outer = image); the output rows follow line set `out`.
+// n/2. `total` rows run, `rows` per image: n (the padded rows), or m (the image
+// rows alone, when the caller knows the others to be zero). Line set `in`
+// lists the image rows, `out` the padded rows, n per image.
 template <int KIND>
 __global__ void rfft_rows_kernel(const void *in, line_set in_rows, int m, const float *scales,
-	int64_t scale_stride, float2 *out, line_set out_rows, fft_plan plan, const float2 *tw, int pairs, float half)
+	int64_t scale_stride, float2 *out, line_set out_rows, fft_plan plan, const float2 *tw, int pairs, float half, int rows, int64_t total)
 {
 	extern __shared__ float2 lds[];
 	const int n = plan.n;
@@ -220,7 +221,6 @@ __global__ void rfft_rows_kernel(const void *in, line_set in_rows, int m, const 
 	{
 		twl[i] = tw[i];
 	}
-	const int64_t total = out_rows.count; // padded rows of all images
 	const int offset = n / 2 - m / 2;
 	for (int64_t first = blockIdx.x * static_cast<int64_t>(2 * pairs); first < total;
 		first += static_cast<int64_t>(gridDim.x) * 2 * pairs)
@@ -233,8 +233,8 @@ __global__ void rfft_rows_kernel(const void *in, line_set in_rows, int m, const 
 			float scale = 1.0f;
 			if (row < total)
 			{
-				const int64_t image = row / n;
-				const int r = static_cast<int>(row - image * n) - offset;
+				const int64_t image = row / rows;
+				const int r = static_cast<int>(row - image * rows) - (rows == n ? offset : 0);
 				if (r >= 0 && r < m)
 				{
 					src = line_offset(in_rows, image * m + r);
@@ -243,7 +243,7 @@ __global__ void rfft_rows_kernel(const void *in, line_set in_rows, int m, const 
 						scale = scales[image * scale_stride];
 					}
 				}
-				dst = line_offset(out_rows, row);
+				dst = line_offset(out_rows, image * n + r + offset);
 			}
 			row_in[q] = src;
 			row_out[q] = dst;
@@ -356,7 +356,7 @@ __global__ void fft_lines_kernel(const float2 *src, line_set src_lines, float2 *
 // image, are zeros, as in rfft_rows_kernel.
 template <int KIND, bool VEC>
 __global__ __launch_bounds__(256) void rfft256_rows_kernel(const void *in, line_set in_rows, int m,
-	const float *scales, int64_t scale_stride, float2 *out, line_set out_rows, const float2 *tw, float half)
+	const float *scales, int64_t scale_stride, float2 *out, line_set out_rows, const float2 *tw, float half, int rows, int64_t total)
 {
 	constexpr int n = 256;
 	constexpr int h = n / 2 + 1;
@@ -369,7 +369,6 @@ __global__ __launch_bounds__(256) void rfft256_rows_kernel(const void *in, line_
 	const int j = t & 15;
 	const int l = t >> 4;
 	twl[t] = tw[t];
-	const int64_t total = out_rows.count; // padded rows of all images
 	const int offset = n / 2 - m / 2;
 	for (int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(2 * fft256_lines); first < total;
 		first += static_cast<int64_t>(gridDim.x) * 2 * fft256_lines)
@@ -382,8 +381,8 @@ __global__ __launch_bounds__(256) void rfft256_rows_kernel(const void *in, line_
 			float scale = 1.0f;
 			if (row < total)
 			{
-				const int64_t image = row / n;
-				const int r = static_cast<int>(row - image * n) - offset;
+				const int64_t image = row / rows;
+				const int r = static_cast<int>(row - image * rows) - (rows == n ? offset : 0);
 				if (r >= 0 && r < m)
 				{
 					src = line_offset(in_rows, image * m + r);
@@ -392,7 +391,7 @@ __global__ __launch_bounds__(256) void rfft256_rows_kernel(const void *in, line_
 						scale = scales[image * scale_stride];
 					}
 				}
-				dst = line_offset(out_rows, row);
+				dst = line_offset(out_rows, image * n + r + offset);
 			}
 			row_in[t] = src;
 			row_out[t] = dst;
@@ -595,7 +594,7 @@ __global__ void irfft_rows_kernel(const float2 *src, line_set src_rows, float *d
 // 0.52 ms through the Stockham stages (0.8 GB: 4.0 against 1.6 TB/s).
 template <int KIND, int WIDTH, int CLASS>
 __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void rfft_rows_two_kernel(const void *in, line_set in_rows, int m,
-	const float *scales, int64_t scale_stride, float2 *out, line_set out_rows, two_factor::plan p, const float2 *tw, float half)
+	const float *scales, int64_t scale_stride, float2 *out, line_set out_rows, two_factor::plan p, const float2 *tw, float half, int rows, int64_t total)
 {
 	extern __shared__ float2 lds[];
 	const int j = threadIdx.x;
@@ -606,7 +605,6 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void rfft_rows_two_k
 	float2 *twl = lds + p.lines * p.line;
 	float2 *x = lds + l * p.line;
 	two_factor::stage_twiddles(p, twl, tw, l * threads + j, threads * blockDim.y);
-	const int64_t total = out_rows.count; // padded rows of all images
 	const int offset = n / 2 - m / 2;
 	// One group of lines per block: a loop over groups would hoist the
 	// twiddles of every register length out of it, into registers.
@@ -628,8 +626,8 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void rfft_rows_two_k
 		scale[q] = 1.0f;
 		if (row < total)
 		{
-			const int64_t image = row / n;
-			const int r = static_cast<int>(row - image * n) - offset;
+			const int64_t image = row / rows;
+			const int r = static_cast<int>(row - image * rows) - (rows == n ? offset : 0);
 			if (r >= 0 && r < m)
 			{
 				src[q] = line_offset(in_rows, image * m + r);
@@ -638,7 +636,7 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void rfft_rows_two_k
 					scale[q] = scales[image * scale_stride];
 				}
 			}
-			dst[q] = line_offset(out_rows, row);
+			dst[q] = line_offset(out_rows, image * n + r + offset);
 		}
 	}
 	// Loads of WIDTH elements, two steps of both rows in flight.
@@ -844,13 +842,15 @@ static void check_length(int64_t n, bool any_length)
 
 void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, const float *scales,
 	int64_t scale_stride, float2 *out, const line_set &out_rows, int64_t n, hipStream_t stream, bool any_length,
-	float scale)
+	float scale, bool image_rows)
 {
+	const int rows = static_cast<int>(image_rows ? m : n);
+	const int64_t total = image_rows ? out_rows.count / n * m : out_rows.count;
 	check_length(n, any_length);
 	const float2 *tw = twiddles(n);
 	if (n == 256)
 	{
-		const unsigned blocks = xcd_grid(grid_for(out_rows.count, 2 * fft256_lines));
+		const unsigned blocks = xcd_grid(grid_for(total, 2 * fft256_lines));
 		// Rows take loads of 4 elements when every run of 4 elements is
 		// aligned and contiguous.
 		const std::uintptr_t element = kind == real_f32 ? 4 : 2;
@@ -861,7 +861,8 @@ void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, 
 		auto launch = [&](auto kind_constant, auto vec_constant)
 		{
 			rfft256_rows_kernel<decltype(kind_constant)::value, decltype(vec_constant)::value>
-				<<<blocks, 256, 0, stream>>>(in, in_rows, m, scales, scale_stride, out, out_rows, tw, 0.5f * scale);
+				<<<blocks, 256, 0, stream>>>(in, in_rows, m, scales, scale_stride, out, out_rows, tw, 0.5f * scale,
+					rows, total);
 		};
 		using vec = std::true_type;
 		using scalar = std::false_type;
@@ -886,7 +887,7 @@ void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, 
 	const two_factor::plan two = two_factor::make_plan(n);
 	if (two.n != 0)
 	{
-		const unsigned blocks = two_factor::blocks_for(out_rows.count, 2 * two.lines);
+		const unsigned blocks = two_factor::blocks_for(total, 2 * two.lines);
 		// Rows take loads of 4 (or 2) elements when every run of them is
 		// aligned and contiguous.
 		const std::uintptr_t element = kind == real_f32 ? 4 : 2;
@@ -905,7 +906,7 @@ void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, 
 				{
 					rfft_rows_two_kernel<decltype(kind_constant)::value, decltype(width_constant)::value, CLASS>
 						<<<blocks, dim3(two.b, two.lines), two_factor::shared_bytes(two), stream>>>(in, in_rows, m, scales,
-							scale_stride, out, out_rows, two, tw, 0.5f * scale);
+							scale_stride, out, out_rows, two, tw, 0.5f * scale, rows, total);
 				};
 				const auto with_width = [&](auto kind_constant)
 				{
@@ -936,11 +937,11 @@ void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, 
 	const int pairs = std::max(1, lines_per_group(static_cast<int>(n)) / 2);
 	// Two buffers, the twiddles, then per row two offsets and a scale.
 	const std::size_t shared = sizeof(float2) * (2 * pairs * (n + 1) + n) + 2 * pairs * (2 * sizeof(int64_t) + 4);
-	const unsigned grid = grid_for(out_rows.count, 2 * pairs);
+	const unsigned grid = grid_for(total, 2 * pairs);
 	const auto launch = [&](auto kind_constant)
 	{
 		rfft_rows_kernel<decltype(kind_constant)::value><<<grid, 256, shared, stream>>>(in, in_rows, m, scales,
-			scale_stride, out, out_rows, plan, tw, pairs, 0.5f * scale);
+			scale_stride, out, out_rows, plan, tw, pairs, 0.5f * scale, rows, total);
 	};
 	switch (kind)
 	{

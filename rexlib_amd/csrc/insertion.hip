@@ -46,8 +46,9 @@ constexpr double pi_d = 3.14159265358979323846;
 // Settle: one block per slice.
 // ---------------------------------------------------------------------------
 
-__global__ void settle_kernel(insertion_params p)
+__global__ __launch_bounds__(128) void settle_kernel(insertion_params p)
 {
+	__shared__ int last_shells[2];
 	const int n = p.n;
 	const int h = p.h;
 	for (int64_t s = blockIdx.x; s < p.slice_count; s += gridDim.x)
@@ -67,6 +68,25 @@ __global__ void settle_kernel(insertion_params p)
 		const double centre = static_cast<double>(n / 2);
 		const int64_t radial_offset = offset(slot_radial);
 
+		// The last shell with a weight: the threads scan the shells side by side
+		// (one thread after another through 129 loads took 20 us of a call).
+		const float *radial = p.radial + radial_offset;
+		int found = -1;
+		for (int shell = threadIdx.x; shell < h; shell += blockDim.x)
+		{
+			found = radial[shell * p.radial_s0] != 0.0f ? shell : found;
+		}
+		for (int offset_lanes = 32; offset_lanes > 0; offset_lanes /= 2)
+		{
+			found = max(found, __shfl_xor(found, offset_lanes, 64));
+		}
+		__syncthreads(); // the previous slice's value is read
+		if ((threadIdx.x & 63) == 0)
+		{
+			last_shells[threadIdx.x >> 6] = found;
+		}
+		__syncthreads();
+
 		if (threadIdx.x == 0)
 		{
 			slice_entry e;
@@ -79,15 +99,7 @@ __global__ void settle_kernel(insertion_params p)
 				e.x_step[a] = static_cast<float>(xs);
 				e.y_step[a] = ys;
 			}
-			int last = -1;
-			const float *radial = p.radial + radial_offset;
-			for (int shell = 0; shell < h; ++shell)
-			{
-				if (radial[shell * p.radial_s0] != 0.0f)
-				{
-					last = shell;
-				}
-			}
+			const int last = max(last_shells[0], last_shells[1]);
 			// A non-finite frame bounds no rows (src/backends/cpu/kernels/row_interval.cpp).
 			e.last_shell = finite ? last : -1;
 			e.ctf_radial = e.ctf_axial = e.ctf_diagonal = e.ctf_phase = 0.0f;
@@ -129,10 +141,10 @@ __global__ void settle_kernel(insertion_params p)
 		}
 
 		// Shift phases exp(2 pi i k (c + t) / n) (axis_phase.inl:14-36), in
-		// double, rounded to float.
+		// double (angles in units of pi), rounded to float.
 		float2 *table = p.tables + s * static_cast<int64_t>(h + n);
-		const double x_scale = 2.0 * pi_d * (centre + at(0, 3)) / static_cast<double>(n);
-		const double y_scale = 2.0 * pi_d * (centre + at(1, 3)) / static_cast<double>(n);
+		const double x_scale = 2.0 * (centre + at(0, 3)) / static_cast<double>(n);
+		const double y_scale = 2.0 * (centre + at(1, 3)) / static_cast<double>(n);
 		for (int j = threadIdx.x; j < h + n; j += blockDim.x)
 		{
 			double angle;
@@ -147,7 +159,7 @@ __global__ void settle_kernel(insertion_params p)
 				angle = y_scale * static_cast<double>(f);
 			}
 			double sn, cs;
-			sincos(angle, &sn, &cs);
+			sincospi(angle, &sn, &cs);
 			table[j] = make_float2(static_cast<float>(cs), static_cast<float>(sn));
 		}
 	}
@@ -532,6 +544,15 @@ __global__ __launch_bounds__(256) void prepare_kernel(insertion_params p, slice_
 	}
 }
 
+// The rows [begin, end) of row-transformed slices that may hold other values
+// than zero (the image rows of a padded slice); the column passes read only
+// these.
+struct row_range
+{
+	int begin;
+	int end;
+};
+
 // The column transforms of 256-point slices fused with the preparation.
 // The rows of each slice are transformed already (in p.slices, at the
 // slices' own offsets and strides); a block transforms 16 columns k_x of one of
@@ -545,7 +566,7 @@ __global__ __launch_bounds__(256) void prepare_kernel(insertion_params p, slice_
 // % of the SIMD cycles: 0.75 ms for 4,096 slices).
 template <int VARIANT>
 __global__ __launch_bounds__(256) void columns_prepare256_kernel(insertion_params p, slice_chunk chunk,
-	const float2 *tw, prepared_sample *prepared)
+	row_range held, const float2 *tw, prepared_sample *prepared)
 {
 	constexpr int n = 256;
 	constexpr int h = n / 2 + 1;
@@ -575,7 +596,8 @@ __global__ __launch_bounds__(256) void columns_prepare256_kernel(insertion_param
 #pragma unroll
 	for (int k = 0; k < 16; ++k)
 	{
-		v[k] = in[k * in_step];
+		const int row = j + 16 * k;
+		v[k] = row >= held.begin && row < held.end ? in[k * in_step] : make_float2(0.0f, 0.0f);
 	}
 	twl[t] = tw[t];
 	row_phase[t] = table[h + t];
@@ -619,7 +641,7 @@ __global__ __launch_bounds__(256) void columns_prepare256_kernel(insertion_param
 // column), numbered j columns + column, where columns is n/2 for even n
 // (the Nyquist column, never inserted, is skipped) and n/2 + 1 for odd n.
 template <int VARIANT>
-__global__ __launch_bounds__(256) void columns_prepare_kernel(insertion_params p, slice_chunk chunk, fft_plan plan,
+__global__ __launch_bounds__(256) void columns_prepare_kernel(insertion_params p, slice_chunk chunk, row_range held, fft_plan plan,
 	const float2 *tw, int group, prepared_sample *prepared)
 {
 	extern __shared__ float2 lds[];
@@ -663,7 +685,8 @@ __global__ __launch_bounds__(256) void columns_prepare_kernel(insertion_params p
 			const int l = t - e * group;
 			if (l < lines)
 			{
-				a[l * stride + e] = p.slices[line_src[l] + e * p.slice_s0];
+				a[l * stride + e] = e >= held.begin && e < held.end ? p.slices[line_src[l] + e * p.slice_s0] :
+					make_float2(0.0f, 0.0f);
 			}
 		}
 		__syncthreads();
@@ -696,7 +719,7 @@ __global__ __launch_bounds__(256) void columns_prepare_kernel(insertion_params p
 // threads prepare the elements from LDS.
 template <int VARIANT, int CLASS>
 __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void columns_prepare_two_kernel(insertion_params p, slice_chunk chunk,
-	two_factor::plan plan, const float2 *tw, prepared_sample *prepared)
+	row_range held, two_factor::plan plan, const float2 *tw, prepared_sample *prepared)
 {
 	extern __shared__ float2 lds[];
 	const int l = threadIdx.x;
@@ -724,7 +747,7 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void columns_prepare
 	const slice_entry &e = p.entries[slice];
 	const float2 *in = p.slices + e.slice_offset + column * p.slice_s1;
 	two_factor::transform_line<CLASS, false, true>(plan, x, twl, j, -1.0f,
-		[&](int i) { return live ? in[i * p.slice_s0] : make_float2(0.0f, 0.0f); },
+		[&](int i) { return live && i >= held.begin && i < held.end ? in[i * p.slice_s0] : make_float2(0.0f, 0.0f); },
 		[&](int k, float2 v) { x[k] = v; });
 	__syncthreads();
 	if (live)
@@ -1728,7 +1751,7 @@ void dispatch_prepare(const insertion_params &p, slice_chunk chunk, prepared_sam
 }
 
 template <int VARIANT>
-void launch_columns_prepare(const insertion_params &p, slice_chunk chunk, prepared_sample *prepared,
+void launch_columns_prepare(const insertion_params &p, slice_chunk chunk, row_range held, prepared_sample *prepared,
 	hipStream_t stream)
 {
 	const int n = p.n;
@@ -1742,7 +1765,7 @@ void launch_columns_prepare(const insertion_params &p, slice_chunk chunk, prepar
 		two_factor::with_class(two, [&](auto kind_class)
 			{
 				columns_prepare_two_kernel<VARIANT, decltype(kind_class)::value><<<blocks, dim3(two.lines, two.b),
-					two_factor::shared_bytes(two), stream>>>(p, chunk, two, tw, prepared);
+					two_factor::shared_bytes(two), stream>>>(p, chunk, held, two, tw, prepared);
 			});
 		return;
 	}
@@ -1750,10 +1773,10 @@ void launch_columns_prepare(const insertion_params &p, slice_chunk chunk, prepar
 	const int group = lines_per_group(n);
 	const std::size_t shared = sizeof(float2) * (2 * group * (n + 1) + n) + group * (3 * sizeof(int64_t) + sizeof(int));
 	const unsigned grid = xcd_grid(static_cast<unsigned>(std::min<int64_t>((lines + group - 1) / group, 1 << 20)));
-	columns_prepare_kernel<VARIANT><<<grid, 256, shared, stream>>>(p, chunk, plan, tw, group, prepared);
+	columns_prepare_kernel<VARIANT><<<grid, 256, shared, stream>>>(p, chunk, held, plan, tw, group, prepared);
 }
 
-void dispatch_columns_prepare(const insertion_params &p, slice_chunk chunk, prepared_sample *prepared,
+void dispatch_columns_prepare(const insertion_params &p, slice_chunk chunk, row_range held, prepared_sample *prepared,
 	hipStream_t stream)
 {
 	if (p.n != 256)
@@ -1761,13 +1784,13 @@ void dispatch_columns_prepare(const insertion_params &p, slice_chunk chunk, prep
 		switch (p.variant)
 		{
 		case variant_plain:
-			launch_columns_prepare<variant_plain>(p, chunk, prepared, stream);
+			launch_columns_prepare<variant_plain>(p, chunk, held, prepared, stream);
 			break;
 		case variant_weighted:
-			launch_columns_prepare<variant_weighted>(p, chunk, prepared, stream);
+			launch_columns_prepare<variant_weighted>(p, chunk, held, prepared, stream);
 			break;
 		default:
-			launch_columns_prepare<variant_ctf>(p, chunk, prepared, stream);
+			launch_columns_prepare<variant_ctf>(p, chunk, held, prepared, stream);
 			break;
 		}
 		return;
@@ -1778,13 +1801,13 @@ void dispatch_columns_prepare(const insertion_params &p, slice_chunk chunk, prep
 	switch (p.variant)
 	{
 	case variant_plain:
-		columns_prepare256_kernel<variant_plain><<<grid, 256, 0, stream>>>(p, chunk, tw, prepared);
+		columns_prepare256_kernel<variant_plain><<<grid, 256, 0, stream>>>(p, chunk, held, tw, prepared);
 		break;
 	case variant_weighted:
-		columns_prepare256_kernel<variant_weighted><<<grid, 256, 0, stream>>>(p, chunk, tw, prepared);
+		columns_prepare256_kernel<variant_weighted><<<grid, 256, 0, stream>>>(p, chunk, held, tw, prepared);
 		break;
 	default:
-		columns_prepare256_kernel<variant_ctf><<<grid, 256, 0, stream>>>(p, chunk, tw, prepared);
+		columns_prepare256_kernel<variant_ctf><<<grid, 256, 0, stream>>>(p, chunk, held, tw, prepared);
 		break;
 	}
 }
@@ -2027,8 +2050,10 @@ void clear_insertion_tuning()
 	tuning_table.clear();
 }
 
-// The row transforms of images [first, last) of a pending image insertion.
-void launch_rows(const pending_columns &columns, int64_t first, int64_t last, hipStream_t stream)
+// The row transforms of images [first, last) of a pending image insertion;
+// `image_rows`: the zero rows of the padding are left out (the column pass
+// that follows does not read them).
+void launch_rows(const pending_columns &columns, int64_t first, int64_t last, bool image_rows, hipStream_t stream)
 {
 	const pending_rows &rows = *columns.rows;
 	if (last <= first)
@@ -2043,7 +2068,7 @@ void launch_rows(const pending_columns &columns, int64_t first, int64_t last, hi
 		first * rows.in_rows.s_outer * static_cast<int64_t>(rows.element_bytes);
 	const float *scales = rows.scales != nullptr ? rows.scales + first * rows.scale_stride : nullptr;
 	launch_rfft_rows(rows.kind, images, in, rows.m, scales, rows.scale_stride,
-		columns.spectra + first * rows.out_rows.s_outer, out, rows.n, stream);
+		columns.spectra + first * rows.out_rows.s_outer, out, rows.n, stream, false, 1.0f, image_rows);
 }
 
 // Host entry of every insertion: fills the workspace and launches.
@@ -2154,7 +2179,7 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 	const bool chunk_rows = fused_columns && columns->rows != nullptr && p.map.kept_count == 1;
 	if (columns != nullptr && columns->rows != nullptr && !chunk_rows)
 	{
-		launch_rows(*columns, 0, columns->rows->in_rows.count / columns->rows->m, stream);
+		launch_rows(*columns, 0, columns->rows->in_rows.count / columns->rows->m, fused_columns, stream);
 	}
 	if (columns != nullptr && !fused_columns && columns->lines.count > 0)
 	{
@@ -2166,6 +2191,9 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 
 	if (brick)
 	{
+		// The rows of the slices that hold image rows; the others are zero.
+		const row_range held = columns != nullptr && columns->rows != nullptr ?
+			row_range{n / 2 - columns->rows->m / 2, n / 2 - columns->rows->m / 2 + columns->rows->m} : row_range{0, n};
 		int count = 0;
 		int split = 0; // tasks of split bricks, the first ones
 		const int4 *tasks = brick_tasks(p.big, chunk_count, tuning, layout_taps, voxels, workspace, stream, count, split);
@@ -2176,12 +2204,12 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 			const slice_chunk chunk{begin, std::min(chunk_count, p.map.reduced_count - begin)};
 			if (chunk_rows)
 			{
-				launch_rows(*columns, chunk.begin, chunk.begin + chunk.count, stream);
+				launch_rows(*columns, chunk.begin, chunk.begin + chunk.count, true, stream);
 			}
 			const int prepare_token = timing_begin(REXLIB_HIP_KERNEL_PREPARE, stream);
 			if (fused_columns)
 			{
-				dispatch_columns_prepare(p, chunk, prepared, stream);
+				dispatch_columns_prepare(p, chunk, held, prepared, stream);
 			}
 			else
 			{

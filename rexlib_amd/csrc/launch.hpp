@@ -120,10 +120,11 @@ void timing_end(int token, hipStream_t stream);
 void kernel_timing(int kernel, double *total_ms, int64_t *launches);
 
 // `any_length`: also the lengths with factors 7, 11 and 13 that the two-factor
-// kernels take (false: 2-3-5 lengths, others are refused).
+// kernels take (false: 2-3-5 lengths, others are refused). `image_rows`: only
+// the m rows of each image run, the zero rows of the padding are not written.
 void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, const float *scales,
 	int64_t scale_stride, float2 *out, const line_set &out_rows, int64_t n, hipStream_t stream,
-	bool any_length = false, float scale = 1.0f);
+	bool any_length = false, float scale = 1.0f, bool image_rows = false);
 
 void launch_fft_lines(const float2 *src, const line_set &src_lines, float2 *dst, const line_set &dst_lines,
 	int64_t n, float sign, float scale, hipStream_t stream, bool any_length = false);

@@ -58,9 +58,13 @@ __device__ double window_transform(int profile, double half_width, double shape,
 // out (crop^3 per volume) = the central crop^3 of in (big^3 per volume),
 // divided by the window's transform along each axis. The crop starts at
 // big/2 - crop/2, so that the volume's centre big/2 stays at crop/2 (the
-// central n^3 of a reconstruction inserted with 2x padding).
-__global__ void gridding_kernel(const float *in, float *out, int big, int crop, int64_t volumes, int profile,
-	double half_width, double shape)
+// central n^3 of a reconstruction inserted with 2x padding). A wavefront takes
+// rows (volume, z, y): the divisions and two of the three factors are made
+// once per row, and the double-precision table once per block, of which there
+// are few (8,192 blocks with three 64-bit divisions per voxel took 0.12 ms at
+// 320^3, 2.2 TB/s).
+__global__ __launch_bounds__(256) void gridding_kernel(const float *in, float *out, int big, int crop, int64_t rows,
+	int profile, double half_width, double shape)
 {
 	extern __shared__ float table[];
 	const int offset = big / 2 - crop / 2;
@@ -70,21 +74,22 @@ __global__ void gridding_kernel(const float *in, float *out, int big, int crop, 
 		table[i] = static_cast<float>(1.0 / window_transform(profile, half_width, shape, u));
 	}
 	__syncthreads();
-	const int64_t volume = static_cast<int64_t>(crop) * crop * crop;
-	const int64_t big_volume = static_cast<int64_t>(big) * big * big;
-	const int64_t count = volume * volumes;
-	for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < count;
-		i += static_cast<int64_t>(gridDim.x) * blockDim.x)
+	const int lane = threadIdx.x & 63;
+	for (int64_t row = blockIdx.x * 4ll + (threadIdx.x >> 6); row < rows; row += gridDim.x * 4ll)
 	{
-		const int64_t b = i / volume;
-		int64_t v = i - b * volume;
-		const int x = static_cast<int>(v % crop);
-		v /= crop;
-		const int y = static_cast<int>(v % crop);
-		const int z = static_cast<int>(v / crop);
-		const int64_t source = b * big_volume + ((static_cast<int64_t>(z + offset) * big + (y + offset)) * big) +
-			(x + offset);
-		out[i] = in[source] * table[x] * table[y] * table[z];
+		const int64_t plane = row / crop;
+		const int y = static_cast<int>(row - plane * crop);
+		const int64_t b = plane / crop;
+		const int z = static_cast<int>(plane - b * crop);
+		const float *source = in + ((b * big + z + offset) * big + (y + offset)) * big + offset;
+		float *target = out + row * crop;
+		const float ty = table[y];
+		const float tz = table[z];
+#pragma unroll 4
+		for (int x = lane; x < crop; x += 64)
+		{
+			target[x] = source[x] * table[x] * ty * tz;
+		}
 	}
 }
 
@@ -160,9 +165,9 @@ void launch_normalize(const float2 *num, const float *den, float2 *out, int64_t 
 void launch_gridding(const float *in, float *out, int big, int crop, int64_t volumes, int profile,
 	double half_width, double shape, hipStream_t stream)
 {
-	const int64_t count = static_cast<int64_t>(crop) * crop * crop * volumes;
-	gridding_kernel<<<blocks_for(count), 256, sizeof(float) * crop, stream>>>(in, out, big, crop, volumes, profile,
-		half_width, shape);
+	const int64_t rows = static_cast<int64_t>(crop) * crop * volumes;
+	const unsigned blocks = static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>((rows + 3) / 4, 2048)));
+	gridding_kernel<<<blocks, 256, sizeof(float) * crop, stream>>>(in, out, big, crop, rows, profile, half_width, shape);
 	REXLIB_HIP_CHECK(hipGetLastError());
 }
 

@@ -147,6 +147,19 @@ __host__ __device__ inline float phase_sin(float x)
 	return (q & 2) ? -v : v;
 }
 
+// chi(k) of a slice (contrast_transfer_function.inl:73-87), with the fused
+// products written out: left to the compiler, the kernels that prepare samples
+// contract the sum differently, and chi, hundreds of radians, moves by its
+// last bit between them.
+__device__ inline float ctf_chi(const slice_entry &e, float aberration, float xx, float yy, float xy)
+{
+	const float norm = xx + yy;
+	const float radial = e.ctf_radial * norm;
+	const float astigmatic = __builtin_fmaf(e.ctf_axial, xx - yy, radial);
+	const float defocus = __builtin_fmaf(e.ctf_diagonal, xy, astigmatic);
+	return __builtin_fmaf(-(norm * norm), aberration, defocus) + e.ctf_phase;
+}
+
 // The element's value comes from `load`, called only for inserted samples.
 template <int VARIANT, typename Load>
 __device__ inline bool prepare_value(const insertion_params &p, const slice_entry &e, int64_t s, int row,
@@ -186,9 +199,7 @@ __device__ inline bool prepare_value(const insertion_params &p, const slice_entr
 		const float fy = static_cast<float>(ky);
 		const float xx = fx * fx;
 		const float yy = fy * fy;
-		const float norm = xx + yy;
-		const float chi = e.ctf_radial * norm + e.ctf_axial * (xx - yy) + e.ctf_diagonal * (fx * fy) -
-			static_cast<float>(p.ctf_aberration) * (norm * norm) + e.ctf_phase;
+		const float chi = ctf_chi(e, static_cast<float>(p.ctf_aberration), xx, yy, fx * fy);
 		numerator_weight = phase_sin(chi);
 		denominator_weight = numerator_weight * numerator_weight;
 	}
@@ -330,8 +341,7 @@ __device__ inline prepared_sample prepare_unbranched(const insertion_params &p, 
 	}
 	else if (VARIANT == variant_ctf)
 	{
-		const float chi = e.ctf_radial * norm + e.ctf_axial * (xx - yy) + e.ctf_diagonal * (fx * fy) -
-			static_cast<float>(p.ctf_aberration) * (norm * norm) + e.ctf_phase;
+		const float chi = ctf_chi(e, static_cast<float>(p.ctf_aberration), xx, yy, fx * fy);
 		numerator_weight = phase_sin(chi);
 		denominator_weight = numerator_weight * numerator_weight;
 	}
