@@ -218,44 +218,25 @@ __global__ void volume_phase_kernel(float2 *table, int big)
 	table[j] = make_float2(static_cast<float>(cs), static_cast<float>(sn));
 }
 
-// Out-of-place insertions start from a copy of the accumulators: a wavefront
-// copies a row (kept, z, y), so that the batch offsets and the divisions are
-// made once per row. SHARED copies only the rows that hold the frequencies
-// +-N/2 of an even N along y or z (2 N - 1 of a volume's N^2): what bricks
-// that own voxels need. A row per wavefront moves 1.6 GB at 512^3 in 0.29 ms
-// where a division chain per voxel took 0.36 ms.
-template <bool SHARED>
-__global__ __launch_bounds__(256) void copy_accumulators_kernel(insertion_params p, const float2 *num_in, int64_t ni0,
-	int64_t ni1, int64_t ni2, const float *den_in, int64_t di0, int64_t di1, int64_t di2)
+// Out-of-place insertions start from a copy of the accumulators.
+__global__ void copy_accumulators_kernel(insertion_params p, const float2 *num_in, int64_t ni0, int64_t ni1,
+	int64_t ni2, const float *den_in, int64_t di0, int64_t di1, int64_t di2)
 {
-	const int lane = threadIdx.x & 63;
-	const int big = p.big;
-	const int64_t rows = SHARED ? 2 * static_cast<int64_t>(big) - 1 : static_cast<int64_t>(big) * big;
-	const int64_t total = rows * p.map.kept_count;
-	for (int64_t i = blockIdx.x * 4ll + (threadIdx.x >> 6); i < total; i += gridDim.x * 4ll)
+	const int64_t volume = static_cast<int64_t>(p.big) * p.big * p.half;
+	const int64_t total = volume * p.map.kept_count;
+	for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < total;
+		i += static_cast<int64_t>(gridDim.x) * blockDim.x)
 	{
-		const int64_t kept = i / rows;
-		const int64_t r = i - kept * rows;
-		int64_t z, y;
-		if (SHARED)
-		{
-			z = r < big ? big / 2 : (r - big < big / 2 ? r - big : r - big + 1);
-			y = r < big ? r : big / 2;
-		}
-		else
-		{
-			z = r / big;
-			y = r - z * big;
-		}
-		const float2 *num = num_in + kept_offset(p.map, slot_numerator, kept) + z * ni0 + y * ni1;
-		const float *den = den_in + kept_offset(p.map, slot_denominator, kept) + z * di0 + y * di1;
-		float2 *num_out = p.numerator + kept_offset(p.map, slot_numerator_out, kept) + z * p.num_s0 + y * p.num_s1;
-		float *den_out = p.denominator + kept_offset(p.map, slot_denominator_out, kept) + z * p.den_s0 + y * p.den_s1;
-		for (int x = lane; x < p.half; x += 64)
-		{
-			num_out[x * p.num_s2] = num[x * ni2];
-			den_out[x * p.den_s2] = den[x * di2];
-		}
+		const int64_t kept = i / volume;
+		int64_t v = i % volume;
+		const int64_t x = v % p.half;
+		v /= p.half;
+		const int64_t y = v % p.big;
+		const int64_t z = v / p.big;
+		const float2 a = num_in[kept_offset(p.map, slot_numerator, kept) + z * ni0 + y * ni1 + x * ni2];
+		const float b = den_in[kept_offset(p.map, slot_denominator, kept) + z * di0 + y * di1 + x * di2];
+		p.numerator[kept_offset(p.map, slot_numerator_out, kept) + z * p.num_s0 + y * p.num_s1 + x * p.num_s2] = a;
+		p.denominator[kept_offset(p.map, slot_denominator_out, kept) + z * p.den_s0 + y * p.den_s1 + x * p.den_s2] = b;
 	}
 }
 
@@ -916,36 +897,60 @@ __device__ inline void clip_row(int ky, int first, int widest, float radius, con
 	}
 }
 
-// The inputs of the bricks that own voxels but are split into shares (the
-// first `gridDim.x` tasks hold them all): their shares add with atomics.
+// Before bricks that own voxels: the inputs that reach the outputs by atomics.
+// Blocks up to `split` copy the bricks split into shares (the first `split`
+// tasks hold them all), the others the rows of the frequencies +-N/2 of an even
+// N along y or z (2 N - 1 of a volume's N^2), which two bricks reach.
 template <int T>
-__global__ __launch_bounds__(64) void copy_split_bricks_kernel(insertion_params p, const int4 *tasks,
+__global__ __launch_bounds__(64) void copy_shared_inputs_kernel(insertion_params p, const int4 *tasks, int split,
 	accumulator_input input)
 {
+	const int64_t kept = blockIdx.y;
+	const int big = p.big;
+	const int he = big / 2;
+	const int lane = threadIdx.x;
+	const float2 *num = input.numerator + kept_offset(p.map, input.num_slot, kept);
+	const float *den = input.denominator + kept_offset(p.map, input.den_slot, kept);
+	float2 *num_out = p.numerator + kept_offset(p.map, slot_numerator_out, kept);
+	float *den_out = p.denominator + kept_offset(p.map, slot_denominator_out, kept);
+	const auto copy = [&](int64_t z, int64_t y, int64_t x)
+	{
+		num_out[z * p.num_s0 + y * p.num_s1 + x * p.num_s2] =
+			num[z * input.num_s0 + y * input.num_s1 + x * input.num_s2];
+		den_out[z * p.den_s0 + y * p.den_s1 + x * p.den_s2] =
+			den[z * input.den_s0 + y * input.den_s1 + x * input.den_s2];
+	};
+	if (static_cast<int>(blockIdx.x) >= split)
+	{
+		const int r = static_cast<int>(blockIdx.x) - split;
+		const int z = r < big ? he : (r - big < he ? r - big : r - big + 1);
+		const int y = r < big ? r : he;
+		for (int x = lane; x < p.half; x += 64)
+		{
+			copy(z, y, x);
+		}
+		return;
+	}
 	const brick_box box = unpack_brick(tasks[2 * blockIdx.x]);
 	const int4 share = tasks[2 * blockIdx.x + 1];
 	if (share.x != 0 || share.y == 1)
 	{
 		return;
 	}
-	const int64_t kept = blockIdx.y;
-	const int he = p.big / 2;
-	const int ex = box.ext[0] - (T - 1), ey = box.ext[1] - (T - 1), ez = box.ext[2] - (T - 1);
-	for (int v = threadIdx.x; v < ex * ey * ez; v += 64)
+	const int x = box.lo[0] + T - 1 + lane % 8;
+	const int ey = box.ext[1] - (T - 1);
+	const int ez = box.ext[2] - (T - 1);
+	for (int xs = x; xs <= min(he, box.lo[0] + box.ext[0] - 1); xs += 8)
 	{
-		const int x = box.lo[0] + T - 1 + v % ex;
-		const int y = box.lo[1] + T - 1 + (v / ex) % ey;
-		const int z = box.lo[2] + T - 1 + v / (ex * ey);
-		if (x <= he && y <= he && z <= he)
+		for (int r = lane / 8; r < ey * ez; r += 8)
 		{
-			const int64_t sy = y < 0 ? y + p.big : y;
-			const int64_t sz = z < 0 ? z + p.big : z;
-			p.numerator[kept_offset(p.map, slot_numerator_out, kept) + sz * p.num_s0 + sy * p.num_s1 + x * p.num_s2] =
-				input.numerator[kept_offset(p.map, input.num_slot, kept) + sz * input.num_s0 + sy * input.num_s1 +
-					x * input.num_s2];
-			p.denominator[kept_offset(p.map, slot_denominator_out, kept) + sz * p.den_s0 + sy * p.den_s1 + x * p.den_s2] =
-				input.denominator[kept_offset(p.map, input.den_slot, kept) + sz * input.den_s0 + sy * input.den_s1 +
-					x * input.den_s2];
+			const int y = box.lo[1] + T - 1 + r % ey;
+			const int z = box.lo[2] + T - 1 + r / ey;
+			// (+-N/2 of an even N is the rows' above: both write the same input.)
+			if (y <= he && z <= he)
+			{
+				copy(z < 0 ? z + big : z, y < 0 ? y + big : y, xs);
+			}
 		}
 	}
 }
@@ -1501,15 +1506,47 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 			const int x_count = min(box.ext[0] - (T - 1), he + 1 - (box.lo[0] + T - 1));
 			const int y_count = min(box.ext[1] - (T - 1), he + 1 - (box.lo[1] + T - 1));
 			const int z_count = min(box.ext[2] - (T - 1), he + 1 - (box.lo[2] + T - 1));
+			// Rows of 7 voxels, 8 lanes each. Every input is loaded before any
+			// output is written, so a brick waits for memory once (row by row, the
+			// seven round trips were a third of the time of a sparse call).
 			constexpr int row = EX - T + 1 <= 8 ? 8 : 16; // lanes along x
+			constexpr int steps = ((EY - T + 1) * (EZ - T + 1) + 64 / row - 1) / (64 / row);
 			const int lx = lane % row;
-			if (lx < x_count)
+			const int x = box.lo[0] + T - 1 + lx;
+			float2 in_value[steps];
+			float in_weight[steps];
+#pragma unroll
+			for (int step = 0; step < steps; ++step)
 			{
-				const int x = box.lo[0] + T - 1 + lx;
-				for (int r = lane / row; r < y_count * z_count; r += 64 / row)
+				const int r = lane / row + step * (64 / row);
+				const int lz = r / (EY - T + 1);
+				const int ly = r - lz * (EY - T + 1);
+				const int y = box.lo[1] + T - 1 + ly;
+				const int z = box.lo[2] + T - 1 + lz;
+				const int sy = y < 0 ? y + big : y;
+				const int sz = z < 0 ? z + big : z;
+				const int v = (lx + T - 1) + L::pitch_y * (ly + T - 1) + L::pitch_z * (lz + T - 1);
+				in_value[step] = make_float2(0.0f, 0.0f);
+				in_weight[step] = 0.0f;
+				const bool inside = lx < x_count && ly < y_count && lz < z_count && !split;
+				// (In place, voxels without a sum keep what they hold.)
+				if (inside && (!input.in_place ||
+					!(acc_value[v].x == 0.0f && acc_value[v].y == 0.0f && acc_weight[v] == 0.0f)))
 				{
-					const int lz = r / y_count;
-					const int ly = r - lz * y_count;
+					in_value[step] =
+						input.numerator[num_in + sz * input.num_s0 + sy * input.num_s1 + x * input.num_s2];
+					in_weight[step] =
+						input.denominator[den_in + sz * input.den_s0 + sy * input.den_s1 + x * input.den_s2];
+				}
+			}
+#pragma unroll
+			for (int step = 0; step < steps; ++step)
+			{
+				const int r = lane / row + step * (64 / row);
+				const int lz = r / (EY - T + 1);
+				const int ly = r - lz * (EY - T + 1);
+				if (lx < x_count && ly < y_count && lz < z_count)
+				{
 					const int v = (lx + T - 1) + L::pitch_y * (ly + T - 1) + L::pitch_z * (lz + T - 1);
 					const float2 sum = touched ? acc_value[v] : make_float2(0.0f, 0.0f);
 					const float weight = touched ? acc_weight[v] : 0.0f;
@@ -1533,10 +1570,8 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 					}
 					else if (!(none && input.in_place))
 					{
-						const float2 a = input.numerator[num_in + sz * input.num_s0 + sy * input.num_s1 + x * input.num_s2];
-						const float d = input.denominator[den_in + sz * input.den_s0 + sy * input.den_s1 + x * input.den_s2];
-						*target = make_float2(a.x + value.x, a.y + value.y);
-						*dtarget = d + weight;
+						*target = make_float2(in_value[step].x + value.x, in_value[step].y + value.y);
+						*dtarget = in_weight[step] + weight;
 					}
 				}
 			}
@@ -1997,7 +2032,7 @@ const int4 *brick_tasks(int big, int64_t slices, const brick_tuning &tuning, int
 // of its T - 1 lower cell layers a second time (512 / 343 of the samples for 8
 // x 8 x 8 and two taps). The line is at the density where the one costs what
 // the other does, in samples per voxel of the stored half: 256 slices of 256^2
-// into 512^3 (0.1 samples per voxel) take 1.25 against 1.75 ms, 512 of 256^2
+// into 512^3 (0.1 samples per voxel) take 1.15 against 1.75 ms, 512 of 256^2
 // into 256^3 (1.6) 0.47 against 0.51 ms, 1,024 (3.1) 0.75 against 0.71 ms. Four
 // taps would insert 4 times the samples; a fixed workspace buffer keeps the
 // smaller task list of cells.
@@ -2006,6 +2041,24 @@ bool bricks_own_voxels(const insertion_params &p, int64_t slices, int taps, cons
 	const double samples = 0.125 * 3.14159265 * p.n * p.n * static_cast<double>(slice_bucket(slices));
 	const double voxels = 0.5 * p.big * p.big * static_cast<double>(p.big);
 	return taps <= 2 && workspace.arena == nullptr && samples < 1.6 * voxels;
+}
+
+// Whether an out-of-place call of bricks that own voxels still copies the inputs
+// first and inserts in place. The bricks' own copy runs in rows of 7 voxels,
+// whose ends share cache lines with other bricks: an empty brick copies at half
+// the rate of copy_accumulators_kernel, but a brick with samples saves a pass.
+// The line is at 0.04 samples per voxel of the stored half: 16 slices of 256^2
+// into 512^3 (0.006) take 0.64 copied against 0.88 ms, 64 (0.025) 0.89 against
+// 0.93, 128 (0.05) 1.05 against 0.98; 32 of 128^2 into 256^3 (0.025) 118 against
+// 128 us, 128 (0.1) 149 against 144. Where inputs and outputs fit the L2s (8 x 4
+// MiB), the copy costs less still: 64 of 64^2 into 128^3 (0.1) 52.5 against 55.7
+// us, 64 of 99^2 into 99^3 (0.5) 50.8 against 54.6.
+bool copy_first(const insertion_params &p, int64_t slices)
+{
+	const double samples = 0.125 * 3.14159265 * p.n * p.n * static_cast<double>(slices);
+	const double voxels = 0.5 * p.big * p.big * static_cast<double>(p.big);
+	const double bytes = 2.0 * (sizeof(float2) + sizeof(float)) * voxels * static_cast<double>(p.map.kept_count);
+	return samples < 0.04 * voxels || bytes <= 8.0 * (4 << 20);
 }
 
 } // anonymous namespace
@@ -2097,23 +2150,21 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 	p.kb_table = kb;
 	p.volume_phase = vphase;
 
-	const auto copy_inputs = [&](bool shared_only)
+	const auto copy_inputs = [&]()
 	{
-		const int64_t rows = (shared_only ? 2 * static_cast<int64_t>(p.big) - 1 : static_cast<int64_t>(p.big) * p.big) *
-			p.map.kept_count;
-		if (in_place || rows == 0)
+		const int64_t total = static_cast<int64_t>(p.big) * p.big * p.half * p.map.kept_count;
+		if (in_place || total == 0)
 		{
 			return;
 		}
-		const unsigned blocks = static_cast<unsigned>(std::min<int64_t>((rows + 3) / 4, 1 << 20));
-		const auto kernel = shared_only ? copy_accumulators_kernel<true> : copy_accumulators_kernel<false>;
-		kernel<<<blocks, 256, 0, stream>>>(p, num_in, num_in_strides[0], num_in_strides[1], num_in_strides[2], den_in,
-			den_in_strides[0], den_in_strides[1], den_in_strides[2]);
+		const unsigned blocks = static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 1 << 20));
+		copy_accumulators_kernel<<<blocks, 256, 0, stream>>>(p, num_in, num_in_strides[0], num_in_strides[1],
+			num_in_strides[2], den_in, den_in_strides[0], den_in_strides[1], den_in_strides[2]);
 		REXLIB_HIP_CHECK(hipGetLastError());
 	};
 	if (slices == 0)
 	{
-		copy_inputs(false);
+		copy_inputs();
 		return;
 	}
 
@@ -2164,11 +2215,12 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 	{
 		tuning = voxel_tuning;
 	}
-	// Bricks that own voxels read the inputs themselves, but for the elements
-	// that two of them add to.
-	if (!voxels || p.big % 2 == 0)
+	// Bricks that own voxels read the inputs themselves, unless most of them
+	// would have nothing to add.
+	const bool copied = !voxels || copy_first(p, chunk_count);
+	if (copied)
 	{
-		copy_inputs(voxels);
+		copy_inputs();
 	}
 	// Pending column transforms run inside the preparation of each chunk on
 	// the brick schedule; on the scatter schedule they run here, in place.
@@ -2218,18 +2270,18 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 			REXLIB_HIP_CHECK(hipGetLastError());
 			timing_end(prepare_token, stream);
 			const int brick_token = timing_begin(REXLIB_HIP_KERNEL_BRICK, stream);
-			const bool from_outputs = in_place || begin > 0;
+			const bool from_outputs = in_place || copied || begin > 0;
 			const accumulator_input input = from_outputs ?
 				accumulator_input{p.numerator, p.num_s0, p.num_s1, p.num_s2, p.denominator, p.den_s0, p.den_s1, p.den_s2,
 					slot_numerator_out, slot_denominator_out, true} :
 				accumulator_input{num_in, num_in_strides[0], num_in_strides[1], num_in_strides[2], den_in,
 					den_in_strides[0], den_in_strides[1], den_in_strides[2], slot_numerator, slot_denominator, false};
-			if (voxels && !input.in_place && split > 0)
+			const unsigned shared_blocks = static_cast<unsigned>(split + (p.big % 2 == 0 ? 2 * p.big - 1 : 0));
+			if (voxels && !input.in_place && shared_blocks > 0)
 			{
-				const dim3 grid(static_cast<unsigned>(split), static_cast<unsigned>(p.map.kept_count));
-				const auto kernel = layout_taps == 1 ? copy_split_bricks_kernel<1> :
-					(layout_taps == 2 ? copy_split_bricks_kernel<2> : copy_split_bricks_kernel<4>);
-				kernel<<<grid, 64, 0, stream>>>(p, tasks, input);
+				const dim3 grid(shared_blocks, static_cast<unsigned>(p.map.kept_count));
+				const auto kernel = layout_taps == 1 ? copy_shared_inputs_kernel<1> : copy_shared_inputs_kernel<2>;
+				kernel<<<grid, 64, 0, stream>>>(p, tasks, split, input);
 				REXLIB_HIP_CHECK(hipGetLastError());
 			}
 			dispatch_brick(p, chunk, prepared, tasks, count, tuning, voxels ? &input : nullptr, stream);

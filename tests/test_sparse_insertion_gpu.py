@@ -29,9 +29,11 @@ def geometry(inputs, rng):
 
 # 1.6 samples per voxel of the stored half divide the two: n = N = 16 with 5
 # slices (0.4: bucket 8) and with 60 (3.1); N around 7 (voxels per brick), 8 and
-# 14; odd and even.
+# 14; odd and even. At N = 145 and 146 the inputs exceed the L2s: out of place, 60
+# slices (0.06 samples per voxel) let the bricks copy them, 20 (0.02) do not.
 @pytest.mark.parametrize("n,big,slices", [(16, 16, 5), (16, 16, 60), (6, 7, 2), (7, 13, 3), (8, 14, 3), (9, 15, 1),
-                                          (12, 24, 9), (12, 29, 9), (20, 33, 4)])
+                                          (12, 24, 9), (12, 29, 9), (20, 33, 4), (64, 145, 60), (64, 146, 60),
+                                          (64, 146, 20)])
 @pytest.mark.parametrize("in_place", [True, False])
 def test_sparse_and_dense_insertions_match_the_oracle(n, big, slices, in_place):
     inputs = geometry(make_case("plain", n, big, seed=n + big, slices=slices), np.random.default_rng(big))
@@ -42,8 +44,10 @@ def test_sparse_and_dense_insertions_match_the_oracle(n, big, slices, in_place):
     assert np.abs(den - ref[1]).max() <= BAR * max(1.0, float(np.abs(ref[1]).max()))
 
 
-def test_sparse_insertion_into_strided_batched_accumulators():
-    n, big, kept, slices = 10, 20, 2, 3
+# (Two volumes of 116^3 exceed the L2s: the bricks copy the inputs.)
+@pytest.mark.parametrize("n,big,slices", [(10, 20, 3), (64, 116, 30)])
+def test_sparse_insertion_into_strided_batched_accumulators(n, big, slices):
+    kept = 2
     rng = np.random.default_rng(4)
     inputs = make_case("plain", n, big, seed=9, slices=slices, accumulator_batch=(kept, 1))
     inputs = geometry(inputs, rng)
