@@ -449,119 +449,6 @@ __device__ inline half8_t join(half4_t lo, half4_t hi)
 	return half8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
 }
 
-// Load the B operand tile (rows k0.., columns n0..) of a row-major K x N
-// float16 matrix in LDS with row length `cols`.
-__device__ inline half4_t load_b(const _Float16 *w, int cols, int k0, int n0, int lane)
-{
-	half4_t b;
-	const int k = k0 + 4 * (lane >> 4);
-	const int n = n0 + (lane & 15);
-	for (int j = 0; j < 4; ++j)
-	{
-		b[j] = w[(k + j) * cols + n];
-	}
-	return b;
-}
-
-// Load the A operand tile (rows m0.., columns k0..) of a row-major M x K
-// float16 matrix in LDS with row length `cols`.
-__device__ inline half4_t load_a(const _Float16 *m, int cols, int m0, int k0, int lane)
-{
-	half4_t a;
-	const int row = m0 + (lane & 15);
-	const int k = k0 + 4 * (lane >> 4);
-	for (int j = 0; j < 4; ++j)
-	{
-		a[j] = m[row * cols + k + j];
-	}
-	return a;
-}
-
-// A operand of the transpose of a row-major K x M matrix: A[m][k] = T[k][m].
-__device__ inline half4_t load_a_transposed(const _Float16 *t, int cols, int m0, int k0, int lane)
-{
-	half4_t a;
-	const int m = m0 + (lane & 15);
-	const int k = k0 + 4 * (lane >> 4);
-	for (int j = 0; j < 4; ++j)
-	{
-		a[j] = t[(k + j) * cols + m];
-	}
-	return a;
-}
-
-// B operand of the transpose of a row-major N x K matrix: B[k][n] = T[n][k].
-__device__ inline half4_t load_b_transposed(const _Float16 *t, int cols, int k0, int n0, int lane)
-{
-	half4_t b;
-	const int k = k0 + 4 * (lane >> 4);
-	const int n = n0 + (lane & 15);
-	for (int j = 0; j < 4; ++j)
-	{
-		b[j] = t[n * cols + k + j];
-	}
-	return b;
-}
-
-// One dense layer on a 16-row tile: out (16 x 64) = act(in (16 x K) W (K x 64) + b).
-template <int K, bool RELU>
-__device__ inline void dense_tile(const _Float16 *in, const _Float16 *w, const float *b, _Float16 *out, int lane)
-{
-	for (int nt = 0; nt < hidden / 16; ++nt)
-	{
-		float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-		for (int kt = 0; kt < K / 16; ++kt)
-		{
-			acc = mfma16(load_a(in, K, 0, kt * 16, lane), load_b(w, hidden, kt * 16, nt * 16, lane), acc);
-		}
-		const int col = nt * 16 + (lane & 15);
-		for (int j = 0; j < 4; ++j)
-		{
-			const int row = 4 * (lane >> 4) + j;
-			float v = acc[j] + b[col];
-			if (RELU)
-			{
-				v = fmaxf(v, 0.0f);
-			}
-			out[row * hidden + col] = static_cast<_Float16>(v);
-		}
-	}
-}
-
-// Stage the float16 parameters and float32 biases in LDS.
-struct mlp_lds
-{
-	_Float16 w[off_b1];
-	float b[parameter_count - off_b1];
-};
-
-__device__ inline void stage_parameters(mlp_lds &s, const _Float16 *params_h, const float *params_f)
-{
-	for (int i = threadIdx.x; i < off_b1; i += blockDim.x)
-	{
-		s.w[i] = params_h[i];
-	}
-	for (int i = threadIdx.x; i < parameter_count - off_b1; i += blockDim.x)
-	{
-		s.b[i] = params_f[off_b1 + i];
-	}
-	__syncthreads();
-}
-
-// Per-wave activations: the input tile and the three hidden layers.
-struct tile_lds
-{
-	_Float16 x[16 * inputs];
-	_Float16 h1[16 * hidden];
-	_Float16 h2[16 * hidden];
-	_Float16 h3[16 * hidden];
-	float g[16 * hidden]; // gradient of one layer's output
-	_Float16 gh[16 * hidden]; // gradients as float16 MFMA operands, two in turn
-	_Float16 gh2[16 * hidden];
-};
-
-constexpr int mlp_waves = 4;
-
 // The perceptron in transposed form: each layer computes Y^T = W^T X^T on a
 // tile of 16 samples, the 16 columns of the B operand. The weights are the A
 // operands and stay in registers for the whole kernel. An MFMA's output
@@ -911,178 +798,343 @@ __global__ __launch_bounds__(64) void density_scale_kernel(const double *partial
 	}
 }
 
-// Add the gradient of a weight matrix: dW (K x 64) += act_in^T (K x 16) dY (16 x 64), for one tile.
-template <int K>
-__device__ inline void accumulate_weight_gradient(const _Float16 *act_in, int in_cols, const _Float16 *dy,
-	float *grad, float scale, int lane)
-{
-	for (int mt = 0; mt < K / 16; ++mt)
-	{
-		for (int nt = 0; nt < hidden / 16; ++nt)
-		{
-			float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-			acc = mfma16(load_a_transposed(act_in, in_cols, mt * 16, 0, lane), load_b(dy, hidden, 0, nt * 16, lane),
-				acc);
-			const int col = nt * 16 + (lane & 15);
-			for (int j = 0; j < 4; ++j)
-			{
-				const int row = mt * 16 + 4 * (lane >> 4) + j;
-				atomicAdd(&grad[row * hidden + col], acc[j] * scale);
-			}
-		}
-	}
-}
-
-// dX (16 x K) = dY (16 x 64) W^T (64 x K) masked by act_x > 0; written to t.g and t.gh.
-template <int K>
-__device__ inline void backward_input(const _Float16 *dy, const _Float16 *w, const _Float16 *act_x, float *g,
-	_Float16 *gh, int lane)
-{
-	for (int nt = 0; nt < K / 16; ++nt)
-	{
-		float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-		for (int kt = 0; kt < hidden / 16; ++kt)
-		{
-			acc = mfma16(load_a(dy, hidden, 0, kt * 16, lane), load_b_transposed(w, hidden, kt * 16, nt * 16, lane),
-				acc);
-		}
-		const int col = nt * 16 + (lane & 15);
-		for (int j = 0; j < 4; ++j)
-		{
-			const int row = 4 * (lane >> 4) + j;
-			const float v = static_cast<float>(act_x[row * K + col]) > 0.0f ? acc[j] : 0.0f;
-			g[row * hidden + col] = v;
-			gh[row * hidden + col] = static_cast<_Float16>(v);
-		}
-	}
-}
-
 // One pass of forward and backward over `count` samples: the mean squared
 // error of MLP(features) against `target`, scaled by `loss_scale` for the
 // float16 gradients; grads (float32, parameter layout) and loss[0] accumulate.
-__global__ __launch_bounds__(64 * mlp_waves) void mlp_backward_kernel(const __half *features, const float *target,
-	const _Float16 *params_h, const float *params_f, float *grads, float *loss, int64_t count, float loss_scale)
+//
+// A wavefront takes tiles of 16 samples in the transposed form of the forward
+// pass. The gradient of a layer's output, dY^T, has the layout of its
+// activations, so dX^T = W dY^T runs on the same fragments (W's rows as A
+// operands). A weight gradient dW = X^T dY contracts over the samples, which
+// lie across lanes: both fragments pass through LDS with the samples of a unit
+// side by side and come back as 8-byte operands. All sums stay in registers
+// over the wavefront's tiles (one wavefront per SIMD holds them with the
+// weights); the four wavefronts of a block then hand theirs over through LDS,
+// fragment by fragment (plain adds in LDS, one wavefront after another, took 15
+// us, LDS atomics 40), and a block adds 9.4 thousand sums to memory. 8,192 rows
+// take 25 us; with one atomic per parameter and tile, on operands gathered from
+// LDS two bytes at a time, 57.
+constexpr int backward_waves = 4;
+constexpr int sample_pitch = 20; // halves per unit: 16 samples, padded to 40 bytes
+
+// The 16 x 16 tiles of the weight gradients of layers 1 (4), 2 and 3 (16 each),
+// and how many of them the wavefronts exchange at a time.
+constexpr int gradient_tiles = 4 + 16 + 16;
+constexpr int exchanged_tiles = 12;
+// Per wavefront: W4's, the three layers' biases', b4's gradients and the error.
+constexpr int small_sums = 4 * hidden + 2;
+
+struct backward_operands
 {
-	__shared__ mlp_lds s;
-	__shared__ tile_lds tiles[mlp_waves];
-	stage_parameters(s, params_h, params_f);
+	_Float16 weights[off_b1];
+	_Float16 left[backward_waves][hidden * sample_pitch];
+	_Float16 right[backward_waves][hidden * sample_pitch];
+};
+
+union backward_lds
+{
+	backward_operands operands;
+	float4_t tiles[backward_waves][exchanged_tiles][64];
+	float small[backward_waves][small_sums];
+};
+
+// A fragment (lane (g, c): units unit0 + 4 g + j of sample c) into LDS, a unit's
+// samples side by side.
+__device__ __forceinline__ void put_samples(_Float16 *lds, int unit0, int g, int c, half4_t v)
+{
+#pragma unroll
+	for (int j = 0; j < 4; ++j)
+	{
+		lds[(unit0 + 4 * g + j) * sample_pitch + c] = v[j];
+	}
+}
+
+// Samples 4 g .. 4 g + 3 of unit unit0 + c: an operand of a product over the
+// samples.
+__device__ __forceinline__ half4_t get_samples(const _Float16 *lds, int unit0, int g, int c)
+{
+	return *reinterpret_cast<const half4_t *>(lds + (unit0 + c) * sample_pitch + 4 * g);
+}
+
+// sums[4 k + n] += sum over the samples of left[16 k ..] right[16 n ..], K tiles
+// of left units and 4 of right units.
+template <int K>
+__device__ __forceinline__ void add_products(const _Float16 *left, const _Float16 *right, int g, int c, float4_t *sums)
+{
+	half4_t r[4];
+#pragma unroll
+	for (int n = 0; n < 4; ++n)
+	{
+		r[n] = get_samples(right, 16 * n, g, c);
+	}
+#pragma unroll
+	for (int k = 0; k < K; ++k)
+	{
+		const half4_t l = get_samples(left, 16 * k, g, c);
+#pragma unroll
+		for (int n = 0; n < 4; ++n)
+		{
+			sums[4 * k + n] = mfma16(l, r[n], sums[4 * k + n]);
+		}
+	}
+}
+
+__global__ __launch_bounds__(64 * backward_waves, 1) void mlp_backward_kernel(const __half *features,
+	const float *target, const _Float16 *params_h, const float *params_f, float *grads, float *loss, int64_t count,
+	float loss_scale)
+{
+	__shared__ backward_lds s;
 	const int lane = threadIdx.x & 63;
 	const int wave = threadIdx.x >> 6;
-	tile_lds &t = tiles[wave];
-	const int64_t tiles_total = (count + 15) / 16;
-	const float inverse = 1.0f / static_cast<float>(count);
-	for (int64_t tile = blockIdx.x * static_cast<int64_t>(mlp_waves) + wave; tile < tiles_total;
-		tile += static_cast<int64_t>(gridDim.x) * mlp_waves)
+	const int g = lane >> 4;
+	const int c = lane & 15;
+	_Float16 *staged = s.operands.weights;
+	for (int i = threadIdx.x; i < off_b1; i += 64 * backward_waves)
 	{
-		const int64_t row0 = tile * 16;
-		for (int e = lane; e < 16 * inputs; e += 64)
+		staged[i] = params_h[i];
+	}
+	__syncthreads();
+	half4_t w1[4];
+	half8_t w2[4][2], w3[4][2], w4[2];   // W^T as A operands (forward)
+	half8_t b2[4][2], b3[4][2];          // W as A operands (backward)
+	float w4_unit[4][4];                 // W4's column per held unit
+	float4_t bias[3][4];
+#pragma unroll
+	for (int mt = 0; mt < 4; ++mt)
+	{
+#pragma unroll
+		for (int j = 0; j < 4; ++j)
 		{
-			const int64_t r = row0 + e / inputs;
-			t.x[e] = r < count ? static_cast<_Float16>(__half2float(features[r * inputs + e % inputs])) : _Float16(0);
+			w1[mt][j] = staged[off_w1 + (4 * g + j) * hidden + mt * 16 + c];
+			w4_unit[mt][j] = static_cast<float>(staged[off_w4 + (16 * mt + 4 * g + j) * 16]);
+#pragma unroll
+			for (int layer = 0; layer < 3; ++layer)
+			{
+				bias[layer][mt][j] = params_f[off_b1 + layer * hidden + 16 * mt + 4 * g + j];
+			}
 		}
-		wave_order();
-		dense_tile<inputs, true>(t.x, s.w + off_w1, s.b, t.h1, lane);
-		wave_order();
-		dense_tile<hidden, true>(t.h1, s.w + off_w2, s.b + (off_b2 - off_b1), t.h2, lane);
-		wave_order();
-		dense_tile<hidden, true>(t.h2, s.w + off_w3, s.b + (off_b3 - off_b1), t.h3, lane);
-		wave_order();
-		float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-		for (int kt = 0; kt < hidden / 16; ++kt)
+#pragma unroll
+		for (int t = 0; t < 2; ++t)
 		{
-			acc = mfma16(load_a(t.h3, hidden, 0, kt * 16, lane), load_b(s.w + off_w4, 16, kt * 16, 0, lane), acc);
+#pragma unroll
+			for (int j = 0; j < 8; ++j)
+			{
+				const int unit = 32 * t + (j < 4 ? 4 * g + j : 16 + 4 * g + j - 4);
+				w2[mt][t][j] = staged[off_w2 + unit * hidden + mt * 16 + c];
+				w3[mt][t][j] = staged[off_w3 + unit * hidden + mt * 16 + c];
+				b2[mt][t][j] = staged[off_w2 + (mt * 16 + c) * hidden + unit];
+				b3[mt][t][j] = staged[off_w3 + (mt * 16 + c) * hidden + unit];
+				w4[t][j] = staged[off_w4 + unit * 16 + c];
+			}
 		}
+	}
+	const float b4 = params_f[off_b4];
+	__syncthreads();
+
+	const float4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+	float4_t tile_sums[gradient_tiles];
+	float4_t unit_sums[4][4]; // W4's and the three biases' gradients, per held unit and sample
+#pragma unroll
+	for (int i = 0; i < gradient_tiles; ++i)
+	{
+		tile_sums[i] = zero;
+	}
+#pragma unroll
+	for (int i = 0; i < 4; ++i)
+	{
+		unit_sums[0][i] = unit_sums[1][i] = unit_sums[2][i] = unit_sums[3][i] = zero;
+	}
+	float gb4 = 0.0f;
+	float error = 0.0f;
+	_Float16 *left = s.operands.left[wave];
+	_Float16 *right = s.operands.right[wave];
+	const float inverse = 1.0f / static_cast<float>(count);
+	const int64_t tiles = (count + 15) / 16;
+	for (int64_t tile = blockIdx.x * static_cast<int64_t>(backward_waves) + wave; tile < tiles;
+		tile += static_cast<int64_t>(gridDim.x) * backward_waves)
+	{
+		const int64_t row = tile * 16 + c;
+		half4_t x = {0, 0, 0, 0};
+		if (row < count)
+		{
+			x = *reinterpret_cast<const half4_t *>(features + row * inputs + 4 * g);
+		}
+		half4_t h1[4], h2[4], h3[4];
+#pragma unroll
+		for (int mt = 0; mt < 4; ++mt)
+		{
+			h1[mt] = relu_half(mfma16(w1[mt], x, bias[0][mt]));
+		}
+#pragma unroll
+		for (int mt = 0; mt < 4; ++mt)
+		{
+			h2[mt] = relu_half(mfma32(w2[mt][1], join(h1[2], h1[3]), mfma32(w2[mt][0], join(h1[0], h1[1]), bias[1][mt])));
+		}
+#pragma unroll
+		for (int mt = 0; mt < 4; ++mt)
+		{
+			h3[mt] = relu_half(mfma32(w3[mt][1], join(h2[2], h2[3]), mfma32(w3[mt][0], join(h2[0], h2[1]), bias[2][mt])));
+		}
+		const float4_t y = mfma32(w4[1], join(h3[2], h3[3]), mfma32(w4[0], join(h3[0], h3[1]), zero));
 		// dOut = 2 (out - target) / count, scaled; rows beyond count carry 0.
-		// Lanes with column 0 hold the outputs; share them through t.g.
-		if ((lane & 15) == 0)
+		// The outputs sit in lanes c of group 0.
+		float d = 0.0f;
+		if (g == 0 && row < count)
 		{
+			const float difference = y[0] + b4 - target[row];
+			error += difference * difference * inverse;
+			d = 2.0f * difference * inverse * loss_scale;
+			gb4 += d;
+		}
+		d = __shfl(d, c, 64);
+
+		// Layer 4, and dH3 = dOut W4 where h3 > 0.
+		half4_t dh[4];
+		const auto masked = [](const half4_t &h, const float4_t &v)
+		{
+			float4_t m;
+#pragma unroll
 			for (int j = 0; j < 4; ++j)
 			{
-				const int row = 4 * (lane >> 4) + j;
-				const int64_t r = row0 + row;
-				float d = 0.0f;
-				if (r < count)
+				m[j] = static_cast<float>(h[j]) > 0.0f ? v[j] : 0.0f;
+			}
+			return m;
+		};
+		const auto rounded = [](const float4_t &v)
+		{
+			return half4_t{static_cast<_Float16>(v[0]), static_cast<_Float16>(v[1]), static_cast<_Float16>(v[2]),
+				static_cast<_Float16>(v[3])};
+		};
+#pragma unroll
+		for (int mt = 0; mt < 4; ++mt)
+		{
+			float4_t v;
+#pragma unroll
+			for (int j = 0; j < 4; ++j)
+			{
+				unit_sums[0][mt][j] += static_cast<float>(h3[mt][j]) * d;
+				v[j] = d * w4_unit[mt][j];
+			}
+			v = masked(h3[mt], v);
+			unit_sums[3][mt] += v;
+			dh[mt] = rounded(v);
+			put_samples(left, 16 * mt, g, c, h2[mt]);
+			put_samples(right, 16 * mt, g, c, dh[mt]);
+		}
+		wave_order();
+		add_products<4>(left, right, g, c, tile_sums + 20);
+		wave_order();
+		// dH2 = W3 dH3 where h2 > 0.
+		half4_t next[4];
+#pragma unroll
+		for (int mt = 0; mt < 4; ++mt)
+		{
+			const float4_t v = masked(h2[mt], mfma32(b3[mt][1], join(dh[2], dh[3]),
+				mfma32(b3[mt][0], join(dh[0], dh[1]), zero)));
+			unit_sums[2][mt] += v;
+			next[mt] = rounded(v);
+			put_samples(left, 16 * mt, g, c, h1[mt]);
+			put_samples(right, 16 * mt, g, c, next[mt]);
+		}
+		wave_order();
+		add_products<4>(left, right, g, c, tile_sums + 4);
+		wave_order();
+		// dH1 = W2 dH2 where h1 > 0.
+		put_samples(left, 0, g, c, x);
+#pragma unroll
+		for (int mt = 0; mt < 4; ++mt)
+		{
+			const float4_t v = masked(h1[mt], mfma32(b2[mt][1], join(next[2], next[3]),
+				mfma32(b2[mt][0], join(next[0], next[1]), zero)));
+			unit_sums[1][mt] += v;
+			put_samples(right, 16 * mt, g, c, rounded(v));
+		}
+		wave_order();
+		add_products<1>(left, right, g, c, tile_sums);
+		wave_order();
+	}
+
+	// The samples' sums over the 16 lanes of a group.
+	const auto over_samples = [](float v)
+	{
+#pragma unroll
+		for (int offset = 8; offset > 0; offset /= 2)
+		{
+			v += __shfl_xor(v, offset, 64);
+		}
+		return v;
+	};
+	// The tiles, a few at a time: each wavefront writes its own, and adds up and
+	// sends on a quarter of them all.
+#pragma unroll
+	for (int first = 0; first < gradient_tiles; first += exchanged_tiles)
+	{
+		__syncthreads();
+#pragma unroll
+		for (int i = 0; i < exchanged_tiles; ++i)
+		{
+			s.tiles[wave][i][lane] = tile_sums[first + i];
+		}
+		__syncthreads();
+#pragma unroll
+		for (int i = 0; i < exchanged_tiles / backward_waves; ++i)
+		{
+			const int local = i * backward_waves + wave;
+			float4_t sum = s.tiles[0][local][lane];
+#pragma unroll
+			for (int w = 1; w < backward_waves; ++w)
+			{
+				sum += s.tiles[w][local][lane];
+			}
+			const int tile = first + local;
+			const int k = tile < 4 ? 0 : (tile - 4) % 16 / 4;
+			float *target = grads + (tile < 4 ? off_w1 : (tile < 20 ? off_w2 : off_w3)) + (16 * k + 4 * g) * hidden +
+				16 * (tile % 4) + c;
+#pragma unroll
+			for (int j = 0; j < 4; ++j)
+			{
+				atomicAdd(target + j * hidden, sum[j]);
+			}
+		}
+	}
+	__syncthreads();
+#pragma unroll
+	for (int layer = 0; layer < 4; ++layer)
+	{
+#pragma unroll
+		for (int mt = 0; mt < 4; ++mt)
+		{
+#pragma unroll
+			for (int j = 0; j < 4; ++j)
+			{
+				const float sum = over_samples(unit_sums[layer][mt][j]);
+				if (c == 0)
 				{
-					const float out = acc[j] + s.b[off_b4 - off_b1];
-					const float diff = out - target[r];
-					atomicAdd(loss, diff * diff * inverse);
-					d = 2.0f * diff * inverse * loss_scale;
+					s.small[wave][layer * hidden + 16 * mt + 4 * g + j] = sum;
 				}
-				t.g[row] = d;
 			}
 		}
-		wave_order();
-		// Layer 4: dW4[c][0] += sum_r h3[r][c] dOut[r]; db4 += sum_r dOut[r];
-		// dH3[r][c] = dOut[r] W4[c][0] (h3 > 0).
+	}
+	gb4 = over_samples(gb4);
+	error = over_samples(error);
+	if (lane == 0)
+	{
+		s.small[wave][4 * hidden] = gb4;
+		s.small[wave][4 * hidden + 1] = error;
+	}
+	__syncthreads();
+	for (int i = threadIdx.x; i < small_sums; i += blockDim.x)
+	{
+		float sum = 0.0f;
+		for (int w = 0; w < backward_waves; ++w)
 		{
-			const int c = lane;
-			float sum = 0.0f;
-			for (int r = 0; r < 16; ++r)
-			{
-				sum += static_cast<float>(t.h3[r * hidden + c]) * t.g[r];
-			}
-			atomicAdd(&grads[off_w4 + c * 16], sum);
-			if (lane == 0)
-			{
-				float db = 0.0f;
-				for (int r = 0; r < 16; ++r)
-				{
-					db += t.g[r];
-				}
-				atomicAdd(&grads[off_b4], db);
-			}
-			const float w4 = static_cast<float>(s.w[off_w4 + c * 16]);
-			float dout[16];
-			for (int r = 0; r < 16; ++r)
-			{
-				dout[r] = t.g[r];
-			}
-			wave_order();
-			for (int r = 0; r < 16; ++r)
-			{
-				const float v = static_cast<float>(t.h3[r * hidden + c]) > 0.0f ? dout[r] * w4 : 0.0f;
-				t.g[r * hidden + c] = v;
-				t.gh[r * hidden + c] = static_cast<_Float16>(v);
-			}
+			sum += s.small[w][i];
 		}
-		wave_order();
-		// Layer 3: dW3 += h2^T dH3; db3 += column sums; dH2 = dH3 W3^T (h2 > 0).
-		accumulate_weight_gradient<hidden>(t.h2, hidden, t.gh, grads + off_w3, 1.0f, lane);
-		{
-			float db = 0.0f;
-			for (int r = 0; r < 16; ++r)
-			{
-				db += t.g[r * hidden + lane];
-			}
-			atomicAdd(&grads[off_b3 + lane], db);
-		}
-		wave_order();
-		backward_input<hidden>(t.gh, s.w + off_w3, t.h2, t.g, t.gh2, lane);
-		wave_order();
-		// Layer 2.
-		accumulate_weight_gradient<hidden>(t.h1, hidden, t.gh2, grads + off_w2, 1.0f, lane);
-		{
-			float db = 0.0f;
-			for (int r = 0; r < 16; ++r)
-			{
-				db += t.g[r * hidden + lane];
-			}
-			atomicAdd(&grads[off_b2 + lane], db);
-		}
-		wave_order();
-		backward_input<hidden>(t.gh2, s.w + off_w2, t.h1, t.g, t.gh, lane);
-		wave_order();
-		// Layer 1: dW1 += x^T dH1; db1 += column sums.
-		accumulate_weight_gradient<inputs>(t.x, inputs, t.gh, grads + off_w1, 1.0f, lane);
-		{
-			float db = 0.0f;
-			for (int r = 0; r < 16; ++r)
-			{
-				db += t.g[r * hidden + lane];
-			}
-			atomicAdd(&grads[off_b1 + lane], db);
-		}
-		wave_order();
+		const int unit = i % hidden;
+		const int layer = i / hidden;
+		float *target = i == 4 * hidden + 1 ? loss : (i == 4 * hidden ? grads + off_b4 :
+			grads + (layer == 0 ? off_w4 + unit * 16 : (layer == 1 ? off_b1 : (layer == 2 ? off_b2 : off_b3)) + unit));
+		atomicAdd(target, sum);
 	}
 }
 
@@ -1221,9 +1273,12 @@ void launch_mlp_forward(const void *features, const void *params_h, const float 
 void launch_mlp_backward(const void *features, const float *target, const void *params_h, const float *params_f,
 	float *grads, float *loss, int64_t count, float loss_scale, hipStream_t stream)
 {
-	mlp_backward_kernel<<<blocks_of((count + 15) / 16, mlp_waves), 64 * mlp_waves, 0, stream>>>(
-		static_cast<const __half *>(features), target, static_cast<const _Float16 *>(params_h), params_f, grads, loss,
-		count, loss_scale);
+// Two tiles per wavefront at least, one block per CU at most.
+	const int64_t tiles = (count + 15) / 16;
+	const unsigned blocks = static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>((tiles + 2 * backward_waves - 1) /
+		(2 * backward_waves), 256)));
+	mlp_backward_kernel<<<blocks, 64 * backward_waves, 0, stream>>>(static_cast<const __half *>(features), target,
+		static_cast<const _Float16 *>(params_h), params_f, grads, loss, count, loss_scale);
 	REXLIB_HIP_CHECK(hipGetLastError());
 }
 
