@@ -655,6 +655,21 @@ __global__ __launch_bounds__(256, 2) void mlp_forward_kernel(const __half *featu
 	}
 }
 
+// |g| <= N/2 as learned.inside_nyquist has it, to the last bit: fftfreq scales by
+// 1 / (N (1 / N)) in double, which is not 1 for N = 98, 196, 206, 214, ..., and
+// there the rounding of the separate products and sums decides the voxels at
+// exactly N/2 (a fused one decides some of N = 214 the other way).
+__device__ inline bool inside_nyquist(int x, int y, int z, int big, double frequency_scale)
+{
+#pragma clang fp contract(off)
+	const double fy = y * frequency_scale;
+	const double fz = z * frequency_scale;
+	const double zz = fz * fz;
+	const double yy = fy * fy;
+	const double xx = static_cast<double>(x) * x;
+	return zz + yy + xx <= static_cast<double>(big / 2) * (big / 2);
+}
+
 // The predicted weights of a volume in one pass: W = exp(MLP(features)) / den
 // where den > 0 within the Nyquist sphere, 1 / den beyond it, 0 elsewhere. A
 // lane computes the radius, density and table entry of one of 64 voxels of a
@@ -662,7 +677,8 @@ __global__ __launch_bounds__(256, 2) void mlp_forward_kernel(const __half *featu
 // fractions from the table, and hand the outputs back. The features (270 MB at
 // 256^3), the correction and the masks never reach memory.
 __global__ __launch_bounds__(256, 2) void predicted_weights_kernel(const float *den, const float *table,
-	float density_scale, const _Float16 *params_h, const float *params_f, float *out, int big)
+	float density_scale, const _Float16 *params_h, const float *params_f, float *out, int big,
+	double frequency_scale)
 {
 	__shared__ mlp_biases bias;
 	mlp_weights m;
@@ -740,8 +756,7 @@ __global__ __launch_bounds__(256, 2) void predicted_weights_kernel(const float *
 			// numpy's fftfreq (of an odd N, index N/2 is +N/2).
 			const int y = sy < (big + 1) / 2 ? sy : sy - big;
 			const int z = sz < (big + 1) / 2 ? sz : sz - big;
-			const int64_t r2 = static_cast<int64_t>(x) * x + static_cast<int64_t>(y) * y + static_cast<int64_t>(z) * z;
-			const bool inside = r2 <= static_cast<int64_t>(big / 2) * (big / 2);
+			const bool inside = inside_nyquist(x, y, z, big, frequency_scale);
 			out[i] = d > 0.0f ? (inside ? expf(correction) : 1.0f) / d : 0.0f;
 		}
 	}
@@ -1258,7 +1273,7 @@ void launch_predicted_weights(const float *den, const float *table, float densit
 	// once for dozens of groups.
 	const int64_t groups = static_cast<int64_t>((big * (big / 2 + 1) + 63) / 64) * big;
 	predicted_weights_kernel<<<blocks_of(std::min<int64_t>(groups, 2048), 4), 256, 0, stream>>>(den, table, density_scale,
-		static_cast<const _Float16 *>(params_h), params_f, out, big);
+		static_cast<const _Float16 *>(params_h), params_f, out, big, 1.0 / (big * (1.0 / big)));
 	REXLIB_HIP_CHECK(hipGetLastError());
 }
 
