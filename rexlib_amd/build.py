@@ -1,8 +1,9 @@
 """Build the gfx950 backend in-tree.
 
-- rexlib_amd/librexlib_hip.so: one hipcc invocation compiles every HIP and C++
-  source of rexlib_amd/csrc for gfx950; only the C ABI (rexlib_hip_*) is
-  exported.
+- rexlib_amd/librexlib_hip.so: every HIP and C++ source of rexlib_amd/csrc,
+  compiled for gfx950 one hipcc process per source (the kernel variants take 4
+  minutes one after another, less than two side by side); only the C ABI
+  (rexlib_hip_*) is exported.
 - rexlib_amd/librexlib_host.so: the C++ core of the mirrored rexlib API
   (rexlib_amd/host/core.cpp): services, plugin loader, arrays, the eager
   dispatcher and the em / Fourier functions.
@@ -20,6 +21,8 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -93,14 +96,12 @@ def build_host(verbose: bool = False) -> list:
 def build(verbose: bool = False) -> str:
     exports = os.path.join(CSRC, "exports.map")
     tmp = LIBRARY + ".tmp"
-    cmd = [hipcc(), *HIPCC_FLAGS, "-shared", "-o", tmp, *sources(),
-           f"-Wl,--version-script={exports}", "-lpthread"]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        sys.stderr.write(proc.stdout + proc.stderr)
-        raise RuntimeError("hipcc failed to build librexlib_hip.so")
+    with tempfile.TemporaryDirectory() as objects, ThreadPoolExecutor(max(1, min(8, os.cpu_count() or 1))) as pool:
+        compiled = [(source, os.path.join(objects, os.path.basename(source) + ".o")) for source in sources()]
+        list(pool.map(lambda c: _run([hipcc(), *HIPCC_FLAGS, "-c", c[0], "-o", c[1]], os.path.basename(c[0]), verbose),
+                      compiled))
+        _run([hipcc(), "--offload-arch=gfx950", "-shared", "-o", tmp, *[o for _, o in compiled],
+              f"-Wl,--version-script={exports}", "-lpthread"], "librexlib_hip.so", verbose)
     os.replace(tmp, LIBRARY)
     build_host(verbose)
     return LIBRARY
