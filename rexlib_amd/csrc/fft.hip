@@ -590,7 +590,7 @@ __global__ void irfft_rows_kernel(const float2 *src, line_set src_rows, float *d
 // Real rows, two to a complex line, to half spectra, as rfft_rows_kernel: a
 // block of (b, lines) threads stages its rows in LDS (a line's threads load
 // consecutive elements, 4 at a time where VEC), transforms them and separates
-// the two half spectra. Bound by HBM: 1,000 images 320^2 take 0.20 ms against
+// the two half spectra. Bound by HBM: 1,000 images 320^2 take 0.28 ms against
 // 0.52 ms through the Stockham stages (0.8 GB: 4.0 against 1.6 TB/s).
 template <int KIND, int WIDTH, int CLASS>
 __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void rfft_rows_two_kernel(const void *in, line_set in_rows, int m,

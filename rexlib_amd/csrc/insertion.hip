@@ -1050,8 +1050,9 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 		// sample of the rows, puts its 12 axis weights in LDS, and the wavefront
 		// then adds the samples one after another, each by one read-add-write
 		// of 64 different voxels (no claims, no bank conflicts, every lane
-		// busy). 64 serial taps per lane, claimed as below, took 48 cycles per
-		// CU and sample; this is bound by the LDS pipeline at about 20.
+		// busy). 1,024 slices of 128^2 into 256^3 take 0.80 ms so, 1.35 with 64
+		// serial taps per lane, claimed as below; dense calls lose a little by
+		// it (2,048 of 256^2 into 256^3: 4.4 against 3.75 ms).
 		const int tap_x = lane & 3;
 		const int tap_y = (lane >> 2) & 3;
 		const int tap_z = lane >> 4;
