@@ -649,7 +649,8 @@ int rexlib_hip_rfft2(const rexlib_hip_array *images, const rexlib_hip_array *spe
 		float2 *out = static_cast<float2 *>(spectra->data);
 		const line_set in_rows{batch * n, 1, n, in_stride, 0, core_stride(*images, 2), core_stride(*images, 1)};
 		const line_set out_rows{batch * n, 1, n, out_stride, 0, core_stride(*spectra, 2), core_stride(*spectra, 1)};
-		launch_rfft_rows(real_f32, images->data, in_rows, static_cast<int>(n), nullptr, 0, out, out_rows, n, s);
+		launch_rfft_rows(real_f32, images->data, in_rows, static_cast<int>(n), nullptr, 0, out, out_rows,
+			whole_rows(n, batch * n), n, s);
 		const int64_t h = n / 2 + 1;
 		const line_set columns{batch * h, 1, h, out_stride, 0, core_stride(*spectra, 1), core_stride(*spectra, 2)};
 		launch_fft_lines(out, columns, out, columns, n, -1.0f, 1.0f, s);
@@ -689,7 +690,7 @@ int rexlib_hip_irfft2(const rexlib_hip_array *spectra, const rexlib_hip_array *i
 		launch_fft_lines(static_cast<const float2 *>(spectra->data), columns_in, w, columns_w, n, 1.0f, 1.0f, s);
 		const line_set rows_w{batch * n, 1, n, n * h, 0, h, 1};
 		const line_set rows_out{batch * n, 1, n, out_stride, 0, core_stride(*images, 2), core_stride(*images, 1)};
-		launch_irfft_rows(w, rows_w, static_cast<float *>(images->data), rows_out, n,
+		launch_irfft_rows(w, rows_w, static_cast<float *>(images->data), rows_out, whole_rows(n, batch * n), n,
 			static_cast<float>(1.0 / (static_cast<double>(n) * static_cast<double>(n))), s);
 	});
 }
@@ -737,7 +738,8 @@ int rexlib_hip_irfft3(const rexlib_hip_array *spectrum, const rexlib_hip_array *
 		const line_set x_out{batch * big * big, big, big, out_stride, core_stride(*volume, 3),
 			core_stride(*volume, 2), core_stride(*volume, 1)};
 		const double scale = 1.0 / (static_cast<double>(big) * static_cast<double>(big) * static_cast<double>(big));
-		launch_irfft_rows(w, x_w, static_cast<float *>(volume->data), x_out, big, static_cast<float>(scale), s);
+		launch_irfft_rows(w, x_w, static_cast<float *>(volume->data), x_out, whole_rows(big, batch * big * big), big,
+			static_cast<float>(scale), s);
 	});
 }
 

@@ -198,12 +198,12 @@ __device__ inline void load_reals(const void *base, bool live, int64_t row, int 
 
 // Rows of real images, two at a time, to half spectra. Images of extent m
 // are zero-padded to the transform length n with their origin m/2 moved to
-// n/2. `total` rows run, `rows` per image: n (the padded rows), or m (the image
-// rows alone, when the caller knows the others to be zero). Line set `in`
-// lists the image rows, `out` the padded rows, n per image.
+// n/2. Line set `in` lists the image rows, `out` the padded rows; `lines` says
+// which of them run, and together. A block takes `pairs` lines at a time.
 template <int KIND>
 __global__ void rfft_rows_kernel(const void *in, line_set in_rows, int m, const float *scales,
-	int64_t scale_stride, float2 *out, line_set out_rows, fft_plan plan, const float2 *tw, int pairs, float half, int rows, int64_t total)
+	int64_t scale_stride, float2 *out, line_set out_rows, row_pairs lines, fft_plan plan, const float2 *tw, int pairs,
+	float half)
 {
 	extern __shared__ float2 lds[];
 	const int n = plan.n;
@@ -222,32 +222,19 @@ __global__ void rfft_rows_kernel(const void *in, line_set in_rows, int m, const 
 		twl[i] = tw[i];
 	}
 	const int offset = n / 2 - m / 2;
-	for (int64_t first = blockIdx.x * static_cast<int64_t>(2 * pairs); first < total;
-		first += static_cast<int64_t>(gridDim.x) * 2 * pairs)
+	const int64_t total = line_count(lines);
+	for (int64_t first = blockIdx.x * static_cast<int64_t>(pairs); first < total;
+		first += static_cast<int64_t>(gridDim.x) * pairs)
 	{
-		for (int q = threadIdx.x; q < 2 * pairs; q += blockDim.x)
+		for (int p = threadIdx.x; p < pairs; p += blockDim.x)
 		{
-			const int64_t row = first + q;
-			int64_t src = -1;
-			int64_t dst = -1;
-			float scale = 1.0f;
-			if (row < total)
+			const line_rows l = rows_of(lines, first + p);
+			for (int q = 0; q < 2; ++q)
 			{
-				const int64_t image = row / rows;
-				const int r = static_cast<int>(row - image * rows) - (rows == n ? offset : 0);
-				if (r >= 0 && r < m)
-				{
-					src = line_offset(in_rows, image * m + r);
-					if (scales != nullptr)
-					{
-						scale = scales[image * scale_stride];
-					}
-				}
-				dst = line_offset(out_rows, image * n + r + offset);
+				row_in[2 * p + q] = l.in[q] >= 0 ? line_offset(in_rows, l.in[q]) : -1;
+				row_out[2 * p + q] = l.out[q] >= 0 ? line_offset(out_rows, l.out[q]) : -1;
+				row_scale[2 * p + q] = scales != nullptr && l.in[q] >= 0 ? scales[l.transform * scale_stride] : 1.0f;
 			}
-			row_in[q] = src;
-			row_out[q] = dst;
-			row_scale[q] = scale;
 		}
 		__syncthreads();
 		for (int t = threadIdx.x; t < pairs * n; t += blockDim.x)
@@ -356,7 +343,8 @@ __global__ void fft_lines_kernel(const float2 *src, line_set src_lines, float2 *
 // image, are zeros, as in rfft_rows_kernel.
 template <int KIND, bool VEC>
 __global__ __launch_bounds__(256) void rfft256_rows_kernel(const void *in, line_set in_rows, int m,
-	const float *scales, int64_t scale_stride, float2 *out, line_set out_rows, const float2 *tw, float half, int rows, int64_t total)
+	const float *scales, int64_t scale_stride, float2 *out, line_set out_rows, row_pairs lines, const float2 *tw,
+	float half)
 {
 	constexpr int n = 256;
 	constexpr int h = n / 2 + 1;
@@ -370,32 +358,20 @@ __global__ __launch_bounds__(256) void rfft256_rows_kernel(const void *in, line_
 	const int l = t >> 4;
 	twl[t] = tw[t];
 	const int offset = n / 2 - m / 2;
-	for (int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(2 * fft256_lines); first < total;
-		first += static_cast<int64_t>(gridDim.x) * 2 * fft256_lines)
+	const int64_t total = line_count(lines);
+	for (int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(fft256_lines); first < total;
+		first += static_cast<int64_t>(gridDim.x) * fft256_lines)
 	{
-		if (t < 2 * fft256_lines)
+		if (t < fft256_lines)
 		{
-			const int64_t row = first + t;
-			int64_t src = -1;
-			int64_t dst = -1;
-			float scale = 1.0f;
-			if (row < total)
+			const line_rows r = rows_of(lines, first + t);
+#pragma unroll
+			for (int q = 0; q < 2; ++q)
 			{
-				const int64_t image = row / rows;
-				const int r = static_cast<int>(row - image * rows) - (rows == n ? offset : 0);
-				if (r >= 0 && r < m)
-				{
-					src = line_offset(in_rows, image * m + r);
-					if (scales != nullptr)
-					{
-						scale = scales[image * scale_stride];
-					}
-				}
-				dst = line_offset(out_rows, image * n + r + offset);
+				row_in[2 * t + q] = r.in[q] >= 0 ? line_offset(in_rows, r.in[q]) : -1;
+				row_out[2 * t + q] = r.out[q] >= 0 ? line_offset(out_rows, r.out[q]) : -1;
+				row_scale[2 * t + q] = scales != nullptr && r.in[q] >= 0 ? scales[r.transform * scale_stride] : 1.0f;
 			}
-			row_in[t] = src;
-			row_out[t] = dst;
-			row_scale[t] = scale;
 		}
 		__syncthreads();
 		float2 *x = exchange + l * fft256_line_stride;
@@ -503,7 +479,7 @@ __global__ __launch_bounds__(256) void rfft256_rows_kernel(const void *in, line_
 
 // Half-spectrum rows, two at a time, to real rows, scaled.
 __global__ void irfft_rows_kernel(const float2 *src, line_set src_rows, float *dst, line_set dst_rows,
-	fft_plan plan, const float2 *tw, float scale, int pairs)
+	row_pairs lines, fft_plan plan, const float2 *tw, float scale, int pairs)
 {
 	extern __shared__ float2 lds[];
 	const int n = plan.n;
@@ -518,15 +494,18 @@ __global__ void irfft_rows_kernel(const float2 *src, line_set src_rows, float *d
 	{
 		twl[i] = tw[i];
 	}
-	const int64_t total = src_rows.count;
-	for (int64_t first = blockIdx.x * static_cast<int64_t>(2 * pairs); first < total;
-		first += static_cast<int64_t>(gridDim.x) * 2 * pairs)
+	const int64_t total = line_count(lines);
+	for (int64_t first = blockIdx.x * static_cast<int64_t>(pairs); first < total;
+		first += static_cast<int64_t>(gridDim.x) * pairs)
 	{
-		for (int q = threadIdx.x; q < 2 * pairs; q += blockDim.x)
+		for (int p = threadIdx.x; p < pairs; p += blockDim.x)
 		{
-			const int64_t row = first + q;
-			row_src[q] = row < total ? line_offset(src_rows, row) : -1;
-			row_dst[q] = row < total ? line_offset(dst_rows, row) : -1;
+			const line_rows l = rows_of(lines, first + p);
+			for (int q = 0; q < 2; ++q)
+			{
+				row_src[2 * p + q] = l.in[q] >= 0 ? line_offset(src_rows, l.in[q]) : -1;
+				row_dst[2 * p + q] = l.out[q] >= 0 ? line_offset(dst_rows, l.out[q]) : -1;
+			}
 		}
 		__syncthreads();
 		for (int t = threadIdx.x; t < pairs * n; t += blockDim.x)
@@ -594,7 +573,8 @@ __global__ void irfft_rows_kernel(const float2 *src, line_set src_rows, float *d
 // 0.52 ms through the Stockham stages (0.8 GB: 4.0 against 1.6 TB/s).
 template <int KIND, int WIDTH, int CLASS>
 __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void rfft_rows_two_kernel(const void *in, line_set in_rows, int m,
-	const float *scales, int64_t scale_stride, float2 *out, line_set out_rows, two_factor::plan p, const float2 *tw, float half, int rows, int64_t total)
+	const float *scales, int64_t scale_stride, float2 *out, line_set out_rows, row_pairs lines, two_factor::plan p,
+	const float2 *tw, float half)
 {
 	extern __shared__ float2 lds[];
 	const int j = threadIdx.x;
@@ -608,36 +588,22 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void rfft_rows_two_k
 	const int offset = n / 2 - m / 2;
 	// One group of lines per block: a loop over groups would hoist the
 	// twiddles of every register length out of it, into registers.
-	const int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(2 * p.lines);
-	if (first >= total)
+	const int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(p.lines);
+	if (first >= line_count(lines))
 	{
 		return;
 	}
 	// The two rows of the line: first input element (-1: a zero row of the
-	// padding or past the end), first output element, scale.
+	// padding or none), first output element, scale.
+	const line_rows rows = rows_of(lines, first + l);
 	int64_t src[2], dst[2];
 	float scale[2];
 #pragma unroll
 	for (int q = 0; q < 2; ++q)
 	{
-		const int64_t row = first + 2 * l + q;
-		src[q] = -1;
-		dst[q] = -1;
-		scale[q] = 1.0f;
-		if (row < total)
-		{
-			const int64_t image = row / rows;
-			const int r = static_cast<int>(row - image * rows) - (rows == n ? offset : 0);
-			if (r >= 0 && r < m)
-			{
-				src[q] = line_offset(in_rows, image * m + r);
-				if (scales != nullptr)
-				{
-					scale[q] = scales[image * scale_stride];
-				}
-			}
-			dst[q] = line_offset(out_rows, image * n + r + offset);
-		}
+		src[q] = rows.in[q] >= 0 ? line_offset(in_rows, rows.in[q]) : -1;
+		dst[q] = rows.out[q] >= 0 ? line_offset(out_rows, rows.out[q]) : -1;
+		scale[q] = scales != nullptr && rows.in[q] >= 0 ? scales[rows.transform * scale_stride] : 1.0f;
 	}
 	// Loads of WIDTH elements, two steps of both rows in flight.
 #pragma unroll 2
@@ -680,7 +646,7 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void rfft_rows_two_k
 // irfft_rows_kernel: a coefficient is read once and staged with its mirror.
 template <int CLASS>
 __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void irfft_rows_two_kernel(const float2 *src, line_set src_rows, float *dst,
-	line_set dst_rows, two_factor::plan p, const float2 *tw, float scale)
+	line_set dst_rows, row_pairs lines, two_factor::plan p, const float2 *tw, float scale)
 {
 	extern __shared__ float2 lds[];
 	const int j = threadIdx.x;
@@ -691,17 +657,16 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void irfft_rows_two_
 	float2 *twl = lds + p.lines * p.line;
 	float2 *x = lds + l * p.line;
 	two_factor::stage_twiddles(p, twl, tw, l * threads + j, threads * blockDim.y);
-	const int64_t total = src_rows.count;
-	const int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(2 * p.lines);
-	if (first >= total)
+	const int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(p.lines);
+	if (first >= line_count(lines))
 	{
 		return;
 	}
-	const int64_t row = first + 2 * l;
-	const int64_t src0 = row < total ? line_offset(src_rows, row) : -1;
-	const int64_t src1 = row + 1 < total ? line_offset(src_rows, row + 1) : -1;
-	const int64_t dst0 = row < total ? line_offset(dst_rows, row) : -1;
-	const int64_t dst1 = row + 1 < total ? line_offset(dst_rows, row + 1) : -1;
+	const line_rows rows = rows_of(lines, first + l);
+	const int64_t src0 = rows.in[0] >= 0 ? line_offset(src_rows, rows.in[0]) : -1;
+	const int64_t src1 = rows.in[1] >= 0 ? line_offset(src_rows, rows.in[1]) : -1;
+	const int64_t dst0 = rows.out[0] >= 0 ? line_offset(dst_rows, rows.out[0]) : -1;
+	const int64_t dst1 = rows.out[1] >= 0 ? line_offset(dst_rows, rows.out[1]) : -1;
 	for (int k = j; k < h; k += threads)
 	{
 		float2 va = src0 >= 0 ? src[src0 + k * src_rows.s_elem] : make_float2(0.0f, 0.0f);
@@ -841,16 +806,15 @@ static void check_length(int64_t n, bool any_length)
 }
 
 void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, const float *scales,
-	int64_t scale_stride, float2 *out, const line_set &out_rows, int64_t n, hipStream_t stream, bool any_length,
-	float scale, bool image_rows)
+	int64_t scale_stride, float2 *out, const line_set &out_rows, const row_pairs &pairs, int64_t n, hipStream_t stream,
+	bool any_length, float scale)
 {
-	const int rows = static_cast<int>(image_rows ? m : n);
-	const int64_t total = image_rows ? out_rows.count / n * m : out_rows.count;
+	const int64_t lines = line_count(pairs);
 	check_length(n, any_length);
 	const float2 *tw = twiddles(n);
 	if (n == 256)
 	{
-		const unsigned blocks = xcd_grid(grid_for(total, 2 * fft256_lines));
+		const unsigned blocks = xcd_grid(grid_for(lines, fft256_lines));
 		// Rows take loads of 4 elements when every run of 4 elements is
 		// aligned and contiguous.
 		const std::uintptr_t element = kind == real_f32 ? 4 : 2;
@@ -861,8 +825,7 @@ void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, 
 		auto launch = [&](auto kind_constant, auto vec_constant)
 		{
 			rfft256_rows_kernel<decltype(kind_constant)::value, decltype(vec_constant)::value>
-				<<<blocks, 256, 0, stream>>>(in, in_rows, m, scales, scale_stride, out, out_rows, tw, 0.5f * scale,
-					rows, total);
+				<<<blocks, 256, 0, stream>>>(in, in_rows, m, scales, scale_stride, out, out_rows, pairs, tw, 0.5f * scale);
 		};
 		using vec = std::true_type;
 		using scalar = std::false_type;
@@ -887,7 +850,7 @@ void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, 
 	const two_factor::plan two = two_factor::make_plan(n);
 	if (two.n != 0)
 	{
-		const unsigned blocks = two_factor::blocks_for(total, 2 * two.lines);
+		const unsigned blocks = two_factor::blocks_for(lines, two.lines);
 		// Rows take loads of 4 (or 2) elements when every run of them is
 		// aligned and contiguous.
 		const std::uintptr_t element = kind == real_f32 ? 4 : 2;
@@ -906,7 +869,7 @@ void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, 
 				{
 					rfft_rows_two_kernel<decltype(kind_constant)::value, decltype(width_constant)::value, CLASS>
 						<<<blocks, dim3(two.b, two.lines), two_factor::shared_bytes(two), stream>>>(in, in_rows, m, scales,
-							scale_stride, out, out_rows, two, tw, 0.5f * scale, rows, total);
+							scale_stride, out, out_rows, pairs, two, tw, 0.5f * scale);
 				};
 				const auto with_width = [&](auto kind_constant)
 				{
@@ -934,14 +897,14 @@ void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, 
 		return;
 	}
 	const fft_plan plan = make_fft_plan(n);
-	const int pairs = std::max(1, lines_per_group(static_cast<int>(n)) / 2);
+	const int group = std::max(1, lines_per_group(static_cast<int>(n)) / 2);
 	// Two buffers, the twiddles, then per row two offsets and a scale.
-	const std::size_t shared = sizeof(float2) * (2 * pairs * (n + 1) + n) + 2 * pairs * (2 * sizeof(int64_t) + 4);
-	const unsigned grid = grid_for(total, 2 * pairs);
+	const std::size_t shared = sizeof(float2) * (2 * group * (n + 1) + n) + 2 * group * (2 * sizeof(int64_t) + 4);
+	const unsigned grid = grid_for(lines, group);
 	const auto launch = [&](auto kind_constant)
 	{
 		rfft_rows_kernel<decltype(kind_constant)::value><<<grid, 256, shared, stream>>>(in, in_rows, m, scales,
-			scale_stride, out, out_rows, plan, tw, pairs, 0.5f * scale, rows, total);
+			scale_stride, out, out_rows, pairs, plan, tw, group, 0.5f * scale);
 	};
 	switch (kind)
 	{
@@ -988,27 +951,27 @@ void launch_fft_lines(const float2 *src, const line_set &src_lines, float2 *dst,
 }
 
 void launch_irfft_rows(const float2 *src, const line_set &src_rows, float *dst, const line_set &dst_rows,
-	int64_t n, float scale, hipStream_t stream, bool any_length)
+	const row_pairs &pairs, int64_t n, float scale, hipStream_t stream, bool any_length)
 {
 	check_length(n, any_length);
 	const float2 *tw = twiddles(n);
 	const two_factor::plan two = two_factor::make_plan(n);
 	if (two.n != 0)
 	{
-		const unsigned blocks = two_factor::blocks_for(src_rows.count, 2 * two.lines);
+		const unsigned blocks = two_factor::blocks_for(line_count(pairs), two.lines);
 		two_factor::with_class(two, [&](auto kind_class)
 			{
 				irfft_rows_two_kernel<decltype(kind_class)::value><<<blocks, dim3(two.b, two.lines),
-					two_factor::shared_bytes(two), stream>>>(src, src_rows, dst, dst_rows, two, tw, scale);
+					two_factor::shared_bytes(two), stream>>>(src, src_rows, dst, dst_rows, pairs, two, tw, scale);
 			});
 		REXLIB_HIP_CHECK(hipGetLastError());
 		return;
 	}
 	const fft_plan plan = make_fft_plan(n);
-	const int pairs = std::max(1, lines_per_group(static_cast<int>(n)) / 2);
-	const std::size_t shared = sizeof(float2) * (2 * pairs * (n + 1) + n) + 2 * pairs * 2 * sizeof(int64_t);
-	const unsigned grid = grid_for(src_rows.count, 2 * pairs);
-	irfft_rows_kernel<<<grid, 256, shared, stream>>>(src, src_rows, dst, dst_rows, plan, tw, scale, pairs);
+	const int group = std::max(1, lines_per_group(static_cast<int>(n)) / 2);
+	const std::size_t shared = sizeof(float2) * (2 * group * (n + 1) + n) + 2 * group * 2 * sizeof(int64_t);
+	const unsigned grid = grid_for(line_count(pairs), group);
+	irfft_rows_kernel<<<grid, 256, shared, stream>>>(src, src_rows, dst, dst_rows, pairs, plan, tw, scale, group);
 	REXLIB_HIP_CHECK(hipGetLastError());
 }
 

@@ -40,6 +40,80 @@ __host__ __device__ inline int64_t line_offset(const line_set &l, int64_t line)
 	return outer * l.s_outer + middle * l.s_middle + inner * l.s_inner;
 }
 
+// Which real rows share a complex line: two rows of one transform (an image, or
+// the rows along a transformed axis of a general one), never rows of different
+// ones. Both halves of a line round relative to the larger of its rows, and a
+// NaN or an infinity reaches both, which the transform's other axis does to all of its
+// rows anyway; the rows of another transform, and every row where no other axis
+// is transformed (`rows` = 1), stay as exact as on a line of their own.
+struct row_pairs
+{
+	int64_t transforms;
+	int32_t rows;      // of each transform that run
+	int32_t in_rows;   // input rows of each transform
+	int32_t in_shift;  // the running row of its first input row
+	int32_t out_rows;  // output rows of each transform
+	int32_t out_shift; // the output row of the first running row
+};
+
+__host__ __device__ inline int64_t line_count(const row_pairs &p)
+{
+	return p.transforms * ((p.rows + 1) / 2);
+}
+
+// Transforms of `rows` rows, in and out, `count` rows in all.
+inline row_pairs whole_rows(int64_t rows, int64_t count)
+{
+	const int32_t r = static_cast<int32_t>(rows);
+	return row_pairs{count / rows, r, r, 0, r, 0};
+}
+
+// Images of m rows zero-padded to n, their origin m/2 moved to n/2; `image_rows`:
+// only the m rows run, the zero rows of the padding are not written.
+inline row_pairs padded_rows(int64_t m, int64_t n, int64_t images, bool image_rows)
+{
+	const int32_t offset = static_cast<int32_t>(n / 2 - m / 2);
+	return row_pairs{images, static_cast<int32_t>(image_rows ? m : n), static_cast<int32_t>(m),
+		image_rows ? 0 : offset, static_cast<int32_t>(n), image_rows ? offset : 0};
+}
+
+// The rows of line `line`: the transform, and per row of the line the input and
+// output row among all (-1: none).
+struct line_rows
+{
+	int64_t transform;
+	int64_t in[2];
+	int64_t out[2];
+};
+
+__device__ inline line_rows rows_of(const row_pairs &p, int64_t line)
+{
+	line_rows l{0, {-1, -1}, {-1, -1}};
+	const int pairs = (p.rows + 1) / 2;
+	const int64_t transform = line / pairs;
+	if (transform >= p.transforms)
+	{
+		return l;
+	}
+	const int first = 2 * static_cast<int>(line - transform * pairs);
+	l.transform = transform;
+#pragma unroll
+	for (int q = 0; q < 2; ++q)
+	{
+		const int row = first + q;
+		if (row < p.rows)
+		{
+			const int in = row - p.in_shift;
+			if (in >= 0 && in < p.in_rows)
+			{
+				l.in[q] = transform * p.in_rows + in;
+			}
+			l.out[q] = transform * p.out_rows + row + p.out_shift;
+		}
+	}
+	return l;
+}
+
 fft_plan make_fft_plan(int64_t n);
 
 // Device twiddles exp(-2 pi i m / n), m < n, computed in double, cached per

@@ -6,7 +6,8 @@
 //
 // Transforms between dense operands run their axis passes from the input
 // straight into the output: complex ones over any axes, real ones whose halved
-// axis is the last one in memory (its rows go two to a complex line). Other
+// axis is the last one in memory (rows of one transform go two to a complex
+// line, row_pairs). Other
 // operands are gathered into a contiguous complex buffer; each axis is then a
 // batch of lines (outer, line, inner) transformed in place.
 //
@@ -406,7 +407,7 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void bluestein_lines
 // Real rows, two to a complex line, to half spectra (as rfft_rows_two_kernel).
 template <int CLASS>
 __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void bluestein_rfft_rows_kernel(const float *src,
-	line_set src_rows, float2 *dst, line_set dst_rows, int n, two_factor::plan p, const float2 *tw,
+	line_set src_rows, float2 *dst, line_set dst_rows, row_pairs lines, int n, two_factor::plan p, const float2 *tw,
 	const float2 *chirps, float scale)
 {
 	extern __shared__ float2 lds[];
@@ -416,21 +417,22 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void bluestein_rfft_
 	float2 *x = lds + l * p.line;
 	two_factor::stage_twiddles(p, twl, tw, l * blockDim.x + j, blockDim.x * blockDim.y);
 	__syncthreads();
-	const int64_t row = (xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(p.lines) + l) * 2;
-	if (row - 2 * l >= src_rows.count)
+	const int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(p.lines);
+	if (first >= line_count(lines))
 	{
 		return;
 	}
-	const bool live0 = row < src_rows.count;
-	const bool live1 = row + 1 < src_rows.count;
-	const float *in0 = src + (live0 ? line_offset(src_rows, row) : 0);
-	const float *in1 = src + (live1 ? line_offset(src_rows, row + 1) : 0);
+	const line_rows rows = rows_of(lines, first + l);
+	const bool live0 = rows.in[0] >= 0;
+	const bool live1 = rows.in[1] >= 0;
+	const float *in0 = src + (live0 ? line_offset(src_rows, rows.in[0]) : 0);
+	const float *in1 = src + (live1 ? line_offset(src_rows, rows.in[1]) : 0);
 	bluestein_line<CLASS, false, true>(p, n, x, twl, j, chirps,
 		[&](int i) { return make_float2(live0 ? in0[i * src_rows.s_elem] : 0.0f, live1 ? in1[i * src_rows.s_elem] : 0.0f); },
 		[&](int k, float2 v) { x[k] = v; });
 	__syncthreads();
-	float2 *out0 = dst + (live0 ? line_offset(dst_rows, row) : 0);
-	float2 *out1 = dst + (live1 ? line_offset(dst_rows, row + 1) : 0);
+	float2 *out0 = dst + (live0 ? line_offset(dst_rows, rows.out[0]) : 0);
+	float2 *out1 = dst + (live1 ? line_offset(dst_rows, rows.out[1]) : 0);
 	const float half = 0.5f * scale;
 	for (int k = j; k < n / 2 + 1; k += blockDim.x)
 	{
@@ -452,7 +454,7 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void bluestein_rfft_
 // Half-spectrum rows, two at a time, to real rows (as irfft_rows_two_kernel).
 template <int CLASS>
 __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void bluestein_irfft_rows_kernel(const float2 *src,
-	line_set src_rows, float *dst, line_set dst_rows, int n, two_factor::plan p, const float2 *tw,
+	line_set src_rows, float *dst, line_set dst_rows, row_pairs lines, int n, two_factor::plan p, const float2 *tw,
 	const float2 *chirps, float scale)
 {
 	extern __shared__ float2 lds[];
@@ -461,15 +463,16 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void bluestein_irfft
 	float2 *twl = lds + p.lines * p.line;
 	float2 *x = lds + l * p.line;
 	two_factor::stage_twiddles(p, twl, tw, l * blockDim.x + j, blockDim.x * blockDim.y);
-	const int64_t row = (xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(p.lines) + l) * 2;
-	if (row - 2 * l >= src_rows.count)
+	const int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(p.lines);
+	if (first >= line_count(lines))
 	{
 		return;
 	}
-	const bool live0 = row < src_rows.count;
-	const bool live1 = row + 1 < src_rows.count;
-	const float2 *in0 = src + (live0 ? line_offset(src_rows, row) : 0);
-	const float2 *in1 = src + (live1 ? line_offset(src_rows, row + 1) : 0);
+	const line_rows rows = rows_of(lines, first + l);
+	const bool live0 = rows.in[0] >= 0;
+	const bool live1 = rows.in[1] >= 0;
+	const float2 *in0 = src + (live0 ? line_offset(src_rows, rows.in[0]) : 0);
+	const float2 *in1 = src + (live1 ? line_offset(src_rows, rows.in[1]) : 0);
 	for (int k = j; k < n / 2 + 1; k += blockDim.x)
 	{
 		float2 va = live0 ? in0[k * src_rows.s_elem] : make_float2(0.0f, 0.0f);
@@ -486,8 +489,8 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void bluestein_irfft
 		x[k] = make_float2(va.x - vb.y, va.y + vb.x);
 	}
 	__syncthreads();
-	float *out0 = dst + (live0 ? line_offset(dst_rows, row) : 0);
-	float *out1 = dst + (live1 ? line_offset(dst_rows, row + 1) : 0);
+	float *out0 = dst + (live0 ? line_offset(dst_rows, rows.out[0]) : 0);
+	float *out1 = dst + (live1 ? line_offset(dst_rows, rows.out[1]) : 0);
 	bluestein_line<CLASS, true, false>(p, n, x, twl, j, chirps, [&](int i) { return x[i]; },
 		[&](int k, float2 v)
 		{
@@ -546,12 +549,13 @@ bool direct_rows(int64_t n)
 	return n > 1 && (direct_length(n) || n <= longest_fused);
 }
 
-void launch_forward_rows(const float *src, const line_set &src_rows, float2 *dst, const line_set &dst_rows, int64_t n,
-	float scale, hipStream_t stream)
+void launch_forward_rows(const float *src, const line_set &src_rows, float2 *dst, const line_set &dst_rows,
+	const row_pairs &pairs, int64_t n, float scale, hipStream_t stream)
 {
 	if (direct_length(n))
 	{
-		launch_rfft_rows(real_f32, src, src_rows, static_cast<int>(n), nullptr, 0, dst, dst_rows, n, stream, true, scale);
+		launch_rfft_rows(real_f32, src, src_rows, static_cast<int>(n), nullptr, 0, dst, dst_rows, pairs, n, stream, true,
+			scale);
 		return;
 	}
 	const int64_t m = bluestein_length(n);
@@ -560,19 +564,19 @@ void launch_forward_rows(const float *src, const line_set &src_rows, float2 *dst
 	const float2 *tw = twiddles(m);
 	two_factor::with_class(p, [&](auto kind)
 		{
-			bluestein_rfft_rows_kernel<decltype(kind)::value><<<two_factor::blocks_for(src_rows.count, 2 * p.lines),
-				dim3(p.b, p.lines), two_factor::shared_bytes(p), stream>>>(src, src_rows, dst, dst_rows,
+			bluestein_rfft_rows_kernel<decltype(kind)::value><<<two_factor::blocks_for(line_count(pairs), p.lines),
+				dim3(p.b, p.lines), two_factor::shared_bytes(p), stream>>>(src, src_rows, dst, dst_rows, pairs,
 				static_cast<int>(n), p, tw, chirps, scale);
 		});
 	REXLIB_HIP_CHECK(hipGetLastError());
 }
 
-void launch_inverse_rows(const float2 *src, const line_set &src_rows, float *dst, const line_set &dst_rows, int64_t n,
-	float sign, float scale, hipStream_t stream)
+void launch_inverse_rows(const float2 *src, const line_set &src_rows, float *dst, const line_set &dst_rows,
+	const row_pairs &pairs, int64_t n, float sign, float scale, hipStream_t stream)
 {
 	if (direct_length(n))
 	{
-		launch_irfft_rows(src, src_rows, dst, dst_rows, n, scale, stream, true);
+		launch_irfft_rows(src, src_rows, dst, dst_rows, pairs, n, scale, stream, true);
 		return;
 	}
 	const int64_t m = bluestein_length(n);
@@ -581,8 +585,8 @@ void launch_inverse_rows(const float2 *src, const line_set &src_rows, float *dst
 	const float2 *tw = twiddles(m);
 	two_factor::with_class(p, [&](auto kind)
 		{
-			bluestein_irfft_rows_kernel<decltype(kind)::value><<<two_factor::blocks_for(src_rows.count, 2 * p.lines),
-				dim3(p.b, p.lines), two_factor::shared_bytes(p), stream>>>(src, src_rows, dst, dst_rows,
+			bluestein_irfft_rows_kernel<decltype(kind)::value><<<two_factor::blocks_for(line_count(pairs), p.lines),
+				dim3(p.b, p.lines), two_factor::shared_bytes(p), stream>>>(src, src_rows, dst, dst_rows, pairs,
 				static_cast<int>(n), p, tw, chirps, scale);
 		});
 	REXLIB_HIP_CHECK(hipGetLastError());
@@ -843,11 +847,23 @@ bool direct_transform(int kind, const rexlib_hip_array *in, const rexlib_hip_arr
 	}
 	const line_set rows = axis_lines(full, last);
 	const line_set half_rows = axis_lines(half, last);
+	// Consecutive rows belong to one transform along the axis before `last` (of
+	// those longer than 1) if it is transformed too, else to one each.
+	int64_t together = 1;
+	for (int a = last - 1; a >= 0; --a)
+	{
+		if (full[a] != 1)
+		{
+			together = std::find(live.begin(), live.end(), a) != live.end() ? full[a] : 1;
+			break;
+		}
+	}
+	const row_pairs pairs = whole_rows(together, rows.count);
 	if (kind == 1)
 	{
 		float2 *dst = static_cast<float2 *>(out->data);
-		launch_forward_rows(static_cast<const float *>(in->data), rows, dst, half_rows, n, live.empty() ? scale : 1.0f,
-			stream);
+		launch_forward_rows(static_cast<const float *>(in->data), rows, dst, half_rows, pairs, n,
+			live.empty() ? scale : 1.0f, stream);
 		for (std::size_t i = 0; i < live.size(); ++i)
 		{
 			const line_set lines = axis_lines(half, live[i]);
@@ -866,7 +882,7 @@ bool direct_transform(int kind, const rexlib_hip_array *in, const rexlib_hip_arr
 			src = work;
 		}
 	}
-	launch_inverse_rows(src, half_rows, static_cast<float *>(out->data), rows, n, sign, scale, stream);
+	launch_inverse_rows(src, half_rows, static_cast<float *>(out->data), rows, pairs, n, sign, scale, stream);
 	return true;
 }
 

@@ -2122,7 +2122,8 @@ void launch_rows(const pending_columns &columns, int64_t first, int64_t last, bo
 		first * rows.in_rows.s_outer * static_cast<int64_t>(rows.element_bytes);
 	const float *scales = rows.scales != nullptr ? rows.scales + first * rows.scale_stride : nullptr;
 	launch_rfft_rows(rows.kind, images, in, rows.m, scales, rows.scale_stride,
-		columns.spectra + first * rows.out_rows.s_outer, out, rows.n, stream, false, 1.0f, image_rows);
+		columns.spectra + first * rows.out_rows.s_outer, out, padded_rows(rows.m, rows.n, last - first, image_rows), rows.n,
+		stream);
 }
 
 // Host entry of every insertion: fills the workspace and launches.

@@ -119,18 +119,18 @@ int timing_begin(int kernel, hipStream_t stream);
 void timing_end(int token, hipStream_t stream);
 void kernel_timing(int kernel, double *total_ms, int64_t *launches);
 
+// `pairs` says which rows of `in_rows` and `out_rows` run, and together.
 // `any_length`: also the lengths with factors 7, 11 and 13 that the two-factor
-// kernels take (false: 2-3-5 lengths, others are refused). `image_rows`: only
-// the m rows of each image run, the zero rows of the padding are not written.
+// kernels take (false: 2-3-5 lengths, others are refused).
 void launch_rfft_rows(int kind, const void *in, const line_set &in_rows, int m, const float *scales,
-	int64_t scale_stride, float2 *out, const line_set &out_rows, int64_t n, hipStream_t stream,
-	bool any_length = false, float scale = 1.0f, bool image_rows = false);
+	int64_t scale_stride, float2 *out, const line_set &out_rows, const row_pairs &pairs, int64_t n, hipStream_t stream,
+	bool any_length = false, float scale = 1.0f);
 
 void launch_fft_lines(const float2 *src, const line_set &src_lines, float2 *dst, const line_set &dst_lines,
 	int64_t n, float sign, float scale, hipStream_t stream, bool any_length = false);
 
 void launch_irfft_rows(const float2 *src, const line_set &src_rows, float *dst, const line_set &dst_rows,
-	int64_t n, float scale, hipStream_t stream, bool any_length = false);
+	const row_pairs &pairs, int64_t n, float scale, hipStream_t stream, bool any_length = false);
 
 void launch_normalize(const float2 *num, const float *den, float2 *out, int64_t count, double threshold,
 	hipStream_t stream);
