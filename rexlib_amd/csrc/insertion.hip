@@ -1056,7 +1056,16 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 		const int tap_x = lane & 3;
 		const int tap_y = (lane >> 2) & 3;
 		const int tap_z = lane >> 4;
-		const int tap_voxel = tap_x + L::pitch_y * tap_y + L::pitch_z * tap_z;
+		// A sample's voxel times `reached` plus `tap_voxel` is the tap's. Windows of
+		// fewer than 4 taps send the surplus lanes to the padding of the rows,
+		// which is never added to the accumulators (64 rows at least, one a lane):
+		// their weights are 0, but a sample that is not finite times 0 is not.
+		// (Switching the lanes off for the access takes 4.4 to 5.3 ms below.)
+		const bool within = max(max(tap_x, tap_y), tap_z) < p.taps;
+		const int reached = within ? 1 : 0;
+		static_assert(T < 4 || (L::pitch_y > L::lx && L::ly * L::lz >= 64), "a padding voxel per lane");
+		const int tap_voxel = within ? tap_x + L::pitch_y * tap_y + L::pitch_z * tap_z :
+			L::lx + L::pitch_y * (lane % L::ly) + L::pitch_z * (lane / L::ly);
 		auto wide_round = [&]()
 		{
 			if constexpr (T == 4)
@@ -1110,7 +1119,7 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 				float wz = weights[12 * s + 8 + tap_z];
 				while (left != 0)
 				{
-					const int at = __builtin_amdgcn_readlane(voxel, s) + tap_voxel;
+					const int at = __mul24(__builtin_amdgcn_readlane(voxel, s), reached) + tap_voxel;
 					const float wt = wz * wy * wx;
 					const float re = lane_value(q.re, s);
 					const float imaginary = lane_value(im, s);

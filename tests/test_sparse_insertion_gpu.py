@@ -79,3 +79,23 @@ def test_kaiser_bessel_bricks_match_the_oracle(half_width, shape, n, big, slices
     # The reference's bar for this window (5e-4: its table and its edge).
     assert np.abs(num - ref[0]).max() <= 5e-4 * max(1.0, float(np.abs(ref[0]).max()))
     assert np.abs(den - ref[1]).max() <= 5e-4 * max(1.0, float(np.abs(ref[1]).max()))
+
+
+# 2 taps (half-width 1), 3 (1.2, 1.5) and 4 of the layout's 4.
+@pytest.mark.parametrize("half_width", [1.0, 1.2, 1.5, 2.0])
+@pytest.mark.parametrize("big", [16, 17])
+def test_an_infinite_sample_stays_within_its_kaiser_bessel_window(half_width, big):
+    n = 8
+    taps = int(np.ceil(2 * half_width))
+    inputs = make_case("plain", n, big, seed=1, slices=1, zero_accumulators=True)
+    inputs[2][...] = 0.0
+    inputs[2][0, 1, 2] = np.inf  # k = (2, 1)
+    inputs[3][...] = [[[0.9, 0.1, 0.0, 0.0], [-0.1, 0.8, 0.3, 0.0], [0.0, 0.0, 1.0, 0.0]]]
+    inputs[4][...] = 1.0
+    position = (big / n) * (2 * inputs[3][0, 0, :3] + inputs[3][0, 1, :3])
+    reach = [{int(f) % big for f in np.floor(c - half_width) + 1 + np.arange(taps)} for c in position]
+    num, _ = hip_insert("plain", inputs, oracle.Window.kaiser_bessel(half_width, 6.0))
+    spoilt = np.argwhere(~np.isfinite(num))
+    assert len(spoilt) > 0
+    for z, y, x in spoilt:
+        assert x in reach[0] and y in reach[1] and z in reach[2]
