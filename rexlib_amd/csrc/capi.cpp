@@ -1055,6 +1055,10 @@ int rexlib_hip_predicted_weights(const rexlib_hip_array *denominator, const rexl
 		expect_dtype(*parameters_f16, REXLIB_HIP_FLOAT16, "mlp float16 parameters");
 		expect_dtype(*parameters_f32, REXLIB_HIP_FLOAT32, "mlp float32 parameters");
 		const int64_t big = core_extent(*denominator, 3);
+		if (big < 1)
+		{
+			fail(REXLIB_HIP_INVALID_ARGUMENT, "predicted_weights: the volume extent must be at least 1");
+		}
 		expect_core(*denominator, "predicted_weights denominator", {big, big, big / 2 + 1});
 		expect_core(*table, "predicted_weights table", {8, 33, 64, 8});
 		check_same_shape(*denominator, *weights, "predicted_weights output");

@@ -245,3 +245,14 @@ def test_insertion_tuning_for_one_window_family():
                                          table["256"]["extent_z"]), table["256"]["share"])
     finally:
         tune.clear_tuning()
+
+
+def test_predicted_weights_of_an_empty_grid_are_refused():
+    """The kernel divides by the groups of a plane, which extent 0 has none of."""
+    lib = N.library()
+    count = lib.rexlib_hip_mlp_parameter_count()
+    den, out = fake((0, 0, 1), N.FLOAT32), fake((0, 0, 1), N.FLOAT32, 0x2000)
+    table = fake((8, 33, 64, 8), N.FLOAT32, 0x3000)
+    f16, f32 = fake((count,), N.FLOAT16, 0x4000), fake((count,), N.FLOAT32, 0x5000)
+    assert lib.rexlib_hip_predicted_weights(ctypes.byref(den), ctypes.byref(table), 1.0, ctypes.byref(f16),
+                                            ctypes.byref(f32), ctypes.byref(out), None) == N.INVALID_ARGUMENT
