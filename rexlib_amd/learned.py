@@ -65,8 +65,14 @@ def coverage_table(transforms: torch.Tensor, big: int) -> torch.Tensor:
 
 def density_scale(den: torch.Tensor) -> float:
     """1 / mean of the positive weights (1 when there are none)."""
-    out = torch.empty(1, dtype=torch.float64, device=den.device)
-    N.check(N.library().rexlib_hip_density_scale(N.array(den.contiguous()), ctypes.c_void_p(out.data_ptr()), _stream()))
+    if not (den.is_cuda and den.dtype == torch.float32):
+        # The kernel reads float32 in device memory; any other tensor is torch's.
+        positive = den[den > 0]
+        return 1.0 / float(positive.mean()) if positive.numel() else 1.0
+    with torch.cuda.device(den.device):
+        out = torch.empty(1, dtype=torch.float64, device=den.device)
+        N.check(N.library().rexlib_hip_density_scale(N.array(den.contiguous()), ctypes.c_void_p(out.data_ptr()),
+                                                     _stream()))
     return float(out)
 
 

@@ -2,9 +2,11 @@
 density compensation, pinned on the CPU."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from oracle import mlp
+from rexlib_amd import learned
 
 P = sum(int(np.prod(s)) for _, s in mlp.SHAPES)
 
@@ -153,3 +155,13 @@ def test_features_take_the_nyquist_index_as_negative():
     f = oracle.compensation_features(den, table, 1.0)
     assert np.array_equal(f[8, 0, 0, 2:], np.arange(8))
     assert np.array_equal(f[0, 8, 0, 2:], 10 + np.arange(8))
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32, torch.bfloat16])
+def test_density_scale_of_any_device_and_type(device, dtype):
+    den = torch.tensor([[4.0, 0.0, -1.0], [2.0, 6.0, float("nan")]], dtype=dtype, device=device)
+    assert learned.density_scale(den) == pytest.approx(0.25, rel=1e-6)
+    assert learned.density_scale(den.t()) == pytest.approx(0.25, rel=1e-6)
+    assert learned.density_scale(torch.zeros((3, 2), dtype=dtype, device=device)) == 1.0
+    assert learned.density_scale(torch.zeros((0, 0, 1), dtype=dtype, device=device)) == 1.0
