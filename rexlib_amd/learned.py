@@ -65,7 +65,7 @@ def coverage_table(transforms: torch.Tensor, big: int) -> torch.Tensor:
 
 def density_scale(den: torch.Tensor) -> float:
     """1 / mean of the positive weights (1 when there are none)."""
-    if not (den.is_cuda and den.dtype == torch.float32):
+    if not (den.is_cuda and den.dtype == torch.float32 and den.numel()):
         # The kernel reads float32 in device memory; any other tensor is torch's.
         positive = den[den > 0]
         return 1.0 / float(positive.mean()) if positive.numel() else 1.0
