@@ -330,9 +330,10 @@ struct voxel_features
 
 __device__ inline voxel_features features_of(float den, float density_scale, int x, int sy, int sz, int big)
 {
-	// Signed frequencies as numpy's fftfreq: index N/2 is -N/2.
-	const int y = sy < big / 2 ? sy : sy - big;
-	const int z = sz < big / 2 ? sz : sz - big;
+	// Signed frequencies as numpy's fftfreq: index N/2 is -N/2 of an even N, +N/2
+	// of an odd one.
+	const int y = sy < (big + 1) / 2 ? sy : sy - big;
+	const int z = sz < (big + 1) / 2 ? sz : sz - big;
 	// log(1 + v) by the hardware logarithm, corrected for the rounding of
 	// 1 + v: with u = fl(1 + v), log(u) v / (u - 1) keeps the relative error
 	// near one ulp for small v as well (u = 1 gives v itself).

@@ -55,3 +55,27 @@ def test_density_scale_is_the_reciprocal_mean_of_the_positive_weights():
     positive = den[den > 0].double()
     assert abs(learned.density_scale(den) * float(positive.mean()) - 1.0) < 1e-12
     assert learned.density_scale(torch.zeros((4, 4, 3), device="cuda")) == 1.0
+
+
+# Index N/2 of an odd N is the frequency +N/2 (of an even N, -N/2).
+@pytest.mark.parametrize("big", [15, 16, 33, 45])
+def test_features_of_odd_and_even_extents_match_the_oracle(big):
+    den = weight_volume(big, big)
+    table = np.random.default_rng(big).uniform(size=(8, 33, 64, 8)).astype(np.float32)
+    got = learned.features(torch.from_numpy(den).cuda(), torch.from_numpy(table).cuda(), 0.7).float().cpu().numpy()
+    ref = oracle.compensation_features(den, table, 0.7)
+    np.testing.assert_allclose(got[..., :2], ref[..., :2], rtol=2e-3, atol=2e-3)  # float16
+    # (A direction within a float32 rounding of two grid directions may take either.)
+    same = np.all(np.abs(got[..., 2:10] - ref[..., 2:]) <= 2e-3, axis=-1)
+    assert same.mean() > 0.999
+
+
+@pytest.mark.parametrize("big", [15, 16, 33])
+def test_predicted_weights_of_a_plane_that_mirrors_itself(big):
+    # A table that depends on the radius alone: (0, y, z) and (0, -y, -z) have
+    # the same features, so the same weights, to the last bit.
+    den = torch.from_numpy(weight_volume(big, 5)).cuda()
+    table = torch.rand((8, 1, 1, 8), generator=torch.Generator().manual_seed(2)).expand(8, 33, 64, 8).contiguous().cuda()
+    plane = learned.CompensationModel(seed=3).weights(den, table)[..., 0]
+    index = (-torch.arange(big)) % big
+    assert torch.equal(plane, plane[index][:, index])
