@@ -60,6 +60,8 @@ EXPORTS = [
     "rexlib_hip_set_insertion_tuning",
     "rexlib_hip_set_insertion_tuning_for_window",
     "rexlib_hip_get_insertion_tuning",
+    "rexlib_hip_insertion_bricks",
+    "rexlib_hip_drop_insertion_tuning",
     "rexlib_hip_clear_insertion_tuning",
     "rexlib_hip_insert_slices",
     "rexlib_hip_insert_weighted_slices",
@@ -121,6 +123,10 @@ def library() -> ctypes.CDLL:
     lib.rexlib_hip_set_insertion_tuning_for_window.restype = ctypes.c_int
     lib.rexlib_hip_get_insertion_tuning.argtypes = [ctypes.c_int32] + [P(ctypes.c_int32)] * 4
     lib.rexlib_hip_get_insertion_tuning.restype = ctypes.c_int
+    lib.rexlib_hip_insertion_bricks.argtypes = [ctypes.c_int32] * 3 + [ctypes.c_int64] + [P(ctypes.c_int32)] * 5
+    lib.rexlib_hip_insertion_bricks.restype = ctypes.c_int
+    lib.rexlib_hip_drop_insertion_tuning.argtypes = [ctypes.c_int32] * 2 + [P(ctypes.c_int32)] * 4
+    lib.rexlib_hip_drop_insertion_tuning.restype = ctypes.c_int
     lib.rexlib_hip_clear_insertion_tuning.argtypes = []
     lib.rexlib_hip_clear_insertion_tuning.restype = None
     lib.rexlib_hip_insert_slices.argtypes = [A, A, A, A, A, W, A, A, vp]

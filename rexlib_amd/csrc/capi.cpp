@@ -520,6 +520,36 @@ int rexlib_hip_get_insertion_tuning(int32_t extent, int32_t *extent_x, int32_t *
 		});
 }
 
+int rexlib_hip_insertion_bricks(int32_t n, int32_t extent, int32_t taps, int64_t slices, int32_t *extent_x,
+	int32_t *extent_y, int32_t *extent_z, int32_t *share, int32_t *own_voxels)
+{
+	return guarded([&]
+	{
+		if (extent_x == nullptr || extent_y == nullptr || extent_z == nullptr || share == nullptr ||
+			own_voxels == nullptr)
+		{
+			fail(REXLIB_HIP_INVALID_ARGUMENT, "insertion_bricks: null output");
+		}
+		rexlib_hip::insertion_bricks(n, extent, taps, slices, extent_x, extent_y, extent_z, share, own_voxels);
+	});
+}
+
+int rexlib_hip_drop_insertion_tuning(int32_t extent, int32_t taps, int32_t *extent_x, int32_t *extent_y,
+	int32_t *extent_z, int32_t *share)
+{
+	return guarded([&]
+	{
+		if (extent_x == nullptr || extent_y == nullptr || extent_z == nullptr || share == nullptr)
+		{
+			fail(REXLIB_HIP_INVALID_ARGUMENT, "drop_insertion_tuning: null output");
+		}
+		if (!rexlib_hip::drop_insertion_tuning(extent, taps, extent_x, extent_y, extent_z, share))
+		{
+			*extent_x = *extent_y = *extent_z = *share = 0;
+		}
+	});
+}
+
 void rexlib_hip_clear_insertion_tuning(void)
 {
 	rexlib_hip::clear_insertion_tuning();

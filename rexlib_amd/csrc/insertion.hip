@@ -1656,9 +1656,6 @@ struct brick_tuning
 	int share;
 };
 
-// What the getter reports for an extent without an entry.
-constexpr brick_tuning default_brick_tuning{16, 8, 6, 256};
-
 // What calls take without an entry: over 64 to 512 voxels and 16 to 2,048
 // slices, 8 x 8 x 8 bricks and 512 plane hits per task stay within a tenth of
 // the fastest shape for up to two taps per axis, and 8 x 6 x 6 for four (16 x
@@ -1668,7 +1665,8 @@ constexpr brick_tuning untuned_bricks{8, 8, 8, 512};
 constexpr brick_tuning untuned_wide_bricks{8, 6, 6, 512};
 
 // Bricks that own voxels: a cell shell of T - 1 is walked twice, so the brick
-// has to be a large one of the small ones.
+// has to be a large one of the small ones. (The share is an entry's, if there
+// is one.)
 constexpr brick_tuning voxel_tuning{8, 8, 8, 512};
 
 std::mutex tuning_mutex;
@@ -2044,13 +2042,38 @@ const int4 *brick_tasks(int big, int64_t slices, const brick_tuning &tuning, int
 // the other does, in samples per voxel of the stored half: 256 slices of 256^2
 // into 512^3 (0.1 samples per voxel) take 1.15 against 1.75 ms, 512 of 256^2
 // into 256^3 (1.6) 0.47 against 0.51 ms, 1,024 (3.1) 0.75 against 0.71 ms. Four
-// taps would insert 4 times the samples; a fixed workspace buffer keeps the
-// smaller task list of cells.
-bool bricks_own_voxels(const insertion_params &p, int64_t slices, int taps, const workspace_source &workspace)
+// taps would insert 4 times the samples; a fixed workspace buffer (`fixed`) keeps
+// the smaller task list of cells.
+bool bricks_own_voxels(int n, int big, int64_t slices, int taps, bool fixed)
 {
-	const double samples = 0.125 * 3.14159265 * p.n * p.n * static_cast<double>(slice_bucket(slices));
-	const double voxels = 0.5 * p.big * p.big * static_cast<double>(p.big);
-	return taps <= 2 && workspace.arena == nullptr && samples < 1.6 * voxels;
+	const double samples = 0.125 * 3.14159265 * n * n * static_cast<double>(slice_bucket(slices));
+	const double voxels = 0.5 * big * big * static_cast<double>(big);
+	return taps <= 2 && !fixed && samples < 1.6 * voxels;
+}
+
+// The bricks of cells of a window of `taps` per axis of the brick layout.
+brick_tuning cell_bricks(int big, int taps)
+{
+	return tuning_for(big, taps, taps == 4 ? untuned_wide_bricks : untuned_bricks);
+}
+
+// The bricks of voxels: their own shape, an entry's share.
+brick_tuning voxel_bricks(int big, int taps)
+{
+	brick_tuning t = tuning_for(big, taps, voxel_tuning);
+	t.ex = voxel_tuning.ex;
+	t.ey = voxel_tuning.ey;
+	t.ez = voxel_tuning.ez;
+	return t;
+}
+
+// Prepared samples take 12 bytes per stored element of a slice; a chunk of slices
+// stays within 4 GiB.
+constexpr int64_t prepared_limit = int64_t(4) << 30;
+
+int64_t prepared_bytes(int n)
+{
+	return static_cast<int64_t>(n) * (n / 2 + 1) * static_cast<int64_t>(sizeof(prepared_sample));
 }
 
 // Whether an out-of-place call of bricks that own voxels still copies the inputs
@@ -2100,11 +2123,58 @@ void set_insertion_tuning(int extent, int taps, int extent_x, int extent_y, int 
 
 void get_insertion_tuning(int extent, int *extent_x, int *extent_y, int *extent_z, int *share)
 {
-	const brick_tuning t = tuning_for(extent, 0, default_brick_tuning);
+	const brick_tuning t = tuning_for(extent, 0, untuned_bricks);
 	*extent_x = t.ex;
 	*extent_y = t.ey;
 	*extent_z = t.ez;
 	*share = t.share;
+}
+
+static void check_window_taps(int taps)
+{
+	if (taps != 1 && taps != 2 && taps != 4)
+	{
+		fail(REXLIB_HIP_INVALID_ARGUMENT, "insertion tuning: taps per axis of a window are 1 (nearest), 2 (trilinear) "
+			"or 4 (Kaiser-Bessel)");
+	}
+}
+
+void insertion_bricks(int n, int extent, int taps, int64_t slices, int *extent_x, int *extent_y, int *extent_z,
+	int *share, int *own_voxels)
+{
+	check_window_taps(taps);
+	if (n < 1 || extent < 1 || slices < 1)
+	{
+		fail(REXLIB_HIP_INVALID_ARGUMENT, "insertion bricks: the extents and the number of slices must be positive");
+	}
+	const int64_t chunk = std::min(slices, std::max<int64_t>(1, prepared_limit / prepared_bytes(n)));
+	const bool voxels = bricks_own_voxels(n, extent, chunk, taps, false);
+	const brick_tuning t = voxels ? voxel_bricks(extent, taps) : cell_bricks(extent, taps);
+	*extent_x = t.ex;
+	*extent_y = t.ey;
+	*extent_z = t.ez;
+	*share = t.share;
+	*own_voxels = voxels ? 1 : 0;
+}
+
+bool drop_insertion_tuning(int extent, int taps, int *extent_x, int *extent_y, int *extent_z, int *share)
+{
+	if (taps != 0)
+	{
+		check_window_taps(taps);
+	}
+	std::lock_guard<std::mutex> lock(tuning_mutex);
+	const auto found = tuning_table.find(extent + taps * taps_key);
+	if (extent < 0 || extent >= taps_key || found == tuning_table.end())
+	{
+		return false;
+	}
+	*extent_x = found->second.ex;
+	*extent_y = found->second.ey;
+	*extent_z = found->second.ez;
+	*share = found->second.share;
+	tuning_table.erase(found);
+	return true;
 }
 
 void clear_insertion_tuning()
@@ -2189,18 +2259,16 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 		volume_phase_kernel<<<(p.big + 255) / 256, 256, 0, stream>>>(vphase, p.big);
 		REXLIB_HIP_CHECK(hipGetLastError());
 	}
-	// Prepared samples take 12 bytes per stored element; the slices of one
-	// call go through in chunks that keep them within 4 GiB, and with a fixed
-	// workspace buffer within what it has left beside the task list. The
+	// The slices of one call go through in chunks whose prepared samples stay
+	// within prepared_limit, and with a fixed workspace buffer within what it has
+	// left beside the task list. The
 	// brick schedule needs the window to span at most 4 voxels; wider
 	// Kaiser-Bessel windows take the scatter schedule, and so do calls whose
 	// workspace buffer cannot hold one slice's prepared samples.
-	const int64_t per_slice = static_cast<int64_t>(p.n) * p.h * static_cast<int64_t>(sizeof(prepared_sample)) *
-		p.map.kept_count;
-	const int64_t limit = int64_t(4) << 30;
+	const int64_t per_slice = prepared_bytes(p.n) * p.map.kept_count;
 	// Taps per axis of the brick layout: 1, 2, or 4 for every Kaiser-Bessel window.
 	const int layout_taps = p.profile == REXLIB_HIP_BOX ? 1 : (p.profile == REXLIB_HIP_TRIANGLE ? 2 : 4);
-	brick_tuning tuning = tuning_for(p.big, layout_taps, layout_taps == 4 ? untuned_wide_bricks : untuned_bricks);
+	brick_tuning tuning = cell_bricks(p.big, layout_taps);
 	int64_t chunk_count = 0;
 	if (schedule != schedule_scatter && p.taps <= 4 && p.map.kept_count <= 65535)
 	{
@@ -2208,7 +2276,7 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 		{
 			const std::size_t left = workspace.remaining();
 			return left <= reserved + 512 ? int64_t(0) :
-				std::min<int64_t>(limit, static_cast<int64_t>(std::min<std::size_t>(left - reserved - 512,
+				std::min<int64_t>(prepared_limit, static_cast<int64_t>(std::min<std::size_t>(left - reserved - 512,
 					std::size_t(1) << 40)));
 		};
 		chunk_count = std::min<int64_t>(p.map.reduced_count, room(0) / per_slice);
@@ -2221,10 +2289,10 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 		}
 	}
 	const bool brick = chunk_count >= 1;
-	const bool voxels = brick && bricks_own_voxels(p, chunk_count, layout_taps, workspace);
+	const bool voxels = brick && bricks_own_voxels(p.n, p.big, chunk_count, layout_taps, workspace.arena != nullptr);
 	if (voxels)
 	{
-		tuning = voxel_tuning;
+		tuning = voxel_bricks(p.big, layout_taps);
 	}
 	// Bricks that own voxels read the inputs themselves, unless most of them
 	// would have nothing to add.

@@ -112,6 +112,12 @@ void insert_ctf_slices_within(const rexlib_hip_array *numerator, const rexlib_hi
 void set_insertion_tuning(int extent, int taps, int extent_x, int extent_y, int extent_z, int share);
 void get_insertion_tuning(int extent, int *extent_x, int *extent_y, int *extent_z, int *share);
 void clear_insertion_tuning();
+// The bricks that a call without a fixed workspace takes (own_voxels: 1 when they
+// own voxels, whose shape is no entry's).
+void insertion_bricks(int n, int extent, int taps, int64_t slices, int *extent_x, int *extent_y, int *extent_z,
+	int *share, int *own_voxels);
+// Removes one entry and gives its values; false when there is none.
+bool drop_insertion_tuning(int extent, int taps, int *extent_x, int *extent_y, int *extent_z, int *share);
 
 // Event timing of single kernels (ids as REXLIB_HIP_KERNEL_*).
 void set_kernel_timing(bool enable);

@@ -5,7 +5,9 @@ the insertion on the device for every brick shape the library holds (the
 brick's first-tap cells along x, y and z) and several shares (expected plane
 hits per task, which split busy bricks), checks every configuration's sums
 against the first one's, and records the fastest per volume extent N in a
-JSON table. ``apply_all()`` hands the
+JSON table. A sparse workload (below 1.6 samples per voxel, at most two taps)
+takes bricks of one fixed shape: only its shares are timed, and nothing is
+recorded. ``apply_all()`` hands the
 whole table to the library, which then picks each call's entry by its volume
 extent, so reconstructions of different sizes need no switching between
 calls.
@@ -28,7 +30,8 @@ TABLE = os.path.join(HERE, "tuning.json")
 # (x, y, z) extents of the bricks the library is built for.
 SHAPES = ((16, 8, 6), (16, 8, 8), (16, 16, 8), (8, 8, 8), (8, 8, 6), (8, 8, 4), (8, 6, 6))
 SHARES = (32, 64, 128, 256, 512, 1024)
-DEFAULT = {"extent_x": 16, "extent_y": 8, "extent_z": 6, "share": 256}
+# What calls take without an entry (with a Kaiser-Bessel window: 8, 6, 6 and 512).
+DEFAULT = {"extent_x": 8, "extent_y": 8, "extent_z": 8, "share": 512}
 
 
 def load_table(path: str = TABLE) -> dict:
@@ -52,11 +55,32 @@ def set_tuning(extent: int, shape, share: int, taps: int = 0) -> None:
 
 
 def get_tuning(extent: int):
-    """((extent_x, extent_y, extent_z), share) that calls with volume extent ``extent`` use."""
+    """((extent_x, extent_y, extent_z), share) that calls with volume extent
+    ``extent`` take unless their window family has an entry of its own
+    (``bricks_of``: what one call takes)."""
     from . import _native as N
     v = [ctypes.c_int32() for _ in range(4)]
     N.check(N.library().rexlib_hip_get_insertion_tuning(int(extent), *[ctypes.byref(x) for x in v]))
     return (v[0].value, v[1].value, v[2].value), v[3].value
+
+
+def bricks_of(n: int, big: int, slices: int, taps: int = 2):
+    """((extent_x, extent_y, extent_z), share, own voxels) of a call of
+    ``slices`` slices of extent ``n`` into a volume of extent ``big``. Bricks
+    that own voxels (sparse calls) have a shape that no entry changes."""
+    from . import _native as N
+    v = [ctypes.c_int32() for _ in range(5)]
+    N.check(N.library().rexlib_hip_insertion_bricks(int(n), int(big), int(taps), int(slices),
+                                                    *[ctypes.byref(x) for x in v]))
+    return (v[0].value, v[1].value, v[2].value), v[3].value, bool(v[4].value)
+
+
+def drop_tuning(extent: int, taps: int = 0):
+    """Drops one entry; (shape, share) it held, or None."""
+    from . import _native as N
+    v = [ctypes.c_int32() for _ in range(4)]
+    N.check(N.library().rexlib_hip_drop_insertion_tuning(int(extent), int(taps), *[ctypes.byref(x) for x in v]))
+    return ((v[0].value, v[1].value, v[2].value), v[3].value) if v[3].value else None
 
 
 def clear_tuning() -> None:
@@ -138,13 +162,16 @@ def rel_l2(a, b) -> float:
 
 def tune(n: int, big: int, launch: int, path: str = TABLE, verbose: bool = True, taps: int = 0) -> dict:
     """Time every brick shape and share; record the fastest under "N" (taps
-    0: every window, timed with trilinear) or "N/taps" (one window family)."""
+    0: every window, timed with trilinear) or "N/taps" (one window family).
+    The library's other entries stay as they are, and so does this one when the
+    workload reads only its share ("recorded" is False then) or a trial fails."""
     slices, transforms, ctf = workload(n, big, launch)
     results = []
     reference = None
-    previous = get_tuning(big)
+    shape, _, sparse = bricks_of(n, big, launch, taps or 2)
+    previous = drop_tuning(big, taps)
     try:
-        for shape in SHAPES:
+        for shape in (shape,) if sparse else SHAPES:
             for share in SHARES:
                 set_tuning(big, shape, share, taps)
                 ms, sums = time_insertion(n, big, slices, transforms, ctf, taps=taps)
@@ -160,8 +187,14 @@ def tune(n: int, big: int, launch: int, path: str = TABLE, verbose: bool = True,
                     print(f"n={n} N={big} L={launch} brick {shape[0]}x{shape[1]}x{shape[2]} share={share}: "
                           f"{ms:.3f} ms (rel-L2 to the first {error:.1e})", flush=True)
     finally:
-        set_tuning(big, *previous)
+        drop_tuning(big, taps)
+        if previous is not None:
+            set_tuning(big, *previous, taps)
     best = min(results, key=lambda r: r["ms"])
+    if sparse:
+        if verbose:
+            print(f"n={n} N={big} L={launch}: bricks that own voxels have one shape; no entry recorded", flush=True)
+        return {"best": best, "all": results, "recorded": False}
     table = load_table(path)
     table[f"{big}/{taps}" if taps else str(big)] = {
         "extent_x": best["extent_x"], "extent_y": best["extent_y"], "extent_z": best["extent_z"],
@@ -170,7 +203,7 @@ def tune(n: int, big: int, launch: int, path: str = TABLE, verbose: bool = True,
     with open(path, "w") as f:
         json.dump(table, f, indent=1, sort_keys=True)
     set_tuning(big, (best["extent_x"], best["extent_y"], best["extent_z"]), best["share"], taps)
-    return {"best": best, "all": results}
+    return {"best": best, "all": results, "recorded": True}
 
 
 def main():

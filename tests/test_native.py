@@ -208,10 +208,10 @@ def test_insertion_tuning_is_a_table_per_volume_extent():
     lib = N.library()
     tune.clear_tuning()
     try:
-        assert tune.get_tuning(256) == ((16, 8, 6), 256)
+        assert tune.get_tuning(256) == ((8, 8, 8), 512)
         tune.set_tuning(256, (16, 16, 8), 128)
         assert tune.get_tuning(256) == ((16, 16, 8), 128)
-        assert tune.get_tuning(64) == ((16, 8, 6), 256)
+        assert tune.get_tuning(64) == ((8, 8, 8), 512)
         tune.set_tuning(0, (8, 8, 8), 64)
         assert tune.get_tuning(64) == ((8, 8, 8), 64)
         assert tune.get_tuning(256) == ((16, 16, 8), 128)
@@ -222,7 +222,7 @@ def test_insertion_tuning_is_a_table_per_volume_extent():
         assert tune.get_tuning(96) == ((8, 8, 8), 64)
     finally:
         tune.clear_tuning()
-    assert tune.get_tuning(256) == ((16, 8, 6), 256)
+    assert tune.get_tuning(256) == ((8, 8, 8), 512)
 
 
 def test_insertion_tuning_for_one_window_family():
@@ -256,3 +256,78 @@ def test_predicted_weights_of_an_empty_grid_are_refused():
     f16, f32 = fake((count,), N.FLOAT16, 0x4000), fake((count,), N.FLOAT32, 0x5000)
     assert lib.rexlib_hip_predicted_weights(ctypes.byref(den), ctypes.byref(table), 1.0, ctypes.byref(f16),
                                             ctypes.byref(f32), ctypes.byref(out), None) == N.INVALID_ARGUMENT
+
+
+def test_the_bricks_a_call_takes():
+    """What the getter and bricks_of report is what calls take: the defaults
+    per window family, the entries, and the fixed shape of sparse calls."""
+    from rexlib_amd import tune
+    lib = N.library()
+    tune.clear_tuning()
+    try:
+        dense, sparse = (256, 256, 4096), (256, 512, 256)
+        assert tune.bricks_of(*dense) == (*tune.get_tuning(256), False)
+        assert tune.get_tuning(256) == ((tune.DEFAULT["extent_x"], tune.DEFAULT["extent_y"],
+                                         tune.DEFAULT["extent_z"]), tune.DEFAULT["share"])
+        assert tune.bricks_of(*dense, taps=4) == ((8, 6, 6), 512, False)
+        assert tune.bricks_of(*sparse) == ((8, 8, 8), 512, True)
+        assert tune.bricks_of(*sparse, taps=4) == ((8, 6, 6), 512, False)  # four taps keep cells
+        tune.set_tuning(256, (16, 8, 6), 64)
+        tune.set_tuning(512, (16, 8, 6), 64)
+        tune.set_tuning(256, (8, 8, 4), 32, taps=4)
+        assert tune.bricks_of(*dense, taps=1) == ((16, 8, 6), 64, False)
+        assert tune.bricks_of(*dense, taps=4) == ((8, 8, 4), 32, False)
+        assert tune.bricks_of(*sparse) == ((8, 8, 8), 64, True)  # the entry's share
+        # The line between them: the slices' next power of two.
+        assert tune.bricks_of(256, 256, 512)[2] and not tune.bricks_of(256, 256, 513)[2]
+        assert tune.drop_tuning(256, 1) is None
+        assert tune.drop_tuning(256, 4) == ((8, 8, 4), 32)
+        assert tune.bricks_of(*dense, taps=4) == ((16, 8, 6), 64, False)
+        assert tune.drop_tuning(256) == ((16, 8, 6), 64) and tune.drop_tuning(256) is None
+        v = [ctypes.byref(ctypes.c_int32()) for _ in range(5)]
+        assert lib.rexlib_hip_insertion_bricks(256, 256, 3, 1, *v) == N.INVALID_ARGUMENT
+        assert lib.rexlib_hip_insertion_bricks(0, 256, 2, 1, *v) == N.INVALID_ARGUMENT
+        assert lib.rexlib_hip_insertion_bricks(256, 256, 2, 0, *v) == N.INVALID_ARGUMENT
+        assert lib.rexlib_hip_drop_insertion_tuning(256, 3, *v[:4]) == N.INVALID_ARGUMENT
+    finally:
+        tune.clear_tuning()
+
+
+def test_tuning_one_window_family_leaves_the_others(tmp_path, monkeypatch):
+    """The autotuner's trials, timed by a stand-in: every other entry (or the
+    lack of one) is as before; a failure and a sparse workload, which has one
+    shape, record nothing."""
+    from rexlib_amd import tune
+    path = str(tmp_path / "table.json")
+    monkeypatch.setattr(tune, "workload", lambda *a: (None, None, None))
+    monkeypatch.setattr(tune, "rel_l2", lambda a, b: 0.0)
+    tried = []
+
+    def timed(n, big, *rest, taps=0):
+        shape, share, _ = tune.bricks_of(n, big, launch, taps or 2)
+        tried.append((shape, share))
+        if shape == broken:
+            raise RuntimeError("no time")
+        return (1.0 if (shape, share) == ((8, 8, 4), 64) else 2.0), (0, 0)
+
+    monkeypatch.setattr(tune, "time_insertion", timed)
+    tune.clear_tuning()
+    try:
+        launch, broken = 4096, None
+        tune.tune(256, 256, launch, path, verbose=False, taps=4)
+        assert tried == [(shape, share) for shape in tune.SHAPES for share in tune.SHARES]
+        assert tune.bricks_of(256, 256, launch, 4) == ((8, 8, 4), 64, False)
+        assert tune.bricks_of(256, 256, launch, 2) == (*tune.get_tuning(256), False) == ((8, 8, 8), 512, False)
+        broken = (16, 16, 8)
+        for taps, before in ((4, ((8, 8, 4), 64, False)), (0, ((8, 8, 8), 512, False))):
+            with pytest.raises(RuntimeError):
+                tune.tune(256, 256, launch, path, verbose=False, taps=taps)
+            assert tune.bricks_of(256, 256, launch, taps or 2) == before
+        recorded = tune.load_table(path)
+        assert list(recorded) == ["256/4"]
+        launch, broken, tried[:] = 64, None, []
+        assert tune.tune(64, 512, launch, path, verbose=False)["recorded"] is False
+        assert tried == [((8, 8, 8), share) for share in tune.SHARES]
+        assert tune.load_table(path) == recorded and tune.drop_tuning(512) is None
+    finally:
+        tune.clear_tuning()
