@@ -95,7 +95,7 @@ def _lib():
         i64 = ctypes.c_int64
         p = ctypes.c_void_p
         _oracle.oracle_insert_f64.argtypes = [ctypes.c_int, ctypes.c_int, d, d, i64, i64, i64, i64,
-                                              p, p, p, p, p, p, d, d, d, d]
+                                              p, p, p, p, p, p, d, d, d, d, ctypes.c_int]
         _oracle.oracle_insert_f64.restype = None
         _oracle.oracle_bessel_i0.argtypes = [d]
         _oracle.oracle_bessel_i0.restype = d
@@ -232,8 +232,12 @@ def _run_expanded(variant, inputs, fn):
     return out_num.reshape(inputs[0].shape), out_den.reshape(inputs[1].shape)
 
 
-def insert_f64(variant: str, inputs, window: Window, optics: Optics = Optics(), pixel_size: float = 1.0):
-    """Brute-force FP64 insertion; ``inputs`` in the operation's operand order."""
+def insert_f64(variant: str, inputs, window: Window, optics: Optics = Optics(), pixel_size: float = 1.0,
+               float32_positions: bool = False):
+    """Brute-force FP64 insertion; ``inputs`` in the operation's operand order.
+    With ``float32_positions`` the sample positions round as the float32
+    kernels' do (the sums stay in float64): a nearest window then puts every
+    sample in the same voxel."""
     lib = _lib()
 
     def fn(K, B, num, den, slices, transforms, radial, extra):
@@ -248,7 +252,7 @@ def insert_f64(variant: str, inputs, window: Window, optics: Optics = Optics(), 
         lib.oracle_insert_f64(VARIANTS[variant], PROFILES[window.profile], window.half_width,
                               window.shape, n, big, K, B, _ptr(num), _ptr(den), _ptr(sl), _ptr(tr),
                               _ptr(ra), _ptr(ex), optics.voltage, optics.spherical_aberration,
-                              optics.amplitude_contrast, float(pixel_size))
+                              optics.amplitude_contrast, float(pixel_size), int(float32_positions))
         return num, den
 
     return _run_expanded(variant, inputs, fn)

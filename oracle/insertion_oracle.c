@@ -67,11 +67,18 @@ double oracle_window_weight(int profile, double half_width, double shape, double
 
 /* The voxels a sample at `c` reaches along one axis, as [first, last]
  * (fixture slice_insertion_cases.hpp:327-358). Box rounds halves away from 0
- * like std::round. */
-static void reached(int profile, double half_width, double c, int64_t *first, int64_t *last)
+ * like std::round; in float32 the half is added in float32
+ * (box_window.inl:16-34). */
+static void reached(int profile, double half_width, double c, int float32_positions, int64_t *first, int64_t *last)
 {
 	switch (profile) {
 	case PROFILE_BOX:
+		if (float32_positions) {
+			const float f = (float)c;
+			const float moved = f + (f < 0.0f ? -0.5f : 0.5f);
+			*first = *last = (int64_t)moved;
+			return;
+		}
 		*first = *last = (int64_t)round(c);
 		return;
 	case PROFILE_TRIANGLE:
@@ -107,12 +114,18 @@ double oracle_ctf(const double *p, int64_t extent, double pixel_size,
  *   slices: K*B x n x h complex; transforms: K*B x 12 (row-major 3x4);
  *   radial: K*B x h; extra: K*B x 4 (ctf) or K*B x n x h (weighted) or NULL.
  * The accumulators are updated in place.
+ *
+ * float32_positions: the sample positions round as the float32 row kernel's do
+ * (row_insertion_kernel.inl:157-166): the frame's x step to float, the row base
+ * k_y Y formed in double and rounded, then base + k_x X in float. A sample within
+ * such a rounding of a box window's half-voxel boundary falls in the same voxel
+ * then; everything else stays in double.
  */
 void oracle_insert_f64(int variant, int profile, double half_width, double shape,
 	int64_t n, int64_t big, int64_t K, int64_t B,
 	double *num, double *den,
 	const double *slices, const double *transforms, const double *radial, const double *extra,
-	double voltage_kv, double cs_mm, double amplitude_contrast, double pixel_size)
+	double voltage_kv, double cs_mm, double amplitude_contrast, double pixel_size, int float32_positions)
 {
 	const int64_t h = n / 2 + 1;
 	const int64_t half = big / 2 + 1;
@@ -165,13 +178,21 @@ void oracle_insert_f64(int variant, int profile, double half_width, double shape
 				const double value_r = vr;
 				const double value_i = sign > 0 ? vi : -vi;
 				double big_k[3];
-				for (int j = 0; j < 3; ++j)
-					big_k[j] = sign * scale * (k_x * t[j] + k_y * t[4 + j]);
+				for (int j = 0; j < 3; ++j) {
+					if (float32_positions) {
+						const float base = (float)(k_y * (sign * (t[4 + j] * scale)));
+						const float step = (float)sign * (float)(t[j] * scale);
+						const float along = (float)k_x * step;
+						big_k[j] = base + along;
+					} else {
+						big_k[j] = sign * scale * (k_x * t[j] + k_y * t[4 + j]);
+					}
+				}
 
 				int64_t z0, z1, y0, y1, x0, x1;
-				reached(profile, half_width, big_k[2], &z0, &z1);
-				reached(profile, half_width, big_k[1], &y0, &y1);
-				reached(profile, half_width, big_k[0], &x0, &x1);
+				reached(profile, half_width, big_k[2], float32_positions, &z0, &z1);
+				reached(profile, half_width, big_k[1], float32_positions, &y0, &y1);
+				reached(profile, half_width, big_k[0], float32_positions, &x0, &x1);
 				for (int64_t gz = z0; gz <= z1; ++gz)
 				for (int64_t gy = y0; gy <= y1; ++gy)
 				for (int64_t gx = x0; gx <= x1; ++gx) {

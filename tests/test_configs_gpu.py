@@ -37,10 +37,10 @@ THREADS = max(1, min(16, os.cpu_count() or 1))
 
 def reference_insert(inputs, window=oracle.Window.linear()):
     """The reference's float32 kernels where oracle/_ref is built, else the
-    float64 contract."""
+    float64 contract at their float32 positions."""
     if oracle.ref_available():
         return oracle.ref_insert("ctf", inputs, window, pixel_size=1.5, dtype=np.float32, threads=THREADS)
-    return oracle.insert_f64("ctf", inputs, window, pixel_size=1.5)
+    return oracle.insert_f64("ctf", inputs, window, pixel_size=1.5, float32_positions=True)
 
 
 def host_spectra(images):

@@ -394,3 +394,40 @@ def test_standardization_without_background_or_spread():
     image[2, 2] = 9.0
     out = oracle.standardize_background(image, 7, 0.5, -1e9, 1e9)
     assert out[2, 2] == 5.0 and out[0, 0] == 0.0
+
+
+def test_float32_positions_put_a_nearest_window_where_float32_kernels_do():
+    # Sample counts per voxel, positions in numpy float32: row base k_y Y in
+    # double, rounded; base + k_x X in float32; halves away from 0 in float32.
+    n = big = 48
+    rng = np.random.default_rng(3)
+    count = 60
+    transforms = np.zeros((count, 3, 4), np.float32)
+    transforms[:, :, :3] = np.linalg.qr(rng.normal(size=(count, 3, 3)))[0]
+    # Half of them steps of whole and half voxels but for float32's rounding.
+    transforms[::2, :2, :3] = np.round(transforms[::2, :2, :3] * 10) / 10
+    h = n // 2 + 1
+    acc = np.zeros((big, big, big // 2 + 1), np.complex64)
+    inputs = [acc, acc.real.copy(), np.zeros((count, n, h), np.complex64), transforms, np.ones(h, np.float32)]
+    expected = np.zeros(acc.shape)
+    ky, kx = np.meshgrid(np.arange(-(n // 2) + 1, n // 2), np.arange(h - 1), indexing="ij")
+    keep = np.floor(np.sqrt(kx ** 2 + ky ** 2) + 0.5) < h
+    ky, kx = ky[keep], kx[keep]
+    for t in transforms:
+        for sign in (1, -1):
+            c = []
+            for a in range(3):
+                base = (ky * (sign * np.float64(t[1, a]))).astype(np.float32)
+                c.append(base + kx.astype(np.float32) * np.float32(sign * t[0, a]))
+            g = [np.trunc(p + np.where(p < 0, np.float32(-0.5), np.float32(0.5))).astype(int) for p in c]
+            ok = (g[0] >= 0) & (g[0] <= big // 2) & (abs(g[1]) <= big // 2) & (abs(g[2]) <= big // 2)
+            ok &= (kx > 0) if sign < 0 else True
+            np.add.at(expected, (g[2][ok] % big, g[1][ok] % big, g[0][ok]), 1.0)
+    _, den = oracle.insert_f64("plain", inputs, oracle.Window.nearest(), float32_positions=True)
+    np.testing.assert_array_equal(den, expected)
+    _, den64 = oracle.insert_f64("plain", inputs, oracle.Window.nearest())
+    assert np.any(den64 != expected)
+    # A window without a boundary there moves by the positions' rounding alone.
+    a = oracle.insert_f64("plain", inputs, oracle.Window.linear(), float32_positions=True)[1]
+    b = oracle.insert_f64("plain", inputs, oracle.Window.linear())[1]
+    assert oracle.rel_l2(a, b) < 1e-5
