@@ -23,6 +23,7 @@
 #include "fft_two.hpp"
 #include "launch.hpp"
 #include "sample.hpp"
+#include "section_bounds.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -751,152 +752,6 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void columns_prepare
 	}
 }
 
-// The section of a slice's plane with the box [lower, upper], as real ranges
-// of k_x and k_y (of the +k copy; the -k copy's are the negated ones). With
-// p = k_x X + k_y Y, eliminating k_x or k_y between the axes a and b gives
-//   k_y n = X_a p_b - X_b p_a,  k_x n = Y_b p_a - Y_a p_b,  n = X_a Y_b - X_b Y_a,
-// and the three pairs of axes bound each frequency exactly: the section is
-// the intersection of three strips, whose projections are the intersections
-// of the strips' pairwise ones. The per-axis bound of the reference
-// (row_interval.cpp:34-136) takes each axis over the whole k_x range; it kept
-// 28 rows per (slice, brick) at 256^3 where 7.4 hold samples, these keep 9.
-// The box is widened by 0.01 voxel, the roundings here stay within
-// 1e-4 (|X_a| + |X_b|) of the products, which the widening covers.
-__device__ inline void bound_section(const float *x_step, const float *y_step, const float *normal, const float *lower,
-	const float *upper, float *kx, float *ky)
-{
-	kx[0] = ky[0] = -3.0e38f;
-	kx[1] = ky[1] = 3.0e38f;
-#pragma unroll
-	for (int c = 0; c < 3; ++c)
-	{
-		const int a = (c + 1) % 3;
-		const int b = (c + 2) % 3;
-		if (fabsf(normal[c]) > 1e-30f)
-		{
-			const float inv = __builtin_amdgcn_rcpf(normal[c]);
-			const auto narrow = [&](float p, float q, int i, int j, float *range)
-			{
-				// p [lower_i, upper_i] - q [lower_j, upper_j], over the normal.
-				const float p0 = p * lower[i], p1 = p * upper[i];
-				const float q0 = q * lower[j], q1 = q * upper[j];
-				const float l = (fminf(p0, p1) - fmaxf(q0, q1)) * inv;
-				const float u = (fmaxf(p0, p1) - fminf(q0, q1)) * inv;
-				range[0] = fmaxf(range[0], fminf(l, u));
-				range[1] = fminf(range[1], fmaxf(l, u));
-			};
-			narrow(x_step[a], x_step[b], b, a, ky);
-			narrow(y_step[b], y_step[a], a, b, kx);
-		}
-	}
-}
-
-// The rows [r0, r1) of one sign of a slice whose samples k_x in [first,
-// widest] can reach the box [lower, upper], given the section's ranges of
-// k_x and k_y (all already of that sign: the -k copy passes the negated box
-// and ranges); r0 >= r1 when none. `inv_y` holds 1 / y_step (0 where the step
-// is 0). Evaluated per lane, one slice per lane.
-__device__ inline void bound_rows(const insertion_params &p, const float *x_step, const float *y_step,
-	const float *inv_y, int last_shell, const float *lower, const float *upper, float kx_low, float kx_high,
-	float ky_low, float ky_high, int first, int &r0, int &r1)
-{
-	r0 = 0;
-	r1 = 0;
-	const int n = p.n;
-	const int h = p.h;
-	const bool even = n % 2 == 0;
-	const int last_column = h - (even ? 2 : 1);
-	const int highest_row = even ? n / 2 - 1 : n / 2;
-	const int widest = min(last_column, last_shell);
-	const int last_row = min(highest_row, widest);
-	const float k_low = ceilf(fmaxf(kx_low, static_cast<float>(first)));
-	const float k_high = floorf(fminf(kx_high, static_cast<float>(widest)));
-	float low = fmaxf(ky_low, -static_cast<float>(last_row));
-	float high = fminf(ky_high, static_cast<float>(last_row));
-	bool none = last_shell < 0 || k_low > k_high;
-#pragma unroll
-	for (int a = 0; a < 3; ++a)
-	{
-		const float at_first = k_low * x_step[a];
-		const float at_last = k_high * x_step[a];
-		const float lo = lower[a] - fmaxf(at_first, at_last);
-		const float hi = upper[a] - fminf(at_first, at_last);
-		if (y_step[a] == 0.0f)
-		{
-			none = none || !(lo <= 0.0f && 0.0f <= hi);
-		}
-		else
-		{
-			const float l = lo * inv_y[a];
-			const float u = hi * inv_y[a];
-			low = fmaxf(low, fminf(l, u));
-			high = fminf(high, fmaxf(l, u));
-		}
-	}
-	if (none || low > high)
-	{
-		return;
-	}
-	// The box is already widened past the window, so rounding inwards keeps
-	// every sample that can reach it.
-	r0 = static_cast<int>(ceilf(low));
-	r1 = static_cast<int>(floorf(high)) + 1;
-}
-
-// Position of sample k_x along one axis from its row's base and step (the
-// sign applied): the row base k_y * Y is formed in double and rounded to
-// float once per row, then base + k_x * X in float, uncontracted
-// (row_insertion_kernel.inl:157-166).
-__device__ inline float row_position(float base, float step, int kx)
-{
-#pragma clang fp contract(off)
-	const float product = static_cast<float>(kx) * step;
-	return base + product;
-}
-
-// clip_row of one row k_y and sign: the samples k_x in [begin, end) (end <=
-// begin when none) within the shell radius whose positions can fall in
-// [lower, upper], a box widened by 0.01 voxel beyond every rounding here.
-// `inv_step` holds 1 / step per axis (0 where the step is 0); a product with
-// it stands for the division.
-__device__ inline void clip_row(int ky, int first, int widest, float radius, const float *step, const float *y_step,
-	const float *inv_step, const float *lower, const float *upper, int &begin, int &end)
-{
-	begin = 0;
-	end = 0;
-	const float kyf = static_cast<float>(ky);
-	const float room = radius * radius - kyf * kyf;
-	if (room < 0.0f)
-	{
-		return;
-	}
-	const int last = min(widest, static_cast<int>(sqrtf(room)));
-	float lo_k = static_cast<float>(first);
-	float hi_k = static_cast<float>(last);
-	bool none = first > last;
-#pragma unroll
-	for (int a = 0; a < 3; ++a)
-	{
-		const float base = kyf * y_step[a];
-		if (step[a] == 0.0f)
-		{
-			none = none || !(lower[a] <= base && base <= upper[a]);
-		}
-		else
-		{
-			const float l = (lower[a] - base) * inv_step[a];
-			const float u = (upper[a] - base) * inv_step[a];
-			lo_k = fmaxf(lo_k, fminf(l, u));
-			hi_k = fminf(hi_k, fmaxf(l, u));
-		}
-	}
-	if (!none && lo_k <= hi_k)
-	{
-		begin = max(static_cast<int>(ceilf(lo_k)), first);
-		end = max(begin, min(static_cast<int>(floorf(hi_k)) + 1, last + 1));
-	}
-}
-
 // Before bricks that own voxels: the inputs that reach the outputs by atomics.
 // Blocks up to `split` copy the bricks split into shares (the first `split`
 // tasks hold them all), the others the rows of the frequencies +-N/2 of an even
@@ -984,10 +839,7 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 	const int h = p.h;
 	const int64_t elements = static_cast<int64_t>(n) * h;
 	const int64_t kept = blockIdx.y;
-	const int last_column = h - (n % 2 == 0 ? 2 : 1);
-	// A first tap f holds the positions [f + offset, f + 1 + offset).
-	const float cell_offset = PROFILE == REXLIB_HIP_BOX ? -0.5f :
-		(PROFILE == REXLIB_HIP_TRIANGLE ? 0.0f : p.kb_half_width - 1.0f);
+	const float cell_offset = first_tap_offset(T, p.kb_half_width);
 	const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
 
 	for (int ti = blockIdx.x; ti < task_count; ti += gridDim.x)
@@ -996,8 +848,6 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 		const int4 share = tasks[2 * ti + 1];
 		const int64_t share_begin = chunk.count * share.x / share.y;
 		const int64_t share_end = chunk.count * (share.x + 1) / share.y;
-		// The positions whose first tap lies in the brick, widened so that
-		// rounding never drops a sample (each sample is then tested exactly).
 		float lower[3];
 		float upper[3];
 		float centre[3];
@@ -1005,8 +855,7 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 		float half_diagonal2 = 0.0f;
 		for (int a = 0; a < 3; ++a)
 		{
-			lower[a] = static_cast<float>(box.lo[a]) + cell_offset - 0.01f;
-			upper[a] = static_cast<float>(box.lo[a] + box.ext[a]) + cell_offset + 0.01f;
+			cell_positions(box.lo[a], box.ext[a], cell_offset, lower[a], upper[a]);
 			centre[a] = 0.5f * (lower[a] + upper[a]);
 			half_extent[a] = 0.5f * (upper[a] - lower[a]) + 0.01f;
 			half_diagonal2 += half_extent[a] * half_extent[a];
@@ -1310,36 +1159,19 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 				y1 = static_cast<float>(e.y_step[1]);
 				y2 = static_cast<float>(e.y_step[2]);
 			}
-			// bound_rows of both signs, one slice per lane, and the
-			// reciprocal steps of the frame (shared by both signs).
-			int r0_plus = 0, r1_plus = 0, r0_minus = 0, r1_minus = 0;
-			float ix0 = 0.0f, ix1 = 0.0f, ix2 = 0.0f;
+			// The rows of both copies, one slice per lane, and the reciprocal steps
+			// of the frame.
+			int plus[2] = {0, 0}, minus_range[2] = {0, 0};
+			float inv_x[3] = {0.0f, 0.0f, 0.0f};
 			if (near)
 			{
 				const float xs[3] = {x0, x1, x2};
 				const float ys[3] = {y0, y1, y2};
-				// The hardware reciprocal (within 1 ulp): the bounds it feeds
-				// are widened by 0.01 voxel, far beyond its error.
-				float iy[3];
-				for (int a = 0; a < 3; ++a)
-				{
-					iy[a] = ys[a] == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(ys[a]);
-				}
-				ix0 = x0 == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(x0);
-				ix1 = x1 == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(x1);
-				ix2 = x2 == 0.0f ? 0.0f : __builtin_amdgcn_rcpf(x2);
-				const float normal[3] = {x1 * y2 - x2 * y1, x2 * y0 - x0 * y2, x0 * y1 - x1 * y0};
-				float kx[2];
-				float ky[2];
-				bound_section(xs, ys, normal, lower, upper, kx, ky);
-				bound_rows(p, xs, ys, iy, last_shell, lower, upper, kx[0], kx[1], ky[0], ky[1], 0, r0_plus, r1_plus);
-				const float mirrored_lower[3] = {-upper[0], -upper[1], -upper[2]};
-				const float mirrored_upper[3] = {-lower[0], -lower[1], -lower[2]};
-				bound_rows(p, xs, ys, iy, last_shell, mirrored_lower, mirrored_upper, -kx[1], -kx[0], -ky[1], -ky[0], 1,
-					r0_minus, r1_minus);
+				bound_slice(n, xs, ys, last_shell, lower, upper, [](float v) { return __builtin_amdgcn_rcpf(v); }, plus,
+					minus_range, inv_x);
 			}
-			const int plus_rows = near ? max(r1_plus - r0_plus, 0) : 0;
-			const int minus_rows = near ? max(r1_minus - r0_minus, 0) : 0;
+			const int plus_rows = near ? max(plus[1] - plus[0], 0) : 0;
+			const int minus_rows = near ? max(minus_range[1] - minus_range[0], 0) : 0;
 			const int rows = plus_rows + minus_rows;
 			const int rows_inclusive = wave_inclusive_scan(rows);
 			const int rows_first = rows_inclusive - rows;
@@ -1364,14 +1196,14 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 				// from a source lane that is switched off.
 				const int idx = r - __shfl(rows_first, s, 64);
 				const int np = __shfl(plus_rows, s, 64);
-				const int first_plus = __shfl(r0_plus, s, 64);
-				const int first_minus = __shfl(r0_minus, s, 64);
+				const int first_plus = __shfl(plus[0], s, 64);
+				const int first_minus = __shfl(minus_range[0], s, 64);
 				const bool minus = idx >= np;
 				const int ky = minus ? first_minus + (idx - np) : first_plus + idx;
 				const float sign = minus ? -1.0f : 1.0f;
 				const float frame_x[3] = {__shfl(x0, s, 64), __shfl(x1, s, 64), __shfl(x2, s, 64)};
 				const float frame_y[3] = {__shfl(y0, s, 64), __shfl(y1, s, 64), __shfl(y2, s, 64)};
-				const float frame_ix[3] = {__shfl(ix0, s, 64), __shfl(ix1, s, 64), __shfl(ix2, s, 64)};
+				const float frame_ix[3] = {__shfl(inv_x[0], s, 64), __shfl(inv_x[1], s, 64), __shfl(inv_x[2], s, 64)};
 				const int shell = __shfl(last_shell, s, 64);
 				const int js = __shfl(js_lane, s, 64);
 				float step[3];
@@ -1391,8 +1223,7 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 						base[a] = static_cast<float>(static_cast<double>(ky) *
 							(minus ? -e.y_step[a] : e.y_step[a]));
 					}
-					clip_row(ky, minus ? 1 : 0, min(last_column, shell), static_cast<float>(shell) + 0.5f, step, y_step,
-						inv_step, lower, upper, begin, end);
+					clip_row(n, ky, minus ? 1 : 0, shell, step, y_step, inv_step, lower, upper, begin, end);
 				}
 				else
 				{

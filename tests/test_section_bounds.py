@@ -1,89 +1,123 @@
-"""The brick kernel's section bound (bound_section and bound_rows in
-rexlib_amd/csrc/insertion.hip), restated in float32 numpy, against brute force
-over random planes and bricks: every row that holds a sample whose first tap
-lies in the brick is kept, for both copies of a slice, and few others are."""
+"""The brick kernel's bounds of rows and samples (bound_slice and clip_row of
+rexlib_amd/csrc/section_bounds.hpp), compiled for the CPU and compared with a
+walk over every sample of a slice: no sample whose first tap lies in a brick is
+dropped, for both copies of a slice, every window, brick shape, extent and last
+shell; no sample that the slice does not insert is kept (its prepared value is
+not written); and few rows without a sample are kept. The reciprocals, which
+are approximate on the device, are off by up to two units in the last place
+either way; the functions are built with and without fused multiply-adds."""
+import ctypes
+import os
+import shutil
+import subprocess
+
 import numpy as np
 import pytest
 
-f32 = np.float32
-LARGE = f32(3.0e38)
+from rexlib_amd import tune
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "rexlib_amd", "csrc")
+COMPILER = next((c for c in ("/opt/rocm/bin/amdclang++", "/opt/rocm/llvm/bin/clang++", shutil.which("clang++"))
+                 if c and os.path.exists(c)), None)
+# Half-width and layout taps: nearest, trilinear, Kaiser-Bessel of 3 and 4 taps.
+WINDOWS = [(0.5, 1), (1.0, 2), (1.2, 4), (1.5, 4), (2.0, 4)]
+
+
+@pytest.fixture(scope="module", params=["fused", "unfused"])
+def check(request, tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("bounds") / "check.so")
+    flags = ["-mfma", "-ffp-contract=fast"] if request.param == "fused" else ["-ffp-contract=off"]
+    subprocess.run([COMPILER, "-std=c++17", "-O2", "-fPIC", "-shared", *flags, "-I", CSRC, "-o", path,
+                    os.path.join(HERE, "section_bounds_check.cpp")], check=True)
+    function = ctypes.CDLL(path).section_bounds_check
+    p = ctypes.c_void_p
+    function.argtypes = [ctypes.c_int, p, p, ctypes.c_int, ctypes.c_int, ctypes.c_float, p, p, ctypes.c_int, p]
+    function.restype = None
+
+    def run(n, frame, last_shell, window, low, extent, ulps, out):
+        x, y = frame[0].astype(np.float32), np.ascontiguousarray(frame[1], np.float64)
+        low, extent = np.asarray(low, np.int32), np.asarray(extent, np.int32)
+        function(n, x.ctypes.data, y.ctypes.data, last_shell, window[1], window[0], low.ctypes.data, extent.ctypes.data,
+                 ulps, out.ctypes.data)
+
+    return run
 
 
 def rotation(rng):
-    q = rng.normal(size=4)
-    a, b, c, d = q / np.linalg.norm(q)
-    return np.array([[a * a + b * b - c * c - d * d, 2 * (b * c - a * d), 2 * (b * d + a * c)],
-                     [2 * (b * c + a * d), a * a - b * b + c * c - d * d, 2 * (c * d - a * b)],
-                     [2 * (b * d - a * c), 2 * (c * d + a * b), a * a - b * b - c * c + d * d]])
+    q, _ = np.linalg.qr(rng.normal(size=(3, 3)))
+    return q
 
 
-def narrowed(p, q, i, j, lower, upper, inv, bounds):
-    p0, p1, q0, q1 = f32(p * lower[i]), f32(p * upper[i]), f32(q * lower[j]), f32(q * upper[j])
-    l = f32(f32(min(p0, p1) - max(q0, q1)) * inv)
-    u = f32(f32(max(p0, p1) - min(q0, q1)) * inv)
-    return max(bounds[0], min(l, u)), min(bounds[1], max(l, u))
+def frame_of(kind, rng):
+    """Steps of k_x and k_y for N = n: rotations; planes along the lattice's
+    axes (zero steps and zero normals); matrices of any shape, as the insertion
+    accepts; axes a small angle apart."""
+    if kind == "rotation":
+        return rotation(rng)[:2]
+    if kind == "axes":
+        return (np.eye(3)[rng.permutation(3)] * rng.choice([-1.0, 1.0], 3)[:, None])[:2]
+    if kind == "any":
+        return rng.uniform(-1, 1, (2, 3))
+    if kind == "one axis":
+        # k_x runs along an axis, k_y nearly so.
+        f = np.eye(3)[rng.permutation(3)][:2]
+        f[1] = f[0] + rng.uniform(-1, 1, 3) * 10.0 ** rng.uniform(-6, 0)
+        return f
+    r = rotation(rng)
+    return np.stack([r[0], r[0] + r[1] * 10.0 ** rng.uniform(-3, 0)])
 
 
-def section(xs, ys, lower, upper):
-    kx = ky = (-LARGE, LARGE)
-    for c in range(3):
-        a, b = (c + 1) % 3, (c + 2) % 3
-        normal = f32(f32(xs[a] * ys[b]) - f32(xs[b] * ys[a]))
-        if abs(normal) > 1e-30:
-            inv = f32(f32(1) / normal)
-            ky = narrowed(xs[a], xs[b], b, a, lower, upper, inv, ky)
-            kx = narrowed(ys[b], ys[a], a, b, lower, upper, inv, kx)
-    return kx, ky
+def transforms_as_float32(frame):
+    return frame.astype(np.float32).astype(np.float64)
 
 
-def rows(xs, ys, lower, upper, kx, ky, first, widest):
-    k_low, k_high = np.ceil(max(kx[0], f32(first))), np.floor(min(kx[1], f32(widest)))
-    low, high = max(ky[0], f32(-widest)), min(ky[1], f32(widest))
-    if k_low > k_high:
-        return 0, 0
-    for a in range(3):
-        at_first, at_last = f32(k_low * xs[a]), f32(k_high * xs[a])
-        lo, hi = f32(lower[a] - max(at_first, at_last)), f32(upper[a] - min(at_first, at_last))
-        if ys[a] == 0:
-            if not lo <= 0 <= hi:
-                return 0, 0
-        else:
-            l, u = f32(lo * f32(1 / ys[a])), f32(hi * f32(1 / ys[a]))
-            low, high = max(low, min(l, u)), min(high, max(l, u))
-    return (int(np.ceil(low)), int(np.floor(high)) + 1) if low <= high else (0, 0)
+@pytest.mark.parametrize("kind", ["rotation", "axes", "any", "one axis", "near"])
+@pytest.mark.parametrize("n", [5, 8, 63, 128, 255])
+def test_no_sample_of_a_brick_is_dropped(check, kind, n):
+    rng = np.random.default_rng(n)
+    out = np.zeros(5, np.int64)
+    for case in range(400):
+        scale = rng.choice([1.0, 2.0, 0.7, rng.uniform(0.3, 8.0)])
+        frame = transforms_as_float32(frame_of(kind, rng)) * scale
+        last = int(rng.choice([n // 2, n // 2, n // 3, 1, 0]))
+        window = WINDOWS[rng.integers(len(WINDOWS))]
+        extent = tune.SHAPES[rng.integers(len(tune.SHAPES))]
+        # A brick around some sample of the slice.
+        centre = rng.uniform(-last, last, 2) @ frame * rng.choice([-1, 1])
+        low = np.floor(centre - np.array(extent) * rng.uniform(0, 1, 3)).astype(int)
+        before = out.copy()
+        check(n, frame, last, window, low, extent, int(rng.integers(-2, 3)), out)
+        assert out[1] == before[1], (case, frame, last, window, low, extent)
+        assert out[4] == before[4], (case, frame, last, window, low, extent)
+    assert out[0] > 400
+    if kind == "rotation" and n > 100:
+        # At most one row in three holds no sample (those of few samples per
+        # voxel among them).
+        assert out[2] < 1.5 * out[3]
 
 
-@pytest.mark.parametrize("scale", [1.0, 2.0, 0.7])
-@pytest.mark.parametrize("axes", [False, True])
-def test_every_row_with_a_sample_is_kept(scale, axes):
-    rng = np.random.default_rng(11)
-    n, widest, edge = 256, 127, 8
-    kept = held = 0
-    for case in range(300):
-        r = rotation(rng)
-        if axes:
-            # Planes along the lattice's axes: zero steps and zero normals.
-            r = np.eye(3)[rng.permutation(3)] * rng.choice([-1, 1], 3)[:, None]
-        xs, ys = (scale * r[0]).astype(f32), (scale * r[1]).astype(f32)
-        centre = rng.uniform(-100, 100, 2) @ (scale * r[:2]) + rng.uniform(-2, 2) * r[2]
-        lo = np.floor(centre) - edge // 2
-        lower, upper = (lo - 0.01).astype(f32), (lo + edge + 0.01).astype(f32)
-        kx, ky = section(xs, ys, lower, upper)
-        for mirrored in (False, True):
-            if mirrored:
-                r0, r1 = rows(xs, ys, -upper, -lower, (-kx[1], -kx[0]), (-ky[1], -ky[0]), 1, widest)
-            else:
-                r0, r1 = rows(xs, ys, lower, upper, kx, ky, 0, widest)
-            k_y = np.arange(-widest, widest + 1)[:, None]
-            k_x = np.arange(1 if mirrored else 0, widest + 1)[None, :]
-            sign = f32(-1 if mirrored else 1)
-            base = (k_y.astype(np.float64)[..., None] * (sign * ys.astype(np.float64))).astype(f32)
-            position = base + (k_x.astype(f32)[..., None] * (sign * xs)).astype(f32)
-            cell = np.floor(position)
-            inside = np.all((cell >= lo) & (cell < lo + edge), axis=-1) & (k_x * k_x + k_y * k_y <= (n // 2) ** 2)
-            found = np.unique(np.nonzero(inside)[0] - widest)
-            assert np.all((found >= r0) & (found < r1)), (case, mirrored, found, r0, r1)
-            kept += max(r1 - r0, 0)
-            held += found.size
-    # On generic planes at most one row in three holds no sample.
-    assert held > 300 and (axes or kept < 1.5 * held)
+# The longest extents that are not written past the last shell (4,095), and the
+# first whose shells are found without the rounded square root's correction.
+@pytest.mark.parametrize("n", [719, 721, 2048, 4095])
+def test_large_extents(check, n):
+    rng = np.random.default_rng(n)
+    out = np.zeros(5, np.int64)
+    for case in range(12):
+        frame = transforms_as_float32(rotation(rng)[:2])
+        last = int(rng.choice([n // 2, n // 2 - 1, n // 3]))
+        centre = rng.uniform(-last, last, 2) / 1.5 @ frame
+        check(n, frame, last, WINDOWS[case % len(WINDOWS)], np.floor(centre).astype(int) - 4, (16, 16, 8), 0, out)
+    assert out[0] > 12 and out[1] == 0 and out[4] == 0
+
+
+# Rows along the lattice's x axis in a brick at its edge: the clipped rows end at
+# the shell itself.
+@pytest.mark.parametrize("n", [255, 256, 1024, 4094, 4095])
+def test_rows_end_at_the_last_shell(check, n):
+    out = np.zeros(5, np.int64)
+    frame = np.array([[1.0, 0.0, 0.0], [0.0, 1.0, 0.0]])
+    for last in (n // 2, n // 2 - 1, n // 2 - 7):
+        check(n, frame, last, (1.0, 2), (last - 12, -n // 2, -4), (40, n + 2, 8), 0, out)
+        check(n, frame, last, (1.0, 2), (0, -n // 2, -4), (n, n + 2, 8), 0, out)
+    assert out[0] > 100 and out[1] == 0 and out[4] == 0
