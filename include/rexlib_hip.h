@@ -101,13 +101,14 @@ int32_t rexlib_hip_device_count(void);
  * (16, 8, 8), (16, 16, 8), (8, 8, 8), (8, 8, 6), (8, 8, 4) or (8, 6, 6) --
  * and the expected plane hits per task, in [16, 2^20], that splits busy
  * bricks into shares of their slices. Each call reads its extent's entry
- * once; without entries calls take (8, 8, 8) and 512, with a Kaiser-Bessel
- * window (8, 6, 6) and 512. Sparse calls with at most two taps (below 1.6
- * samples per voxel) take bricks of a fixed shape, (8, 8, 8), and only the
- * entry's share. Returns REXLIB_HIP_INVALID_ARGUMENT for other values. The
- * getter gives what calls of the extent take without a window family's entry
- * (without any entry: the values for up to two taps);
- * rexlib_hip_insertion_bricks what one call takes.
+ * once; without entries calls take (8, 8, 8) and 512. Sparse calls with at
+ * most two taps (below 1.6 samples per voxel) take bricks of a fixed shape, (8, 8,
+ * 8), and the entry's share up to 512. Kaiser-Bessel calls without an entry take (8,
+ * 6, 6) and 512, or, with many samples or a window of up to 3 taps, (8, 8, 6) and
+ * 128, or, sparse into 200^3 and more, (16, 8, 6) and 128; the latter two take an
+ * entry's share up to 128. Returns REXLIB_HIP_INVALID_ARGUMENT for other values.
+ * The getter gives what calls of the extent with up to two taps take
+ * without a window family's entry; rexlib_hip_insertion_bricks what one call takes.
  * No reference counterpart (the reference's CPU tuning is
  * slice_insertion_tuning, src/backends/cpu/builders/em/reconstruction/slice_insertion_tuning.cpp:10-13);
  * set by the autotuner (rexlib_amd/tune.py). */
@@ -122,9 +123,10 @@ int rexlib_hip_get_insertion_tuning(int32_t extent, int32_t *extent_x, int32_t *
 int rexlib_hip_set_insertion_tuning_for_window(int32_t extent, int32_t taps, int32_t extent_x, int32_t extent_y,
 	int32_t extent_z, int32_t share);
 /* The bricks that a call inserting `slices` slices of extent n into each volume
- * of extent `extent` takes, with a window of `taps` per axis of the brick layout
- * (1, 2 or 4) and no fixed workspace buffer; own_voxels is 1 for the sparse
- * calls whose brick shape is no entry's. No reference counterpart. */
+ * of extent `extent` takes, with a window of `taps` per axis (1 nearest, 2
+ * trilinear, 3 a Kaiser-Bessel one of up to 3, 4 a Kaiser-Bessel one) and no
+ * fixed workspace buffer; own_voxels is 1 for the sparse calls whose brick shape
+ * is no entry's. No reference counterpart. */
 int rexlib_hip_insertion_bricks(int32_t n, int32_t extent, int32_t taps, int64_t slices, int32_t *extent_x,
 	int32_t *extent_y, int32_t *extent_z, int32_t *share, int32_t *own_voxels);
 /* Drops the entry of an extent (taps 0) or of one window family, and gives its

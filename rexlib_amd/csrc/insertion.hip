@@ -421,6 +421,16 @@ void dispatch_scatter(const insertion_params &p, hipStream_t stream)
 // ---------------------------------------------------------------------------
 
 
+// How the rounds of a brick add its samples (see above): each lane its own,
+// after claiming its cell, or one sample after another by all 64 lanes, with all
+// 4 taps per axis of the layout or fewer.
+enum brick_rounds : int
+{
+	claimed_rounds = 0,
+	wide_rounds = 1,
+	wide_narrow_rounds = 2
+};
+
 // Taps per axis an LDS brick is laid out for: the window's own (box 1,
 // triangle 2), at most 4 for Kaiser-Bessel windows on this schedule.
 template <int PROFILE>
@@ -434,26 +444,26 @@ struct brick_reach
 // 64 lanes of an access are the 4 x 4 x 4 taps of one sample: a y pitch of 4
 // modulo 8 and a z pitch of 16 modulo 32 put every 32 of them in 32 different
 // residues, without a bank conflict.
-constexpr int brick_pitch_y(int taps, int lx)
+constexpr int brick_pitch_y(bool wide, int lx)
 {
-	return taps == 4 ? (lx + 3) / 8 * 8 + 4 : (lx % 2 == 0 ? lx + 1 : lx);
+	return wide ? (lx + 3) / 8 * 8 + 4 : (lx % 2 == 0 ? lx + 1 : lx);
 }
 
-constexpr int brick_pitch_z(int taps, int pitch_y, int ly)
+constexpr int brick_pitch_z(bool wide, int pitch_y, int ly)
 {
-	return taps == 4 ? (pitch_y * ly + 15) / 32 * 32 + 16 : (pitch_y * ly) % 2 == 0 ? pitch_y * ly + 1 : pitch_y * ly;
+	return wide ? (pitch_y * ly + 15) / 32 * 32 + 16 : (pitch_y * ly) % 2 == 0 ? pitch_y * ly + 1 : pitch_y * ly;
 }
 
 // LDS layout of a brick of first-tap cells EX x EY x EZ with the taps - 1
 // voxels above them.
-template <int T, int EX, int EY, int EZ>
+template <int T, bool WIDE, int EX, int EY, int EZ>
 struct brick_layout
 {
 	static constexpr int lx = EX + T - 1;
 	static constexpr int ly = EY + T - 1;
 	static constexpr int lz = EZ + T - 1;
-	static constexpr int pitch_y = brick_pitch_y(T, lx);
-	static constexpr int pitch_z = brick_pitch_z(T, pitch_y, ly);
+	static constexpr int pitch_y = brick_pitch_y(WIDE, lx);
+	static constexpr int pitch_z = brick_pitch_z(WIDE, pitch_y, ly);
 	static_assert(pitch_y >= lx && pitch_z >= pitch_y * ly, "the pitches hold a row and a plane");
 	static constexpr int voxels = pitch_z * lz;
 	static constexpr int cells = EX * EY * EZ;
@@ -813,21 +823,38 @@ __global__ __launch_bounds__(64) void copy_shared_inputs_kernel(insertion_params
 // A wavefront owns the brick of one task (a brick and a share of the
 // slices): EX x EY x EZ first-tap cells and the voxels their taps reach, in
 // LDS.
-template <int PROFILE, bool ODD, bool VOXELS, int EX, int EY, int EZ>
-__global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chunk chunk, const prepared_sample *prepared,
+// Wavefronts per SIMD that the register budget of a kernel is held to: as many
+// as the LDS of claimed Kaiser-Bessel bricks allows, four (128 registers) for 8 x
+// 6 x 6, which take 137 left alone. 0 leaves the others to the compiler.
+template <int PROFILE, int ROUNDS, int EX, int EY, int EZ>
+constexpr int brick_waves()
+{
+	if (PROFILE != REXLIB_HIP_KAISER_BESSEL || ROUNDS != claimed_rounds)
+	{
+		return 0;
+	}
+	using L = brick_layout<brick_reach<PROFILE>::taps, false, EX, EY, EZ>;
+	const int per_cu = 160 * 1024 / (L::voxels * 12 + L::cells + 2 * 64 * 4);
+	return per_cu >= 13 ? 4 : (per_cu + 3) / 4;
+}
+
+template <int PROFILE, bool ODD, bool VOXELS, int ROUNDS, int EX, int EY, int EZ>
+__global__ __launch_bounds__(64, (brick_waves<PROFILE, ROUNDS, EX, EY, EZ>())) void brick_kernel(insertion_params p,
+	slice_chunk chunk, const prepared_sample *prepared,
 	const int4 *tasks, int task_count, accumulator_input input)
 {
 	constexpr int T = brick_reach<PROFILE>::taps;
-	using L = brick_layout<T, EX, EY, EZ>;
+	constexpr bool WIDE = ROUNDS != claimed_rounds;
+	using L = brick_layout<T, WIDE, EX, EY, EZ>;
 	// The voxels as two arrays, value and weight. A tap is then a 64-bit and a
 	// 32-bit access at even and odd bank pitches; one array of 12-byte voxels
 	// took 217 cycles per CU for the 8 taps of 48 lanes, the two arrays 184.
 	__shared__ float2 acc_value[L::voxels];
 	__shared__ float acc_weight[L::voxels];
-	// Up to 2 taps, per first-tap cell: the lane that last claimed it.
-	__shared__ unsigned char claim[T == 4 ? 1 : L::cells];
-	// 4 taps: the axis weights of the samples in the lanes, x, y, z.
-	__shared__ float4 axis_weights[T == 4 ? 64 * 3 : 1];
+	// Claimed rounds, per first-tap cell: the lane that last claimed it.
+	__shared__ unsigned char claim[WIDE ? 1 : L::cells];
+	// Wide rounds: the axis weights of the samples in the lanes, x, y, z.
+	__shared__ float4 axis_weights[WIDE ? 64 * 3 : 1];
 	// Per lane: the last row (or slice) starting at or before it.
 	__shared__ int marker[64];
 	// Slices that hit the brick, waiting for their rows to be bounded.
@@ -910,14 +937,14 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 		// which is never added to the accumulators (64 rows at least, one a lane):
 		// their weights are 0, but a sample that is not finite times 0 is not.
 		// (Switching the lanes off for the access takes 4.4 to 5.3 ms below.)
-		const bool within = max(max(tap_x, tap_y), tap_z) < p.taps;
+		const bool within = ROUNDS != wide_narrow_rounds || max(max(tap_x, tap_y), tap_z) < p.taps;
 		const int reached = within ? 1 : 0;
-		static_assert(T < 4 || (L::pitch_y > L::lx && L::ly * L::lz >= 64), "a padding voxel per lane");
+		static_assert(!WIDE || (L::pitch_y > L::lx && L::ly * L::lz >= 64), "a padding voxel per lane");
 		const int tap_voxel = within ? tap_x + L::pitch_y * tap_y + L::pitch_z * tap_z :
 			L::lx + L::pitch_y * (lane % L::ly) + L::pitch_z * (lane / L::ly);
 		auto wide_round = [&]()
 		{
-			if constexpr (T == 4)
+			if constexpr (WIDE)
 			{
 				const int take = min(64, total - next);
 				marker[lane] = lane == 0 ? current : 0;
@@ -968,7 +995,8 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 				float wz = weights[12 * s + 8 + tap_z];
 				while (left != 0)
 				{
-					const int at = __mul24(__builtin_amdgcn_readlane(voxel, s), reached) + tap_voxel;
+					const int first = __builtin_amdgcn_readlane(voxel, s);
+					const int at = (ROUNDS == wide_narrow_rounds ? __mul24(first, reached) : first) + tap_voxel;
 					const float wt = wz * wy * wx;
 					const float re = lane_value(q.re, s);
 					const float imaginary = lane_value(im, s);
@@ -1068,12 +1096,20 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 					wz[0] = 1.0f - held_w[2];
 					wz[1] = held_w[2];
 				}
-				else
+				else if constexpr (PROFILE == REXLIB_HIP_BOX)
 				{
 					wx[0] = 1.0f;
 					wy[0] = 1.0f;
 					wz[0] = 1.0f;
 				}
+				else
+				{
+					window_taps<PROFILE>::template place<T>(p, held_w[0], wx);
+					window_taps<PROFILE>::template place<T>(p, held_w[1], wy);
+					window_taps<PROFILE>::template place<T>(p, held_w[2], wz);
+				}
+				// (Of the layout's 4 taps a Kaiser-Bessel window takes its own.)
+				const int taps = PROFILE == REXLIB_HIP_KAISER_BESSEL ? p.taps : T;
 #pragma unroll
 				for (int tz = 0; tz < T; ++tz)
 				{
@@ -1084,6 +1120,7 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 #pragma unroll
 						for (int tx = 0; tx < T; ++tx)
 						{
+							if (tx < taps && ty < taps && tz < taps)
 							{
 								const float wt = wzy * wx[tx];
 								const int at = base + tx + L::pitch_y * ty + L::pitch_z * tz;
@@ -1114,7 +1151,7 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 				for (int a = 0; a < 3; ++a)
 				{
 					f[a] = window_taps<PROFILE>::first_float(p, c[a]);
-					w[a] = c[a] - f[a];
+					w[a] = PROFILE == REXLIB_HIP_KAISER_BESSEL ? c[a] : c[a] - f[a];
 					f[a] -= middle[a];
 				}
 				const bool own = fabsf(f[0]) < 0.5f * EX && fabsf(f[1]) < 0.5f * EY && fabsf(f[2]) < 0.5f * EZ;
@@ -1247,7 +1284,7 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 				current = 0;
 				while (next < total)
 				{
-					if constexpr (T == 4)
+					if constexpr (WIDE)
 					{
 						wide_round();
 					}
@@ -1314,7 +1351,7 @@ __global__ __launch_bounds__(64) void brick_kernel(insertion_params p, slice_chu
 			queued += count;
 		}
 		// Samples still held after the last rows.
-		if constexpr (T < 4)
+		if constexpr (!WIDE)
 		{
 			while (__ballot(pending) != 0)
 			{
@@ -1489,15 +1526,16 @@ struct brick_tuning
 
 // What calls take without an entry: over 64 to 512 voxels and 16 to 2,048
 // slices, 8 x 8 x 8 bricks and 512 plane hits per task stay within a tenth of
-// the fastest shape for up to two taps per axis, and 8 x 6 x 6 for four (16 x
-// 8 x 6 and 256, the default before the slices were culled 64 at a time, is up
-// to a third slower on dense stacks).
+// the fastest shape for up to two taps per axis (16 x 8 x 6 and 256, the
+// default before the slices were culled 64 at a time, is up to a third slower
+// on dense stacks). Kaiser-Bessel windows: kaiser_bessel_bricks.
 constexpr brick_tuning untuned_bricks{8, 8, 8, 512};
 constexpr brick_tuning untuned_wide_bricks{8, 6, 6, 512};
+constexpr brick_tuning untuned_claimed_bricks{8, 8, 6, 128};
+constexpr brick_tuning untuned_sparse_bricks{16, 8, 6, 128};
 
 // Bricks that own voxels: a cell shell of T - 1 is walked twice, so the brick
-// has to be a large one of the small ones. (The share is an entry's, if there
-// is one.)
+// has to be a large one of the small ones.
 constexpr brick_tuning voxel_tuning{8, 8, 8, 512};
 
 std::mutex tuning_mutex;
@@ -1513,10 +1551,10 @@ bool valid_brick_shape(int ex, int ey, int ez)
 // the taps per axis of the brick layout (1, 2 or 4) for one window family.
 constexpr int taps_key = 1 << 20;
 
-// The tuning of an extent for a window of `taps` per axis (0: any window):
-// the window's own entry, else the extent's, else the entry for every
-// extent, else `fallback`.
-brick_tuning tuning_for(int extent, int taps, const brick_tuning &fallback)
+// The entry of an extent for a window of `taps` per axis (0: any window): the
+// window's own entry, else the extent's, else the entry for every extent, else
+// none (false).
+bool find_tuning(int extent, int taps, brick_tuning &t)
 {
 	std::lock_guard<std::mutex> lock(tuning_mutex);
 	auto found = taps > 0 ? tuning_table.find(extent + taps * taps_key) : tuning_table.end();
@@ -1528,79 +1566,116 @@ brick_tuning tuning_for(int extent, int taps, const brick_tuning &fallback)
 	{
 		found = tuning_table.find(0);
 	}
-	return found != tuning_table.end() ? found->second : fallback;
+	if (found == tuning_table.end())
+	{
+		return false;
+	}
+	t = found->second;
+	return true;
 }
+
+// The same, or `fallback` without an entry.
+brick_tuning tuning_for(int extent, int taps, const brick_tuning &fallback)
+{
+	brick_tuning t = fallback;
+	find_tuning(extent, taps, t);
+	return t;
+}
+
+// The bricks of one call.
+struct brick_choice
+{
+	brick_tuning bricks;
+	bool voxels; // they own voxels
+	bool wide;   // wide rounds
+};
 
 template <int PROFILE, int EX, int EY, int EZ>
 void launch_brick_shape(const insertion_params &p, slice_chunk chunk, const prepared_sample *prepared, const int4 *tasks,
-	int task_count, const accumulator_input *input, hipStream_t stream)
+	int task_count, bool wide, const accumulator_input *input, hipStream_t stream)
 {
 	const dim3 grid(static_cast<unsigned>(task_count), static_cast<unsigned>(p.map.kept_count));
-	const auto launch = [&](auto odd, auto voxels)
+	const auto launch = [&](auto odd, auto voxels, auto rounds)
 	{
-		brick_kernel<PROFILE, decltype(odd)::value, decltype(voxels)::value, EX, EY, EZ><<<grid, 64, 0, stream>>>(p, chunk,
-			prepared, tasks, task_count, input != nullptr ? *input : accumulator_input{});
+		brick_kernel<PROFILE, decltype(odd)::value, decltype(voxels)::value, decltype(rounds)::value, EX, EY, EZ>
+			<<<grid, 64, 0, stream>>>(p, chunk, prepared, tasks, task_count,
+				input != nullptr ? *input : accumulator_input{});
 	};
+	if constexpr (PROFILE == REXLIB_HIP_KAISER_BESSEL)
+	{
+		if (wide)
+		{
+			const auto launch_wide = [&](auto odd)
+			{
+				p.taps == 4 ? launch(odd, std::false_type(), std::integral_constant<int, wide_rounds>()) :
+					launch(odd, std::false_type(), std::integral_constant<int, wide_narrow_rounds>());
+			};
+			p.big % 2 == 1 ? launch_wide(std::true_type()) : launch_wide(std::false_type());
+			return;
+		}
+	}
+	constexpr std::integral_constant<int, claimed_rounds> claimed{};
 	if constexpr (PROFILE != REXLIB_HIP_KAISER_BESSEL && EX == voxel_tuning.ex && EY == voxel_tuning.ey &&
 		EZ == voxel_tuning.ez)
 	{
 		if (input != nullptr)
 		{
-			p.big % 2 == 1 ? launch(std::true_type(), std::true_type()) : launch(std::false_type(), std::true_type());
+			p.big % 2 == 1 ? launch(std::true_type(), std::true_type(), claimed) :
+				launch(std::false_type(), std::true_type(), claimed);
 			return;
 		}
 	}
-	p.big % 2 == 1 ? launch(std::true_type(), std::false_type()) : launch(std::false_type(), std::false_type());
+	p.big % 2 == 1 ? launch(std::true_type(), std::false_type(), claimed) :
+		launch(std::false_type(), std::false_type(), claimed);
 }
 
 template <int PROFILE>
 void launch_brick(const insertion_params &p, slice_chunk chunk, const prepared_sample *prepared, const int4 *tasks,
-	int task_count, const brick_tuning &t, const accumulator_input *input, hipStream_t stream)
+	int task_count, const brick_tuning &t, bool wide, const accumulator_input *input, hipStream_t stream)
 {
 	if (t.ex == 16 && t.ey == 8 && t.ez == 8)
 	{
-		launch_brick_shape<PROFILE, 16, 8, 8>(p, chunk, prepared, tasks, task_count, input, stream);
+		launch_brick_shape<PROFILE, 16, 8, 8>(p, chunk, prepared, tasks, task_count, wide, input, stream);
 	}
 	else if (t.ex == 16 && t.ey == 16)
 	{
-		launch_brick_shape<PROFILE, 16, 16, 8>(p, chunk, prepared, tasks, task_count, input, stream);
+		launch_brick_shape<PROFILE, 16, 16, 8>(p, chunk, prepared, tasks, task_count, wide, input, stream);
 	}
 	else if (t.ex == 8 && t.ey == 8 && t.ez == 8)
 	{
-		launch_brick_shape<PROFILE, 8, 8, 8>(p, chunk, prepared, tasks, task_count, input, stream);
+		launch_brick_shape<PROFILE, 8, 8, 8>(p, chunk, prepared, tasks, task_count, wide, input, stream);
 	}
 	else if (t.ex == 8 && t.ey == 8 && t.ez == 6)
 	{
-		launch_brick_shape<PROFILE, 8, 8, 6>(p, chunk, prepared, tasks, task_count, input, stream);
+		launch_brick_shape<PROFILE, 8, 8, 6>(p, chunk, prepared, tasks, task_count, wide, input, stream);
 	}
 	else if (t.ex == 8 && t.ey == 8)
 	{
-		launch_brick_shape<PROFILE, 8, 8, 4>(p, chunk, prepared, tasks, task_count, input, stream);
+		launch_brick_shape<PROFILE, 8, 8, 4>(p, chunk, prepared, tasks, task_count, wide, input, stream);
 	}
 	else if (t.ex == 8)
 	{
-		launch_brick_shape<PROFILE, 8, 6, 6>(p, chunk, prepared, tasks, task_count, input, stream);
+		launch_brick_shape<PROFILE, 8, 6, 6>(p, chunk, prepared, tasks, task_count, wide, input, stream);
 	}
 	else
 	{
-		launch_brick_shape<PROFILE, 16, 8, 6>(p, chunk, prepared, tasks, task_count, input, stream);
+		launch_brick_shape<PROFILE, 16, 8, 6>(p, chunk, prepared, tasks, task_count, wide, input, stream);
 	}
 }
 
 void dispatch_brick(const insertion_params &p, slice_chunk chunk, const prepared_sample *prepared, const int4 *tasks,
-	int task_count, const brick_tuning &tuning, const accumulator_input *input,
-	hipStream_t stream)
+	int task_count, const brick_choice &choice, const accumulator_input *input, hipStream_t stream)
 {
 	switch (p.profile)
 	{
 	case REXLIB_HIP_BOX:
-		launch_brick<REXLIB_HIP_BOX>(p, chunk, prepared, tasks, task_count, tuning, input, stream);
+		launch_brick<REXLIB_HIP_BOX>(p, chunk, prepared, tasks, task_count, choice.bricks, choice.wide, input, stream);
 		break;
 	case REXLIB_HIP_TRIANGLE:
-		launch_brick<REXLIB_HIP_TRIANGLE>(p, chunk, prepared, tasks, task_count, tuning, input, stream);
+		launch_brick<REXLIB_HIP_TRIANGLE>(p, chunk, prepared, tasks, task_count, choice.bricks, choice.wide, input, stream);
 		break;
 	default:
-		launch_brick<REXLIB_HIP_KAISER_BESSEL>(p, chunk, prepared, tasks, task_count, tuning, input, stream);
+		launch_brick<REXLIB_HIP_KAISER_BESSEL>(p, chunk, prepared, tasks, task_count, choice.bricks, choice.wide, input, stream);
 		break;
 	}
 }
@@ -1787,7 +1862,7 @@ struct task_list
 };
 
 std::mutex task_mutex;
-std::map<std::tuple<int, int, int64_t, int, int, int, int, int, bool>, task_list> task_cache;
+std::map<std::tuple<int, int, int64_t, int, int, int, int, int, bool, bool>, task_list> task_cache;
 
 int64_t slice_bucket(int64_t slices)
 {
@@ -1800,12 +1875,15 @@ int64_t slice_bucket(int64_t slices)
 }
 
 // The cached list for a call (made on first use); the caller holds task_mutex.
-task_list &brick_task_list(int big, int64_t slices, const brick_tuning &tuning, int taps, bool voxels)
+task_list &brick_task_list(int big, int64_t slices, const brick_choice &choice, int taps)
 {
+	const brick_tuning &tuning = choice.bricks;
+	const bool wide = choice.wide;
 	int device = 0;
 	REXLIB_HIP_CHECK(hipGetDevice(&device));
 	const int64_t bucket = slice_bucket(slices);
-	const auto key = std::make_tuple(device, big, bucket, tuning.share, tuning.ex, tuning.ey, tuning.ez, taps, voxels);
+	const auto key = std::make_tuple(device, big, bucket, tuning.share, tuning.ex, tuning.ey, tuning.ez, taps, wide,
+		choice.voxels);
 	auto found = task_cache.find(key);
 	if (found == task_cache.end())
 	{
@@ -1815,12 +1893,12 @@ task_list &brick_task_list(int big, int64_t slices, const brick_tuning &tuning, 
 		int units = 0;
 		REXLIB_HIP_CHECK(hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device));
 		const int lx = tuning.ex + taps - 1, ly = tuning.ey + taps - 1, lz = tuning.ez + taps - 1;
-		const int pitch_z = brick_pitch_z(taps, brick_pitch_y(taps, lx), ly);
+		const int pitch_z = brick_pitch_z(wide, brick_pitch_y(wide, lx), ly);
 		const int lds = static_cast<int>(align_up(static_cast<std::size_t>(pitch_z * lz * 12 +
-			(taps == 4 ? 64 * 48 : tuning.ex * tuning.ey * tuning.ez) + 2 * 64 * 4), 512));
+			(wide ? 64 * 48 : tuning.ex * tuning.ey * tuning.ez) + 2 * 64 * 4), 512));
 		found = task_cache.emplace(key, task_list{}).first;
 		found->second.host = brick_task_items(big, bucket, tuning.share, tuning.ex, tuning.ey, tuning.ez, taps,
-			units * std::max(1, (160 * 1024) / lds), voxels);
+			units * std::max(1, (160 * 1024) / lds), choice.voxels);
 		for (std::size_t i = 0; i < found->second.host.size(); i += 2)
 		{
 			if (found->second.host[i + 1].y > 1)
@@ -1833,20 +1911,20 @@ task_list &brick_task_list(int big, int64_t slices, const brick_tuning &tuning, 
 }
 
 // Workspace bytes the task list of a call takes (with its alignment).
-std::size_t brick_task_bytes(int big, int64_t slices, const brick_tuning &tuning, int taps, bool voxels)
+std::size_t brick_task_bytes(int big, int64_t slices, const brick_choice &choice, int taps)
 {
 	std::lock_guard<std::mutex> lock(task_mutex);
-	return align_up(sizeof(int4) * brick_task_list(big, slices, tuning, taps, voxels).host.size(), 256) + 256;
+	return align_up(sizeof(int4) * brick_task_list(big, slices, choice, taps).host.size(), 256) + 256;
 }
 
 // The device copy of a call's tasks. With a fixed workspace buffer the list
 // is copied into it from the host copy the cache keeps (nothing allocated);
 // otherwise the device copy is made once and cached.
-const int4 *brick_tasks(int big, int64_t slices, const brick_tuning &tuning, int taps, bool voxels,
+const int4 *brick_tasks(int big, int64_t slices, const brick_choice &choice, int taps,
 	workspace_source &workspace, hipStream_t stream, int &count, int &split)
 {
 	std::lock_guard<std::mutex> lock(task_mutex);
-	task_list &list = brick_task_list(big, slices, tuning, taps, voxels);
+	task_list &list = brick_task_list(big, slices, choice, taps);
 	count = static_cast<int>(list.host.size() / 2);
 	split = list.split;
 	const std::size_t bytes = sizeof(int4) * list.host.size();
@@ -1882,20 +1960,68 @@ bool bricks_own_voxels(int n, int big, int64_t slices, int taps, bool fixed)
 	return taps <= 2 && !fixed && samples < 1.6 * voxels;
 }
 
-// The bricks of cells of a window of `taps` per axis of the brick layout.
-brick_tuning cell_bricks(int big, int taps)
+// Kaiser-Bessel windows of 4 taps add one sample at a time, its taps on the 64
+// lanes (wide rounds), while the call has too few samples to keep every
+// wavefront's claims busy: 256 slices of 128^2 into 256^3 (1.6 million samples)
+// take 0.53 ms against 0.78, 1,024 (6.6 million) 0.81 against 0.92, but 300 of
+// 256^2 (7.7 million) 0.82 against 0.71, 1,500 3.3 against 2.7 and 2,048 of 128^2
+// into 128^3 (13 million) 1.4 against 1.1. Narrower windows leave those lanes
+// idle (3 taps, 300 of 256^2: 1.13 against 0.53 ms); 3 taps take wide rounds only
+// in small calls into twice the slices' extent and below 200^3, whose bricks meet
+// few samples of a slice: 512 of 64^2 into 128^3 0.18 against 0.24 ms.
+//
+// A task of claimed rounds takes several times as long per plane hit as one of
+// two taps, so an entry's share is cut to 128 (300 of 256^2: 0.71 against 0.99 ms
+// with 512).
+//
+// Sparse calls into large volumes (below 0.25 samples per voxel of the stored
+// half, from 200^3 on) spend their time on the atomics of the bricks' faces, of
+// which large bricks have fewer: claimed rounds in 16 x 8 x 6 bricks take 0.90 ms
+// for 100 slices of 256^2 into 384^3 against 1.20 wide in 8 x 6 x 6, 0.55 against
+// 0.75 for 150 of 200^2 into 300^3, 2.4 against 3.2 for 256 of 256^2 into 512^3.
+// Below 200^3 the small bricks' tasks win (16 of 128^2 into 128^3 87 against 106
+// us), and so do wide rounds for a slice or two (1 of 256^2 into 256^3 63 against
+// 72 us).
+brick_choice kaiser_bessel_bricks(int n, int big, int64_t slices, int64_t volumes, int window_taps)
 {
-	return tuning_for(big, taps, taps == 4 ? untuned_wide_bricks : untuned_bricks);
+	const double samples = 0.125 * 3.14159265 * n * n * static_cast<double>(slices);
+	const double voxels = 0.5 * big * big * static_cast<double>(big);
+	brick_choice c{untuned_wide_bricks, false, false};
+	const bool entry = find_tuning(big, 4, c.bricks);
+	const bool sparse = !entry && big >= 200 && samples < 0.25 * voxels && samples >= 5e4;
+	const double all = samples * static_cast<double>(volumes);
+	c.wide = window_taps == 4 ? !sparse && all < 7e6 :
+		window_taps == 3 && big >= 2 * n && big < 200 && all < 1e6;
+	if (!c.wide)
+	{
+		if (!entry)
+		{
+			c.bricks = sparse ? untuned_sparse_bricks : untuned_claimed_bricks;
+		}
+		c.bricks.share = std::min(c.bricks.share, untuned_claimed_bricks.share);
+	}
+	return c;
 }
 
-// The bricks of voxels: their own shape, an entry's share.
-brick_tuning voxel_bricks(int big, int taps)
+// The bricks of a call of `slices` slices into each of `volumes` volumes, for a
+// brick layout of `taps` and a window of `window_taps` per axis.
+brick_choice choose_bricks(int n, int big, int64_t slices, int64_t volumes, int taps, int window_taps, bool fixed)
 {
-	brick_tuning t = tuning_for(big, taps, voxel_tuning);
-	t.ex = voxel_tuning.ex;
-	t.ey = voxel_tuning.ey;
-	t.ez = voxel_tuning.ez;
-	return t;
+	if (taps == 4)
+	{
+		return kaiser_bessel_bricks(n, big, slices, volumes, window_taps);
+	}
+	brick_choice c{untuned_bricks, bricks_own_voxels(n, big, slices, taps, fixed), false};
+	const bool entry = find_tuning(big, taps, c.bricks);
+	if (c.voxels)
+	{
+		// Their own shape, and an entry's share up to their own: 1,024 slices of
+		// 128^2 into 256^3 take 0.31 ms with 512 and 0.38 with 1,024.
+		const int share = entry ? c.bricks.share : voxel_tuning.share;
+		c.bricks = voxel_tuning;
+		c.bricks.share = std::min(share, voxel_tuning.share);
+	}
+	return c;
 }
 
 // Prepared samples take 12 bytes per stored element of a slice; a chunk of slices
@@ -1961,38 +2087,33 @@ void get_insertion_tuning(int extent, int *extent_x, int *extent_y, int *extent_
 	*share = t.share;
 }
 
-static void check_window_taps(int taps)
-{
-	if (taps != 1 && taps != 2 && taps != 4)
-	{
-		fail(REXLIB_HIP_INVALID_ARGUMENT, "insertion tuning: taps per axis of a window are 1 (nearest), 2 (trilinear) "
-			"or 4 (Kaiser-Bessel)");
-	}
-}
-
 void insertion_bricks(int n, int extent, int taps, int64_t slices, int *extent_x, int *extent_y, int *extent_z,
 	int *share, int *own_voxels)
 {
-	check_window_taps(taps);
+	if (taps < 1 || taps > 4)
+	{
+		fail(REXLIB_HIP_INVALID_ARGUMENT, "insertion bricks: taps per axis are 1 (nearest), 2 (trilinear), 3 (a "
+			"Kaiser-Bessel window of up to 3 taps) or 4 (Kaiser-Bessel)");
+	}
 	if (n < 1 || extent < 1 || slices < 1)
 	{
 		fail(REXLIB_HIP_INVALID_ARGUMENT, "insertion bricks: the extents and the number of slices must be positive");
 	}
 	const int64_t chunk = std::min(slices, std::max<int64_t>(1, prepared_limit / prepared_bytes(n)));
-	const bool voxels = bricks_own_voxels(n, extent, chunk, taps, false);
-	const brick_tuning t = voxels ? voxel_bricks(extent, taps) : cell_bricks(extent, taps);
-	*extent_x = t.ex;
-	*extent_y = t.ey;
-	*extent_z = t.ez;
-	*share = t.share;
-	*own_voxels = voxels ? 1 : 0;
+	const brick_choice c = choose_bricks(n, extent, chunk, 1, taps >= 3 ? 4 : taps, taps, false);
+	*extent_x = c.bricks.ex;
+	*extent_y = c.bricks.ey;
+	*extent_z = c.bricks.ez;
+	*share = c.bricks.share;
+	*own_voxels = c.voxels ? 1 : 0;
 }
 
 bool drop_insertion_tuning(int extent, int taps, int *extent_x, int *extent_y, int *extent_z, int *share)
 {
-	if (taps != 0)
+	if (taps != 0 && taps != 1 && taps != 2 && taps != 4)
 	{
-		check_window_taps(taps);
+		fail(REXLIB_HIP_INVALID_ARGUMENT, "insertion tuning: taps per axis are 0 (every window), 1 (nearest), "
+			"2 (trilinear) or 4 (Kaiser-Bessel)");
 	}
 	std::lock_guard<std::mutex> lock(tuning_mutex);
 	const auto found = tuning_table.find(extent + taps * taps_key);
@@ -2099,8 +2220,8 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 	const int64_t per_slice = prepared_bytes(p.n) * p.map.kept_count;
 	// Taps per axis of the brick layout: 1, 2, or 4 for every Kaiser-Bessel window.
 	const int layout_taps = p.profile == REXLIB_HIP_BOX ? 1 : (p.profile == REXLIB_HIP_TRIANGLE ? 2 : 4);
-	brick_tuning tuning = cell_bricks(p.big, layout_taps);
 	int64_t chunk_count = 0;
+	brick_choice choice{untuned_bricks, false, false};
 	if (schedule != schedule_scatter && p.taps <= 4 && p.map.kept_count <= 65535)
 	{
 		const auto room = [&](std::size_t reserved)
@@ -2111,20 +2232,21 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 					std::size_t(1) << 40)));
 		};
 		chunk_count = std::min<int64_t>(p.map.reduced_count, room(0) / per_slice);
+		if (chunk_count >= 1)
+		{
+			choice = choose_bricks(p.n, p.big, chunk_count, p.map.kept_count, layout_taps, p.taps,
+				workspace.arena != nullptr);
+		}
 		if (chunk_count >= 1 && workspace.arena != nullptr)
 		{
 			// Tasks made for more slices stay valid for fewer (their shares
 			// are fractions of a chunk).
 			chunk_count = std::min<int64_t>(chunk_count,
-				room(brick_task_bytes(p.big, chunk_count, tuning, layout_taps, false)) / per_slice);
+				room(brick_task_bytes(p.big, chunk_count, choice, layout_taps)) / per_slice);
 		}
 	}
 	const bool brick = chunk_count >= 1;
-	const bool voxels = brick && bricks_own_voxels(p.n, p.big, chunk_count, layout_taps, workspace.arena != nullptr);
-	if (voxels)
-	{
-		tuning = voxel_bricks(p.big, layout_taps);
-	}
+	const bool voxels = brick && choice.voxels;
 	// Bricks that own voxels read the inputs themselves, unless most of them
 	// would have nothing to add.
 	const bool copied = !voxels || copy_first(p, chunk_count);
@@ -2158,7 +2280,7 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 			row_range{n / 2 - columns->rows->m / 2, n / 2 - columns->rows->m / 2 + columns->rows->m} : row_range{0, n};
 		int count = 0;
 		int split = 0; // tasks of split bricks, the first ones
-		const int4 *tasks = brick_tasks(p.big, chunk_count, tuning, layout_taps, voxels, workspace, stream, count, split);
+		const int4 *tasks = brick_tasks(p.big, chunk_count, choice, layout_taps, workspace, stream, count, split);
 		prepared_sample *prepared = static_cast<prepared_sample *>(workspace.take(area_prepared,
 			static_cast<std::size_t>(per_slice * chunk_count), stream));
 		for (int64_t begin = 0; begin < p.map.reduced_count; begin += chunk_count)
@@ -2194,7 +2316,7 @@ void run_insertion(insertion_params p, int schedule, const float2 *num_in, const
 				kernel<<<grid, 64, 0, stream>>>(p, tasks, split, input);
 				REXLIB_HIP_CHECK(hipGetLastError());
 			}
-			dispatch_brick(p, chunk, prepared, tasks, count, tuning, voxels ? &input : nullptr, stream);
+			dispatch_brick(p, chunk, prepared, tasks, count, choice, voxels ? &input : nullptr, stream);
 			REXLIB_HIP_CHECK(hipGetLastError());
 			timing_end(brick_token, stream);
 		}

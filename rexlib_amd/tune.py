@@ -7,7 +7,7 @@ hits per task, which split busy bricks), checks every configuration's sums
 against the first one's, and records the fastest per volume extent N in a
 JSON table. A sparse workload (below 1.6 samples per voxel, at most two taps)
 takes bricks of one fixed shape: only its shares are timed, and nothing is
-recorded. ``apply_all()`` hands the
+recorded. Settings that a call takes alike are timed once. ``apply_all()`` hands the
 whole table to the library, which then picks each call's entry by its volume
 extent, so reconstructions of different sizes need no switching between
 calls.
@@ -30,7 +30,7 @@ TABLE = os.path.join(HERE, "tuning.json")
 # (x, y, z) extents of the bricks the library is built for.
 SHAPES = ((16, 8, 6), (16, 8, 8), (16, 16, 8), (8, 8, 8), (8, 8, 6), (8, 8, 4), (8, 6, 6))
 SHARES = (32, 64, 128, 256, 512, 1024)
-# What calls take without an entry (with a Kaiser-Bessel window: 8, 6, 6 and 512).
+# What calls take without an entry with up to two taps (bricks_of: any call).
 DEFAULT = {"extent_x": 8, "extent_y": 8, "extent_z": 8, "share": 512}
 
 
@@ -55,9 +55,9 @@ def set_tuning(extent: int, shape, share: int, taps: int = 0) -> None:
 
 
 def get_tuning(extent: int):
-    """((extent_x, extent_y, extent_z), share) that calls with volume extent
-    ``extent`` take unless their window family has an entry of its own
-    (``bricks_of``: what one call takes)."""
+    """((extent_x, extent_y, extent_z), share) that calls with volume
+    extent ``extent`` and up to two taps take unless their window family has an
+    entry of its own (``bricks_of``: what one call takes)."""
     from . import _native as N
     v = [ctypes.c_int32() for _ in range(4)]
     N.check(N.library().rexlib_hip_get_insertion_tuning(int(extent), *[ctypes.byref(x) for x in v]))
@@ -66,8 +66,10 @@ def get_tuning(extent: int):
 
 def bricks_of(n: int, big: int, slices: int, taps: int = 2):
     """((extent_x, extent_y, extent_z), share, own voxels) of a call of
-    ``slices`` slices of extent ``n`` into a volume of extent ``big``. Bricks
-    that own voxels (sparse calls) have a shape that no entry changes."""
+    ``slices`` slices of extent ``n`` into a volume of extent ``big``, with a
+    window of ``taps`` per axis (1 nearest, 2 trilinear, 3 a Kaiser-Bessel one
+    of up to 3, 4 a Kaiser-Bessel one). Bricks that own voxels (sparse calls)
+    have a shape that no entry changes."""
     from . import _native as N
     v = [ctypes.c_int32() for _ in range(5)]
     N.check(N.library().rexlib_hip_insertion_bricks(int(n), int(big), int(taps), int(slices),
@@ -168,12 +170,16 @@ def tune(n: int, big: int, launch: int, path: str = TABLE, verbose: bool = True,
     slices, transforms, ctf = workload(n, big, launch)
     results = []
     reference = None
-    shape, _, sparse = bricks_of(n, big, launch, taps or 2)
+    timed = set()
     previous = drop_tuning(big, taps)
     try:
-        for shape in (shape,) if sparse else SHAPES:
-            for share in SHARES:
-                set_tuning(big, shape, share, taps)
+        for trial in SHAPES:
+            for limit in SHARES:
+                set_tuning(big, trial, limit, taps)
+                shape, share, sparse = bricks_of(n, big, launch, taps or 2)
+                if (shape, share) in timed:
+                    continue
+                timed.add((shape, share))
                 ms, sums = time_insertion(n, big, slices, transforms, ctf, taps=taps)
                 if reference is None:
                     reference = sums

@@ -269,15 +269,27 @@ def test_the_bricks_a_call_takes():
         assert tune.bricks_of(*dense) == (*tune.get_tuning(256), False)
         assert tune.get_tuning(256) == ((tune.DEFAULT["extent_x"], tune.DEFAULT["extent_y"],
                                          tune.DEFAULT["extent_z"]), tune.DEFAULT["share"])
-        assert tune.bricks_of(*dense, taps=4) == ((8, 6, 6), 512, False)
         assert tune.bricks_of(*sparse) == ((8, 8, 8), 512, True)
-        assert tune.bricks_of(*sparse, taps=4) == ((8, 6, 6), 512, False)  # four taps keep cells
+        # Kaiser-Bessel: a sample at a time with few samples, claims otherwise
+        # and for narrower windows, larger bricks for sparse calls into large
+        # volumes. Four taps keep cells.
+        assert tune.bricks_of(128, 256, 256, taps=4) == ((16, 8, 6), 128, False)  # 0.2 samples per voxel
+        assert tune.bricks_of(128, 192, 256, taps=4) == ((8, 6, 6), 512, False)
+        assert tune.bricks_of(128, 192, 256, taps=3) == ((8, 8, 6), 128, False)
+        assert tune.bricks_of(16, 128, 4, taps=4) == ((8, 6, 6), 512, False)
+        assert tune.bricks_of(*dense, taps=4) == ((8, 8, 6), 128, False)
+        assert tune.bricks_of(*sparse, taps=4) == tune.bricks_of(*sparse, taps=3) == ((16, 8, 6), 128, False)
         tune.set_tuning(256, (16, 8, 6), 64)
         tune.set_tuning(512, (16, 8, 6), 64)
         tune.set_tuning(256, (8, 8, 4), 32, taps=4)
         assert tune.bricks_of(*dense, taps=1) == ((16, 8, 6), 64, False)
         assert tune.bricks_of(*dense, taps=4) == ((8, 8, 4), 32, False)
-        assert tune.bricks_of(*sparse) == ((8, 8, 8), 64, True)  # the entry's share
+        tune.set_tuning(192, (8, 8, 8), 1024)
+        assert tune.bricks_of(128, 192, 256, taps=4) == ((8, 8, 8), 1024, False)
+        assert tune.bricks_of(128, 192, 256, taps=3) == ((8, 8, 8), 128, False)
+        assert tune.bricks_of(*sparse) == ((8, 8, 8), 64, True)  # the entry's share, up to 512
+        tune.set_tuning(512, (16, 8, 6), 1024)
+        assert tune.bricks_of(*sparse) == ((8, 8, 8), 512, True)
         # The line between them: the slices' next power of two.
         assert tune.bricks_of(256, 256, 512)[2] and not tune.bricks_of(256, 256, 513)[2]
         assert tune.drop_tuning(256, 1) is None
@@ -285,7 +297,8 @@ def test_the_bricks_a_call_takes():
         assert tune.bricks_of(*dense, taps=4) == ((16, 8, 6), 64, False)
         assert tune.drop_tuning(256) == ((16, 8, 6), 64) and tune.drop_tuning(256) is None
         v = [ctypes.byref(ctypes.c_int32()) for _ in range(5)]
-        assert lib.rexlib_hip_insertion_bricks(256, 256, 3, 1, *v) == N.INVALID_ARGUMENT
+        assert lib.rexlib_hip_insertion_bricks(256, 256, 0, 1, *v) == N.INVALID_ARGUMENT
+        assert lib.rexlib_hip_insertion_bricks(256, 256, 5, 1, *v) == N.INVALID_ARGUMENT
         assert lib.rexlib_hip_insertion_bricks(0, 256, 2, 1, *v) == N.INVALID_ARGUMENT
         assert lib.rexlib_hip_insertion_bricks(256, 256, 2, 0, *v) == N.INVALID_ARGUMENT
         assert lib.rexlib_hip_drop_insertion_tuning(256, 3, *v[:4]) == N.INVALID_ARGUMENT
@@ -315,8 +328,13 @@ def test_tuning_one_window_family_leaves_the_others(tmp_path, monkeypatch):
     try:
         launch, broken = 4096, None
         tune.tune(256, 256, launch, path, verbose=False, taps=4)
-        assert tried == [(shape, share) for shape in tune.SHAPES for share in tune.SHARES]
+        # Dense Kaiser-Bessel calls take shares up to 128.
+        assert tried == [(shape, share) for shape in tune.SHAPES for share in tune.SHARES if share <= 128]
         assert tune.bricks_of(256, 256, launch, 4) == ((8, 8, 4), 64, False)
+        launch = 200
+        assert tune.tune(64, 64, launch, path, verbose=False)["recorded"] and tune.drop_tuning(64)
+        assert tried[-42:] == [(shape, share) for shape in tune.SHAPES for share in tune.SHARES]
+        launch = 4096
         assert tune.bricks_of(256, 256, launch, 2) == (*tune.get_tuning(256), False) == ((8, 8, 8), 512, False)
         broken = (16, 16, 8)
         for taps, before in ((4, ((8, 8, 4), 64, False)), (0, ((8, 8, 8), 512, False))):
@@ -324,10 +342,10 @@ def test_tuning_one_window_family_leaves_the_others(tmp_path, monkeypatch):
                 tune.tune(256, 256, launch, path, verbose=False, taps=taps)
             assert tune.bricks_of(256, 256, launch, taps or 2) == before
         recorded = tune.load_table(path)
-        assert list(recorded) == ["256/4"]
+        assert sorted(recorded) == ["256/4", "64"]
         launch, broken, tried[:] = 64, None, []
         assert tune.tune(64, 512, launch, path, verbose=False)["recorded"] is False
-        assert tried == [((8, 8, 8), share) for share in tune.SHARES]
+        assert tried == [((8, 8, 8), share) for share in tune.SHARES if share <= 512]
         assert tune.load_table(path) == recorded and tune.drop_tuning(512) is None
     finally:
         tune.clear_tuning()

@@ -10,7 +10,7 @@ import torch
 import oracle
 from cases import make_case
 from gpu_helpers import OPTICS, hip_insert, hip_window, to_device
-from rexlib_amd import em
+from rexlib_amd import em, tune
 
 pytestmark = pytest.mark.gpu
 
@@ -99,3 +99,27 @@ def test_an_infinite_sample_stays_within_its_kaiser_bessel_window(half_width, bi
     assert len(spoilt) > 0
     for z, y, x in spoilt:
         assert x in reach[0] and y in reach[1] and z in reach[2]
+
+
+# The rounds of a Kaiser-Bessel brick: claimed (3 taps in every brick shape; 4
+# taps, sparse into 200^3 and more), one sample at a time (4 taps; 3 into twice
+# the slices' extent).
+@pytest.mark.parametrize("half_width,n,big,slices", [(1.5, 24, 37, 20), (1.0, 20, 40, 12), (1.2, 16, 32, 9),
+                                                     (1.5, 17, 35, 9), (2.0, 100, 200, 13), (2.0, 100, 201, 13)])
+def test_kaiser_bessel_rounds_match_the_oracle(half_width, n, big, slices):
+    # (The same positions: the window steps at its edge, by 1 / I0(6) = 0.015 of a sample.)
+    window = oracle.Window.kaiser_bessel(half_width, 6.0)
+    inputs = geometry(make_case("plain", n, big, seed=n, slices=slices), np.random.default_rng(n))
+    inputs = [a.astype(np.complex64 if np.iscomplexobj(a) else np.float32) for a in inputs]
+    ref = oracle.insert_f64("plain", inputs, window, float32_positions=True)
+    shapes = tune.SHAPES if big < 40 else (None,)
+    tune.clear_tuning()
+    try:
+        for shape in shapes:
+            if shape is not None:
+                tune.set_tuning(big, shape, 64)
+            num, den = hip_insert("plain", inputs, window)
+            assert np.abs(num - ref[0]).max() <= 5e-4 * max(1.0, float(np.abs(ref[0]).max())), shape
+            assert np.abs(den - ref[1]).max() <= 5e-4 * max(1.0, float(np.abs(ref[1]).max())), shape
+    finally:
+        tune.clear_tuning()
