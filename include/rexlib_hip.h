@@ -101,13 +101,14 @@ int32_t rexlib_hip_device_count(void);
  * (16, 8, 8), (16, 16, 8), (8, 8, 8), (8, 8, 6), (8, 8, 4) or (8, 6, 6) --
  * and the expected plane hits per task, in [16, 2^20], that splits busy
  * bricks into shares of their slices. Each call reads its extent's entry
- * once; without entries calls take (8, 8, 8) and 512. Sparse calls with at
+ * once; without entries calls take (8, 8, 8) and 512, or, below 3 million
+ * samples, (16, 8, 6) and 256. Sparse calls with at
  * most two taps (below 1.6 samples per voxel) take bricks of a fixed shape, (8, 8,
  * 8), and the entry's share up to 512. Kaiser-Bessel calls without an entry take (8,
  * 6, 6) and 512, or, with many samples or a window of up to 3 taps, (8, 8, 6) and
  * 128, or, sparse into 200^3 and more, (16, 8, 6) and 128; the latter two take an
  * entry's share up to 128. Returns REXLIB_HIP_INVALID_ARGUMENT for other values.
- * The getter gives what calls of the extent with up to two taps take
+ * The getter gives what large calls of the extent with up to two taps take
  * without a window family's entry; rexlib_hip_insertion_bricks what one call takes.
  * No reference counterpart (the reference's CPU tuning is
  * slice_insertion_tuning, src/backends/cpu/builders/em/reconstruction/slice_insertion_tuning.cpp:10-13);

@@ -1524,12 +1524,17 @@ struct brick_tuning
 	int share;
 };
 
-// What calls take without an entry: over 64 to 512 voxels and 16 to 2,048
-// slices, 8 x 8 x 8 bricks and 512 plane hits per task stay within a tenth of
-// the fastest shape for up to two taps per axis (16 x 8 x 6 and 256, the
-// default before the slices were culled 64 at a time, is up to a third slower
-// on dense stacks). Kaiser-Bessel windows: kaiser_bessel_bricks.
+// What calls of up to two taps per axis take without an entry: 8 x 8 x 8 bricks
+// and 512 plane hits per task (over 64 to 512 voxels and up to 4,096 slices within
+// a fifth of the fastest shape), or, with fewer than 3 million samples, larger
+// bricks, whose fewer faces count there for more than their tasks: 300 slices of
+// 108^2 into 108^3 take 104 us in 16 x 8 x 6 and 117 in 8 x 8 x 8, 1,000 of 32^2
+// into 48^3 85 against 92, but 4,000 of 100^2 into 100^3 (16 million) 0.49 ms in
+// the one against 0.45, 2,000 of 225^2 into 225^3 0.89 against 0.82. Sparse calls on
+// cells (a fixed workspace) are all faces and take the larger bricks too.
+// Kaiser-Bessel windows: kaiser_bessel_bricks.
 constexpr brick_tuning untuned_bricks{8, 8, 8, 512};
+constexpr brick_tuning untuned_small_bricks{16, 8, 6, 256};
 constexpr brick_tuning untuned_wide_bricks{8, 6, 6, 512};
 constexpr brick_tuning untuned_claimed_bricks{8, 8, 6, 128};
 constexpr brick_tuning untuned_sparse_bricks{16, 8, 6, 128};
@@ -2011,7 +2016,9 @@ brick_choice choose_bricks(int n, int big, int64_t slices, int64_t volumes, int 
 	{
 		return kaiser_bessel_bricks(n, big, slices, volumes, window_taps);
 	}
-	brick_choice c{untuned_bricks, bricks_own_voxels(n, big, slices, taps, fixed), false};
+	const double samples = 0.125 * 3.14159265 * n * n * static_cast<double>(slices);
+	const bool small = samples * static_cast<double>(volumes) < 3e6 || bricks_own_voxels(n, big, slices, taps, false);
+	brick_choice c{small ? untuned_small_bricks : untuned_bricks, bricks_own_voxels(n, big, slices, taps, fixed), false};
 	const bool entry = find_tuning(big, taps, c.bricks);
 	if (c.voxels)
 	{

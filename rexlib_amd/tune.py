@@ -30,7 +30,7 @@ TABLE = os.path.join(HERE, "tuning.json")
 # (x, y, z) extents of the bricks the library is built for.
 SHAPES = ((16, 8, 6), (16, 8, 8), (16, 16, 8), (8, 8, 8), (8, 8, 6), (8, 8, 4), (8, 6, 6))
 SHARES = (32, 64, 128, 256, 512, 1024)
-# What calls take without an entry with up to two taps (bricks_of: any call).
+# What large calls take without an entry with up to two taps (bricks_of: any call).
 DEFAULT = {"extent_x": 8, "extent_y": 8, "extent_z": 8, "share": 512}
 
 
@@ -55,7 +55,7 @@ def set_tuning(extent: int, shape, share: int, taps: int = 0) -> None:
 
 
 def get_tuning(extent: int):
-    """((extent_x, extent_y, extent_z), share) that calls with volume
+    """((extent_x, extent_y, extent_z), share) that large calls with volume
     extent ``extent`` and up to two taps take unless their window family has an
     entry of its own (``bricks_of``: what one call takes)."""
     from . import _native as N

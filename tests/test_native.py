@@ -270,6 +270,7 @@ def test_the_bricks_a_call_takes():
         assert tune.get_tuning(256) == ((tune.DEFAULT["extent_x"], tune.DEFAULT["extent_y"],
                                          tune.DEFAULT["extent_z"]), tune.DEFAULT["share"])
         assert tune.bricks_of(*sparse) == ((8, 8, 8), 512, True)
+        assert tune.bricks_of(32, 48, 1000) == ((16, 8, 6), 256, False)  # 0.4 million samples
         # Kaiser-Bessel: a sample at a time with few samples, claims otherwise
         # and for narrower windows, larger bricks for sparse calls into large
         # volumes. Four taps keep cells.
