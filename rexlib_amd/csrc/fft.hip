@@ -226,15 +226,12 @@ __global__ void rfft_rows_kernel(const void *in, line_set in_rows, int m, const 
 	for (int64_t first = blockIdx.x * static_cast<int64_t>(pairs); first < total;
 		first += static_cast<int64_t>(gridDim.x) * pairs)
 	{
-		for (int p = threadIdx.x; p < pairs; p += blockDim.x)
+		for (int q = threadIdx.x; q < 2 * pairs; q += blockDim.x)
 		{
-			const line_rows l = rows_of(lines, first + p);
-			for (int q = 0; q < 2; ++q)
-			{
-				row_in[2 * p + q] = l.in[q] >= 0 ? line_offset(in_rows, l.in[q]) : -1;
-				row_out[2 * p + q] = l.out[q] >= 0 ? line_offset(out_rows, l.out[q]) : -1;
-				row_scale[2 * p + q] = scales != nullptr && l.in[q] >= 0 ? scales[l.transform * scale_stride] : 1.0f;
-			}
+			const line_row r = row_of(lines, first + q / 2, q & 1);
+			row_in[q] = r.in >= 0 ? line_offset(in_rows, r.in) : -1;
+			row_out[q] = r.out >= 0 ? line_offset(out_rows, r.out) : -1;
+			row_scale[q] = scales != nullptr && r.in >= 0 ? scales[r.transform * scale_stride] : 1.0f;
 		}
 		__syncthreads();
 		for (int t = threadIdx.x; t < pairs * n; t += blockDim.x)
@@ -362,16 +359,12 @@ __global__ __launch_bounds__(256) void rfft256_rows_kernel(const void *in, line_
 	for (int64_t first = xcd_block(blockIdx.x, gridDim.x) * static_cast<int64_t>(fft256_lines); first < total;
 		first += static_cast<int64_t>(gridDim.x) * fft256_lines)
 	{
-		if (t < fft256_lines)
+		if (t < 2 * fft256_lines)
 		{
-			const line_rows r = rows_of(lines, first + t);
-#pragma unroll
-			for (int q = 0; q < 2; ++q)
-			{
-				row_in[2 * t + q] = r.in[q] >= 0 ? line_offset(in_rows, r.in[q]) : -1;
-				row_out[2 * t + q] = r.out[q] >= 0 ? line_offset(out_rows, r.out[q]) : -1;
-				row_scale[2 * t + q] = scales != nullptr && r.in[q] >= 0 ? scales[r.transform * scale_stride] : 1.0f;
-			}
+			const line_row r = row_of(lines, first + t / 2, t & 1);
+			row_in[t] = r.in >= 0 ? line_offset(in_rows, r.in) : -1;
+			row_out[t] = r.out >= 0 ? line_offset(out_rows, r.out) : -1;
+			row_scale[t] = scales != nullptr && r.in >= 0 ? scales[r.transform * scale_stride] : 1.0f;
 		}
 		__syncthreads();
 		float2 *x = exchange + l * fft256_line_stride;
@@ -498,14 +491,11 @@ __global__ void irfft_rows_kernel(const float2 *src, line_set src_rows, float *d
 	for (int64_t first = blockIdx.x * static_cast<int64_t>(pairs); first < total;
 		first += static_cast<int64_t>(gridDim.x) * pairs)
 	{
-		for (int p = threadIdx.x; p < pairs; p += blockDim.x)
+		for (int q = threadIdx.x; q < 2 * pairs; q += blockDim.x)
 		{
-			const line_rows l = rows_of(lines, first + p);
-			for (int q = 0; q < 2; ++q)
-			{
-				row_src[2 * p + q] = l.in[q] >= 0 ? line_offset(src_rows, l.in[q]) : -1;
-				row_dst[2 * p + q] = l.out[q] >= 0 ? line_offset(dst_rows, l.out[q]) : -1;
-			}
+			const line_row r = row_of(lines, first + q / 2, q & 1);
+			row_src[q] = r.in >= 0 ? line_offset(src_rows, r.in) : -1;
+			row_dst[q] = r.out >= 0 ? line_offset(dst_rows, r.out) : -1;
 		}
 		__syncthreads();
 		for (int t = threadIdx.x; t < pairs * n; t += blockDim.x)
@@ -595,15 +585,15 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void rfft_rows_two_k
 	}
 	// The two rows of the line: first input element (-1: a zero row of the
 	// padding or none), first output element, scale.
-	const line_rows rows = rows_of(lines, first + l);
 	int64_t src[2], dst[2];
 	float scale[2];
 #pragma unroll
 	for (int q = 0; q < 2; ++q)
 	{
-		src[q] = rows.in[q] >= 0 ? line_offset(in_rows, rows.in[q]) : -1;
-		dst[q] = rows.out[q] >= 0 ? line_offset(out_rows, rows.out[q]) : -1;
-		scale[q] = scales != nullptr && rows.in[q] >= 0 ? scales[rows.transform * scale_stride] : 1.0f;
+		const line_row r = row_of(lines, first + l, q);
+		src[q] = r.in >= 0 ? line_offset(in_rows, r.in) : -1;
+		dst[q] = r.out >= 0 ? line_offset(out_rows, r.out) : -1;
+		scale[q] = scales != nullptr && r.in >= 0 ? scales[r.transform * scale_stride] : 1.0f;
 	}
 	// Loads of WIDTH elements, two steps of both rows in flight.
 #pragma unroll 2
@@ -662,11 +652,12 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void irfft_rows_two_
 	{
 		return;
 	}
-	const line_rows rows = rows_of(lines, first + l);
-	const int64_t src0 = rows.in[0] >= 0 ? line_offset(src_rows, rows.in[0]) : -1;
-	const int64_t src1 = rows.in[1] >= 0 ? line_offset(src_rows, rows.in[1]) : -1;
-	const int64_t dst0 = rows.out[0] >= 0 ? line_offset(dst_rows, rows.out[0]) : -1;
-	const int64_t dst1 = rows.out[1] >= 0 ? line_offset(dst_rows, rows.out[1]) : -1;
+	const line_row row0 = row_of(lines, first + l, 0);
+	const line_row row1 = row_of(lines, first + l, 1);
+	const int64_t src0 = row0.in >= 0 ? line_offset(src_rows, row0.in) : -1;
+	const int64_t src1 = row1.in >= 0 ? line_offset(src_rows, row1.in) : -1;
+	const int64_t dst0 = row0.out >= 0 ? line_offset(dst_rows, row0.out) : -1;
+	const int64_t dst1 = row1.out >= 0 ? line_offset(dst_rows, row1.out) : -1;
 	for (int k = j; k < h; k += threads)
 	{
 		float2 va = src0 >= 0 ? src[src0 + k * src_rows.s_elem] : make_float2(0.0f, 0.0f);

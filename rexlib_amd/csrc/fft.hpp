@@ -77,41 +77,34 @@ inline row_pairs padded_rows(int64_t m, int64_t n, int64_t images, bool image_ro
 		image_rows ? 0 : offset, static_cast<int32_t>(n), image_rows ? offset : 0};
 }
 
-// The rows of line `line`: the transform, and per row of the line the input and
-// output row among all (-1: none).
-struct line_rows
+// Row `q` (0 or 1) of a line: its transform, and the input and output row among
+// all (-1: none).
+struct line_row
 {
 	int64_t transform;
-	int64_t in[2];
-	int64_t out[2];
+	int64_t in;
+	int64_t out;
 };
 
-__device__ inline line_rows rows_of(const row_pairs &p, int64_t line)
+__device__ inline line_row row_of(const row_pairs &p, int64_t line, int q)
 {
-	line_rows l{0, {-1, -1}, {-1, -1}};
 	const int pairs = (p.rows + 1) / 2;
 	const int64_t transform = line / pairs;
-	if (transform >= p.transforms)
+	if (p.rows % 2 == 0 && p.in_rows == p.rows && p.out_rows == p.rows)
 	{
-		return l;
+		// Whole pairs of whole transforms: no division (it costs a row kernel 1 to 2 %
+		// where nothing else takes the transform).
+		const int64_t all = 2 * line + q;
+		return all < p.transforms * p.rows ? line_row{transform, all, all} : line_row{0, -1, -1};
 	}
-	const int first = 2 * static_cast<int>(line - transform * pairs);
-	l.transform = transform;
-#pragma unroll
-	for (int q = 0; q < 2; ++q)
+	const int row = 2 * static_cast<int>(line - transform * pairs) + q;
+	if (transform >= p.transforms || row >= p.rows)
 	{
-		const int row = first + q;
-		if (row < p.rows)
-		{
-			const int in = row - p.in_shift;
-			if (in >= 0 && in < p.in_rows)
-			{
-				l.in[q] = transform * p.in_rows + in;
-			}
-			l.out[q] = transform * p.out_rows + row + p.out_shift;
-		}
+		return line_row{0, -1, -1};
 	}
-	return l;
+	const int in = row - p.in_shift;
+	return line_row{transform, in >= 0 && in < p.in_rows ? transform * p.in_rows + in : -1,
+		transform * p.out_rows + row + p.out_shift};
 }
 
 fft_plan make_fft_plan(int64_t n);

@@ -422,17 +422,18 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void bluestein_rfft_
 	{
 		return;
 	}
-	const line_rows rows = rows_of(lines, first + l);
-	const bool live0 = rows.in[0] >= 0;
-	const bool live1 = rows.in[1] >= 0;
-	const float *in0 = src + (live0 ? line_offset(src_rows, rows.in[0]) : 0);
-	const float *in1 = src + (live1 ? line_offset(src_rows, rows.in[1]) : 0);
+	const line_row row0 = row_of(lines, first + l, 0);
+	const line_row row1 = row_of(lines, first + l, 1);
+	const bool live0 = row0.in >= 0;
+	const bool live1 = row1.in >= 0;
+	const float *in0 = src + (live0 ? line_offset(src_rows, row0.in) : 0);
+	const float *in1 = src + (live1 ? line_offset(src_rows, row1.in) : 0);
 	bluestein_line<CLASS, false, true>(p, n, x, twl, j, chirps,
 		[&](int i) { return make_float2(live0 ? in0[i * src_rows.s_elem] : 0.0f, live1 ? in1[i * src_rows.s_elem] : 0.0f); },
 		[&](int k, float2 v) { x[k] = v; });
 	__syncthreads();
-	float2 *out0 = dst + (live0 ? line_offset(dst_rows, rows.out[0]) : 0);
-	float2 *out1 = dst + (live1 ? line_offset(dst_rows, rows.out[1]) : 0);
+	float2 *out0 = dst + (live0 ? line_offset(dst_rows, row0.out) : 0);
+	float2 *out1 = dst + (live1 ? line_offset(dst_rows, row1.out) : 0);
 	const float half = 0.5f * scale;
 	for (int k = j; k < n / 2 + 1; k += blockDim.x)
 	{
@@ -468,11 +469,12 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void bluestein_irfft
 	{
 		return;
 	}
-	const line_rows rows = rows_of(lines, first + l);
-	const bool live0 = rows.in[0] >= 0;
-	const bool live1 = rows.in[1] >= 0;
-	const float2 *in0 = src + (live0 ? line_offset(src_rows, rows.in[0]) : 0);
-	const float2 *in1 = src + (live1 ? line_offset(src_rows, rows.in[1]) : 0);
+	const line_row row0 = row_of(lines, first + l, 0);
+	const line_row row1 = row_of(lines, first + l, 1);
+	const bool live0 = row0.in >= 0;
+	const bool live1 = row1.in >= 0;
+	const float2 *in0 = src + (live0 ? line_offset(src_rows, row0.in) : 0);
+	const float2 *in1 = src + (live1 ? line_offset(src_rows, row1.in) : 0);
 	for (int k = j; k < n / 2 + 1; k += blockDim.x)
 	{
 		float2 va = live0 ? in0[k * src_rows.s_elem] : make_float2(0.0f, 0.0f);
@@ -489,8 +491,8 @@ __global__ __launch_bounds__(512, two_factor::waves<CLASS>) void bluestein_irfft
 		x[k] = make_float2(va.x - vb.y, va.y + vb.x);
 	}
 	__syncthreads();
-	float *out0 = dst + (live0 ? line_offset(dst_rows, rows.out[0]) : 0);
-	float *out1 = dst + (live1 ? line_offset(dst_rows, rows.out[1]) : 0);
+	float *out0 = dst + (live0 ? line_offset(dst_rows, row0.out) : 0);
+	float *out1 = dst + (live1 ? line_offset(dst_rows, row1.out) : 0);
 	bluestein_line<CLASS, true, false>(p, n, x, twl, j, chirps, [&](int i) { return x[i]; },
 		[&](int k, float2 v)
 		{
