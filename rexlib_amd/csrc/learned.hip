@@ -68,18 +68,22 @@ __device__ inline bool voxel_of_thread(int big, int half, int &x, int &y, int &z
 // den > 0, else 0. It starts from P = den (W = 1), and the last pass divides by
 // den; the passes between touch P alone. A block takes a tile of `width` x
 // height voxels (x, y), an even share of the row, and walks
-// compensation_planes planes along z: a plane goes to LDS with its halo of
+// `planes` planes along z: a plane goes to LDS with its halo of
 // one, is convolved there along x and y, and the three z taps come from
 // registers, so a voxel is loaded once per pass and tile (1.4 times with the
 // halo). 27 gathers of W and den per voxel took 166 us a pass at 256^3; this
 // takes 31 us (68 MB of P read and written), bound by the latency of a plane's
 // loads and barrier.
-constexpr int compensation_planes = 16;
+constexpr int compensation_planes = 16; // at most
+// Small volumes walk fewer planes per block, until this many blocks run (each
+// plane waits for its loads and a barrier): ten passes at 33^3 take 39 us so, 94
+// with 16 planes, at 64^3 42 against 95; from 180^3 on 16 fill the chip.
+constexpr int compensation_blocks = 512;
 constexpr int compensation_width = 40; // at most
 
 template <bool FIRST, bool LAST>
 __global__ __launch_bounds__(256) void compensation_pass_kernel(const float *den, const float *p_in, float *out,
-	int big, int width, int height, float floor_value)
+	int big, int width, int height, int planes, float floor_value)
 {
 	// A plane of the tile with its halo, at most two elements per thread.
 	__shared__ float product[2][512];
@@ -89,8 +93,8 @@ __global__ __launch_bounds__(256) void compensation_pass_kernel(const float *den
 	const int tx = t - ty * width;
 	const int x0 = blockIdx.x * width;
 	const int y0 = blockIdx.y * height;
-	const int z0 = blockIdx.z * compensation_planes;
-	const int z1 = min(z0 + compensation_planes, big);
+	const int z0 = blockIdx.z * planes;
+	const int z1 = min(z0 + planes, big);
 	const int x = x0 + tx;
 	const int y = y0 + ty;
 	const bool live = ty < height && x < half && y < big;
@@ -1209,14 +1213,20 @@ void launch_compensation(const float *den, float *w, float *scratch, int big, in
 	const int width = (half + columns - 1) / columns;
 	// As many rows as 256 threads and 512 halo elements take.
 	const int height = std::min(256 / width, 512 / (width + 2) - 2);
+	const int64_t plane_tiles = static_cast<int64_t>(columns) * ((big + height - 1) / height);
+	int planes = compensation_planes;
+	while (planes > 2 && plane_tiles * ((big + planes - 1) / planes) < compensation_blocks)
+	{
+		planes /= 2;
+	}
 	const dim3 tiles(static_cast<unsigned>(columns), static_cast<unsigned>((big + height - 1) / height),
-		static_cast<unsigned>((big + compensation_planes - 1) / compensation_planes));
+		static_cast<unsigned>((big + planes - 1) / planes));
 	for (int p = 0; p < passes; ++p)
 	{
 		const bool first = p == 0, last = p + 1 == passes;
 		const auto kernel = first ? (last ? compensation_pass_kernel<true, true> : compensation_pass_kernel<true, false>) :
 			(last ? compensation_pass_kernel<false, true> : compensation_pass_kernel<false, false>);
-		kernel<<<tiles, 256, 0, stream>>>(den, first ? den : a, b, big, width, height, floor_value);
+		kernel<<<tiles, 256, 0, stream>>>(den, first ? den : a, b, big, width, height, planes, floor_value);
 		float *t = a;
 		a = b;
 		b = t;
