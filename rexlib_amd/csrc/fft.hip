@@ -1,14 +1,15 @@
 // Batched FFTs on gfx950.
 //
-// Lengths of two register factors (every 2-3-5 length from 48 to 625 but 125,
-// 243 and few others, fft_two.hpp) hold a line in the registers of its
+// Lengths of two register factors (every 2-3-5 length from 48 to 1,024 but
+// 125, 243, 972 and 1,000, fft_two.hpp) hold a line in the registers of its
 // threads and exchange it once through LDS: 4.5 to 5.5 TB/s of the operand
-// read and written, from 64 to 512 points, where the LDS stages below reach 1.7
-// to 2.9. The other lengths stage a group of lines in LDS, run the
+// read and written, from 64 to 512 points, where the LDS stages below reach
+// 1.7 to 2.9. The other lengths stage a group of lines in LDS, run the
 // radix-4/2/3/5 Stockham stages there (ping-pong between two LDS buffers, one
-// butterfly per thread per step), and write the lines back. Real transforms pack two real rows
-// into one complex line and separate the two half spectra afterwards, so a
-// real row costs half a complex transform.
+// butterfly per thread per step), and write the lines back. Real transforms
+// pack two real rows of one transform (row_pairs) into one complex line and
+// separate the two half spectra afterwards, so a real row costs half a complex
+// transform.
 //
 // Conventions follow pocketfft as rexlib calls it
 // (src/backends/cpu/kernels/pocketfft_fourier_transform.cpp:74-163): the

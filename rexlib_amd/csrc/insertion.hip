@@ -386,10 +386,10 @@ void dispatch_scatter(const insertion_params &p, hipStream_t stream)
 // packed densely over the lanes (64 rows at a time, each with its base
 // position, step and first sample in its lane's registers), and their samples
 // over the lanes (64 at a time), so a lane carries a sample whatever slice it
-// comes from. The kernel is bound by its vector instructions (88 % of the
-// SIMD cycles at 4,096 slices of 256^2 into 256^3): bounding the 2.2 hits of
-// each 64 slices on their own spent half of them, and the queue took the
-// launch from 1.9 to 1.2 ms.
+// comes from. Bounding the 2.2 hits of each 64 slices on their own spent half
+// of the vector instructions, and the queue took a launch of 4,096 slices of
+// 256^2 into 256^3 from 1.9 to 1.18 ms. It is bound by LDS now: the index unit is
+// busy 84 % of the CU cycles, 48 % of that bank conflicts, the vector units 56 %.
 //
 // The samples are added by plain LDS read-modify-write, not LDS float
 // atomics (which retire at about a third of a lane per clock per CU on
@@ -397,8 +397,9 @@ void dispatch_scatter(const insertion_params &p, hipStream_t stream)
 // holding a sample claims its first-tap cell (a byte per cell: it writes its
 // lane, then reads it back); the lanes that read their own lane add their
 // taps one after another, the others keep their sample for the next round,
-// whose new samples go to the free lanes only. (With 4 taps the 64 lanes are
-// the taps of one sample instead: wide_round.) No two lanes of one tap
+// whose new samples go to the free lanes only. (Smaller Kaiser-Bessel calls make
+// the 64 lanes the taps of one sample instead: wide_round, kaiser_bessel_bricks.)
+// No two lanes of one tap
 // instruction then touch one voxel (a tap is a constant offset from the
 // cell). LDS runs a wavefront's accesses in program order and lds_order
 // keeps the compiler from moving them; the wavefront is the brick's only
@@ -555,7 +556,9 @@ struct row_range
 // 8 blocks, and everything of the slice is uniform over a block (scalar
 // registers; its row phases and radial weights in LDS). It was bound by its
 // vector instructions (99 per sample and a 64-bit division chain per line, 66
-// % of the SIMD cycles: 0.75 ms for 4,096 slices).
+// % of the SIMD cycles: 0.75 ms for 4,096 slices, 0.60 now). It and the 256-point
+// row kernel keep their place beside the two-factor kernels that take 256 too:
+// a launch of 4,096 images takes 2.29 ms through them, 2.37 through the others.
 template <int VARIANT>
 __global__ __launch_bounds__(256) void columns_prepare256_kernel(insertion_params p, slice_chunk chunk,
 	row_range held, const float2 *tw, prepared_sample *prepared)
@@ -922,13 +925,12 @@ __global__ __launch_bounds__(64, (brick_waves<PROFILE, ROUNDS, EX, EY, EZ>())) v
 		float4 row_base = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 		float4 row_step = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 		uint32_t row_index = 0;
-		// With 4 taps a sample's 64 taps are the 64 lanes: each lane takes one
+		// Wide rounds: a sample's 64 taps are the 64 lanes. Each lane takes one
 		// sample of the rows, puts its 12 axis weights in LDS, and the wavefront
 		// then adds the samples one after another, each by one read-add-write
 		// of 64 different voxels (no claims, no bank conflicts, every lane
-		// busy). 1,024 slices of 128^2 into 256^3 take 0.80 ms so, 1.35 with 64
-		// serial taps per lane, claimed as below; dense calls lose a little by
-		// it (2,048 of 256^2 into 256^3: 4.4 against 3.75 ms).
+		// busy, but each sample waits for the one before). kaiser_bessel_bricks
+		// says when, with both sides' times.
 		const int tap_x = lane & 3;
 		const int tap_y = (lane >> 2) & 3;
 		const int tap_z = lane >> 4;
@@ -936,7 +938,8 @@ __global__ __launch_bounds__(64, (brick_waves<PROFILE, ROUNDS, EX, EY, EZ>())) v
 		// fewer than 4 taps send the surplus lanes to the padding of the rows,
 		// which is never added to the accumulators (64 rows at least, one a lane):
 		// their weights are 0, but a sample that is not finite times 0 is not.
-		// (Switching the lanes off for the access takes 4.4 to 5.3 ms below.)
+		// (Switching the lanes off for the access took 2,048 slices of 256^2 into
+		// 256^3 from 4.4 to 5.3 ms.)
 		const bool within = ROUNDS != wide_narrow_rounds || max(max(tap_x, tap_y), tap_z) < p.taps;
 		const int reached = within ? 1 : 0;
 		static_assert(!WIDE || (L::pitch_y > L::lx && L::ly * L::lz >= 64), "a padding voxel per lane");

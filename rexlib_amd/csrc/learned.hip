@@ -32,24 +32,6 @@ namespace rexlib_hip
 namespace
 {
 
-// The stored index of full-spectrum frequency (x, y, z), each taken modulo
-// N, for x in [-1, N) and y, z in [-N, 2N) (the neighbours of a stored
-// voxel): frequencies with x >= N/2 + 1 are read at their Hermitian mirror
-// (-x, -y, -z).
-__device__ inline int64_t neighbour_index(int x, int y, int z, int big, int half)
-{
-	x = x < 0 ? x + big : x;
-	y = y < 0 ? y + big : (y >= big ? y - big : y);
-	z = z < 0 ? z + big : (z >= big ? z - big : z);
-	if (x >= half)
-	{
-		x = big - x;
-		y = y == 0 ? 0 : big - y;
-		z = z == 0 ? 0 : big - z;
-	}
-	return (static_cast<int64_t>(z) * big + y) * half + x;
-}
-
 // Threads over a (ceil(N half / blockDim), N) grid: (x, y) of plane z.
 __device__ inline bool voxel_of_thread(int big, int half, int &x, int &y, int &z)
 {
